@@ -1,15 +1,27 @@
-// bf16 MFMA GEMM for gfx950:  C[M,N] = epilogue(A[M,K] * W[N,K]^T)
+// bf16 MFMA GEMM for gfx950:  C[M,N] = epilogue(A[M,K] * W[N,K]^T), one output tile per workgroup
 //
-// Both operands are K-contiguous, which is the layout v_mfma_f32_32x32x16_bf16 wants for its
-// A and B fragments (8 consecutive k per lane).  One workgroup computes a BM x BN tile of C:
-//   - global -> registers -> LDS with a one-tile look-ahead, two LDS stages, one barrier per k-tile
-//   - LDS rows are 128 B (64 bf16) and 16-byte chunks are XOR-swizzled over a 256 B double row so
-//     that both the ds_write_b128 of the loader and the ds_read_b128 of the fragment reads spread
-//     over all banks
-//   - the weight fragment is the first MFMA operand, so a lane ends up with 4 consecutive n for
-//     one m and the epilogue stores 8 B (bf16) / 16 B (f32) vectors
-//   - blockIdx is remapped so that each XCD (blockIdx % 8) works on a contiguous range of tiles,
-//     n fastest, which keeps the A row panels of a range in that XCD's L2
+// For the problems that do not give the 256 x 256 persistent kernel (gemm_persistent.hip) enough tiles to fill the chip.
+// What bounds those is latency: a handful of k-tiles per workgroup, each a round trip to L2, and the first loads and the
+// epilogue on top of them.  Hence 64 x 64 tiles (four waves of 32 x 32, 48 KB of LDS: three workgroups per CU, free of each
+// other, so one's first loads and epilogue fall under another's main loop), three k-tiles in flight, every epilogue
+// operand requested ahead of the main loop, and little code (fetched cold: the kernel before this one, 128 x 128
+// register-staged with every epilogue option in one body, took 18-24 us for what takes 4-5 us here).  Measured before -> after:
+// 2048 x 128 x 128 17.9 -> 3.8 us, 2048 x 128 x 512 22.1 -> 5.3 us, 2048 x 256 x 1024 32.1 -> 8.3 us, 8192 x 256 x 256 25.0 ->
+// 7.0 us.  128 x 128 tiles of the same kernel take what neither this size nor the persistent kernel can (odd N, unaligned
+// rows, W of 2 GiB and more, SiLU).
+//   - global loads go straight into LDS (buffer_load ... lds, 16 bytes per lane); a load instruction of a wave fetches
+//     8 rows x 128 B and the lane -> chunk map is the inverse of the LDS swizzle (swz_off), so fragment reads are
+//     conflict-free ds_read_b128 and nothing is staged through registers
+//   - STAGES k-tiles of 64 in LDS, one barrier per k-tile: the loads of k-tile j + STAGES - 1 are issued right behind the
+//     barrier that ends the reading of k-tile j - 1, and waited for with a counted vmcnt
+//   - v_mfma_f32_16x16x32_bf16 with the weight fragment first and accumulators that start at the bias: the same
+//     arithmetic in the same order as the persistent kernel, bit for bit
+//   - the epilogue works on the accumulators where they are: a lane holds 4 consecutive n of one row; for bf16 C two column
+//     fragments are swapped between lane rows (v_permlane16_swap) into 8 consecutive n, 16 bytes.  No LDS staging: the
+//     64-byte row pieces cost store bandwidth, which the other workgroup's main loop hides, and a short epilogue
+//     matters more here - the kernels this file is for run a few microseconds, and code that is fetched cold counts
+//   - blockIdx is remapped so that each XCD (blockIdx % 8) works on a contiguous range of tiles, groups of GM row panels
+//     x all column tiles, which keeps the panels in use in that XCD's L2
 // Epilogue (all optional, fused): + bias[n], GELU / SiLU / SwiGLU, * gate[b, n], + residual[m, n].
 #include "common.h"
 #include "gemm_common.h"
@@ -17,239 +29,423 @@
 
 namespace aeris {
 
-template <int BM, int BN, int WM, int WN, bool SWIGLU, bool VEC>
-__global__ void __launch_bounds__(WM* WN * 64) gemm_bf16_nt_kernel(GemmParams p) {
-  constexpr int NT = WM * WN * 64;
-  constexpr int BK = 64;
-  constexpr int FM = BM / WM / 32;
-  constexpr int FN = BN / WN / 32;
-  constexpr int A_BYTES = BM * BK * 2;
-  constexpr int B_BYTES = BN * BK * 2;
-  constexpr int STAGE = A_BYTES + B_BYTES;
-  constexpr int RP = NT / 8;  // tile rows covered by one pass of the loader
-  constexpr int A_IT = BM / RP;
-  constexpr int B_IT = BN / RP;
-  static_assert(!SWIGLU || FN == 2, "SwiGLU pairs fragment 0 (gate) with fragment 1 (up)");
-  static_assert(RP % 16 == 0, "swizzle phase must repeat across loader passes");
+namespace {
+constexpr int BK = 64;
+constexpr int NT = 256;
+constexpr int GM = 8;  // row panels per L2 group
 
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+// ends a wave's use of a k-tile: its LDS reads have returned, all but its n newest loads have arrived, then the barrier
+// (one asm statement: nothing the compiler schedules may come between, and no LDS access may cross it)
+template <int N>
+__device__ __forceinline__ void wait_barrier() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+}  // namespace
 
-  // ---- tile selection with XCD-contiguous remap
-  const int np = gridDim.x;
+// VEC: C and the residual are accessed 4 / 8 columns at a time (N % 4 == 0, rows 4-element aligned); else one by one
+template <int BM, int BN, int STAGES, int ACT, bool OUT_F32, bool VEC>
+__global__ void __launch_bounds__(NT, 2) gemm_bf16_nt_tile_kernel(GemmParams p) {
+  constexpr bool SWIGLU = ACT == AERIS_ACT_SWIGLU;
+  constexpr int FM = BM / 32, FN = BN / 32;  // 16 x 16 fragments per wave (2 x 2 waves)
+  constexpr int A_BYTES = BM * BK * 2, B_BYTES = BN * BK * 2, STAGE = A_BYTES + B_BYTES;
+  constexpr int A_LD = BM / 32, B_LD = BN / 32;  // load instructions of a wave per k-tile (8 rows each)
+  constexpr int LPT = A_LD + B_LD;
+  constexpr int BN_OUT = SWIGLU ? BN / 2 : BN;
+  constexpr int NJ = SWIGLU ? FN / 2 : FN;  // column fragments of the output
+  static_assert(BM % 32 == 0 && BN % 64 == 0 && STAGES >= 2 && (STAGES - 2) * LPT < 64, "tile shape");
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+
+  // ---- tile of this workgroup: XCD-contiguous remap, then groups of GM row panels x all column tiles
   int pid = blockIdx.x;
   {
+    const int np = gridDim.x;
     const int per = (np + 7) >> 3;
     int tall = np & 7;
     if (tall == 0) tall = 8;
     const int xcd = pid & 7, loc = pid >> 3;
     pid = (xcd < tall) ? xcd * per + loc : tall * per + (xcd - tall) * (per - 1) + loc;
   }
-  const int tile_m = pid / p.tiles_n;
-  const int tile_n = pid - tile_m * p.tiles_n;
-  const int64_t m0 = (int64_t)tile_m * BM;
-  constexpr int BN_OUT = SWIGLU ? BN / 2 : BN;
-  const int n0 = tile_n * BN_OUT;
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave / WN, wn = wave % WN;
-  const int l31 = lane & 31, hi = lane >> 5;
-
-  // ---- loader mapping: thread -> (row lr + i*RP, chunk lc)
-  const int lc = tid & 7, lr = tid >> 3;
-  const int K = p.K;
-  uint32_t a_goff[A_IT], b_goff[B_IT];  // element offsets from the tile's first row
-  const uint16_t* a_base;
-  const uint16_t* b_base;
+  int tile_m, tile_n;
   {
-    const int64_t last = p.M - 1 - m0;  // >= 0
-#pragma unroll
-    for (int i = 0; i < A_IT; ++i) {
-      int64_t r = lr + i * RP;
-      if (r > last) r = last;
-      a_goff[i] = (uint32_t)(r * K + lc * 8);
-    }
-    a_base = p.A + m0 * K;
-    const int wrows = SWIGLU ? 2 * p.N : p.N;
-    int first_row;
-    if (SWIGLU) first_row = 0; else first_row = n0;
-#pragma unroll
-    for (int i = 0; i < B_IT; ++i) {
-      const int j = lr + i * RP;  // tile row
-      int r;
-      if (SWIGLU) {
-        constexpr int WNW = BN / WN;  // tile columns owned by one wave: [gate 32 | up 32]
-        const int wv = j / WNW, within = j % WNW;
-        const int oc = n0 + wv * 32 + (within & 31);
-        r = ((within >> 5) ? p.N : 0) + (oc < p.N ? oc : p.N - 1);
-      } else {
-        r = n0 + j;
-        if (r > wrows - 1) r = wrows - 1;
-        r -= first_row;
-      }
-      b_goff[i] = (uint32_t)((int64_t)r * K + lc * 8);
-    }
-    b_base = p.W + (int64_t)first_row * K;
+    const int gsz = GM * p.tiles_n;
+    const int grp = pid / gsz, within = pid - grp * gsz;
+    int gm = p.tiles_m - grp * GM;
+    if (gm > GM) gm = GM;
+    tile_n = within / gm;
+    tile_m = grp * GM + (within - tile_n * gm);
   }
-  const uint32_t w_off = swz_off(lr, lc);
-
-  // ---- fragment read offsets (per k16 step)
-  uint32_t a_roff[4], b_roff[4];
-#pragma unroll
-  for (int ks = 0; ks < 4; ++ks) {
-    a_roff[ks] = swz_off(wm * (BM / WM) + l31, ks * 2 + hi);
-    b_roff[ks] = A_BYTES + swz_off(wn * (BN / WN) + l31, ks * 2 + hi);
-  }
-
-  f32x16 acc[FM][FN];
-#pragma unroll
-  for (int i = 0; i < FM; ++i)
-#pragma unroll
-    for (int j = 0; j < FN; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-
-  u32x4 ra[A_IT], rb[B_IT];
-  auto gload = [&](int kt) {
-    const uint16_t* ab = a_base + (int64_t)kt * BK;
-    const uint16_t* bb = b_base + (int64_t)kt * BK;
-#pragma unroll
-    for (int i = 0; i < A_IT; ++i) ra[i] = *reinterpret_cast<const u32x4*>(ab + a_goff[i]);
-#pragma unroll
-    for (int i = 0; i < B_IT; ++i) rb[i] = *reinterpret_cast<const u32x4*>(bb + b_goff[i]);
-  };
-  auto lstore = [&](int stage) {
-    unsigned char* s = smem + stage * STAGE;
-#pragma unroll
-    for (int i = 0; i < A_IT; ++i) *reinterpret_cast<u32x4*>(s + w_off + i * RP * 128) = ra[i];
-#pragma unroll
-    for (int i = 0; i < B_IT; ++i) *reinterpret_cast<u32x4*>(s + A_BYTES + w_off + i * RP * 128) = rb[i];
-  };
-
+  const int64_t m0 = (int64_t)tile_m * BM;
+  const int n0 = tile_n * BN_OUT;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+  const int l15 = lane & 15, q = lane >> 4;
+  const int K = p.K, N = p.N;
   const int KT = K / BK;
-  gload(0);
-  lstore(0);
-  __syncthreads();
 
+  // ---- loads: a wave brings in BM / 4 rows of A and BN / 4 rows of W per k-tile.  Rows past the end of A or W are
+  // outside the descriptors (size in bytes: whole rows) and arrive as zeros; they feed only what is never stored.
+  constexpr int AR = BM / 4, BR = BN / 4;
+  // The row part of an offset is in the per-lane offset, which is what the range check looks at; the k part is not.
+  constexpr int LD_MAX = A_LD > B_LD ? A_LD : B_LD;
+  uint32_t ld_voff[LD_MAX];  // lane part of the source offset, per 8-row block
+  {
+    const int dr = lane >> 4, pos = lane & 15;
+#pragma unroll
+    for (int i = 0; i < LD_MAX; ++i) {
+      const int logical = pos ^ ((i & 1) * 4 + dr);
+      ld_voff[i] = (uint32_t)((i * 8 + dr * 2 + (logical >> 3)) * K * 2 + (logical & 7) * 16);
+    }
+  }
+  auto rows_rsrc = [&](const uint16_t* base, int64_t row, int64_t limit, int count) {
+    int64_t have = limit - row;
+    if (have > count) have = count;
+    if (have < 0) { have = 0; row = 0; }
+    return make_lds_dma_rsrc(base + row * K, (uint32_t)(have * K * 2));
+  };
+  const lds_dma_rsrc rs_a = rows_rsrc(p.A, m0 + wave * AR, p.M, AR);
+  // SwiGLU: a wave column's BN / 2 tile rows are the gate rows, then the up rows, of BN / 4 output columns
+  const int w_out = n0 + (SWIGLU ? (wave >> 1) : wave) * BR;
+  const int64_t w_first = (SWIGLU ? (int64_t)(wave & 1) * N : 0) + w_out;
+  const lds_dma_rsrc rs_w = rows_rsrc(p.W, w_first, w_out < N ? w_first + (N - w_out) : w_first, BR);
+  const uint32_t lds0 = lds_byte_address(smem);
+  auto issue = [&](int kt, int stage) {
+    const uint32_t sa = lds0 + stage * STAGE + wave * (AR * 128), sw = lds0 + stage * STAGE + A_BYTES + wave * (BR * 128);
+    const uint32_t k_off = (uint32_t)kt * (BK * 2);
+#pragma unroll
+    for (int i = 0; i < A_LD; ++i) lds_dma_load16(rs_a, sa + i * 1024, ld_voff[i], k_off);
+#pragma unroll
+    for (int i = 0; i < B_LD; ++i) lds_dma_load16(rs_w, sw + i * 1024, ld_voff[i], k_off);
+  };
+
+  // ---- per-column and (small tiles) per-element operands are requested ahead of the first k-tile: their latency is
+  // that of the first loads instead of a second one at the end
+  const int n_w = n0 + wn * (BN_OUT / 2);  // first output column of this wave
+  f32x4 acc[FM][FN];
+  u32x2 bq[FN];
+#pragma unroll
+  for (int j = 0; j < FN; ++j) {
+    bq[j] = u32x2{0u, 0u};
+    if (p.bias) {
+      const uint16_t* b = p.bias + (SWIGLU && j >= NJ ? N : 0);
+      const int n = n_w + (SWIGLU ? j % NJ : j) * 16 + q * 4;
+      if (VEC) {
+        bq[j] = *reinterpret_cast<const u32x2*>(b + (n < N ? n : N - 4));
+      } else {
+        uint32_t h[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) h[e] = b[n + e < N ? n + e : N - 1];
+        bq[j] = u32x2{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
+      }
+    }
+  }
+  const int m_w = wm * (BM / 2);  // first row of this wave in the tile
+  const int rows = (int)(p.M - m0 < BM ? p.M - m0 : BM);
+  const int64_t rs = c_row_stride(p);
+  // residual of fragment (i, j), f32 or bf16, at this lane's 4 columns
+  auto load_res = [&](int i, int j) -> u32x4 {
+    int r = m_w + i * 16 + l15, n = n_w + j * 16 + q * 4;
+    if (r > rows - 1) r = rows - 1;  // rows and columns outside the matrix: any valid address, the values are not stored
+    if (n > N - 4) n = N - 4;
+    const int64_t off = (m0 + r) * p.ldc + n;
+    if (p.res_dtype == AERIS_F32) return *reinterpret_cast<const u32x4*>(reinterpret_cast<const float*>(p.residual) + off);
+    const u32x2 h = *reinterpret_cast<const u32x2*>(reinterpret_cast<const uint16_t*>(p.residual) + off);
+    return u32x4{h.x << 16, h.x & 0xffff0000u, h.y << 16, h.y & 0xffff0000u};
+  };
+  u32x4 res[VEC ? FM : 1][VEC ? NJ : 1];
+  auto load_all_res = [&]() {
+    if (p.res_dtype < 0) return;
+    if (p.res_dtype == AERIS_F32) {
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) res[VEC ? i : 0][VEC ? j : 0] = load_res(i, j);
+    } else {
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) res[VEC ? i : 0][VEC ? j : 0] = load_res(i, j);
+    }
+  };
+  constexpr bool RES_EARLY = VEC && FM * NJ <= 4;
+  if (RES_EARLY) load_all_res();
+#pragma unroll
+  for (int s = 0; s < STAGES - 1; ++s)
+    if (s < KT) issue(s, s);
+#pragma unroll
+  for (int j = 0; j < FN; ++j) {
+    const f32x4 b = {bf16_lo(bq[j].x), bf16_hi(bq[j].x), bf16_lo(bq[j].y), bf16_hi(bq[j].y)};
+#pragma unroll
+    for (int i = 0; i < FM; ++i) acc[i][j] = b;
+  }
+
+  // ---- main loop
+  uint32_t a_roff[2], b_roff[2];  // fragment read offsets per k-step of 32
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks) {
+    a_roff[ks] = swz_off(m_w + l15, ks * 4 + q);
+    b_roff[ks] = A_BYTES + swz_off(wn * (BN / 2) + l15, ks * 4 + q);
+  }
+  int rd = 0, wr = STAGES - 1;
   for (int kt = 0; kt < KT; ++kt) {
-    const bool more = kt + 1 < KT;
-    if (more) gload(kt + 1);
-    const unsigned char* s = smem + (kt & 1) * STAGE;
+    // k-tile kt has arrived when at most the loads of the min(STAGES - 2, KT - 1 - kt) k-tiles behind it are outstanding
+    const int behind = KT - 1 - kt;
+    static_assert(STAGES <= 4, "one more wait per further stage");
+    if (STAGES > 2 && behind >= STAGES - 2) wait_barrier<(STAGES - 2) * LPT>();
+    else if (STAGES > 3 && behind == 1) wait_barrier<LPT>();
+    else wait_barrier<0>();
+    if (behind >= STAGES - 1) issue(kt + STAGES - 1, wr);
+    const unsigned char* st = smem + rd * STAGE;
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      bf16x8 af[FM], bfr[FN];
+    for (int ks = 0; ks < 2; ++ks) {
+      bf16x8 af[FM], bf[FN];
 #pragma unroll
-      for (int i = 0; i < FM; ++i) af[i] = *reinterpret_cast<const bf16x8*>(s + a_roff[ks] + i * 32 * 128);
+      for (int i = 0; i < FM; ++i) af[i] = *reinterpret_cast<const bf16x8*>(st + a_roff[ks] + i * 16 * 128);
 #pragma unroll
-      for (int j = 0; j < FN; ++j) bfr[j] = *reinterpret_cast<const bf16x8*>(s + b_roff[ks] + j * 32 * 128);
+      for (int j = 0; j < FN; ++j) bf[j] = *reinterpret_cast<const bf16x8*>(st + b_roff[ks] + j * 16 * 128);
 #pragma unroll
       for (int i = 0; i < FM; ++i)
 #pragma unroll
         for (int j = 0; j < FN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bfr[j], af[i], acc[i][j], 0, 0, 0);
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[j], af[i], acc[i][j], 0, 0, 0);
     }
-    if (more) lstore((kt + 1) & 1);
-    __syncthreads();
+    if (++rd == STAGES) rd = 0;
+    if (++wr == STAGES) wr = 0;
   }
 
-  // ---- epilogue: lane holds, per (i, j, g), 4 consecutive n for row m
-  const int N = p.N;
-  constexpr int FN_OUT = SWIGLU ? 1 : FN;
+  // ---- epilogue
+  if (VEC && !RES_EARLY) load_all_res();
+  if (p.q_cols > n_w) {  // query part of a qkv projection: scaled in fp32 ahead of its only rounding
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float s = n_w + j * 16 + q * 4 + e < p.q_cols ? p.q_scale : 1.0f;
+#pragma unroll
+        for (int i = 0; i < FM; ++i) acc[i][j][e] *= s;
+      }
+  }
+  // gate row of tile row r: the tile's first row is in batch entry b0, row `g_off` of it
+  const float* gate0 = p.gate;
+  int64_t g_off = 0;
+  if (p.gate && p.gate_batch_stride) {
+    const int64_t b0 = (p.row0 + m0) / p.rows_per_batch;
+    g_off = p.row0 + m0 - b0 * p.rows_per_batch;
+    gate0 += b0 * p.gate_batch_stride;
+  }
+  auto gate_row = [&](int r) -> const float* {
+    if (!p.gate_batch_stride) return gate0;
+    const int64_t in = g_off + r;
+    if (in < p.rows_per_batch) return gate0;
+    // (a tile spans further entries only when an entry has fewer rows than a tile: small numbers then)
+    return gate0 + (in < 2 * p.rows_per_batch ? 1 : (int64_t)((uint32_t)in / (uint32_t)p.rows_per_batch)) * p.gate_batch_stride;
+  };
+  auto activated = [&](int i, int j, float (&v)[4]) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float x = acc[i][j][e];
+      if (SWIGLU) x = silu_f(x) * acc[i][j + NJ][e];
+      else if (ACT == AERIS_ACT_GELU) x = gelu_erf_f(x);
+      else if (ACT == AERIS_ACT_SILU) x = silu_f(x);
+      v[e] = x;
+    }
+  };
 #pragma unroll
   for (int i = 0; i < FM; ++i) {
-    const int64_t m = m0 + wm * (BM / WM) + i * 32 + l31;
-    const bool m_ok = m < p.M;
-    const float* gate_row = nullptr;
-    if (p.gate) gate_row = p.gate + (p.gate_batch_stride ? (m / p.rows_per_batch) * p.gate_batch_stride : 0);
+    const int r = m_w + i * 16 + l15;
+    const bool row_ok = r < rows;
+    const float* gr = p.gate ? gate_row(row_ok ? r : rows - 1) : nullptr;
+    float v[NJ][4];
 #pragma unroll
-    for (int j = 0; j < FN_OUT; ++j) {
+    for (int j = 0; j < NJ; ++j) {
+      activated(i, j, v[j]);
+      const int n = n_w + j * 16 + q * 4;
+      if (VEC) {
+        if (p.gate) {
+          const f32x4 g = *reinterpret_cast<const f32x4*>(gr + (n < N ? n : N - 4));
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int n = SWIGLU ? n0 + wn * 32 + g * 8 + hi * 4 : n0 + wn * (BN / WN) + j * 32 + g * 8 + hi * 4;
-        if (m_ok && n < N) {
-        float v[4];
+          for (int e = 0; e < 4; ++e) v[j][e] *= g[e];
+        }
+        if (p.res_dtype >= 0) {
+          const u32x4 x = res[VEC ? i : 0][VEC ? j : 0];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[j][e] += __uint_as_float(x[e]);
+        }
+      } else {
+        const int64_t off = (m0 + r) * rs + c_col_off(p, n);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const int nn = (n + e < N) ? n + e : N - 1;
-          float x = acc[i][j][g * 4 + e];
-          if (SWIGLU) {
-            float u = acc[i][1][g * 4 + e];
-            if (p.bias) {
-              x += bf16_bits_to_f32(p.bias[nn]);
-              u += bf16_bits_to_f32(p.bias[N + nn]);
-            }
-            x = silu_f(x) * u;
-          } else {
-            if (p.bias) x += bf16_bits_to_f32(p.bias[nn]);
-            if (p.act == AERIS_ACT_GELU) x = gelu_erf_f(x);
-            else if (p.act == AERIS_ACT_SILU) x = silu_f(x);
-          }
-          if (gate_row) x *= gate_row[nn];
-          if (nn < p.q_cols) x *= p.q_scale;
-          v[e] = x;
-        }
-        const int64_t off = m * c_row_stride(p) + c_col_off(p, n);
-        if (VEC) {
-          if (p.res_dtype == AERIS_BF16) {
-            const u32x2 r = *reinterpret_cast<const u32x2*>(reinterpret_cast<const uint16_t*>(p.residual) + off);
-            v[0] += bf16_lo(r.x); v[1] += bf16_hi(r.x); v[2] += bf16_lo(r.y); v[3] += bf16_hi(r.y);
-          } else if (p.res_dtype == AERIS_F32) {
-            const f32x4 r = *reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(p.residual) + off);
-            v[0] += r.x; v[1] += r.y; v[2] += r.z; v[3] += r.w;
-          }
-          if (p.c_dtype == AERIS_BF16) {
-            u32x2 o;
-            o.x = pack_bf16x2(v[0], v[1]);
-            o.y = pack_bf16x2(v[2], v[3]);
-            *reinterpret_cast<u32x2*>(reinterpret_cast<uint16_t*>(p.C) + off) = o;
-          } else {
-            f32x4 o = {v[0], v[1], v[2], v[3]};
-            *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(p.C) + off) = o;
-          }
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            if (n + e < N) {
-            float x = v[e];
+          if (row_ok && n + e < N) {
+            float x = v[j][e];
+            if (p.gate) x *= gr[n + e];
             if (p.res_dtype == AERIS_BF16) x += bf16_bits_to_f32(reinterpret_cast<const uint16_t*>(p.residual)[off + e]);
             else if (p.res_dtype == AERIS_F32) x += reinterpret_cast<const float*>(p.residual)[off + e];
-            if (p.c_dtype == AERIS_BF16) reinterpret_cast<uint16_t*>(p.C)[off + e] = (uint16_t)f32_to_bf16_bits(x);
-            else reinterpret_cast<float*>(p.C)[off + e] = x;
-            }
+            if (OUT_F32) reinterpret_cast<float*>(p.C)[off + e] = x;
+            else reinterpret_cast<uint16_t*>(p.C)[off + e] = (uint16_t)f32_to_bf16_bits(x);
           }
         }
+      }
+    }
+    if (!VEC) continue;
+    if (OUT_F32) {
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        const int n = n_w + j * 16 + q * 4;
+        if (row_ok && n < N)
+          *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(p.C) + (m0 + r) * rs + c_col_off(p, n)) =
+              f32x4{v[j][0], v[j][1], v[j][2], v[j][3]};
+      }
+    } else if (NJ == 1) {
+      const int n = n_w + q * 4;
+      if (row_ok && n < N)
+        *reinterpret_cast<u32x2*>(reinterpret_cast<uint16_t*>(p.C) + (m0 + r) * rs + c_col_off(p, n)) =
+            u32x2{pack_bf16x2(v[0][0], v[0][1]), pack_bf16x2(v[0][2], v[0][3])};
+    } else {
+      // lane (l15, q) of the swapped pair of column fragments 2 m, 2 m + 1 holds the columns 32 m + 16 (q & 1) + 8 (q >> 1) ..
+#pragma unroll
+      for (int m = 0; m < NJ / 2; ++m) {
+        const auto x = __builtin_amdgcn_permlane16_swap(pack_bf16x2(v[2 * m][0], v[2 * m][1]), pack_bf16x2(v[2 * m + 1][0], v[2 * m + 1][1]), false, false);
+        const auto y = __builtin_amdgcn_permlane16_swap(pack_bf16x2(v[2 * m][2], v[2 * m][3]), pack_bf16x2(v[2 * m + 1][2], v[2 * m + 1][3]), false, false);
+        const int n = n_w + 32 * m + 16 * (q & 1) + 8 * (q >> 1);
+        if (row_ok && n < N) {
+          // N % 4 == 0: 8 columns are whole or exactly their first half is inside
+          uint16_t* c = reinterpret_cast<uint16_t*>(p.C) + (m0 + r) * rs + c_col_off(p, n);
+          if (n + 8 <= N) *reinterpret_cast<u32x4*>(c) = u32x4{x[0], y[0], x[1], y[1]};
+          else *reinterpret_cast<u32x2*>(c) = u32x2{x[0], y[0]};
         }
       }
     }
   }
 }
 
-template <int BM, int BN, int WM, int WN, bool SWIGLU, bool VEC>
-static hipError_t launch_gemm(const GemmParams& p0, hipStream_t stream) {
+namespace {
+
+template <int BM, int BN, int STAGES, int ACT, bool OUT_F32, bool VEC>
+hipError_t launch_tile(const GemmParams& p0, hipStream_t stream) {
   GemmParams p = p0;
-  constexpr int BN_OUT = SWIGLU ? BN / 2 : BN;
+  constexpr int BN_OUT = ACT == AERIS_ACT_SWIGLU ? BN / 2 : BN;
   const int64_t tiles_m = (p.M + BM - 1) / BM;
   p.tiles_n = (p.N + BN_OUT - 1) / BN_OUT;
-  const int64_t grid = tiles_m * p.tiles_n;
-  constexpr int smem = 2 * (BM + BN) * 64 * 2;
-  auto kern = gemm_bf16_nt_kernel<BM, BN, WM, WN, SWIGLU, VEC>;
-  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(WM * WN * 64), smem, stream, p);
+  p.tiles_m = (int)tiles_m;
+  constexpr int smem = STAGES * (BM + BN) * BK * 2;
+  hipLaunchKernelGGL((gemm_bf16_nt_tile_kernel<BM, BN, STAGES, ACT, OUT_F32, VEC>), dim3((unsigned)(tiles_m * p.tiles_n)), dim3(NT), smem, stream, p);
   return hipGetLastError();
 }
 
-hipError_t gemm_configure_all() {
-  // touch every instantiation so that attribute set-up never happens inside a captured region
-  hipError_t e;
-#define CFG(BM, BN, WM, WN, SG, VC)                                                                          \
-  e = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_bf16_nt_kernel<BM, BN, WM, WN, SG, VC>),          \
-                          hipFuncAttributeMaxDynamicSharedMemorySize, 2 * (BM + BN) * 64 * 2);                 \
-  if (e != hipSuccess) return e;
-  CFG(128, 128, 2, 2, false, true)
-  CFG(128, 128, 2, 2, true, true)
-  CFG(128, 128, 2, 2, false, false)
-  CFG(128, 128, 2, 2, true, false)
-#undef CFG
-  return gemm_persistent_configure();
+template <int BM, int BN, int STAGES, bool VEC>
+hipError_t launch_tile_act(const GemmParams& p, hipStream_t stream) {
+#define GO(A)                                                                              \
+  return p.c_dtype == AERIS_F32 ? launch_tile<BM, BN, STAGES, A, true, VEC>(p, stream) \
+                                : launch_tile<BM, BN, STAGES, A, false, VEC>(p, stream)
+  switch (p.act) {
+    case AERIS_ACT_GELU: GO(AERIS_ACT_GELU);
+    case AERIS_ACT_SWIGLU: GO(AERIS_ACT_SWIGLU);
+    case AERIS_ACT_SILU: GO(AERIS_ACT_SILU);
+    default: GO(AERIS_ACT_NONE);
+  }
+#undef GO
 }
+
+template <int BM, int BN, int STAGES, bool VEC, int ACT>
+hipError_t configure_tile_act() {
+  constexpr int smem = STAGES * (BM + BN) * BK * 2;
+  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_bf16_nt_tile_kernel<BM, BN, STAGES, ACT, false, VEC>),
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+  if (e != hipSuccess) return e;
+  return hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_bf16_nt_tile_kernel<BM, BN, STAGES, ACT, true, VEC>),
+                             hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+}
+template <int BM, int BN, int STAGES, bool VEC>
+hipError_t configure_tile() {
+  hipError_t e = configure_tile_act<BM, BN, STAGES, VEC, AERIS_ACT_NONE>();
+  if (e == hipSuccess) e = configure_tile_act<BM, BN, STAGES, VEC, AERIS_ACT_GELU>();
+  if (e == hipSuccess) e = configure_tile_act<BM, BN, STAGES, VEC, AERIS_ACT_SWIGLU>();
+  if (e == hipSuccess) e = configure_tile_act<BM, BN, STAGES, VEC, AERIS_ACT_SILU>();
+  return e;
+}
+}  // namespace
+
+// touch every instantiation so that attribute set-up never happens inside a captured region
+hipError_t gemm_configure_all() {
+  hipError_t e = configure_tile<64, 64, 3, true>();
+  if (e == hipSuccess) e = configure_tile<128, 128, 2, true>();
+  if (e == hipSuccess) e = configure_tile<128, 128, 2, false>();
+  if (e == hipSuccess) e = gemm_persistent_configure();
+  return e;
+}
+
+namespace {
+
+// ---- which kernel: the one whose estimated time is the smallest.
+// The estimates are fits, in microseconds, to 50 shapes measured on one GPU (M 2048 .. 1 036 800, N 128 .. 6144, K 128 ..
+// 6144, every epilogue; calls replayed from a HIP graph) of the quantities that decide: how many rounds of tiles the
+// busiest CU works through, the k-tiles of a tile, an epilogue term per tile.  They need to order the kernels, not to be
+// exact.  Measured (estimated) us, f32 C with gate and residual:
+//        M,    N,    K   256-row tiles  128-row tiles  64 x 64 tiles
+//     2048,  256, 1024      22.8 (32)      17   (21)      8.3  (9)    32 small tiles on an empty chip: the shortest k-tile
+//     8192,  256, 1024      24.6 (32)      18.4 (21)     11.5 (13)    two small workgroups per CU
+//     8192, 1024, 1024      29.8 (32)      26.0 (22)     35.6 (41)    256 tiles of 128 rows: one round
+//     8192, 1536, 1536      43.7 (42)      50.1 (53)     64.6 (79)    192 tiles of 256 rows: one round
+//    14400, 1536, 6144     259  (269)     264  (264)    497  (570)    342 tiles of 256 rows: two rounds
+enum Kind { TILE64, PERSISTENT128, PERSISTENT256 };
+
+struct Shape {
+  int64_t M;
+  int N, KT, act;
+  bool f32, res;
+};
+
+float epilogue_us(const Shape& s) {  // of a 256 x 256 tile
+  return s.f32 ? 8.0f : s.act == AERIS_ACT_GELU ? 6.5f : s.res || s.act == AERIS_ACT_SWIGLU ? 6.0f : 4.5f;
+}
+
+int64_t tiles_of(const Shape& s, int bm, int bn) {
+  const int bn_out = s.act == AERIS_ACT_SWIGLU ? bn / 2 : bn;
+  return ((s.M + bm - 1) / bm) * ((s.N + bn_out - 1) / bn_out);
+}
+
+float estimate_us(Kind kind, const Shape& s) {
+  if (kind == TILE64) {
+    // n workgroups per CU, up to three of them resident: a k-tile takes 0.31 us with one resident, 0.49 with two, 0.66 with three
+    const float n = (float)((tiles_of(s, 64, 64) + 255) / 256);
+    const float per_k = n <= 3.f ? 0.15f + 0.17f * n : 0.22f * n;
+    return 3.0f + s.KT * per_k + n * (s.f32 ? 1.0f : 0.5f);
+  }
+  const int bm = kind == PERSISTENT256 ? 256 : 128;
+  const int64_t per_xcd = (tiles_of(s, bm, 256) + 7) / 8;
+  const float rounds = (float)((per_xcd + 31) / 32);
+  return bm == 256 ? 3.0f + rounds * (1.30f * s.KT + epilogue_us(s))
+                   : 3.0f + rounds * (0.86f * s.KT + 0.5f * epilogue_us(s) + 0.5f);
+}
+
+Kind best_kind(const Shape& s, float* us) {
+  Kind best = TILE64;
+  *us = estimate_us(TILE64, s);
+  for (Kind k : {PERSISTENT128, PERSISTENT256}) {
+    const float t = estimate_us(k, s);
+    if (t < *us) { *us = t; best = k; }
+  }
+  return best;
+}
+
+hipError_t launch_kind(Kind kind, const GemmParams& p, hipStream_t stream) {
+  if (kind == TILE64) return launch_tile_act<64, 64, 3, true>(p, stream);
+  return gemm_persistent_launch(p, kind == PERSISTENT256 ? 256 : 128, stream);
+}
+
+// the same problem from row `first` on, `rows` of them
+GemmParams rows_of(const GemmParams& p0, int64_t first, int64_t rows) {
+  GemmParams p = p0;
+  p.M = rows;
+  p.row0 = p0.row0 + first;
+  p.A += first * p.K;
+  p.C = reinterpret_cast<unsigned char*>(p.C) + first * (p.split ? p.split : p.ldc) * (p.c_dtype == AERIS_F32 ? 4 : 2);
+  if (p.residual)
+    p.residual = reinterpret_cast<const unsigned char*>(p.residual) + first * p.ldc * (p.res_dtype == AERIS_F32 ? 4 : 2);
+  return p;
+}
+
+}  // namespace
 
 hipError_t gemm_launch(const void* A, const void* W, void* C, const void* bias, const float* gate,
                        const void* residual, int64_t M, int N, int K, int64_t ldc, int act, int res_dtype,
@@ -267,33 +463,47 @@ hipError_t gemm_launch(const void* A, const void* W, void* C, const void* bias, 
   p.gate = gate;
   p.residual = residual;
   p.M = M; p.N = N; p.K = K; p.ldc = ldc;
+  p.row0 = 0;
   p.gate_batch_stride = gate_batch_stride;
   p.rows_per_batch = rows_per_batch > 0 ? rows_per_batch : M;
   p.tiles_n = 0;
   p.act = act;
   p.res_dtype = residual ? res_dtype : -1;
   p.c_dtype = c_dtype;
-  const bool swiglu = act == AERIS_ACT_SWIGLU;
-  // big tiles when they are not mostly padding and there are enough of them to fill 256 CUs
-  const int bn_out = swiglu ? 128 : 256;
-  const bool big = (M >= 256) && (N % bn_out == 0 || N >= 4 * bn_out) &&
-                   ((M + 255) / 256) * ((N + bn_out - 1) / bn_out) >= 256 &&
-                   ((M + 255) / 256) * ((N + bn_out - 1) / bn_out) < (int64_t(1) << 24) &&  // the persistent kernel's tile numbering
-                   M + 512 < (int64_t(1) << 31);  // ... and its 32-bit row numbers
-  // vector epilogue (8 / 16 byte accesses to C and the residual) needs 4-element alignment of every row
-  const bool vec = (split || (ldc & 3) == 0) && ((N & 3) == 0);
-  if (!vec) return swiglu ? launch_gemm<128, 128, 2, 2, true, false>(p, stream) : launch_gemm<128, 128, 2, 2, false, false>(p, stream);
-  // (gate rows must allow 16-byte loads: the stride between batch rows is a multiple of 4 floats)
-  const bool aligned = (reinterpret_cast<uintptr_t>(gate) & 15) == 0 && (reinterpret_cast<uintptr_t>(bias) & 7) == 0;
-  // the persistent kernel addresses W through one buffer descriptor (31-bit size) and loads 16 bytes per lane into LDS
-  // ... and forms row offsets with 24-bit multiplies, gate row offsets and batch numbers in 32 bits
-  const bool dma_ok = (int64_t)(swiglu ? 2 : 1) * N * K * 2 < (int64_t(1) << 31) && (K % 64) == 0 && ldc < (1 << 23) && split < (1 << 23) &&
-                      gate_batch_stride < (int64_t(1) << 31) && (rows_per_batch <= 0 || M / rows_per_batch < (int64_t(1) << 31)) &&
-                      ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(W)) & 15) == 0;
-  // (the persistent kernel scales whole 64-column wave blocks of the query part)
-  if (big && dma_ok && act != AERIS_ACT_SILU && (gate_batch_stride & 3) == 0 && aligned && q_cols % 64 == 0)
-    return gemm_persistent_launch(p, stream);
-  return swiglu ? launch_gemm<128, 128, 2, 2, true, true>(p, stream) : launch_gemm<128, 128, 2, 2, false, true>(p, stream);
+  // vector epilogue: 8 / 16-byte accesses to C and the residual (4-element alignment of every row), to bias and gate rows
+  const bool vec = (split || (ldc & 3) == 0) && (N & 3) == 0 && (reinterpret_cast<uintptr_t>(gate) & 15) == 0 &&
+                   (gate_batch_stride & 3) == 0 && (reinterpret_cast<uintptr_t>(bias) & 7) == 0;
+  if (!vec) return launch_tile_act<128, 128, 2, false>(p, stream);
+  // what the persistent kernel cannot take: it addresses W through one buffer descriptor (31-bit size), forms row offsets
+  // with 24-bit multiplies, row numbers, gate row offsets and batch numbers in 32 bits, numbers its tiles in 24 bits and
+  // scales whole 64-column wave blocks of the query part
+  const Shape s = {M, N, K / BK, act, c_dtype == AERIS_F32, residual != nullptr};
+  const bool persistent_ok = act != AERIS_ACT_SILU && (int64_t)(act == AERIS_ACT_SWIGLU ? 2 : 1) * N * K * 2 < (int64_t(1) << 31) &&
+                             ldc < (1 << 23) && split < (1 << 23) && gate_batch_stride < (int64_t(1) << 31) &&
+                             (rows_per_batch <= 0 || M / rows_per_batch < (int64_t(1) << 31)) && M + 512 < (int64_t(1) << 31) &&
+                             tiles_of(s, 128, 256) < (int64_t(1) << 24) && q_cols % 64 == 0 && N >= 64;
+  if (!persistent_ok)
+    return tiles_of(s, 128, 128) < 128 ? launch_tile_act<64, 64, 3, true>(p, stream) : launch_tile_act<128, 128, 2, true>(p, stream);
+  float one = 0.f;
+  const Kind kind = best_kind(s, &one);
+  // Whole rounds of 256-row tiles first, the rows of the last, partly filled round by smaller tiles in a launch of its own:
+  // the rows are split, nothing else.  (14400 x 4608 x 1536: 1026 tiles, two more than four rounds of 256: 177 -> 162 us;
+  // 14400 x 1536 x 6144: 342 tiles: 268 -> 256 us.)
+  const int bn_out = act == AERIS_ACT_SWIGLU ? 128 : 256;
+  const int64_t tiles_n = (N + bn_out - 1) / bn_out, tiles = tiles_of(s, 256, 256);
+  const int64_t panels = (tiles - 1) / 256 * 256 / tiles_n;  // row panels of the rounds before the last
+  if (panels > 0 && panels * 256 < M) {
+    Shape head = s, rest = s;
+    head.M = panels * 256;
+    rest.M = M - head.M;
+    float t_rest = 0.f;
+    const Kind rest_kind = best_kind(rest, &t_rest);
+    if (estimate_us(PERSISTENT256, head) + t_rest < 0.97f * one) {
+      const hipError_t e = launch_kind(PERSISTENT256, rows_of(p, 0, head.M), stream);
+      return e != hipSuccess ? e : launch_kind(rest_kind, rows_of(p, head.M, rest.M), stream);
+    }
+  }
+  return launch_kind(kind, p, stream);
 }
 
 }  // namespace aeris

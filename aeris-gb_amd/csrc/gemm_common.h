@@ -21,6 +21,7 @@ struct GemmParams {
   int64_t plane_stride;
   int64_t gate_batch_stride;
   int64_t rows_per_batch;
+  int64_t row0;  // number of the first row within the whole problem (gate rows are looked up by it)
   int tiles_n;
   // persistent kernel only: tile schedule
   int tiles_m;
@@ -57,8 +58,8 @@ __device__ __forceinline__ uint32_t swz_off(int row, int chunk) {
   return (uint32_t)((row >> 1) * 256 + (((((row & 1) << 3) | chunk) ^ ((row >> 1) & 7)) << 4));
 }
 
-// 256x256 persistent kernel (gemm_persistent.hip); needs N % 4 == 0 and ldc % 4 == 0
+// persistent kernel (gemm_persistent.hip), tiles of tile_height (128 or 256) rows x 256 columns; needs N % 4 == 0 and ldc % 4 == 0
 hipError_t gemm_persistent_configure();
-hipError_t gemm_persistent_launch(const GemmParams& p, hipStream_t stream);
+hipError_t gemm_persistent_launch(const GemmParams& p, int tile_height, hipStream_t stream);
 
 }  // namespace aeris

@@ -1,4 +1,4 @@
-// Persistent bf16 MFMA GEMM for gfx950, 256x256 output tiles, k-tiles of 64:  C[M,N] = epilogue(A[M,K] * W[N,K]^T)
+// Persistent bf16 MFMA GEMM for gfx950, 256x256 (or 128x256) output tiles, k-tiles of 64:  C[M,N] = epilogue(A[M,K] * W[N,K]^T)
 //
 // Same LDS swizzle as the plain tile kernel (gemm.hip), built around what bounds it on MI355X:
 //   - v_mfma_f32_16x16x32_bf16, not 32x32x16: same FLOP per cycle and the same LDS bytes per FLOP (a fragment is
@@ -14,6 +14,8 @@
 //   - the two waves of a SIMD alternate memory slots (LDS fragment reads + load issue) and compute slots (32 MFMAs):
 //     a load instruction holds the issuing wave until the address unit has taken its 64 addresses, which would stall
 //     the MFMA stream if the computing wave issued it
+//   - tiles of 128 rows (same main loop, 16 MFMAs per slot instead of 32) where they fill the chip and 256-row tiles do not:
+//     8192 x 1024 x 1024 with f32 residual 29.8 -> 26 us, 12480 x 384 x 1088 27.8 -> 22 us; per FLOP they are 30 % slower
 //   - tiles are ordered so that the workgroups resident on one XCD (blockIdx % 8) cover a contiguous chunk, 4 row
 //     panels x all column tiles at a time: few distinct A / W k-slices per step compete for that XCD's 4 MB L2
 //   - the epilogue stages through the idle A stage (wave-private 4 KB): fragments (4 consecutive n per lane) are
@@ -27,16 +29,17 @@
 namespace aeris {
 
 namespace {
-constexpr int BM = 256, BN = 256, BK = 64, WM = 2, WN = 4;
+constexpr int BN = 256, BK = 64, WM = 2, WN = 4;
 constexpr int NT = WM * WN * 64;          // 512 threads
-constexpr int FM = BM / WM / 16;          // 8 fragments of 16 rows
 constexpr int FN = BN / WN / 16;          // 4 fragments of 16 columns
-constexpr int A_BYTES = BM * BK * 2;      // 32 KB per stage of the A tile
 constexpr int B_BYTES = BN * BK * 2;      // 32 KB per stage of the W tile
 constexpr int A_STAGES = 2, B_STAGES = 3;
-constexpr int B_OFF = A_STAGES * A_BYTES;
-constexpr int SMEM = A_STAGES * A_BYTES + B_STAGES * B_BYTES;  // 160 KB: all of the CU's LDS
 constexpr int GM = 4;                     // row panels per L2 group
+constexpr int STG_BYTES = 4096;           // staging area of a wave in the epilogue
+// tile height 256: two A stages of 32 KB, the idle one doubles as the staging area (a wave's part of it is 4 KB); height
+// 128: two of 16 KB and a staging area of its own.  160 KB of LDS either way: all of the CU's.
+constexpr int smem_bytes(int bm) { return A_STAGES * bm * BK * 2 + B_STAGES * B_BYTES + (bm == 256 ? 0 : WM * WN * STG_BYTES); }
+static_assert(smem_bytes(256) == 160 * 1024 && smem_bytes(128) == 160 * 1024, "LDS of a CU");
 }  // namespace
 
 // PLAIN: no gate and no residual (qkv, fc1): the epilogue is compiled without those paths - about 2 % faster than
@@ -44,8 +47,12 @@ constexpr int GM = 4;                     // row panels per L2 group
 // fc2 on a bf16 residual stream), compiled as a kernel of its own so that its deeper residual prefetch does not
 // share registers with the general path.  RES_F32: the same for f32 C with an f32 residual (proj, fc2 on an f32
 // residual stream).
-template <int ACT, bool OUT_F32, bool PLAIN, bool RES_BF16 = false, bool RES_F32 = false>
+template <int BM, int ACT, bool OUT_F32, bool PLAIN, bool RES_BF16 = false, bool RES_F32 = false>
 __global__ void __launch_bounds__(NT) gemm_bf16_nt_persistent_kernel(GemmParams p_in) {
+  constexpr int FM = BM / WM / 16;          // 8 (4) fragments of 16 rows
+  constexpr int A_BYTES = BM * BK * 2;      // 32 (16) KB per stage of the A tile
+  constexpr int A_LD = BM / 64;             // load instructions of a wave per k-tile of A (8 rows each); 4 for W
+  constexpr int B_OFF = A_STAGES * A_BYTES;
   static_assert(!(PLAIN && RES_BF16) && !(OUT_F32 && RES_BF16), "RES_BF16 is a non-plain bf16-output form");
   static_assert(!RES_F32 || (OUT_F32 && !PLAIN && !RES_BF16), "RES_F32 is a non-plain f32-output form");
   GemmParams p = p_in;
@@ -125,10 +132,10 @@ __global__ void __launch_bounds__(NT) gemm_bf16_nt_persistent_kernel(GemmParams 
   // records): the number of loads in flight at any point of the k-loop is then the same for every k-tile, and no wait
   // has to be chosen at run time.
   auto issue_a = [&]() {
-    unsigned char* sd = smem + la_stage * A_BYTES + wave_u * 4096;
-    const uint32_t so = (uint32_t)(wave_u * 32) * (uint32_t)(K * 2) + (uint32_t)la_kt * (BK * 2);
+    unsigned char* sd = smem + la_stage * A_BYTES + wave_u * (A_LD * 1024);
+    const uint32_t so = (uint32_t)(wave_u * (A_LD * 8)) * (uint32_t)(K * 2) + (uint32_t)la_kt * (BK * 2);
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < A_LD; ++i)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_a, (lds_ptr)(sd + i * 1024), 16, ld_voff[i & 1],
                                                so + (uint32_t)(i * 8) * (uint32_t)(K * 2), 0, 0);
     la_stage ^= 1;
@@ -215,7 +222,7 @@ __global__ void __launch_bounds__(NT) gemm_bf16_nt_persistent_kernel(GemmParams 
   }
 
   // s_waitcnt immediates: vmcnt in bits 3:0 (and 15:14), expcnt in 6:4 (7 = no wait), lgkmcnt in 11:8 (15 = no wait)
-  constexpr int WAIT_LGKM0 = 0xC07F, WAIT_VM0 = 0x0F70, WAIT_VM4 = 0x0F74, WAIT_VM8_LGKM0 = 0x0078;
+  constexpr int WAIT_LGKM0 = 0xC07F, WAIT_VM0 = 0x0F70, WAIT_VM4 = 0x0F74, WAIT_AW_LGKM0 = 0x0070 | (A_LD + 4);
 
   // ---- epilogue of the tile whose accumulators are complete.
   // Vector memory operations of a wave complete in order, so a wait for a load also waits for every store issued
@@ -240,7 +247,6 @@ __global__ void __launch_bounds__(NT) gemm_bf16_nt_persistent_kernel(GemmParams 
     const int64_t rows_left64 = p.M - m_base;
     const int rows_left = rows_left64 < BM / WM ? (int)rows_left64 : BM / WM;
     const int ld24 = (int)p.ldc, rs24 = (int)c_row_stride(p);
-    const int rrow_t = rrow;
     const int n_wave = tile_n * BN_OUT + (wave_u % WN) * (SWIGLU ? 32 : BN / WN);  // first output column of this wave
     u32x2 bq_next[FN];  // loaded ahead of the last block's stores, used after them
     // The query part of a qkv projection is multiplied by q_scale here, in fp32, before its only rounding.  Whole
@@ -254,8 +260,9 @@ __global__ void __launch_bounds__(NT) gemm_bf16_nt_persistent_kernel(GemmParams 
         for (int j = 0; j < FN; ++j) acc[i][j] *= qs;
     }
     // Staging area of this wave, 32 rows of 128 B: the A stage that the loader fills next is idle during the
-    // epilogue, and the 4 KB of it that this wave's own loads will fill are written by nobody else.
-    unsigned char* stg = smem + la_stage * A_BYTES + wave_u * 4096;
+    // epilogue, and the 4 KB of it that this wave's own loads will fill are written by nobody else (tile height 128: an
+    // area of its own).
+    unsigned char* stg = smem + (BM == 256 ? la_stage * A_BYTES : B_OFF + B_STAGES * B_BYTES) + wave_u * STG_BYTES;
 
     // gate: one row of p.gate per batch.  A tile whose rows are all in one batch (the usual case) loads its gate
     // columns once; otherwise every lane looks up the row of its own fragment row.
@@ -270,16 +277,19 @@ __global__ void __launch_bounds__(NT) gemm_bf16_nt_persistent_kernel(GemmParams 
       if (p.gate_batch_stride == 0) {
         gate_tile = p.gate;
       } else {
-        int64_t last = m_base + BM / WM - 1;
+        // (a group entirely below the matrix looks up the last row's entry: there is no gate row for its own)
+        int64_t first = m_base, last = m_base + BM / WM - 1;
+        if (first > p.M - 1) first = p.M - 1;
         if (last > p.M - 1) last = p.M - 1;
-        const int64_t b0 = (int64_t)(((uint64_t)(uint32_t)m_base * p.rpb_magic) >> p.rpb_shift);
-        const int64_t b1 = (int64_t)(((uint64_t)(uint32_t)last * p.rpb_magic) >> p.rpb_shift);
+        const uint32_t row0 = (uint32_t)p.row0;
+        const int64_t b0 = (int64_t)(((uint64_t)((uint32_t)first + row0) * p.rpb_magic) >> p.rpb_shift);
+        const int64_t b1 = (int64_t)(((uint64_t)((uint32_t)last + row0) * p.rpb_magic) >> p.rpb_shift);
         if (b0 == b1) {
           gate_tile = p.gate + b0 * p.gate_batch_stride;
         } else {
           gate_per_lane = true;
           gate_b0 = (int)b0;
-          gate_r1 = (int)((b0 + 1) * p.rows_per_batch - m_base);
+          gate_r1 = (int)((b0 + 1) * p.rows_per_batch - m_base - p.row0);
           if (p.rows_per_batch < BM / WM) gate_magic = (65536u + (uint32_t)p.rows_per_batch - 1u) / (uint32_t)p.rows_per_batch;
         }
       }
@@ -331,19 +341,15 @@ __global__ void __launch_bounds__(NT) gemm_bf16_nt_persistent_kernel(GemmParams 
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     };
 
-    // Interior tiles of the two forms that gain from it (bf16 residual with an optional per-tile gate: +5 % on
-    // K = 1536; plain GELU: +1 %; plain without activation measured 2 % slower this way and stays on the general
-    // path) take a path without any per-lane condition: every row and column of the group's 128 x 64 block is
-    // inside the matrix.  Straight-line code lets the compiler wait for exactly the loads a block needs (with the
-    // branches of the general path it waited for the next block's residual rows right after the stores), and the
-    // residual rows are requested two blocks ahead: block 0 at the start, block 1 once block 0's accumulators
-    // are staged and their registers free, blocks 2 and 3 after blocks 0 and 1 have been combined.
-    const bool interior = (RES_BF16 || (PLAIN && ACT == AERIS_ACT_GELU)) && !OUT_F32 && !SWIGLU &&
-                          rows_left == BM / WM && n_wave + BN / WN <= N && !gate_per_lane;
+    // Interior tiles (every row and column of the group's 128 x 64 block inside the matrix, one gate row) take paths
+    // without any per-lane condition where that gains (residual forms: +5 % on K = 1536; plain GELU: +1 %; plain without
+    // activation measured 2 % slower this way and stays on the general path): straight-line code lets the compiler wait
+    // for exactly the loads a block needs.
+    const bool inside = rows_left == BM / WM && n_wave + BN_OUT / WN <= N && !gate_per_lane;
+    const bool interior = PLAIN && ACT == AERIS_ACT_GELU && !OUT_F32 && inside;
     // Interior plain SwiGLU tiles skip the staging (in the read-back of the general path half of the lanes idle on
-    // its 64-byte rows; +2 %).  For the other forms this was slower (qkv -4 %, proj -5 %: 64-byte row pieces), although
-    // gate and residual are then applied in fp32 before the only rounding.
-    const bool interior_direct = SWIGLU && PLAIN && !OUT_F32 && rows_left == BM / WM && n_wave + 32 <= N;
+    // its 64-byte rows; +2 %).  For the other forms this was slower (qkv -4 %, proj -5 %: 64-byte row pieces).
+    const bool interior_direct = SWIGLU && PLAIN && !OUT_F32 && inside;
     // Every path ends in a wait of its own.  Nothing that writes a register may be pending when the k-loop is entered:
     // the compiler would guard the fragment registers with a wait for all vector memory operations inside the loop,
     // on every k-tile, which cuts the lead of the W loads to one slot.  The first k-tile needs the oldest loads at once
@@ -380,141 +386,150 @@ __global__ void __launch_bounds__(NT) gemm_bf16_nt_persistent_kernel(GemmParams 
       const int n = n_wave + rch * 8;
       unsigned char* const c_lane =
           reinterpret_cast<unsigned char*>(p.C) + (m_base * c_row_stride(p) + c_col_off(p, n)) * 2;
-      f32x4 gt0 = {1.f, 1.f, 1.f, 1.f}, gt1 = {1.f, 1.f, 1.f, 1.f};
-      if (gate_tile) {
-        gt0 = *reinterpret_cast<const f32x4*>(gate_tile + n);
-        gt1 = *reinterpret_cast<const f32x4*>(gate_tile + n + 4);
-      }
-      const unsigned char* const res_lane =
-          reinterpret_cast<const unsigned char*>(p.residual) + (m_base * p.ldc + n) * 2;
-      u32x4 rq[FM / 2][4];
-      auto load_res = [&](int b) {
-#pragma unroll
-        for (int it = 0; it < 4; ++it)
-          rq[b][it] = *reinterpret_cast<const u32x4*>(res_lane + (int64_t)__mul24(b * 32 + rrow + 8 * it, ld24) * 2);
-      };
-      if (RES_BF16) load_res(0);
 #pragma unroll
       for (int i = 0; i < FM / 2; ++i) {
         stage_block_bf16(i);
-        if (RES_BF16 && i == 0) load_res(1);
         u32x4 out[4];
 #pragma unroll
-        for (int it = 0; it < 4; ++it) {
-          u32x4 w4 = *reinterpret_cast<const u32x4*>(stg + swz_off(rrow + 8 * it, rch));
-          if (RES_BF16) {
-            float o[8];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) { o[2 * e] = bf16_lo(w4[e]); o[2 * e + 1] = bf16_hi(w4[e]); }
-#pragma unroll
-            for (int e = 0; e < 4; ++e) { o[e] *= gt0[e]; o[4 + e] *= gt1[e]; }
-            const u32x4 r4 = rq[i][it];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) { o[2 * e] += bf16_lo(r4[e]); o[2 * e + 1] += bf16_hi(r4[e]); }
-            w4 = u32x4{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]), pack_bf16x2(o[4], o[5]), pack_bf16x2(o[6], o[7])};
-          }
-          out[it] = w4;
-        }
+        for (int it = 0; it < 4; ++it) out[it] = *reinterpret_cast<const u32x4*>(stg + swz_off(rrow + 8 * it, rch));
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
-        // the next loads go ahead of the stores below
-        if (RES_BF16 && i + 2 < FM / 2) load_res(i + 2);
-        if (i + 1 == FM / 2 && r_done + 1 < n_my) load_bias(r_done + 1, bq_next, q);
+        if (i + 1 == FM / 2 && r_done + 1 < n_my) load_bias(r_done + 1, bq_next, q);  // ahead of the stores below
 #pragma unroll
         for (int it = 0; it < 4; ++it)
           *reinterpret_cast<u32x4*>(c_lane + (int64_t)__mul24(i * 32 + rrow + 8 * it, rs24) * 2) = out[it];
       }
       __builtin_amdgcn_s_waitcnt(WAIT_VM4);  // the 4 stores of the last block may still be on their way
+    } else if (!OUT_F32 && !PLAIN) {
+      // bf16 C with gate and / or residual.  (Staged as bf16, with gate and residual applied after that rounding, the same
+      // time: 64800 x 512 x 512 49.8 us, x 2048 125 -> 123 us, at an error of 2.2e-3 of the result instead of 1.7e-3.)  Staged as fp32 (16 rows x 64 columns of 256 B, 16-byte chunks XOR-swizzled
+      // by the row), so that gate and residual are applied before the only rounding, and read back as 8 consecutive
+      // columns per lane: C and a bf16 residual are accessed as full 128-byte row segments.  The residual of row
+      // fragment i + AHEAD is requested ahead of the stores of fragment i.
+      constexpr int CH = NJ * 4, AHEAD = RES_BF16 ? 3 : 1;
+      const auto run = [&](auto inside_tag) {
+        constexpr bool INSIDE = decltype(inside_tag)::value;
+        const int n = n_wave + rch * 8;
+        const bool col_ok = INSIDE || (rch < CH / 2 && n < N);
+        const bool full = INSIDE || n + 8 <= N;  // N % 4 == 0: 8 columns are whole or exactly their first half is inside
+        const int n_ld = INSIDE || n < N - 8 ? n : N - 8;  // 8 columns that exist; half a chunk: its 4 are the upper ones
+        const int n_g0 = INSIDE || n < N - 4 ? n : N - 4, n_g1 = INSIDE || n + 4 < N - 4 ? n + 4 : N - 4;
+        unsigned char* const c_lane = reinterpret_cast<unsigned char*>(p.C) +
+                                      (m_base * c_row_stride(p) + c_col_off(p, col_ok ? n : 0)) * 2;
+        f32x4 g0 = {1.f, 1.f, 1.f, 1.f}, g1 = g0;
+        if (gate_tile) {
+          g0 = *reinterpret_cast<const f32x4*>(gate_tile + n_g0);
+          g1 = *reinterpret_cast<const f32x4*>(gate_tile + n_g1);
+        }
+        const int res_dtype = RES_BF16 ? (int)AERIS_BF16 : p.res_dtype;
+        u32x4 rq[AHEAD + 1][2][RES_BF16 ? 1 : 2];
+        auto load_res = [&](int i) {
+#pragma unroll
+          for (int it = 0; it < 2; ++it) {
+            int r = i * 16 + rrow + 8 * it;
+            if (!INSIDE && r > rows_left - 1) r = rows_left - 1;  // rows below the matrix read its last row (may be negative: M >= 1)
+            const int64_t off = m_base * p.ldc + (int64_t)__mul24(r, ld24);
+            u32x4(&d)[RES_BF16 ? 1 : 2] = rq[i % (AHEAD + 1)][it];
+            if (res_dtype == AERIS_BF16) {
+              d[0] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint16_t*>(p.residual) + off + n_ld);
+            } else {
+              d[0] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const float*>(p.residual) + off + n_g0);
+              d[RES_BF16 ? 0 : 1] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const float*>(p.residual) + off + n_g1);
+            }
+          }
+        };
+        // (the first fragments' accumulators are staged and their registers free before the next ones are requested)
+        if (res_dtype >= 0) load_res(0);
+#pragma unroll
+        for (int i = 0; i < FM; ++i) {
+#pragma unroll
+          for (int j = 0; j < NJ; ++j) {
+            float v[4];
+            fragment(i, j, v);
+            *reinterpret_cast<f32x4*>(stg + l15 * 256 + (((j * 4 + q) ^ (l15 & (CH - 1))) << 4)) = f32x4{v[0], v[1], v[2], v[3]};
+          }
+          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+          __builtin_amdgcn_wave_barrier();
+          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+          if (res_dtype >= 0 && i == 0) {
+#pragma unroll
+            for (int a = 1; a < AHEAD; ++a)
+              if (a < FM) load_res(a);
+          }
+          u32x4 out[2];
+#pragma unroll
+          for (int it = 0; it < 2; ++it) {
+            const int row = rrow + 8 * it, key = row & (CH - 1);
+            const int c0 = (2 * rch) & (CH - 1);
+            f32x4 o0 = *reinterpret_cast<const f32x4*>(stg + row * 256 + ((c0 ^ key) << 4));
+            f32x4 o1 = *reinterpret_cast<const f32x4*>(stg + row * 256 + (((c0 + 1) ^ key) << 4));
+            if (!INSIDE && gate_per_lane) {
+              const float* gr = gate_row_of(i * 16 + row);
+              g0 = *reinterpret_cast<const f32x4*>(gr + n_g0);
+              g1 = *reinterpret_cast<const f32x4*>(gr + n_g1);
+            }
+            o0 *= g0;
+            o1 *= g1;
+            if (res_dtype == AERIS_BF16) {
+              u32x4 r4 = rq[i % (AHEAD + 1)][it][0];
+              if (!full) { r4.x = r4.z; r4.y = r4.w; }
+              o0 += f32x4{bf16_lo(r4.x), bf16_hi(r4.x), bf16_lo(r4.y), bf16_hi(r4.y)};
+              o1 += f32x4{bf16_lo(r4.z), bf16_hi(r4.z), bf16_lo(r4.w), bf16_hi(r4.w)};
+            } else if (res_dtype == AERIS_F32) {
+              const u32x4 a = rq[i % (AHEAD + 1)][it][0], b = rq[i % (AHEAD + 1)][it][RES_BF16 ? 0 : 1];
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                o0[e] += __uint_as_float(a[e]);
+                o1[e] += __uint_as_float(b[e]);
+              }
+            }
+            out[it] = u32x4{pack_bf16x2(o0[0], o0[1]), pack_bf16x2(o0[2], o0[3]), pack_bf16x2(o1[0], o1[1]), pack_bf16x2(o1[2], o1[3])};
+          }
+          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+          __builtin_amdgcn_wave_barrier();
+          // the next loads go ahead of the stores below
+          if (res_dtype >= 0 && i + AHEAD < FM) load_res(i + AHEAD);
+          if (i + 2 == FM && r_done + 1 < n_my) load_bias(r_done + 1, bq_next, q);
+#pragma unroll
+          for (int it = 0; it < 2; ++it) {
+            const int r = i * 16 + rrow + 8 * it;
+            if (INSIDE || (col_ok && r < rows_left)) {
+              unsigned char* cp = c_lane + (int64_t)__mul24(r, rs24) * 2;
+              if (full) *reinterpret_cast<u32x4*>(cp) = out[it];
+              else *reinterpret_cast<u32x2*>(cp) = u32x2{out[it].x, out[it].y};
+            }
+          }
+        }
+      };
+      if (RES_BF16 && !SWIGLU && inside) {
+        run(std::true_type{});
+        __builtin_amdgcn_s_waitcnt(WAIT_VM4);  // the 4 stores of the last two fragments may still be on their way
+      } else {
+        run(std::false_type{});
+        __builtin_amdgcn_s_waitcnt(WAIT_VM0);
+      }
     } else if (!OUT_F32) {
-      // stage 2 (bf16 C): a whole 32 x 64 (SwiGLU: 32 x 32) block through LDS, rows of 128 B, chunk-swizzled; it
-      // is read back as 16-byte chunks, 8 lanes per row, and C / residual are accessed as full row segments
+      // bf16 C without gate and residual: a whole 32 x 64 (SwiGLU: 32 x 32) block through LDS, rows of 128 B,
+      // chunk-swizzled; it is read back as 16-byte chunks, 8 lanes per row, and C is written as full row segments
       constexpr int CHUNKS = SWIGLU ? 4 : 8;  // 16-byte chunks (8 columns) per staged row
       const int n = n_wave + rch * 8;
       const bool col_ok = rch < CHUNKS && n < N;
       const bool full = n + 8 <= N;  // N % 4 == 0: a chunk is whole or exactly its first half is inside
-      // residual: 16 bytes (bf16) or 2 x 16 bytes (f32) per lane and row, from an address that is always valid:
-      // rows are clamped to M - 1, a half chunk reads the 4 columns before it as well (bf16) or its first half
-      // twice (f32)
-      int n_ld = n;
-      if (!col_ok) n_ld = n_wave;
-      else if (!full && (RES_BF16 || p.res_dtype == AERIS_BF16)) n_ld = n - 4;
-      const bool upper = col_ok && !full;  // bf16: the wanted 4 columns are the upper half of what was loaded
-      const int n_g = col_ok ? n : n_wave;
-      // where this lane's chunk of row 0 goes in C / comes from in the residual
+      // where this lane's chunk of row 0 goes in C
       unsigned char* const c_lane =
-          reinterpret_cast<unsigned char*>(p.C) + (m_base * c_row_stride(p) + c_col_off(p, col_ok ? n : n_wave)) * 2;
-      f32x4 gt0 = {1.f, 1.f, 1.f, 1.f}, gt1 = {1.f, 1.f, 1.f, 1.f};
-      if (gate_tile) {
-        gt0 = *reinterpret_cast<const f32x4*>(gate_tile + n_g);
-        gt1 = *reinterpret_cast<const f32x4*>(gate_tile + n_g + (full ? 4 : 0));
-      }
-      const unsigned char* const res_lane = reinterpret_cast<const unsigned char*>(p.residual) +
-                                            (m_base * p.ldc + n_ld) * ((RES_BF16 || p.res_dtype == AERIS_BF16) ? 2 : 4);
-      const int res_dtype = RES_BF16 ? (int)AERIS_BF16 : p.res_dtype;
-      u32x4 rq[4][2];
-      auto load_res = [&](int i) {
-#pragma unroll
-        for (int it = 0; it < 4; ++it) {
-          int r = i * 32 + rrow_t + 8 * it;
-          if (r > rows_left - 1) r = rows_left - 1;  // rows below the matrix read its last row (may be negative: M >= 1)
-          const int64_t off = (int64_t)__mul24(r, ld24);
-          if (res_dtype == AERIS_BF16) {
-            rq[it][0] = *reinterpret_cast<const u32x4*>(res_lane + off * 2);
-          } else {
-            const float* rp = reinterpret_cast<const float*>(res_lane + off * 4);
-            rq[it][0] = *reinterpret_cast<const u32x4*>(rp);
-            rq[it][1] = *reinterpret_cast<const u32x4*>(rp + (full ? 4 : 0));
-          }
-        }
-      };
-      if (res_dtype >= 0) load_res(0);
+          reinterpret_cast<unsigned char*>(p.C) + (m_base * c_row_stride(p) + c_col_off(p, col_ok ? n : 0)) * 2;
 #pragma unroll
       for (int i = 0; i < FM / 2; ++i) {  // blocks of 32 rows = two row fragments
         stage_block_bf16(i);
         u32x4 out[4];
 #pragma unroll
-        for (int it = 0; it < 4; ++it) {
-          const int row = rrow + 8 * it;
-          u32x4 w4 = *reinterpret_cast<const u32x4*>(stg + swz_off(row, rch));
-          if (p.gate || res_dtype >= 0) {
-            float o[8];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) { o[2 * e] = bf16_lo(w4[e]); o[2 * e + 1] = bf16_hi(w4[e]); }
-            if (gate_per_lane) {
-              const float* gr = gate_row_of(i * 32 + row);
-              gt0 = *reinterpret_cast<const f32x4*>(gr + n_g);
-              gt1 = *reinterpret_cast<const f32x4*>(gr + n_g + (full ? 4 : 0));
-            }
-            if (p.gate) {
-#pragma unroll
-              for (int e = 0; e < 4; ++e) { o[e] *= gt0[e]; o[4 + e] *= gt1[e]; }
-            }
-            if (res_dtype == AERIS_BF16) {
-              u32x4 r4 = rq[it][0];
-              if (upper) { r4.x = r4.z; r4.y = r4.w; }
-#pragma unroll
-              for (int e = 0; e < 4; ++e) { o[2 * e] += bf16_lo(r4[e]); o[2 * e + 1] += bf16_hi(r4[e]); }
-            } else if (res_dtype == AERIS_F32) {
-#pragma unroll
-              for (int e = 0; e < 4; ++e) {
-                o[e] += __uint_as_float(rq[it][0][e]);
-                o[4 + e] += __uint_as_float(rq[it][1][e]);
-              }
-            }
-            w4 = u32x4{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]), pack_bf16x2(o[4], o[5]), pack_bf16x2(o[6], o[7])};
-          }
-          out[it] = w4;
-        }
+        for (int it = 0; it < 4; ++it) out[it] = *reinterpret_cast<const u32x4*>(stg + swz_off(rrow + 8 * it, rch));
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
-        if (i + 1 < FM / 2) {
-          if (res_dtype >= 0) load_res(i + 1);  // ahead of the stores below
-        } else if (r_done + 1 < n_my) {
-          load_bias(r_done + 1, bq_next, q);
-        }
+        if (i + 1 == FM / 2 && r_done + 1 < n_my) load_bias(r_done + 1, bq_next, q);  // ahead of the stores below
 #pragma unroll
         for (int it = 0; it < 4; ++it) {
-          const int r = i * 32 + rrow_t + 8 * it;
+          const int r = i * 32 + rrow + 8 * it;
           if (col_ok && r < rows_left) {
             unsigned char* cp = c_lane + (int64_t)__mul24(r, rs24) * 2;
             if (full) *reinterpret_cast<u32x4*>(cp) = out[it];
@@ -601,7 +616,7 @@ __global__ void __launch_bounds__(NT) gemm_bf16_nt_persistent_kernel(GemmParams 
                                               (m_base * p.ldc + n) * (p.res_dtype == AERIS_BF16 ? 2 : 4);
 #pragma unroll
         for (int it = 0; it < 4; ++it) {
-          int r = i * 32 + rrow_t + 8 * it;
+          int r = i * 32 + rrow + 8 * it;
           if (r > rows_left - 1) r = rows_left - 1;
           const int64_t off = (int64_t)__mul24(r, ld24);
           if (p.res_dtype == AERIS_BF16) {
@@ -658,7 +673,7 @@ __global__ void __launch_bounds__(NT) gemm_bf16_nt_persistent_kernel(GemmParams 
             reinterpret_cast<unsigned char*>(p.C) + (m_base * c_row_stride(p) + c_col_off(p, n < N ? n : 0)) * 4;
 #pragma unroll
         for (int it = 0; it < 4; ++it) {
-          const int r = i * 32 + rrow_t + 8 * it;
+          const int r = i * 32 + rrow + 8 * it;
           if (r < rows_left && n < N) *reinterpret_cast<f32x4*>(c_lane + (int64_t)__mul24(r, rs24) * 4) = out[it];
         }
       }
@@ -719,7 +734,7 @@ __global__ void __launch_bounds__(NT) gemm_bf16_nt_persistent_kernel(GemmParams 
         // (group 0 needs its rows of W[j+1] only one slot later and could do without the vmcnt part here; waiting in both
         // groups costs nothing - those loads are a k-tile old - and spares a decision per slot)
         if (half == 0) __builtin_amdgcn_s_waitcnt(WAIT_LGKM0);
-        else __builtin_amdgcn_s_waitcnt(WAIT_VM8_LGKM0);
+        else __builtin_amdgcn_s_waitcnt(WAIT_AW_LGKM0);
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
         // ---- compute slot
@@ -739,34 +754,52 @@ __global__ void __launch_bounds__(NT) gemm_bf16_nt_persistent_kernel(GemmParams 
   }
 }
 
-hipError_t gemm_persistent_configure() {
-  hipError_t e;
-#define CFG1(A, F32, PL)                                                                                   \
-  e = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_bf16_nt_persistent_kernel<A, F32, PL>),         \
-                          hipFuncAttributeMaxDynamicSharedMemorySize, SMEM);                                 \
-  if (e != hipSuccess) return e;
-#define CFG(A, F32) CFG1(A, F32, false) CFG1(A, F32, true)
-  CFG(AERIS_ACT_NONE, false) CFG(AERIS_ACT_NONE, true) CFG(AERIS_ACT_GELU, false) CFG(AERIS_ACT_GELU, true)
-  CFG(AERIS_ACT_SWIGLU, false) CFG(AERIS_ACT_SWIGLU, true)
-#undef CFG
-#undef CFG1
-#define CFGR(A)                                                                                            \
-  e = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_bf16_nt_persistent_kernel<A, false, false, true>), \
-                          hipFuncAttributeMaxDynamicSharedMemorySize, SMEM);                                 \
-  if (e != hipSuccess) return e;
-  CFGR(AERIS_ACT_NONE) CFGR(AERIS_ACT_GELU) CFGR(AERIS_ACT_SWIGLU)
-#undef CFGR
-  e = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_bf16_nt_persistent_kernel<AERIS_ACT_NONE, true, false, false, true>),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, SMEM);
-  if (e != hipSuccess) return e;
-  return hipSuccess;
+namespace {
+
+template <int BM, int ACT, bool OUT_F32, bool PLAIN, bool RES_BF16 = false, bool RES_F32 = false>
+hipError_t configure_one() {
+  return hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_bf16_nt_persistent_kernel<BM, ACT, OUT_F32, PLAIN, RES_BF16, RES_F32>),
+                             hipFuncAttributeMaxDynamicSharedMemorySize, smem_bytes(BM));
+}
+template <int BM, int ACT>
+hipError_t configure_act() {
+  hipError_t e = configure_one<BM, ACT, false, false>();
+  if (e == hipSuccess) e = configure_one<BM, ACT, false, true>();
+  if (e == hipSuccess) e = configure_one<BM, ACT, true, false>();
+  if (e == hipSuccess) e = configure_one<BM, ACT, true, true>();
+  if (e == hipSuccess) e = configure_one<BM, ACT, false, false, true>();
+  return e;
+}
+template <int BM>
+hipError_t configure_all() {
+  hipError_t e = configure_act<BM, AERIS_ACT_NONE>();
+  if (e == hipSuccess) e = configure_act<BM, AERIS_ACT_GELU>();
+  if (e == hipSuccess) e = configure_act<BM, AERIS_ACT_SWIGLU>();
+  if (e == hipSuccess) e = configure_one<BM, AERIS_ACT_NONE, true, false, false, true>();
+  return e;
 }
 
-// p.act must be NONE, GELU or SWIGLU; N % 4 == 0 and ldc % 4 == 0; bias / gate rows 8- / 16-byte aligned
-hipError_t gemm_persistent_launch(const GemmParams& p0, hipStream_t stream) {
-  GemmParams p = p0;
-  const bool swiglu = p.act == AERIS_ACT_SWIGLU;
-  const int bn_out = swiglu ? BN / 2 : BN;
+template <int BM, int ACT>
+void launch_act(const GemmParams& p, dim3 grid, hipStream_t stream) {
+  const bool f32 = p.c_dtype == AERIS_F32, plain = !p.gate && p.res_dtype < 0;
+#define GO(...) hipLaunchKernelGGL((gemm_bf16_nt_persistent_kernel<BM, ACT, __VA_ARGS__>), grid, dim3(NT), smem_bytes(BM), stream, p)
+  if constexpr (ACT == AERIS_ACT_NONE) {
+    if (f32 && p.res_dtype == AERIS_F32 && !p.split) {
+      GO(true, false, false, true);
+      return;
+    }
+  }
+  if (!f32 && p.res_dtype == AERIS_BF16) GO(false, false, true);
+  else if (f32 && plain) GO(true, true);
+  else if (f32) GO(true, false);
+  else if (plain) GO(false, true);
+  else GO(false, false);
+#undef GO
+}
+
+template <int BM>
+hipError_t launch_bm(GemmParams p, hipStream_t stream) {
+  const int bn_out = p.act == AERIS_ACT_SWIGLU ? BN / 2 : BN;
   p.tiles_m = (int)((p.M + BM - 1) / BM);
   p.tiles_n = (p.N + bn_out - 1) / bn_out;
   p.total_tiles = p.tiles_m * p.tiles_n;
@@ -775,7 +808,7 @@ hipError_t gemm_persistent_launch(const GemmParams& p0, hipStream_t stream) {
   if (p.total_tiles >= (1 << 24)) return hipErrorInvalidValue;  // the range of the multiply-shift division
   p.m_gsz = (((uint64_t)1 << 40) + (uint64_t)(GM * p.tiles_n) - 1) / (uint64_t)(GM * p.tiles_n);
   // rows of a tile (first row of a wave group, at most tiles_m * 256 + 128) and rows_per_batch below 2^31
-  if ((int64_t)p.tiles_m * BM + BM >= (int64_t(1) << 31) || p.rows_per_batch <= 0 || p.rows_per_batch >= (int64_t(1) << 31))
+  if (p.row0 + (int64_t)p.tiles_m * BM + BM >= (int64_t(1) << 31) || p.rows_per_batch <= 0 || p.rows_per_batch >= (int64_t(1) << 31))
     return hipErrorInvalidValue;
   {
     int lg = 0;
@@ -783,32 +816,24 @@ hipError_t gemm_persistent_launch(const GemmParams& p0, hipStream_t stream) {
     p.rpb_shift = 31 + lg;
     p.rpb_magic = (uint32_t)((((uint64_t)1 << p.rpb_shift) + (uint64_t)p.rows_per_batch - 1) / (uint64_t)p.rows_per_batch);
   }
-  dim3 grid(8 * p.bpx), block(NT);
-  const bool f32 = p.c_dtype == AERIS_F32;
-  const bool plain = !p.gate && p.res_dtype < 0;
-  const bool res_bf16 = !f32 && p.res_dtype == AERIS_BF16;
-  if (f32 && p.res_dtype == AERIS_F32 && p.act == AERIS_ACT_NONE && !p.split) {
-    hipLaunchKernelGGL((gemm_bf16_nt_persistent_kernel<AERIS_ACT_NONE, true, false, false, true>), grid, block, SMEM, stream, p);
-    return hipGetLastError();
-  }
-#define GO1(A, F32)                                                                                        \
-  do {                                                                                                     \
-    if (plain) hipLaunchKernelGGL((gemm_bf16_nt_persistent_kernel<A, F32, true>), grid, block, SMEM, stream, p);  \
-    else hipLaunchKernelGGL((gemm_bf16_nt_persistent_kernel<A, F32, false>), grid, block, SMEM, stream, p);       \
-  } while (0)
-#define GO(A)                                                                                              \
-  do {                                                                                                     \
-    if (res_bf16)                                                                                            \
-      hipLaunchKernelGGL((gemm_bf16_nt_persistent_kernel<A, false, false, true>), grid, block, SMEM, stream, p);  \
-    else if (f32) GO1(A, true);                                                                              \
-    else GO1(A, false);                                                                                      \
-  } while (0)
-  if (swiglu) GO(AERIS_ACT_SWIGLU);
-  else if (p.act == AERIS_ACT_GELU) GO(AERIS_ACT_GELU);
-  else GO(AERIS_ACT_NONE);
-#undef GO
-#undef GO1
+  const dim3 grid(8 * p.bpx);
+  if (p.act == AERIS_ACT_SWIGLU) launch_act<BM, AERIS_ACT_SWIGLU>(p, grid, stream);
+  else if (p.act == AERIS_ACT_GELU) launch_act<BM, AERIS_ACT_GELU>(p, grid, stream);
+  else launch_act<BM, AERIS_ACT_NONE>(p, grid, stream);
   return hipGetLastError();
+}
+
+}  // namespace
+
+hipError_t gemm_persistent_configure() {
+  hipError_t e = configure_all<256>();
+  if (e == hipSuccess) e = configure_all<128>();
+  return e;
+}
+
+// p.act must be NONE, GELU or SWIGLU; N % 4 == 0 and ldc % 4 == 0; bias / gate rows 8- / 16-byte aligned
+hipError_t gemm_persistent_launch(const GemmParams& p, int tile_height, hipStream_t stream) {
+  return tile_height == 128 ? launch_bm<128>(p, stream) : launch_bm<256>(p, stream);
 }
 
 }  // namespace aeris

@@ -52,7 +52,8 @@ class _timed:
 
 
 def gemm_uses_big_tiles(M, N, act=None):
-    """Mirror of the tile choice in csrc/gemm.hip (256x256 tiles vs 128x128), used to label timings."""
+    """Whether the problem has a chip's worth of 256x256 tiles (csrc/gemm.hip's choice is then the 256x256 kernel for all
+    rows but at most the last partial round's); used to label timings."""
     bn = 128 if act == "swiglu" else 256
     return M >= 256 and (N % bn == 0 or N >= 4 * bn) and ((M + 255) // 256) * ((N + bn - 1) // bn) >= 256 and N % 4 == 0
 
@@ -352,7 +353,7 @@ def gemm(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, 
         if residual.numel() != M * N:
             raise RuntimeError("residual has the wrong size")
     big = gemm_uses_big_tiles(M, N, act) and act != "silu"
-    tag = "gemm_128x128"
+    tag = "gemm_small"
     if big:  # one tag per instantiation of the persistent kernel ("plain": neither gate nor residual in the epilogue;
         # "res": bf16 output with a bf16 residual)
         res_bf16 = residual is not None and residual.dtype == torch.bfloat16 and out.dtype == torch.bfloat16
@@ -392,7 +393,7 @@ def gemm_heads(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], h
         if tuple(out.shape) != (N // head_dim, M, head_dim):
             raise RuntimeError("out has the wrong shape")
     big = gemm_uses_big_tiles(M, N, None)
-    with _timed("gemm_256x256_none_bf16_plain" if big else "gemm_128x128", 2.0 * M * N * K, "flop"):
+    with _timed("gemm_256x256_none_bf16_plain" if big else "gemm_small", 2.0 * M * N * K, "flop"):
         L.call("aeris_gemm_heads_fwd", a.data_ptr(), w.data_ptr(), out.data_ptr(), _ptr(bias), M, N, K, head_dim,
                M * head_dim, float(q_scale), int(q_planes), _stream())
     return out

@@ -89,6 +89,61 @@ def test_gemm_parity(pkg, cuda, case):
     assert torch.isfinite(out).all()
 
 
+GEMM_EDGE_CASES = [
+    # M, N, K, act, bias, gate(batch), residual dtype, out dtype -- the edges of each tile kernel and of the row split
+    (1, 64, 64, None, True, 0, None, torch.bfloat16),                      # 64 x 64 tiles: one row, one k-tile
+    (63, 68, 128, "gelu", True, 0, None, torch.bfloat16),                  # half a 16-byte chunk, fewer k-tiles than stages
+    (65, 132, 192, None, True, 1, torch.bfloat16, torch.bfloat16),
+    (130, 100, 320, "swiglu", True, 0, torch.float32, torch.bfloat16),
+    (200, 192, 64, None, False, 40, torch.float32, torch.float32),         # 5 rows per batch entry: 13 entries in a tile
+    (300, 192, 128, None, True, 3, None, torch.bfloat16),                  # 100 rows per batch entry, gate without residual
+    (2048, 768, 128, "silu", True, 0, None, torch.bfloat16),
+    (8190, 1020, 512, None, True, 0, torch.bfloat16, torch.bfloat16),      # 128-row tiles, ragged in both directions
+    (8200, 1024, 512, None, True, 2, torch.float32, torch.float32),        # a batch boundary inside a 128-row tile
+    (8200, 1024, 512, None, True, 2, torch.bfloat16, torch.bfloat16),
+    (15000, 512, 256, "swiglu", False, 0, None, torch.bfloat16),
+    (14404, 1536, 1536, None, True, 4, torch.float32, torch.float32),      # a round of 256-row tiles + the rest of the rows;
+    (14404, 1536, 1536, None, False, 4, torch.bfloat16, torch.bfloat16),   # batch entries on both sides of the split
+    (9000, 4096, 512, "gelu", True, 0, None, torch.bfloat16),
+]
+
+
+@pytest.mark.parametrize("case", GEMM_EDGE_CASES, ids=lambda c: f"M{c[0]}_N{c[1]}_K{c[2]}_{c[3]}_g{c[5]}")
+def test_gemm_tile_edges(pkg, cuda, case):
+    """Every form rounds its result once.  That alone is at most 2^-7 / sqrt(12) = 2.3e-3 of the result in the 2-norm for
+    bf16 (a uniform error of half an ulp either way, all values at the lower edge of their binade); GELU adds its
+    polynomial's 2e-4.  fp32 results differ from the reference's by the order of the sums: 2e-5."""
+    M, N, K, act, has_bias, gate_b, res_dt, out_dt = case
+    g = torch.Generator().manual_seed(M * 7 + N + K)
+    a = bf(torch.randn(M, K, generator=g)).to(cuda)
+    n_w = 2 * N if act == "swiglu" else N
+    w = bf(torch.randn(n_w, K, generator=g) / math.sqrt(K)).to(cuda)
+    bias = bf(0.5 * torch.randn(n_w, generator=g)).to(cuda) if has_bias else None
+    gate = torch.randn(gate_b, N, generator=g).to(cuda) if gate_b else None
+    res = torch.randn(M, N, generator=g).to(res_dt).to(cuda) if res_dt is not None else None
+    ref = a.float() @ w.float().T
+    if bias is not None:
+        ref = ref + bias.float()
+    if act == "gelu":
+        ref = torch.nn.functional.gelu(ref)
+    elif act == "silu":
+        ref = torch.nn.functional.silu(ref)
+    elif act == "swiglu":
+        ref = torch.nn.functional.silu(ref[:, :N]) * ref[:, N:]
+    if gate is not None:
+        ref = ref * gate.repeat_interleave(M // gate_b, dim=0)
+    if res is not None:
+        ref = ref + res.float()
+    # rows and columns around C must stay as they are: C is the middle of a larger buffer
+    pad = torch.full((M + 2, N), 7.0, dtype=out_dt, device=cuda)
+    out = pad[1:-1] if (N * pad.element_size()) % 16 == 0 else torch.empty(M, N, dtype=out_dt, device=cuda)
+    pkg.ops.gemm(a, w, bias, act=act, gate=gate, residual=res, rows_per_batch=(M // gate_b if gate_b else 0), out=out)
+    torch.cuda.synchronize()
+    err = rel_l2(out, ref)
+    assert err <= (2.5e-3 if out_dt == torch.bfloat16 else 2e-5), err
+    assert bool((pad[0] == 7.0).all()) and bool((pad[-1] == 7.0).all())
+
+
 def test_gemm_gelu_epilogue_pointwise(pkg, cuda):
     """The GELU of the GEMM epilogue, value by value: with one non-zero column in A and ones in W every output is
     GELU(x) for a chosen x.  Against the erf form in float64: the epilogue's polynomial is within 2.1e-4 |x| (a tenth of

@@ -245,7 +245,7 @@ __global__ void __launch_bounds__(NT, 2) gemm_bf16_nt_tile_kernel(GemmParams p) 
     for (int e = 0; e < 4; ++e) {
       float x = acc[i][j][e];
       if (SWIGLU) x = silu_f(x) * acc[i][j + NJ][e];
-      else if (ACT == AERIS_ACT_GELU) x = gelu_erf_f(x);
+      else if (ACT == AERIS_ACT_GELU) x = OUT_F32 ? gelu_erf_f(x) : gelu_erf_bf16_f(x);
       else if (ACT == AERIS_ACT_SILU) x = silu_f(x);
       v[e] = x;
     }
@@ -338,7 +338,8 @@ hipError_t launch_tile_act(const GemmParams& p, hipStream_t stream) {
   return p.c_dtype == AERIS_F32 ? launch_tile<BM, BN, STAGES, A, true, VEC>(p, stream) \
                                 : launch_tile<BM, BN, STAGES, A, false, VEC>(p, stream)
   switch (p.act) {
-    case AERIS_ACT_GELU: GO(AERIS_ACT_GELU);
+    case AERIS_ACT_GELU:
+    case GEMM_ACT_GELU_ERF: GO(AERIS_ACT_GELU);
     case AERIS_ACT_SWIGLU: GO(AERIS_ACT_SWIGLU);
     case AERIS_ACT_SILU: GO(AERIS_ACT_SILU);
     default: GO(AERIS_ACT_NONE);
@@ -396,7 +397,7 @@ struct Shape {
 };
 
 float epilogue_us(const Shape& s) {  // of a 256 x 256 tile
-  return s.f32 ? 8.0f : s.act == AERIS_ACT_GELU ? 6.5f : s.res || s.act == AERIS_ACT_SWIGLU ? 6.0f : 4.5f;
+  return s.f32 ? 8.0f : s.act == GEMM_ACT_GELU_ERF ? 9.0f : s.act == AERIS_ACT_GELU ? 6.5f : s.res || s.act == AERIS_ACT_SWIGLU ? 6.0f : 4.5f;
 }
 
 int64_t tiles_of(const Shape& s, int bm, int bn) {
@@ -477,11 +478,17 @@ hipError_t gemm_launch(const void* A, const void* W, void* C, const void* bias, 
   // what the persistent kernel cannot take: it addresses W through one buffer descriptor (31-bit size), forms row offsets
   // with 24-bit multiplies, row numbers, gate row offsets and batch numbers in 32 bits, numbers its tiles in 24 bits and
   // scales whole 64-column wave blocks of the query part
-  const Shape s = {M, N, K / BK, act, c_dtype == AERIS_F32, residual != nullptr};
-  const bool persistent_ok = act != AERIS_ACT_SILU && (int64_t)(act == AERIS_ACT_SWIGLU ? 2 : 1) * N * K * 2 < (int64_t(1) << 31) &&
+  Shape s = {M, N, K / BK, act, c_dtype == AERIS_F32, residual != nullptr};
+  bool persistent_ok = act != AERIS_ACT_SILU && (int64_t)(act == AERIS_ACT_SWIGLU ? 2 : 1) * N * K * 2 < (int64_t(1) << 31) &&
                              ldc < (1 << 23) && split < (1 << 23) && gate_batch_stride < (int64_t(1) << 31) &&
                              (rows_per_batch <= 0 || M / rows_per_batch < (int64_t(1) << 31)) && M + 512 < (int64_t(1) << 31) &&
                              tiles_of(s, 128, 256) < (int64_t(1) << 24) && q_cols % 64 == 0 && N >= 64;
+  // GELU: the polynomial where there is a chip's worth of 256 x 256 tiles, erf otherwise (whatever the tiles are)
+  if (act == AERIS_ACT_GELU && c_dtype == AERIS_BF16 &&
+      !(M >= 256 && (N % 256 == 0 || N >= 1024) && tiles_of(s, 256, 256) >= 256)) {
+    p.act = s.act = GEMM_ACT_GELU_ERF;
+    persistent_ok = persistent_ok && !gate && !residual;
+  }
   if (!persistent_ok)
     return tiles_of(s, 128, 128) < 128 ? launch_tile_act<64, 64, 3, true>(p, stream) : launch_tile_act<128, 128, 2, true>(p, stream);
   float one = 0.f;

@@ -4,6 +4,10 @@
 
 namespace aeris {
 
+// GELU with bf16 C evaluated to 1.5e-7 instead of by the polynomial of gelu_bf16_f: which of the two a problem gets is part
+// of the interface (aeris_gemm_fwd)
+constexpr int GEMM_ACT_GELU_ERF = 4;
+
 struct GemmParams {
   const uint16_t* A;
   const uint16_t* W;

@@ -302,6 +302,7 @@ __global__ void __launch_bounds__(NT) gemm_bf16_nt_persistent_kernel(GemmParams 
       for (int e = 0; e < 4; ++e) {
         float x = acc[i][j][e];
         if (SWIGLU) x = silu_f(x) * acc[i][j + 2][e];
+        else if (ACT == GEMM_ACT_GELU_ERF) x = gelu_erf_bf16_f(x);
         else if (ACT == AERIS_ACT_GELU) x = OUT_F32 ? gelu_erf_f(x) : gelu_bf16_f(x);
         v[e] = x;
       }
@@ -346,7 +347,7 @@ __global__ void __launch_bounds__(NT) gemm_bf16_nt_persistent_kernel(GemmParams 
     // activation measured 2 % slower this way and stays on the general path): straight-line code lets the compiler wait
     // for exactly the loads a block needs.
     const bool inside = rows_left == BM / WM && n_wave + BN_OUT / WN <= N && !gate_per_lane;
-    const bool interior = PLAIN && ACT == AERIS_ACT_GELU && !OUT_F32 && inside;
+    const bool interior = PLAIN && (ACT == AERIS_ACT_GELU || ACT == GEMM_ACT_GELU_ERF) && !OUT_F32 && inside;
     // Interior plain SwiGLU tiles skip the staging (in the read-back of the general path half of the lanes idle on
     // its 64-byte rows; +2 %).  For the other forms this was slower (qkv -4 %, proj -5 %: 64-byte row pieces).
     const bool interior_direct = SWIGLU && PLAIN && !OUT_F32 && inside;
@@ -776,6 +777,7 @@ hipError_t configure_all() {
   if (e == hipSuccess) e = configure_act<BM, AERIS_ACT_GELU>();
   if (e == hipSuccess) e = configure_act<BM, AERIS_ACT_SWIGLU>();
   if (e == hipSuccess) e = configure_one<BM, AERIS_ACT_NONE, true, false, false, true>();
+  if (e == hipSuccess) e = configure_one<BM, GEMM_ACT_GELU_ERF, false, true>();
   return e;
 }
 
@@ -818,6 +820,8 @@ hipError_t launch_bm(GemmParams p, hipStream_t stream) {
   }
   const dim3 grid(8 * p.bpx);
   if (p.act == AERIS_ACT_SWIGLU) launch_act<BM, AERIS_ACT_SWIGLU>(p, grid, stream);
+  else if (p.act == GEMM_ACT_GELU_ERF)
+    hipLaunchKernelGGL((gemm_bf16_nt_persistent_kernel<BM, GEMM_ACT_GELU_ERF, false, true>), grid, dim3(NT), smem_bytes(BM), stream, p);
   else if (p.act == AERIS_ACT_GELU) launch_act<BM, AERIS_ACT_GELU>(p, grid, stream);
   else launch_act<BM, AERIS_ACT_NONE>(p, grid, stream);
   return hipGetLastError();
@@ -831,7 +835,7 @@ hipError_t gemm_persistent_configure() {
   return e;
 }
 
-// p.act must be NONE, GELU or SWIGLU; N % 4 == 0 and ldc % 4 == 0; bias / gate rows 8- / 16-byte aligned
+// p.act must be NONE, GELU, GELU_ERF (bf16 C without gate and residual) or SWIGLU; N % 4 == 0 and ldc % 4 == 0; bias / gate rows 8- / 16-byte aligned
 hipError_t gemm_persistent_launch(const GemmParams& p, int tile_height, hipStream_t stream) {
   return tile_height == 128 ? launch_bm<128>(p, stream) : launch_bm<256>(p, stream);
 }

@@ -7,21 +7,26 @@
 // (hi = bf16(v), lo = bf16(v - hi)); hi*hi + lo*hi + hi*lo are accumulated in fp32, only lo*lo (2^-16 relative) is
 // dropped.  The bias rides in a spare k column: the input operand holds 1 at k = C and the weight holds b[n] there.
 //
-// A workgroup of four waves owns 256 token rows; a wave builds the split operand of its 64 rows once, keeps it in
-// registers, and then walks over all d output columns in chunks of 64.  The split weight is packed once (when the
+// A workgroup of four waves owns 128 (small problems: 64) token rows; a wave builds the split operand of its 32 (16) rows
+// once, keeps it in registers, and then walks over the output columns in chunks of 64.  (With 64 rows per wave the operand
+// fills the register file: spills, and an eighth of the workgroups when the problem is small.)  The split weight is packed once (when the
 // parameter changes) in the order the MFMA operand wants it - 16 bytes per lane, lanes consecutive, 1 KB per
 // fragment - so a chunk is one contiguous piece of memory that goes to LDS by DMA (buffer_load ... lds), double
 // buffered, and every fragment read is one conflict-free ds_read_b128.  With the weight fragment as first MFMA
-// operand a lane ends up with 4 consecutive output columns of one row: results are stored straight from the
-// accumulators, 16 bytes per lane.
+// operand a lane ends up with 4 consecutive output columns of one row; pieces are exchanged between lanes so that every
+// store instruction writes whole 128-byte lines (in 64-byte pieces the stores alone took longer than everything else).
+// What bounds it now is those stores: without them the kernel takes 1.12 ms where it takes 1.83 ms with them, without
+// two thirds of its MFMAs 1.55 ms.
+// Measured before (64 rows per wave, operand built row by row through an LDS tile, 64-byte stores) -> now: 1 036 800 rows,
+// 138 -> 1536: 2.84 -> 1.83 ms (3.8 TB/s); 259 200 rows, 144 -> 512: 382 -> 170 us (4.0 TB/s); 51 840, 138 -> 320 (bf16): 85 -> 26 us;
+// 14 400, 144 -> 1536: 167 -> 42 us; 8192, 138 -> 1536: 163 -> 23 us; 2048, 138 -> 256: 52 -> 6.7 us.
 #include "common.h"
 #include "kernels.h"
 
 namespace aeris {
 
 namespace {
-constexpr int IS_ROWS = 256, IS_THREADS = 256;
-constexpr int IS_RB = 4;    // 16-row blocks per wave
+constexpr int IS_THREADS = 256;
 constexpr int IS_NBC = 4;   // 16-column blocks per chunk
 constexpr int IS_MAX_KB = 5;
 
@@ -33,6 +38,7 @@ struct InStageParams {
   void* out;
   int64_t M, M_ape;
   int C0, C1, d;
+  int splits;     // workgroups that share the columns of one row tile
   float div0;
 };
 
@@ -68,7 +74,20 @@ __global__ void __launch_bounds__(256) input_pack_weight_kernel(PackParams p) {
   *reinterpret_cast<u32x4*>(p.wp + t * 16) = o;
 }
 
-template <int NKB, bool OUT_F32>
+// a: rows 0-7 of the 16 lanes' pair (x | y), b: rows 8-15; the lower 8 lanes take the x part, the upper 8 the y part
+__device__ __forceinline__ void exchange8(bool upper, u32x4 x, u32x4 y, u32x4& a, u32x4& b) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const uint32_t give = upper ? x[e] : y[e];
+    const uint32_t got = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)give, 0x128, 0xF, 0xF, true);  // row_ror:8
+    a[e] = upper ? got : x[e];
+    b[e] = upper ? y[e] : got;
+  }
+}
+
+// IS_RB: 16-row blocks per wave, i.e. 64 IS_RB rows per workgroup
+// STREAM: non-temporal stores, for token matrices that do not fit the last-level cache
+template <int NKB, int IS_RB, bool OUT_F32, bool STREAM>
 __global__ void __launch_bounds__(IS_THREADS, 2) input_stage_kernel(InStageParams p) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   typedef __attribute__((address_space(3))) void* lds_ptr;
@@ -79,8 +98,11 @@ __global__ void __launch_bounds__(IS_THREADS, 2) input_stage_kernel(InStageParam
 
   const int tid = threadIdx.x, lane = tid & 63, l15 = lane & 15, q = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int64_t m0 = (int64_t)blockIdx.x * IS_ROWS + wave * (16 * IS_RB);
-  const int d = p.d, NCH = d / (16 * IS_NBC);
+  const int tile_m = blockIdx.x / p.splits, part = blockIdx.x - tile_m * p.splits;
+  const int64_t m0 = (int64_t)tile_m * (64 * IS_RB) + wave * (16 * IS_RB);
+  const int d = p.d;
+  // this workgroup's chunks of 64 columns: c_lo .. c_hi
+  const int chunks = d / (16 * IS_NBC), c_lo = part * chunks / p.splits, c_hi = (part + 1) * chunks / p.splits;
   const int C0 = p.C0, C = p.C0 + p.C1;
 
   const __amdgpu_buffer_rsrc_t rs_w =
@@ -92,156 +114,229 @@ __global__ void __launch_bounds__(IS_THREADS, 2) input_stage_kernel(InStageParam
     for (int i = 0; i < DMA_PER_WAVE; ++i)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_w, (lds_ptr)(dst + i * 1024), 16, (uint32_t)lane * 16, src + i * 1024, 0, 0);
   };
-  issue_dma(0, 0);
+  issue_dma(c_lo, 0);
 
-  // ---- the wave's operand: 4 row blocks x NKB k-steps, split into head and remainder, kept in registers.
-  // A row block is read column-wise (lane = channel, row pointers wave-uniform: coalesced loads), summed with the
-  // positional encoding, and turned into the row-wise fragment order through a wave-private 16 x (32 NKB) f32 tile in
-  // the second weight buffer, which is idle until the first chunk has been consumed.  16-byte pieces of a row are
-  // XOR-swizzled with the row number so that the fragment reads (16 rows x 16 bytes per quarter wave) do not collide.
+  // ---- the wave's operand: IS_RB row blocks x NKB k-steps, split into head and remainder, kept in registers.
+  // A lane loads its fragment where it lies: 8 consecutive channels of one row, two 16-byte loads (4-byte aligned, rows
+  // have any length) per k-step, for the input and for the positional encoding.  Only the k-steps that hold the boundary
+  // between x0 and x1 or the end of the row pick their 8 channels one by one.
   bf16x8 a_hi[IS_RB][NKB], a_lo[IS_RB][NKB];
   unsigned char* orow[IS_RB];
-  constexpr int KP = 32 * NKB;             // padded channel count
-  constexpr int NG = (KP + 63) / 64;       // column groups of 64 lanes
-  float* const tile = reinterpret_cast<float*>(smem + CHUNK_BYTES + wave * (CHUNK_BYTES / 4));
   const int64_t last_row = p.M - 1;
   const int64_t m0c = m0 < last_row ? m0 : last_row;
   const int nvalid = (int)(p.M - m0c < 16 * IS_RB ? p.M - m0c : 16 * IS_RB);  // >= 1
-  // the wave's 64 rows wrap around the positional encoding at most once: 64 <= M_ape < 2^31 (checked by the host)
+  // the wave's rows wrap around the positional encoding at most once: 64 <= M_ape < 2^31 (checked by the host)
   const int ape_row0 = (int)(m0c % p.M_ape), ape_rows = (int)p.M_ape;
-  // null pointers are resolved once, here, into valid bases with strides and masks that make them inert: the
-  // per-row code below has no branches, so that the loads of eight rows are in flight together
-  const float* const x0b = p.x0 + m0c * C0;
-  const float* const x1b = p.x1 ? p.x1 + m0c * p.C1 - C0 : x0b;
-  const int x1_stride = p.x1 ? p.C1 : C0;
-  const float* const apeb = p.ape ? p.ape : p.x0;
-  const int ape_stride = p.ape ? C : 0, ape_kmask = p.ape ? -1 : 0;
-  const bool has_ape = p.ape != nullptr;  // wave-uniform
   const float inv_div = 1.0f / p.div0;
+  typedef __attribute__((ext_vector_type(4), aligned(4))) float f32x4_u;  // 16 bytes at any float
 #pragma unroll
   for (int rb = 0; rb < IS_RB; ++rb) {
-    {
-      // Rows below the matrix recompute its last row and store it again (same bits to the same address): every
-      // wave then issues the same number of stores per chunk, which the wait at the end of a chunk counts on.
-      const int roff = min(rb * 16 + l15, nvalid - 1);
-      orow[rb] = reinterpret_cast<unsigned char*>(p.out) + ((m0c + roff) * d + 4 * q) * ESZ;
+    // Rows below the matrix recompute its last row and store it again (same bits to the same address): every
+    // wave then issues the same number of stores per chunk, which the wait at the end of a chunk counts on.
+    const int roff = min(rb * 16 + l15, nvalid - 1);
+    orow[rb] = reinterpret_cast<unsigned char*>(p.out) + (m0c + min(rb * 16 + (l15 & 7), nvalid - 1)) * d * ESZ;
+    int arow = ape_row0 + roff;
+    arow -= arow >= ape_rows ? ape_rows : 0;
+    const float* const r0 = p.x0 + (m0c + roff) * C0;
+    const float* const r1 = p.x1 ? p.x1 + (m0c + roff) * p.C1 - C0 : r0;  // indexed by channel
+    const float* const ra = p.ape ? p.ape + (int64_t)arow * C : nullptr;
+    float v[NKB][8], pe[NKB][8];
+#pragma unroll
+    for (int kb = 0; kb < NKB; ++kb) {
+      const int k0 = 32 * kb + 8 * q;
+      // wave-uniform: all 32 channels of this k-step from one array, none past the end
+      const bool one_part = 32 * kb + 32 <= C && (32 * kb + 32 <= C0 || 32 * kb >= C0);
+      if (one_part) {
+        const float* const src = (32 * kb < C0 ? r0 : r1) + k0;
+        const f32x4_u x = *reinterpret_cast<const f32x4_u*>(src), y = *reinterpret_cast<const f32x4_u*>(src + 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) { v[kb][e] = x[e]; v[kb][4 + e] = y[e]; }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int k = min(k0 + e, C - 1);
+          v[kb][e] = (k < C0 ? r0 : r1)[k];
+        }
+      }
+      if (ra) {
+        if (32 * kb + 32 <= C) {
+          const f32x4_u x = *reinterpret_cast<const f32x4_u*>(ra + k0), y = *reinterpret_cast<const f32x4_u*>(ra + k0 + 4);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) { pe[kb][e] = x[e]; pe[kb][4 + e] = y[e]; }
+        } else {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) pe[kb][e] = ra[min(k0 + e, C - 1)];
+        }
+      }
     }
 #pragma unroll
-    for (int half = 0; half < 2; ++half) {  // eight rows' loads in flight at a time
-      float val[8][NG];
+    for (int kb = 0; kb < NKB; ++kb) {
+      const int k0 = 32 * kb + 8 * q;
+      uint32_t hi[4], lo[4];
 #pragma unroll
-      for (int rr = 0; rr < 8; ++rr) {
-        const int roff = min(rb * 16 + half * 8 + rr, nvalid - 1);  // wave-uniform
-        const float* const b0 = x0b + roff * C0;
-        const float* const b1 = x1b + roff * x1_stride;
-        int arow = ape_row0 + roff;
-        arow -= arow >= ape_rows ? ape_rows : 0;
-        const float* const ba = apeb + (int64_t)arow * ape_stride;
-#pragma unroll
-        for (int g = 0; g < NG; ++g) {
-          const int k = 64 * g + lane;
-          const int kc = k < C ? k : C - 1;
-          const bool first = kc < C0;
-          const float* const src = first ? b0 : b1;
-          const float x = src[kc];
-          const float a = ba[kc & ape_kmask];
+      for (int e = 0; e < 8; ++e) {
+        float x = v[kb][e];
+        if (p.div0 != 1.0f) {
           // x / div0 for the state channels: quotient by reciprocal with one correction step
           float quo = x * inv_div;
           quo = fmaf(fmaf(-quo, p.div0, x), inv_div, quo);
-          // without a positional encoding `a` is a stand-in read from the input itself: a select, not a multiply
-          // by zero, keeps an Inf or NaN there out of every other token
-          const float base = first ? quo : x;
-          const float v = has_ape ? a + base : base;
-          val[rr][g] = k < C ? v : (k == C ? 1.0f : 0.0f);
+          x = k0 + e < C0 ? quo : x;
         }
+        if (ra) x += pe[kb][e];
+        if (32 * kb + 32 > C) x = k0 + e < C ? x : (k0 + e == C ? 1.0f : 0.0f);
+        v[kb][e] = x;
       }
 #pragma unroll
-      for (int rr = 0; rr < 8; ++rr)
-#pragma unroll
-        for (int g = 0; g < NG; ++g) {
-          const int k = 64 * g + lane, r = half * 8 + rr;
-          if (k < KP) tile[r * KP + ((((k >> 2) ^ (r & 7)) << 2) | (k & 3))] = val[rr][g];
-        }
-    }
-    __builtin_amdgcn_wave_barrier();
-#pragma unroll
-    for (int kb = 0; kb < NKB; ++kb) {
-      const int c4 = 8 * kb + 2 * q;  // 16-byte piece of the lane's 8 channels
-      const f32x4 v0 = *reinterpret_cast<const f32x4*>(tile + l15 * KP + ((c4 ^ (l15 & 7)) << 2));
-      const f32x4 v1 = *reinterpret_cast<const f32x4*>(tile + l15 * KP + (((c4 + 1) ^ (l15 & 7)) << 2));
-      uint32_t hi[4], lo[4];
-      hi[0] = pack_bf16x2(v0[0], v0[1]); lo[0] = pack_bf16x2(v0[0] - bf16_lo(hi[0]), v0[1] - bf16_hi(hi[0]));
-      hi[1] = pack_bf16x2(v0[2], v0[3]); lo[1] = pack_bf16x2(v0[2] - bf16_lo(hi[1]), v0[3] - bf16_hi(hi[1]));
-      hi[2] = pack_bf16x2(v1[0], v1[1]); lo[2] = pack_bf16x2(v1[0] - bf16_lo(hi[2]), v1[1] - bf16_hi(hi[2]));
-      hi[3] = pack_bf16x2(v1[2], v1[3]); lo[3] = pack_bf16x2(v1[2] - bf16_lo(hi[3]), v1[3] - bf16_hi(hi[3]));
+      for (int e = 0; e < 4; ++e) {
+        hi[e] = pack_bf16x2(v[kb][2 * e], v[kb][2 * e + 1]);
+        lo[e] = pack_bf16x2(v[kb][2 * e] - bf16_lo(hi[e]), v[kb][2 * e + 1] - bf16_hi(hi[e]));
+      }
       a_hi[rb][kb] = __builtin_bit_cast(bf16x8, u32x4{hi[0], hi[1], hi[2], hi[3]});
       a_lo[rb][kb] = __builtin_bit_cast(bf16x8, u32x4{lo[0], lo[1], lo[2], lo[3]});
     }
-    __builtin_amdgcn_wave_barrier();
   }
+  // second rows of a pair of stores (see below): 8 rows further down, where there are that many
+  int64_t row_step[IS_RB];
+#pragma unroll
+  for (int rb = 0; rb < IS_RB; ++rb)
+    row_step[rb] = (int64_t)(min(rb * 16 + 8 + (l15 & 7), nvalid - 1) - min(rb * 16 + (l15 & 7), nvalid - 1)) * d * ESZ;
   __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0): chunk 0 has landed
   __syncthreads();
 
-  for (int c = 0; c < NCH; ++c) {
+  for (int c = c_lo; c < c_hi; ++c) {
+    const int stage = (c - c_lo) & 1;
     __builtin_amdgcn_sched_barrier(0);
-    if (c + 1 < NCH) issue_dma(c + 1, (c + 1) & 1);
+    if (c + 1 < c_hi) issue_dma(c + 1, stage ^ 1);
     __builtin_amdgcn_sched_barrier(0);
-    const unsigned char* const ws = smem + (c & 1) * CHUNK_BYTES + lane * 16;
+    u32x4 half_line[IS_RB][2];
+    const unsigned char* const ws = smem + stage * CHUNK_BYTES + lane * 16;
+    constexpr int NBG = IS_RB == 1 ? 4 : 2;  // column blocks at a time: four or more independent accumulator chains
+    const bool upper = l15 >= 8;
 #pragma unroll
-    for (int nb = 0; nb < IS_NBC; ++nb) {
-      f32x4 acc[IS_RB];
+    for (int nb0 = 0; nb0 < IS_NBC; nb0 += NBG) {
+      f32x4 acc[NBG][IS_RB];
 #pragma unroll
-      for (int rb = 0; rb < IS_RB; ++rb) acc[rb] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int nb = 0; nb < NBG; ++nb)
+#pragma unroll
+        for (int rb = 0; rb < IS_RB; ++rb) acc[nb][rb] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int kb = 0; kb < NKB; ++kb) {
-        const bf16x8 w_hi = *reinterpret_cast<const bf16x8*>(ws + nb * NB_BYTES + (kb * 2 + 0) * 1024);
-        const bf16x8 w_lo = *reinterpret_cast<const bf16x8*>(ws + nb * NB_BYTES + (kb * 2 + 1) * 1024);
+        bf16x8 w_hi[NBG], w_lo[NBG];
+#pragma unroll
+        for (int nb = 0; nb < NBG; ++nb) {
+          w_hi[nb] = *reinterpret_cast<const bf16x8*>(ws + (nb0 + nb) * NB_BYTES + (kb * 2 + 0) * 1024);
+          w_lo[nb] = *reinterpret_cast<const bf16x8*>(ws + (nb0 + nb) * NB_BYTES + (kb * 2 + 1) * 1024);
+        }
         // weight fragment first: a lane ends up with 4 consecutive output columns of one row
 #pragma unroll
-        for (int rb = 0; rb < IS_RB; ++rb) acc[rb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w_hi, a_hi[rb][kb], acc[rb], 0, 0, 0);
+        for (int nb = 0; nb < NBG; ++nb)
 #pragma unroll
-        for (int rb = 0; rb < IS_RB; ++rb) acc[rb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w_hi, a_lo[rb][kb], acc[rb], 0, 0, 0);
+          for (int rb = 0; rb < IS_RB; ++rb) acc[nb][rb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w_hi[nb], a_hi[rb][kb], acc[nb][rb], 0, 0, 0);
 #pragma unroll
-        for (int rb = 0; rb < IS_RB; ++rb) acc[rb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w_lo, a_hi[rb][kb], acc[rb], 0, 0, 0);
+        for (int nb = 0; nb < NBG; ++nb)
+#pragma unroll
+          for (int rb = 0; rb < IS_RB; ++rb) acc[nb][rb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w_hi[nb], a_lo[rb][kb], acc[nb][rb], 0, 0, 0);
+#pragma unroll
+        for (int nb = 0; nb < NBG; ++nb)
+#pragma unroll
+          for (int rb = 0; rb < IS_RB; ++rb) acc[nb][rb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w_lo[nb], a_hi[rb][kb], acc[nb][rb], 0, 0, 0);
       }
-      const int col_off = (c * (16 * IS_NBC) + nb * 16) * ESZ;
+      // Stores as full 128-byte lines: a lane holds 4 columns of row l15 for each column block; the lanes of rows 0-7 give
+      // their second block's piece for the first block's piece of rows 8-15 (a rotation by 8 within 16 lanes), after which
+      // one store covers 8 rows x 128 B (f32: two column blocks; bf16: four, two of them joined per lane first).
 #pragma unroll
       for (int rb = 0; rb < IS_RB; ++rb) {
         if (OUT_F32) {
-          *reinterpret_cast<f32x4*>(orow[rb] + col_off) = acc[rb];
+#pragma unroll
+          for (int nb = 0; nb < NBG; nb += 2) {
+            u32x4 a, b;
+            exchange8(upper, __builtin_bit_cast(u32x4, acc[nb][rb]), __builtin_bit_cast(u32x4, acc[nb + 1][rb]), a, b);
+            unsigned char* const o = orow[rb] + ((c * IS_NBC + nb0 + nb + (upper ? 1 : 0)) * 16 + 4 * q) * 4;
+            if (STREAM) {
+              __builtin_nontemporal_store(a, reinterpret_cast<u32x4*>(o));
+              __builtin_nontemporal_store(b, reinterpret_cast<u32x4*>(o + row_step[rb]));
+            } else {
+              *reinterpret_cast<u32x4*>(o) = a;
+              *reinterpret_cast<u32x4*>(o + row_step[rb]) = b;
+            }
+          }
         } else {
-          const u32x2 o = {pack_bf16x2(acc[rb][0], acc[rb][1]), pack_bf16x2(acc[rb][2], acc[rb][3])};
-          *reinterpret_cast<u32x2*>(orow[rb] + col_off) = o;
+#pragma unroll
+          for (int nb = 0; nb < NBG; nb += 2) {
+            // (v_permlane16_swap: 8 consecutive columns of the pair of blocks per lane, 16 (q & 1) + 8 (q >> 1) ..)
+            const f32x4 v = acc[nb][rb], w = acc[nb + 1][rb];
+            const auto x = __builtin_amdgcn_permlane16_swap(pack_bf16x2(v[0], v[1]), pack_bf16x2(w[0], w[1]), false, false);
+            const auto y = __builtin_amdgcn_permlane16_swap(pack_bf16x2(v[2], v[3]), pack_bf16x2(w[2], w[3]), false, false);
+            half_line[rb][(nb0 + nb) / 2] = u32x4{x[0], y[0], x[1], y[1]};
+          }
         }
       }
     }
-    // The DMA loads of the next chunk were issued ahead of this chunk's 16 stores and vector memory operations
-    // complete in order: "all but the newest 16" is exactly those loads, without waiting for any store.
-    static_assert(IS_NBC * IS_RB == 16, "the vmcnt(16) below counts one store per 16-column block and 16-row block");
+    if (!OUT_F32) {
+#pragma unroll
+      for (int rb = 0; rb < IS_RB; ++rb) {
+        u32x4 a, b;
+        exchange8(upper, half_line[rb][0], half_line[rb][1], a, b);
+        unsigned char* const o = orow[rb] + (c * 64 + (upper ? 32 : 0) + 16 * (q & 1) + 8 * (q >> 1)) * 2;
+        *reinterpret_cast<u32x4*>(o) = a;
+        *reinterpret_cast<u32x4*>(o + row_step[rb]) = b;
+      }
+    }
+    // The DMA loads of the next chunk were issued ahead of this chunk's stores and vector memory operations complete
+    // in order: "all but the newest STORES" is exactly those loads, without waiting for any of those stores.
+    constexpr int STORES = (OUT_F32 ? IS_NBC : 2) * IS_RB;
+    static_assert(STORES <= 63, "vmcnt");
     __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_waitcnt(0x4F70);  // vmcnt(16)
+    __builtin_amdgcn_s_waitcnt(0x0F70 | (STORES & 15) | ((STORES >> 4) << 14));
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
   }
 }
 
-template <int NKB>
-hipError_t launch_main(const InStageParams& p, bool out_f32, hipStream_t stream) {
-  const dim3 grid((unsigned)((p.M + IS_ROWS - 1) / IS_ROWS)), block(IS_THREADS);
-  const size_t lds = 2 * (size_t)IS_NBC * NKB * 2 * 1024;
-  if (out_f32) hipLaunchKernelGGL((input_stage_kernel<NKB, true>), grid, block, lds, stream, p);
-  else hipLaunchKernelGGL((input_stage_kernel<NKB, false>), grid, block, lds, stream, p);
+constexpr int lds_bytes(int nkb) { return 2 * IS_NBC * nkb * 2 * 1024; }
+
+template <int NKB, int RB>
+hipError_t launch_rb(InStageParams p, bool out_f32, int splits, hipStream_t stream) {
+  p.splits = splits;
+  const int64_t tiles = (p.M + 64 * RB - 1) / (64 * RB);
+  const dim3 grid((unsigned)(tiles * splits)), block(IS_THREADS);
+  // (530 MB of tokens: 198 us with the default cache policy, 170 us non-temporal; 50-90 MB: the same, and the next kernel
+  // finds them in the cache)
+  const bool big = RB == 2 && out_f32 && p.M * p.d * 4 > (int64_t(256) << 20);
+  if (big) hipLaunchKernelGGL((input_stage_kernel<NKB, RB, true, RB == 2>), grid, block, lds_bytes(NKB), stream, p);
+  else if (out_f32) hipLaunchKernelGGL((input_stage_kernel<NKB, RB, true, false>), grid, block, lds_bytes(NKB), stream, p);
+  else hipLaunchKernelGGL((input_stage_kernel<NKB, RB, false, false>), grid, block, lds_bytes(NKB), stream, p);
   return hipGetLastError();
 }
 
 template <int NKB>
+hipError_t launch_main(const InStageParams& p, bool out_f32, hipStream_t stream) {
+  // 128 rows per workgroup where that gives most of two workgroups per CU, else 64 rows and the columns of a row tile
+  // shared by up to four workgroups, each of which builds the row operand for itself.  Measured, us for (RB, splits):
+  //   M = 1 036 800, d 1536:  (2, 1) 1830  (1, 1) 2000  (1, 2) 2125      51 840, d 320:  (2, 1) 25.6  (1, 1) 28.0
+  //   M = 14 400, d 1536:     (2, 1) 60.8  (1, 1) 41.0  (1, 2) 37-42     8192, d 1536:  (1, 1) 36.0  (1, 2) 22.9  (1, 4) 22.7
+  //   M = 2048, d 256:        (2, 1) 14.7  (1, 1) 9.6   (1, 4) 6.7  (1, 8) 6.6
+  if (p.M >= 128 * 320) return launch_rb<NKB, 2>(p, out_f32, 1, stream);
+  int64_t splits = 512 / ((p.M + 63) / 64);
+  if (splits > 4) splits = 4;
+  if (splits > p.d / 64) splits = p.d / 64;
+  if (splits < 1) splits = 1;
+  return launch_rb<NKB, 1>(p, out_f32, (int)splits, stream);
+}
+
+template <int NKB, int RB, bool OUT_F32, bool STREAM>
+hipError_t configure_kernel() {
+  return hipFuncSetAttribute(reinterpret_cast<const void*>(&input_stage_kernel<NKB, RB, OUT_F32, STREAM>),
+                             hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes(NKB));
+}
+template <int NKB>
 hipError_t configure_one() {
-  const int lds = 2 * IS_NBC * NKB * 2 * 1024;
-  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&input_stage_kernel<NKB, true>),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-  if (e != hipSuccess) return e;
-  return hipFuncSetAttribute(reinterpret_cast<const void*>(&input_stage_kernel<NKB, false>),
-                             hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  hipError_t e = configure_kernel<NKB, 2, true, true>();
+  if (e == hipSuccess) e = configure_kernel<NKB, 2, true, false>();
+  if (e == hipSuccess) e = configure_kernel<NKB, 2, false, false>();
+  if (e == hipSuccess) e = configure_kernel<NKB, 1, true, false>();
+  if (e == hipSuccess) e = configure_kernel<NKB, 1, false, false>();
+  return e;
 }
 }  // namespace
 

@@ -97,6 +97,41 @@ def test_input_stage_kernel_against_float64(pkg, cuda, case):
     assert e <= (1e-5 if out_dtype == torch.float32 else 3e-3), (e, ma)
 
 
+@pytest.mark.parametrize("case", [
+    # (M, M_ape, C0, C1, d, out dtype): 128-row workgroups from 40 960 rows on, 64-row ones with shared columns below
+    (1, 0, 5, 0, 64, torch.float32),             # one row, one chunk of columns
+    (65, 0, 33, 30, 320, torch.bfloat16),        # C = 63: the bias takes the last column of the second k-step
+    (8190, 4095, 31, 33, 192, torch.float32),    # two parts whose boundary lies inside a k-step; 2 column shares of 3 chunks
+    (41001, 13667, 32, 32, 128, torch.float32),  # 128-row workgroups, the last one with 41 rows; boundary on a k-step
+    (41001, 0, 69, 69, 64, torch.bfloat16),
+    (70001, 0, 20, 11, 1024, torch.float32),     # tokens beyond the last-level cache: non-temporal stores
+], ids=["one_row", "c63", "split", "large_ragged", "large_bf16", "streaming"])
+def test_input_stage_work_distribution(pkg, cuda, case):
+    """The edges of the input stage's row tiles and column shares, against float64: three products of 16-bit halves leave
+    2^-16 relative per product of the sums (1e-5); a bf16 result adds its rounding, at most 2^-7 / sqrt(12)."""
+    M, M_ape, C0, C1, d, out_dtype = case
+    ops = pkg.ops
+    g = torch.Generator(device="cuda").manual_seed(M + d)
+    C = C0 + C1
+    x0 = torch.randn(M, C0, generator=g, device=cuda)
+    x1 = torch.randn(M, C1, generator=g, device=cuda) if C1 else None
+    ape = torch.randn(M_ape, C, generator=g, device=cuda) if M_ape else None
+    w, b = torch.randn(d, C, generator=g, device=cuda) * 0.1, torch.randn(d, generator=g, device=cuda)
+    buf = torch.full((M + 2, d), 7.0, dtype=out_dtype, device=cuda)
+    ops.input_stage(x0, 2.0, x1, ape, ops.input_stage_pack_weight(w, b), d, out=buf[1:-1])
+    torch.cuda.synchronize()
+    pick = torch.unique(torch.cat([torch.arange(min(M, 600)), torch.arange(max(0, M - 600), M), torch.arange(0, M, 61)]))
+    xin = (x0.cpu()[pick] / 2.0).double()
+    if x1 is not None:
+        xin = torch.cat([xin, x1.cpu()[pick].double()], dim=1)
+    if ape is not None:
+        xin = xin + ape.cpu()[pick % M_ape].double()
+    want = xin @ w.cpu().double().t() + b.cpu().double()
+    e = rel_l2(buf[1:-1].cpu()[pick], want)
+    assert e <= (1e-5 if out_dtype == torch.float32 else 2.4e-3), e
+    assert bool((buf[0] == 7.0).all()) and bool((buf[-1] == 7.0).all())
+
+
 def test_input_stage_without_encoding_keeps_a_non_finite_input_in_its_own_token(pkg, cuda):
     """No positional encoding: an Inf (or NaN) in the first element of the input makes token 0 non-finite, as in the
     reference's Linear, and leaves every other token exactly what it is with a finite value there."""

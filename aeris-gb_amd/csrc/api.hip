@@ -388,8 +388,38 @@ int aeris_modulation_linear_fwd(const float* x, const void* W, const void* bias,
   if (!aligned16(x) || !aligned16(W)) return fail(AERIS_EINVAL, "aeris_modulation_linear_fwd: x/W must be 16-byte aligned");
   if (w_dtype != AERIS_BF16 && w_dtype != AERIS_F32) return fail(AERIS_EINVAL, "aeris_modulation_linear_fwd: bad w_dtype");
   if (act != AERIS_ACT_NONE && act != AERIS_ACT_SILU) return fail(AERIS_EINVAL, "aeris_modulation_linear_fwd: act must be NONE or SILU");
-  hipError_t e = aeris::modulation_linear_launch(x, W, bias, y, B, N, K, w_dtype, act, reinterpret_cast<hipStream_t>(stream));
+  const aeris_modulation_layer layer = {x, W, bias, y, N};
+  hipError_t e = aeris::modulation_linear_launch(&layer, 1, B, K, w_dtype, act, reinterpret_cast<hipStream_t>(stream));
   if (e != hipSuccess) return hip_fail(e, "aeris_modulation_linear_fwd launch");
+  return AERIS_OK;
+}
+
+int aeris_modulation_layers_fwd(const aeris_modulation_layer* layers, int n, int B, int K, int w_dtype, int act, void* stream) {
+  const char* who = "aeris_modulation_layers_fwd";
+  if (!layers || n <= 0) return fail(AERIS_EINVAL, "%s: no layers", who);
+  if (B <= 0 || K <= 0) return fail(AERIS_EINVAL, "%s: B, K must be positive", who);
+  if (K % 8) return fail(AERIS_EUNSUPPORTED, "%s: K=%d must be a multiple of 8", who, K);
+  if (w_dtype != AERIS_BF16 && w_dtype != AERIS_F32) return fail(AERIS_EINVAL, "%s: bad w_dtype", who);
+  if (act != AERIS_ACT_NONE && act != AERIS_ACT_SILU) return fail(AERIS_EINVAL, "%s: act must be NONE or SILU", who);
+  for (int i = 0; i < n; ++i) {
+    const aeris_modulation_layer& l = layers[i];
+    if (!l.x || !l.weight || !l.y) return fail(AERIS_EINVAL, "%s: x/weight/y of layer %d is NULL", who, i);
+    if (!aligned16(l.x) || !aligned16(l.weight)) return fail(AERIS_EINVAL, "%s: x/weight of layer %d must be 16-byte aligned", who, i);
+    if (l.N <= 0 || l.N > 0x7fffffffLL - 4) return fail(AERIS_EINVAL, "%s: N of layer %d out of range", who, i);
+  }
+  hipError_t e = aeris::modulation_linear_launch(layers, n, B, K, w_dtype, act, reinterpret_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return hip_fail(e, "aeris_modulation_layers_fwd launch");
+  return AERIS_OK;
+}
+
+int aeris_heun_update_fwd(const float* x, const float* f0, const float* f1, const float* t, float sigma_data, float* out, int64_t n,
+                          void* stream) {
+  if (!x || !f0 || !t || !out) return fail(AERIS_EINVAL, "aeris_heun_update_fwd: x/f0/t/out is NULL");
+  if (n <= 0) return fail(AERIS_EINVAL, "aeris_heun_update_fwd: n must be positive");
+  if (!aligned16(x) || !aligned16(f0) || !aligned16(out) || (f1 && !aligned16(f1)))
+    return fail(AERIS_EINVAL, "aeris_heun_update_fwd: x/f0/f1/out must be 16-byte aligned");
+  hipError_t e = aeris::heun_update_launch(x, f0, f1, t, sigma_data, out, n, reinterpret_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return hip_fail(e, "aeris_heun_update_fwd launch");
   return AERIS_OK;
 }
 
@@ -463,6 +493,78 @@ int aeris_input_stage_fwd(const float* x0, int C0, float div0, const float* x1, 
   hipError_t e = aeris::input_stage_launch(x0, C0, div0, x1, C1, ape, M_ape, packed_w, out, out_dtype, M, d,
                                            reinterpret_cast<hipStream_t>(stream));
   if (e != hipSuccess) return hip_fail(e, "aeris_input_stage_fwd launch");
+  return AERIS_OK;
+}
+
+// the layouts callers build without this header (ctypes / struct.pack): 8-byte fields, no padding
+static_assert(sizeof(aeris_block) == 20 * 8 && sizeof(aeris_block_config) == 17 * 8 && sizeof(aeris_modulation_layer) == 5 * 8, "ABI");
+
+int aeris_blocks_fwd(const aeris_block_config* c, const aeris_block* blocks, int n, const void* x, void* out,
+                     void* norm_scratch, void* qkv_scratch, void* attn_scratch, void* hidden_scratch, void* const* events,
+                     void* stream) {
+  const char* who = "aeris_blocks_fwd";
+  if (!c || !blocks || n <= 0) return fail(AERIS_EINVAL, "%s: no blocks", who);
+  if (!x || !out || !norm_scratch || !attn_scratch || !hidden_scratch) return fail(AERIS_EINVAL, "%s: x/out/scratch is NULL", who);
+  if (c->mod_ways != 0 && c->mod_ways != 2 && c->mod_ways != 3) return fail(AERIS_EINVAL, "%s: mod_ways must be 0, 2 or 3", who);
+  if (c->mlp_act != AERIS_ACT_GELU && c->mlp_act != AERIS_ACT_SWIGLU) return fail(AERIS_EINVAL, "%s: mlp_act must be GELU or SWIGLU", who);
+  const int64_t in_range[] = {c->B, c->H, c->W, c->dim, c->heads, c->head_dim, c->hidden, c->ws_y, c->ws_x};
+  for (int64_t v : in_range)
+    if (v <= 0 || v > 0x7fffffffLL) return fail(AERIS_EINVAL, "%s: sizes must be positive 32-bit numbers", who);
+  const int B = (int)c->B, H = (int)c->H, W = (int)c->W, d = (int)c->dim, heads = (int)c->heads, hd = (int)c->head_dim;
+  const int hidden = (int)c->hidden, wy = (int)c->ws_y, wx = (int)c->ws_x, xdt = (int)c->x_dtype;
+  const int64_t rows = c->H * c->W, T = c->B * rows, inner = c->heads * c->head_dim;
+  if (3 * inner > 0x7fffffffLL) return fail(AERIS_EINVAL, "%s: heads * head_dim too large", who);
+  const float eps = (float)c->eps, scale = (float)c->scale;
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  int ev = 0;
+  const auto mark = [&]() -> int {
+    if (!events) return AERIS_OK;
+    const hipError_t e = hipEventRecord(reinterpret_cast<hipEvent_t>(events[ev++]), s);
+    return e == hipSuccess ? AERIS_OK : hip_fail(e, "aeris_blocks_fwd: hipEventRecord");
+  };
+#define STEP(call)                    \
+  do {                                \
+    if (int rc = mark()) return rc;   \
+    if (int rc = (call)) return rc;   \
+    if (int rc = mark()) return rc;   \
+  } while (0)
+  for (int i = 0; i < n; ++i) {
+    const aeris_block& b = blocks[i];
+    if (c->mod_ways && !b.modulation) return fail(AERIS_EINVAL, "%s: modulation of block %d is NULL", who, i);
+    const float *shift1 = nullptr, *scale1 = nullptr, *gate1 = nullptr, *shift2 = nullptr, *scale2 = nullptr, *gate2 = nullptr;
+    if (c->mod_ways) {
+      const float* m = b.modulation;
+      shift1 = m; scale1 = m + d;
+      if (c->mod_ways == 3) gate1 = m + 2 * (int64_t)d;
+      m += c->mod_ways * d;
+      shift2 = m; scale2 = m + d;
+      if (c->mod_ways == 3) gate2 = m + 2 * (int64_t)d;
+    }
+    const void* in = i == 0 ? x : out;
+    const int sy = (int)b.shift_y, sx = (int)b.shift_x;
+    STEP(aeris_norm_modulate_fwd(in, xdt, norm_scratch, AERIS_BF16, b.norm1_weight, b.norm1_bias, (int)c->norm_dtype, shift1, scale1,
+                                 b.modulation_stride, B, rows, d, (int)c->norm_kind, (int)c->mod_order, eps, stream));
+    if (b.fuse_qkv && aeris::qkv_attention_supported(wy, wx, hd, d, rows) && 3 * inner * d * 2 < (int64_t(1) << 31)) {
+      STEP(aeris_qkv_window_attention_fwd(norm_scratch, b.qkv_weight, b.qkv_bias, b.bias4, attn_scratch, B, H, W, heads, hd, d, wy, wx,
+                                          sy, sx, (int)b.use_mask, scale, stream));
+    } else {
+      if (!qkv_scratch) return fail(AERIS_EINVAL, "%s: block %d needs qkv_scratch", who, i);
+      constexpr float LOG2E = 1.4426950408889634f;
+      STEP(aeris_gemm_heads_fwd(norm_scratch, b.qkv_weight, qkv_scratch, b.qkv_bias, T, (int)(3 * inner), d, hd, T * hd, scale * LOG2E,
+                                heads, stream));
+      STEP(aeris_window_attention_heads_fwd(qkv_scratch, attn_scratch, b.bias_table, B, H, W, heads, hd, wy, wx, sy, sx,
+                                            (int)b.use_mask, scale, 1, T * hd, stream));
+    }
+    STEP(aeris_gemm_fwd(attn_scratch, b.wo_weight, out, b.wo_bias, gate1, in, T, d, (int)inner, d, AERIS_ACT_NONE, xdt, xdt,
+                        gate1 ? b.modulation_stride : 0, rows, stream));
+    STEP(aeris_norm_modulate_fwd(out, xdt, norm_scratch, AERIS_BF16, b.norm2_weight, b.norm2_bias, (int)c->norm_dtype, shift2, scale2,
+                                 b.modulation_stride, B, rows, d, (int)c->norm_kind, (int)c->mod_order, eps, stream));
+    STEP(aeris_gemm_fwd(norm_scratch, b.up_weight, hidden_scratch, b.up_bias, nullptr, nullptr, T, hidden, d, hidden, (int)c->mlp_act, 0,
+                        AERIS_BF16, 0, T, stream));
+    STEP(aeris_gemm_fwd(hidden_scratch, b.down_weight, out, b.down_bias, gate2, out, T, d, hidden, d, AERIS_ACT_NONE, xdt, xdt,
+                        gate2 ? b.modulation_stride : 0, rows, stream));
+  }
+#undef STEP
   return AERIS_OK;
 }
 

@@ -55,8 +55,9 @@ hipError_t output_stage_launch(const void* x, int x_dtype, const void* gamma, co
                                float* out, int64_t B, int64_t rows_per_batch, int N, int d, int kind, float eps,
                                void* workspace, hipStream_t stream);
 
-hipError_t modulation_linear_launch(const float* x, const void* W, const void* bias, float* y, int B, int N, int K,
-                                    int w_dtype, int act, hipStream_t stream);
+hipError_t modulation_linear_launch(const aeris_modulation_layer* layers, int n, int B, int K, int w_dtype, int act, hipStream_t stream);
+hipError_t heun_update_launch(const float* x, const float* f0, const float* f1, const float* t, float sigma_data, float* out, int64_t n,
+                              hipStream_t stream);
 hipError_t timestep_embedding_launch(const float* t, float* emb, int B, int dim, float max_period, hipStream_t stream);
 hipError_t embed_prepare_launch(const float* x0, int C0, float div0, const float* x1, int C1, const float* ape, void* out,
                                 int64_t M, int64_t M_ape, int K_pad, int split, hipStream_t stream);

@@ -192,6 +192,7 @@ class Attention(nn.Module):
         self.rope = RoPE2D(**{k: v for k, v in rope_kwargs.items() if k in ("window_size", "rope_dim", "rope_base")})
         self.to_qkv = nn.Linear(dim, inner * 3, bias=bias)
         self.wo = nn.Linear(inner, dim, bias=bias)
+        self.table_rows = (2 * self.window_size[0] - 1) * (2 * self.window_size[1] - 1)
         if rel_pos_bias:
             wy, wx = self.window_size
             self.relative_position_bias_table = nn.Parameter(torch.zeros((2 * wy - 1) * (2 * wx - 1), heads))
@@ -272,9 +273,36 @@ def _norm_module(opts: BlockOptions, dim):
     return nn.RMSNorm(dim, eps=opts.eps)
 
 
-def _norm_call(opts: BlockOptions, norm, x, shift, scale, out=None):
-    return ops.norm_modulate(x, norm.weight, getattr(norm, "bias", None), shift, scale, kind=opts.norm,
-                             order=opts.mod_order, eps=opts.norm_eps, out=out)
+def _weight_bias(module):
+    """A module's weight and bias (None if it has none).  Straight from the parameter table where they are plain parameters:
+    a forward looks up a dozen of these per block, and nn.Module's attribute protocol is most of what that costs."""
+    p = module._parameters
+    if "weight" in p and ("bias" in p or not hasattr(module, "bias")):
+        return p["weight"], p.get("bias")
+    return module.weight, getattr(module, "bias", None)
+
+
+def _mlp_params(modulation: nn.Sequential):
+    l0, _, l2 = modulation._modules.values()
+    return *_weight_bias(l0), *_weight_bias(l2)
+
+
+def _mat_ptr(w, rows, cols):
+    """Address of a bf16 weight matrix [rows, cols] on the GPU, checked."""
+    if not (w.is_cuda and w.dtype is torch.bfloat16 and w.is_contiguous() and w.shape[0] == rows and w.shape[1] == cols):
+        ops._dev(w, "w", torch.bfloat16)
+        raise RuntimeError(f"w must be [{rows}, {cols}], got {tuple(w.shape)}")
+    return w.data_ptr()
+
+
+def _vec_ptr(v, n, dtype=torch.bfloat16):
+    """Address of a vector of n elements on the GPU (0 for None), checked."""
+    if v is None:
+        return 0
+    if not (v.is_cuda and v.dtype is dtype and v.is_contiguous() and v.numel() == n):
+        ops._dev(v, "bias / gain", dtype)
+        raise RuntimeError(f"bias / gain must have {n} elements, got {v.numel()}")
+    return v.data_ptr()
 
 
 class SwinLayer(nn.Module):
@@ -315,45 +343,85 @@ class SwinLayer(nn.Module):
             return (self.window_size[0] // 2, self.window_size[1] // 2)
         return (0, 0)
 
-    def block_forward(self, j, x, dt, shift, out=None, tap=None):
-        """One block.  x is not modified; the result is written to ``out`` (allocated if None).
+    def modulations(self):
+        """The parameters (w0, b0, w2, b2) of every block's modulation MLP, for ops.modulation_mlps."""
+        if not self.opts.mod_ways:
+            return []
+        return [_mlp_params(block._modules["4"].modulation) for block in self.modulelist._modules.values()]
 
-        ``tap(name, tensor, block)``, if given, is shown the two intermediates the block holds anyway before they are
-        consumed: "attn" (attention output ahead of the wo projection) and "hidden" (activated MLP hidden ahead of the
-        down projection), both as views of shared scratch that the next kernel overwrites.
-        """
+    def norm_dtype(self):
+        return self.modulelist[0][0].weight.dtype
+
+    def block_records(self, x, mods, shift, norm_dtype):
+        """(records, one-kernel flags) of all blocks for ``run_blocks``; ``mods``: their modulation vectors, f32 [1 | b, 2*ways*d]."""
+        records, fused = [], []
+        for j, block in enumerate(self.modulelist._modules.values()):
+            r, f = self._record(block, x, mods[j] if mods else None, shift, norm_dtype)
+            records.append(r)
+            fused.append(f)
+        return records, fused
+
+    def _record(self, block, x, m, shift, norm_dtype):
         o = self.opts
-        mods = self.modulelist[j]
-        n1, attn, n2, ff = mods[0], mods[1], mods[2], mods[3]
-        b, n, d = x.shape
-        s1 = c1 = g1 = s2 = c2 = g2 = None
-        if o.mod_ways:
-            m = mods[4](dt)  # f32 [1|b, 2*ways*d]
-            parts = m.chunk(2 * o.mod_ways, dim=1)
-            if o.mod_ways == 3:
-                s1, c1, g1, s2, c2, g2 = parts  # model.py:399
+        n1, attn, n2, ff = list(block._modules.values())[:4]
+        b, _, d = x.shape
+        inner = attn.heads * attn.head_dim
+        mod_ptr = mod_stride = 0
+        if m is not None:
+            if m.shape[1] != 2 * o.mod_ways * d or m.shape[0] not in (1, b):
+                raise RuntimeError(f"modulation must be [1 | {b}, {2 * o.mod_ways * d}], got {tuple(m.shape)}")
+            mod_ptr, mod_stride = m.data_ptr(), m.shape[1] if m.shape[0] > 1 else 0
+        sub = ff._modules
+        swiglu = o.mlp == "swiglu"
+        (up_w, up_b), (dn_w, dn_b) = (_weight_bias(sub["w1"]), _weight_bias(sub["w2"])) if swiglu else (
+            _weight_bias(sub["fc1"]), _weight_bias(sub["fc2"]))
+        sub = attn._modules
+        (qkv_w, qkv_b), (wo_w, wo_b) = _weight_bias(sub["to_qkv"]), _weight_bias(sub["wo"])
+        (n1_w, n1_b), (n2_w, n2_b) = _weight_bias(n1), _weight_bias(n2)
+        hid = dn_w.shape[1]
+        up_rows = 2 * hid if swiglu else hid
+        fused = attn.fuse_qkv and ops.qkv_attention_supported(d, attn.heads, attn.head_dim, attn.window_size, attn.image_shape)
+        table_ptr = b4_ptr = 0
+        table = attn.relative_position_bias_table
+        if table is not None:  # the one-kernel attention takes the table in its own form, the attention kernel as it is
+            if fused:
+                b4_ptr = attn._bias4().data_ptr()
             else:
-                s1, c1, s2, c2 = parts
-        # intermediates live in shared scratch buffers (ops.workspace); only `out` is returned
-        y = _norm_call(o, n1, x, s1, c1, out=ops.workspace("norm", (b, n, d), torch.bfloat16, x.device))
-        a = attn.core(y, shift, out=ops.workspace("attn", (b * n, attn.wo.weight.shape[1]), torch.bfloat16, x.device))
-        if tap is not None:
-            tap("attn", a, mods)
+                table_ptr = _vec_ptr(table, attn.table_rows * attn.heads)
+        rec = ops.BLOCK_RECORD.pack(
+            _vec_ptr(n1_w, d, norm_dtype), _vec_ptr(n1_b, d, norm_dtype), _vec_ptr(n2_w, d, norm_dtype), _vec_ptr(n2_b, d, norm_dtype),
+            _mat_ptr(qkv_w, 3 * inner, d), _vec_ptr(qkv_b, 3 * inner), _mat_ptr(wo_w, d, inner), _vec_ptr(wo_b, d),
+            _mat_ptr(up_w, up_rows, d), _vec_ptr(up_b, up_rows), _mat_ptr(dn_w, d, hid), _vec_ptr(dn_b, d), table_ptr, b4_ptr, mod_ptr,
+            mod_stride, shift[0], shift[1], attn.shift_mask and (shift[0] > 0 or shift[1] > 0), fused)
+        return rec, fused
+
+    def run_blocks(self, records, fused, norm_dtype, x, out):
+        """The blocks of ``records`` (this layer's, or several like layers') in one call: x -> out, then in place."""
+        o = self.opts
+        block = next(iter(self.modulelist._modules.values()))
+        _, attn, _, ff = list(block._modules.values())[:4]
+        hid = ff._modules["w2" if o.mlp == "swiglu" else "fc2"].weight.shape[1]
+        return ops.swin_blocks(records, x, out, self.image_shape, attn.heads, attn.head_dim, hid, self.window_size,
+                               norm_dtype=norm_dtype, norm=o.norm, mod_order=o.mod_order, mod_ways=o.mod_ways, mlp=o.mlp,
+                               eps=o.norm_eps, scale=attn.scale, shapes=fused)
+
+    def block_forward(self, j, x, dt, shift, out=None, tap=None):
+        """One block.  x is not modified; the result is written to ``out`` (allocated if None; may be x).
+
+        ``tap(name, tensor, block)``, if given, is shown the two intermediates the block holds anyway: "attn" (attention
+        output ahead of the wo projection) and "hidden" (activated MLP hidden ahead of the down projection), both as views
+        of shared scratch that the next block overwrites.
+        """
+        block = self.modulelist[j]
+        m = ops.modulation_mlps(dt.float().contiguous(), [_mlp_params(block[4].modulation)])[0] if self.opts.mod_ways else None
+        nd = self.norm_dtype()
+        rec, fused = self._record(block, x, m, shift, nd)
         if out is None:
             out = torch.empty_like(x)
-        ops.gemm(a, attn.wo.weight, attn.wo.bias, gate=g1, residual=x, rows_per_batch=n, out=out)
-        z = _norm_call(o, n2, out, s2, c2, out=y)
-        if o.mlp == "swiglu":
-            h = ops.gemm(z, ff.w1.weight, act="swiglu",
-                         out=ops.workspace("hidden", (b, n, ff.w1.weight.shape[0] // 2), torch.bfloat16, x.device))
-            w_dn, b_dn = ff.w2.weight, None
-        else:
-            h = ops.gemm(z, ff.fc1.weight, ff.fc1.bias, act="gelu",
-                         out=ops.workspace("hidden", (b, n, ff.fc1.weight.shape[0]), torch.bfloat16, x.device))
-            w_dn, b_dn = ff.fc2.weight, ff.fc2.bias
+        a, h = self.run_blocks([rec], [fused], nd, x, out)
         if tap is not None:
-            tap("hidden", h, mods)
-        ops.gemm(h, w_dn, b_dn, gate=g2, residual=out, rows_per_batch=n, out=out)  # in place: out += gate * mlp
+            tap("attn", a, block)
+            tap("hidden", h, block)
         return out
 
     def forward(self, x, dt=None, shift=None, tap=None):
@@ -363,9 +431,17 @@ class SwinLayer(nn.Module):
         if x.dtype not in (torch.bfloat16, torch.float32):
             raise TypeError("x must be bf16 or f32")
         x = x.contiguous()
-        for j in range(self.sublayers):
-            x = self.block_forward(j, x, dt, shift, tap=tap)
-        return x
+        if tap is not None:
+            for j in range(self.sublayers):
+                x = self.block_forward(j, x, dt, shift, tap=tap)
+            return x
+        if self.sublayers == 0:
+            return x
+        mods = ops.modulation_mlps(dt.float().contiguous(), self.modulations()) if self.opts.mod_ways else None
+        out = torch.empty_like(x)
+        nd = self.norm_dtype()
+        self.run_blocks(*self.block_records(x, mods, shift, nd), nd, x, out)
+        return out
 
 
 class InputStage(nn.Module):
@@ -462,11 +538,11 @@ class OutputStage(nn.Module):
             self._wcache = (key, w.detach().to(torch.bfloat16).contiguous())
         return self._wcache[1]
 
-    def forward(self, x, dt):
+    def forward(self, x, dt, m=None):
+        """``m``: the modulation vector of ``dt`` where the caller has it already (LocalAERIS, with its blocks')."""
         b, n, d = x.shape
-        l0, l2 = self.modulation[0], self.modulation[2]
-        h = ops.modulation_linear(dt.float().contiguous(), l0.weight, l0.bias, silu=True)
-        m = ops.modulation_linear(h, l2.weight, l2.bias)
+        if m is None:
+            m = ops.modulation_mlps(dt.float().contiguous(), [_mlp_params(self.modulation)])[0]
         shift, scale = m.chunk(2, dim=1)  # model.py:425
         beta = getattr(self.norm, "bias", None)
         w = self.head.weight
@@ -525,20 +601,26 @@ class LocalAERIS(nn.Module):
         tok, t = self.input_stage(x, dt, out_dtype=self.residual_dtype, cond=cond, x_div=x_div)
         if block_hook is not None:
             block_hook(0, tok)
-        k = 0
+        # every modulation MLP of the model depends on the noise level alone: two launches for all of them
+        mods = ops.modulation_mlps(t, [p for layer in self.layers for p in layer.modulations()] +
+                                   [_mlp_params(self.output_stage.modulation)])
         half = (self.window_size[0] // 2, self.window_size[1] // 2)
-        spare = None
+        records, fused, k = [], [], 0
+        nd = self.layers[0].norm_dtype() if len(self.layers) and self.layers[0].sublayers else None
         for i, layer in enumerate(self.layers):
             shift = half if i % 2 == 1 else (0, 0)  # model.py:471-475, folded into the attention kernel
-            for j in range(layer.sublayers):
-                if spare is None:
-                    spare = torch.empty_like(tok)
-                res = layer.block_forward(j, tok, t, shift, out=spare)
-                tok, spare = res, tok
-                k += 1
-                if block_hook is not None:
-                    block_hook(k, tok)
-        out = self.output_stage(tok, t)
+            n_mod = layer.sublayers if self.opts.mod_ways else 0
+            r, f = layer.block_records(tok, mods[k:k + n_mod], shift, nd)
+            k += n_mod
+            records += r
+            fused += f
+        if records and block_hook is None:
+            self.layers[0].run_blocks(records, fused, nd, tok, tok)
+        elif records:
+            for j in range(len(records)):
+                self.layers[0].run_blocks(records[j:j + 1], fused[j:j + 1], nd, tok, tok)
+                block_hook(j + 1, tok)
+        out = self.output_stage(tok, t, mods[-1])
         return (out, tok) if return_hidden else out
 
 

@@ -4,6 +4,8 @@ torch is used for device memory and streams only; all arithmetic happens in liba
 """
 from __future__ import annotations
 
+import math
+import struct
 from typing import Optional, Tuple
 
 import numpy as np
@@ -15,7 +17,8 @@ _DT = {torch.bfloat16: L.BF16, torch.float32: L.F32}
 
 
 def _stream():
-    return torch.cuda.current_stream().cuda_stream
+    # the raw handle, without a torch.cuda.Stream object around it: 0.3 us instead of 3, once or twice per call
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 # Optional per-launch timing (used by bench.py): HIP events recorded on the launch stream around each kernel.
@@ -59,7 +62,7 @@ def gemm_uses_big_tiles(M, N, act=None):
 
 
 _WORKSPACE = {}
-_WS_OWNER = {}  # key -> the stream whose work last used the buffer
+_WS_OWNER = {}  # key -> (raw handle, stream) whose work last used the buffer
 _RETIRED = []  # outgrown buffers stay allocated: a captured HIP graph may still point into them
 
 
@@ -75,26 +78,35 @@ def workspace(tag: str, shape, dtype, device) -> torch.Tensor:
     writing one scratch area at the same time and this raises instead.  Calls made while a stream is being captured
     are not checked, and replays of a captured graph do not pass through here: a graph must not be replayed on one
     stream while model calls run on another."""
-    n = 1
-    for d in shape:
-        n *= int(d)
-    key = (tag, str(device), dtype)
-    if not torch.cuda.is_current_stream_capturing():
-        # (a capture queues no work and nothing may be queried while it runs: it neither checks nor takes the buffer)
-        cur = torch.cuda.current_stream(device)
-        owner = _WS_OWNER.get(key)
-        if owner is not None and owner != cur and not owner.query():
-            raise RuntimeError(f"workspace {tag!r} on {device} is in use by work pending on another stream: the block "
-                               "intermediates are shared per device, run the models of one device on one stream "
-                               "(or synchronise the other stream first)")
-        _WS_OWNER[key] = cur
-    buf = _WORKSPACE.get(key)
-    if buf is None or buf.numel() < n:
-        if buf is not None:
-            _RETIRED.append(buf)
-        buf = torch.empty(n, dtype=dtype, device=device)
-        _WORKSPACE[key] = buf
-    return buf[:n].view(*shape)
+    return workspaces(torch.device(device), (tag, shape, dtype))[0]
+
+
+def workspaces(device, *requests):
+    """``workspace`` for several (tag, shape, dtype) on one device: the stream is looked up once."""
+    # (a capture queues no work and nothing may be queried while it runs: it neither checks nor takes the buffers)
+    capturing = torch._C._cuda_isCurrentStreamCapturing()
+    index = device.index
+    raw = torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice() if index is None else index)
+    got = []
+    for tag, shape, dtype in requests:
+        n = math.prod(shape)
+        key = (tag, device, dtype)
+        if not capturing:
+            owner = _WS_OWNER.get(key)
+            if owner is None or owner[0] != raw:
+                if owner is not None and not owner[1].query():
+                    raise RuntimeError(f"workspace {tag!r} on {device} is in use by work pending on another stream: the block "
+                                       "intermediates are shared per device, run the models of one device on one stream "
+                                       "(or synchronise the other stream first)")
+                _WS_OWNER[key] = (raw, torch.cuda.current_stream(device))
+        buf = _WORKSPACE.get(key)
+        if buf is None or buf.numel() < n:
+            if buf is not None:
+                _RETIRED.append(buf)
+            buf = torch.empty(n, dtype=dtype, device=device)
+            _WORKSPACE[key] = buf
+        got.append(buf[:n].view(shape))
+    return got
 
 
 def _ptr(t: Optional[torch.Tensor]):
@@ -414,6 +426,115 @@ def modulation_linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Ten
         out = torch.empty(B, N, dtype=torch.float32, device=x.device)
     L.call("aeris_modulation_linear_fwd", x.data_ptr(), w.data_ptr(), _ptr(bias), out.data_ptr(), B, N, K, _DT[w.dtype],
            L.ACT_SILU if silu else L.ACT_NONE, _stream())
+    return out
+
+
+def modulation_mlps(x: torch.Tensor, mlps):
+    """Several two-layer modulation MLPs (w0, b0, w2, b2) on the same rows x f32 [B, K]: Linear -> SiLU -> Linear each, all first
+    layers in one launch and all second layers in another.  -> list of f32 [B, N_i]."""
+    _dev(x, "x", torch.float32)
+    B, K = x.shape
+    if not x.is_contiguous():
+        x = x.contiguous()
+    for w0, b0, w2, b2 in mlps:
+        for w, b, k in ((w0, b0, K), (w2, b2, w0.shape[0])):
+            _dev(w, "w")
+            if w.dim() != 2 or w.shape[1] != k or w.dtype not in _DT:
+                raise RuntimeError(f"w must be bf16 or f32 [N, {k}]")
+            if b is not None:
+                _dev(b, "bias", w.dtype)
+                if b.numel() != w.shape[0]:
+                    raise RuntimeError("bias has the wrong size")
+    hidden = torch.empty(sum(m[0].shape[0] for m in mlps) * B, dtype=torch.float32, device=x.device)
+    out = torch.empty(sum(m[2].shape[0] for m in mlps) * B, dtype=torch.float32, device=x.device)
+    res, calls, h_off, o_off = [], {}, 0, 0
+    for w0, b0, w2, b2 in mlps:
+        n0, n2 = w0.shape[0], w2.shape[0]
+        h = hidden.data_ptr() + 4 * h_off
+        y = out[o_off:o_off + B * n2].view(B, n2)
+        calls.setdefault((0, K, w0.dtype), []).append((x.data_ptr(), w0.data_ptr(), _ptr(b0) or 0, h, n0))
+        calls.setdefault((1, n0, w2.dtype), []).append((h, w2.data_ptr(), _ptr(b2) or 0, y.data_ptr(), n2))
+        res.append(y)
+        h_off += B * n0
+        o_off += B * n2
+    for second in (0, 1):
+        for (layer, k, dtype), rows in calls.items():
+            if layer == second:
+                L.call("aeris_modulation_layers_fwd", b"".join(struct.pack("=5q", *r) for r in rows), len(rows), B, k, _DT[dtype],
+                       L.ACT_NONE if second else L.ACT_SILU, _stream())
+    return res
+
+
+BLOCK_RECORD = struct.Struct("=15Q5q")  # struct aeris_block of include/aeris_hip.h
+BLOCK_CONFIG = struct.Struct("=15q2d")  # struct aeris_block_config
+
+
+def swin_blocks(records, x: torch.Tensor, out: torch.Tensor, image_shape, heads: int, head_dim: int, hidden: int, window_size, *,
+                norm_dtype, norm: str, mod_order: str, mod_ways: int, mlp: str, eps: float, scale: float, shapes):
+    """n Swin blocks in one call (aeris_blocks_fwd): x [B, n, d] (bf16 | f32) -> out (may be x; same shape and dtype).
+    ``records``: one packed BLOCK_RECORD per block; ``shapes``: per block whether it runs the one-kernel attention (what the
+    scratch buffers and the timing records follow)."""
+    _dev(x, "x")
+    _dev(out, "out", x.dtype)
+    B, n, d = x.shape
+    T, inner, dev = B * n, heads * head_dim, x.device
+    requests = [("norm", (B, n, d), torch.bfloat16), ("attn", (T, inner), torch.bfloat16), ("hidden", (B, n, hidden), torch.bfloat16)]
+    if not all(shapes):
+        requests.append(("qkv", (3 * heads, T, head_dim), torch.bfloat16))
+    ws = workspaces(dev, *requests)
+    config = BLOCK_CONFIG.pack(B, image_shape[0], image_shape[1], d, heads, head_dim, hidden, window_size[0], window_size[1],
+                               _DT[x.dtype], _DT[norm_dtype], L.NORM_LAYER if norm == "layernorm" else L.NORM_RMS,
+                               L.NORM_THEN_MOD if mod_order == "norm_then_mod" else L.MOD_THEN_NORM, mod_ways,
+                               L.ACT_SWIGLU if mlp == "swiglu" else L.ACT_GELU, eps, scale)
+    events = _block_events(shapes, x, T, n, d, inner, hidden, window_size, mod_ways, mlp) if _profile is not None else None
+    L.call("aeris_blocks_fwd", config, b"".join(records), len(records), x.data_ptr(), out.data_ptr(), ws[0].data_ptr(),
+           ws[3].data_ptr() if len(ws) > 3 else None, ws[1].data_ptr(), ws[2].data_ptr(), events, _stream())
+    return ws[1], ws[2]
+
+
+def _block_events(fused, x, T, n, d, inner, hidden, window_size, mod_ways, mlp):
+    """Events for one swin_blocks call, entered in the running profile with the tags and work of the single ops; -> C array."""
+    norm = ("norm_modulate", float(T * d * (x.element_size() + 2)), "byte")
+    att = 4.0 * T * window_size[0] * window_size[1] * inner
+    qkv = 2.0 * T * 3 * inner * d
+    def gemm_tag(N, K, act, last):
+        if not gemm_uses_big_tiles(T, N, act):
+            return "gemm_small"
+        if not last:
+            return f"gemm_256x256_{act or 'none'}_bf16_plain"
+        return "gemm_256x256_none_f32" if x.dtype == torch.float32 else "gemm_256x256_none_bf16_res"
+    up = "swiglu" if mlp == "swiglu" else "gelu"
+    handles = []
+    for one_kernel in fused:
+        steps = [norm]
+        if one_kernel:
+            steps.append(("qkv_window_attention", qkv + att, "flop"))
+        else:
+            steps += [(gemm_tag(3 * inner, d, None, False), qkv, "flop"), ("window_attention", att, "flop")]
+        steps += [(gemm_tag(d, inner, None, True), 2.0 * T * d * inner, "flop"), norm,
+                  (gemm_tag(hidden, d, up, False), 2.0 * T * hidden * d * (2 if mlp == "swiglu" else 1), "flop"),
+                  (gemm_tag(d, hidden, None, True), 2.0 * T * d * hidden, "flop")]
+        for tag, work, unit in steps:
+            pair = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+            for e in pair:
+                e.record()  # (an event's handle exists from its first record on; the call records it again)
+                handles.append(e.cuda_event)
+            _profile.append((tag, work, unit, *pair))
+    return struct.pack(f"={len(handles)}Q", *handles)
+
+
+def heun_update(x: torch.Tensor, f0: torch.Tensor, f1: Optional[torch.Tensor], times: torch.Tensor, i: int, sigma_data: float):
+    """x + h f0, or with f1 x + (0.5 h) (f0 + f1), h = (times[i + 1] - times[i]) * sigma_data read on the device; f32, new tensor."""
+    _dev(x, "x", torch.float32)
+    _dev(f0, "f0", torch.float32)
+    if f1 is not None:
+        _dev(f1, "f1", torch.float32)
+    _dev(times, "times", torch.float32)
+    if f0.numel() != x.numel() or (f1 is not None and f1.numel() != x.numel()) or not 0 <= i < times.numel() - 1:
+        raise RuntimeError("x, f0, f1 must have one size, i must be a step of times")
+    out = torch.empty_like(x)
+    L.call("aeris_heun_update_fwd", x.data_ptr(), f0.data_ptr(), _ptr(f1), times.data_ptr() + 4 * i, float(sigma_data), out.data_ptr(),
+           x.numel(), _stream())
     return out
 
 

@@ -12,7 +12,7 @@ from typing import Optional
 
 import torch
 
-from . import _lib as L
+from . import _lib as L, ops
 
 
 def sigma_schedule(n_steps, sigma_min=0.2, sigma_max=500.0, sigma_data=1.0, rho=10, device="cpu"):
@@ -123,19 +123,26 @@ class TrigFlowSampler:
         # concatenation happen inside the embedding's operand preparation
         return self.model(x, t, cond=cond, x_div=self.sigma_data)
 
+    def _advance(self, x, F_s, F_t, i):
+        """x + h F_s, or x + (h / 2) (F_s + F_t), h = (t[i + 1] - t[i]) sigma_data  (inference.py:160-178)."""
+        ts, sd = self.t_steps, self.sigma_data
+        if all(v is None or (v.dtype is torch.float32 and v.is_cuda and v.is_contiguous()) for v in (x, F_s, F_t, ts)):
+            return ops.heun_update(x, F_s, F_t, ts, i, sd)
+        step = (ts[i + 1:i + 2] - ts[i:i + 1]) * sd  # another type, or a layout of the caller's own: the result has the promoted type
+        return x + step * F_s if F_t is None else x + (0.5 * step) * (F_s + F_t)
+
     @torch.no_grad()
     def sample(self, cond: torch.Tensor, latents: torch.Tensor) -> torch.Tensor:
         """cond [B, S, C_cond], latents [B, S, C] ~ N(0,1) -> sample [B, S, C]; 2*n_steps-1 denoiser calls."""
-        sd, ts, n = self.sigma_data, self.t_steps, self.n_steps
+        sd, n = self.sigma_data, self.n_steps
         x = latents * sd
+        levels = self.t_steps.split(1)
         for i in range(n):
-            s, t = ts[i:i + 1], ts[i + 1:i + 2]
-            step = (t - s) * sd
-            F_s = self._denoise(x, cond, s)
-            x_euler = x + step * F_s
+            F_s = self._denoise(x, cond, levels[i])
+            x_euler = self._advance(x, F_s, None, i)
             if i < n - 1:
-                F_t = self._denoise(x_euler, cond, t)
-                x = x + (0.5 * step) * (F_s + F_t)
+                F_t = self._denoise(x_euler, cond, levels[i + 1])
+                x = self._advance(x, F_s, F_t, i)
             else:
                 x = x_euler
         return x

@@ -196,8 +196,24 @@ int aeris_gemm_heads_fwd(const void* A, const void* W, void* C, const void* bias
 int aeris_modulation_linear_fwd(const float* x, const void* W, const void* bias, float* y, int B, int N,
                                 int K, int w_dtype, int act, void* stream);
 
+/* The same for n layers (one Linear of several ModulationLinear modules) that share B, K, w_dtype and act: one launch for
+ * up to 48 of them.  x may be the same array for all. */
+typedef struct aeris_modulation_layer {
+  const float* x;     /* f32 [B, K] */
+  const void* weight; /* [N, K], 16-byte aligned */
+  const void* bias;   /* [N] or NULL */
+  float* y;           /* f32 [B, N] */
+  int64_t N;
+} aeris_modulation_layer;
+int aeris_modulation_layers_fwd(const aeris_modulation_layer* layers, int n, int B, int K, int w_dtype, int act, void* stream);
+
 /* Sinusoidal noise-level embedding [sin | cos], t f32 [B] (device) -> emb f32 [B, dim]  (model.py:127-143). */
 int aeris_timestep_embedding_fwd(const float* t, float* emb, int B, int dim, float max_period, void* stream);
+
+/* One update of the Heun sampler (inference.py:160-178), out[n] = x + h f0, or with f1 given x + (0.5 h) (f0 + f1), where
+ * h = (t[1] - t[0]) * sigma_data is formed on the device from two consecutive noise levels.  f32; out may be x. */
+int aeris_heun_update_fwd(const float* x, const float* f0, const float* f1, const float* t, float sigma_data, float* out, int64_t n,
+                          void* stream);
 
 /* A-operand preparation for the input embedding: out bf16 [M, K_pad] = (x f32 [M, C] + ape f32 [M_ape, C] or NULL),
  * zero padded from C to K_pad columns; ape row = m % M_ape.  (model.py:350-352)
@@ -227,6 +243,35 @@ int aeris_input_stage_pack_weight(const float* W, const float* bias, void* packe
 int aeris_input_stage_fwd(const float* x0, int C0, float div0, const float* x1, int C1, const float* ape,
                           int64_t M_ape, const void* packed_w, void* out, int out_dtype, int64_t M, int d,
                           void* stream);
+
+/* n Swin blocks in a row (SwinLayer.forward, model.py:395-403; the loop of model.py:471-475): the calls above in the order
+ *   norm1 (+ modulation) -> to_qkv + window attention -> wo (* gate + residual) -> norm2 (+ modulation) -> MLP up -> MLP
+ *   down (* gate + residual)
+ * for each block, from one call: for small token counts the host's share of a block is otherwise longer than the GPU's.
+ * Block 0 reads x and writes out (which may be x); the blocks after it work in place on out.  Nothing is kept between calls.
+ *   mod_ways 0 | 2 | 3 per branch: modulation f32 [B_mod, 2*mod_ways*dim] = (shift, scale[, gate]) of the attention branch,
+ *   then of the MLP branch (model.py:399); modulation_stride 0: one row for the whole batch, else the rows' distance.
+ *   Scratch (bf16, 16-byte aligned, borrowed): norm_scratch [T, dim], qkv_scratch [3*heads][T, head_dim] (NULL if every block
+ *   takes the one-kernel attention: fuse_qkv and the shape supported), attn_scratch [T, heads*head_dim], hidden_scratch
+ *   [T, hidden] with T = B*H*W.
+ *   events: NULL, or 2 * (7 or, with one-kernel attention, 6) hipEvent_t per block, recorded on the stream before and after
+ *   each of the calls. */
+typedef struct aeris_block {
+  const void *norm1_weight, *norm1_bias, *norm2_weight, *norm2_bias;     /* [dim], norm_dtype; biases may be NULL */
+  const void *qkv_weight, *qkv_bias, *wo_weight, *wo_bias;               /* bf16; biases may be NULL */
+  const void *up_weight, *up_bias, *down_weight, *down_bias;             /* bf16 (w1, w2 | fc1, fc2) */
+  const void *bias_table, *bias4; /* relative-position bias as aeris_window_attention_heads_fwd / aeris_qkv_window_attention_fwd take it, or NULL */
+  const float* modulation;
+  int64_t modulation_stride, shift_y, shift_x, use_mask, fuse_qkv;
+} aeris_block;
+typedef struct aeris_block_config {
+  int64_t B, H, W, dim, heads, head_dim, hidden, ws_y, ws_x;
+  int64_t x_dtype, norm_dtype, norm_kind, mod_order, mod_ways, mlp_act; /* mlp_act: AERIS_ACT_GELU | AERIS_ACT_SWIGLU */
+  double eps, scale;
+} aeris_block_config;
+int aeris_blocks_fwd(const aeris_block_config* config, const aeris_block* blocks, int n, const void* x, void* out,
+                     void* norm_scratch, void* qkv_scratch, void* attn_scratch, void* hidden_scratch, void* const* events,
+                     void* stream);
 
 #ifdef __cplusplus
 }

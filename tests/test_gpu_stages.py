@@ -266,6 +266,34 @@ def test_converted_checkpoint_runs_on_the_gpu(pkg, cuda, tmp_path):
         pkg.convert_inference_checkpoint(str(tmp_path), N, model, map_location="cuda")
 
 
+@pytest.mark.parametrize("n", [1, 3, 4, 1023, 1025, 70001])
+def test_heun_update_equals_the_elementwise_chain(pkg, cuda, n):
+    """One kernel, the same roundings as the chain of element-wise operations: equal bit for bit."""
+    g = torch.Generator(device="cuda").manual_seed(n)
+    x, f0, f1 = (torch.randn(n, generator=g, device=cuda) for _ in range(3))
+    t = torch.tensor([1.5, 1.1, 0.3], device=cuda)
+    for i in range(2):
+        step = (t[i + 1] - t[i]) * 0.7
+        assert torch.equal(pkg.ops.heun_update(x, f0, None, t, i, 0.7), x + step * f0)
+        assert torch.equal(pkg.ops.heun_update(x, f0, f1, t, i, 0.7), x + (0.5 * step) * (f0 + f1))
+
+
+@pytest.mark.parametrize("wdt", [torch.float32, torch.bfloat16])
+def test_modulation_mlps_equal_the_single_layers(pkg, cuda, wdt):
+    """All modulation MLPs of a model in two launches, more of them than fit one launch and of different widths: the same bits as
+    layer by layer, the last bits of the sums included."""
+    g = torch.Generator(device="cuda").manual_seed(4)
+    K, B, ops = 200, 3, pkg.ops
+    x = torch.randn(B, K, generator=g, device=cuda)
+
+    def layer(n, k):
+        return torch.randn(n, k, generator=g, device=cuda).to(wdt), torch.randn(n, generator=g, device=cuda).to(wdt)
+    mlps = [(*layer(K, K), *layer(n, K)) for n in ([5, 1200, 64] * 17)]
+    for got, (w0, b0, w2, b2) in zip(ops.modulation_mlps(x, mlps), mlps):
+        want = ops.modulation_linear(ops.modulation_linear(x, w0, b0, silu=True), w2, b2)
+        assert torch.equal(got, want)
+
+
 def test_workspace_refuses_a_second_stream_while_the_first_is_busy(pkg, cuda):
     """The block intermediates are one set of scratch buffers per device; a second stream asking for them while the
     first still has work pending would overwrite them under that work, so the request raises.  Once the first stream

@@ -182,6 +182,39 @@ def with_of(args, i, v):
     return a
 
 
+def test_packed_records_match_the_header(pkg):
+    """struct.pack layouts of the host side against the structs of include/aeris_hip.h: every field 8 bytes, same count."""
+    header = open(os.path.join(ROOT, "include", "aeris_hip.h")).read()
+    header = re.sub(r"/\*.*?\*/", "", header, flags=re.S)
+
+    def fields(name):
+        body = re.search(r"typedef struct %s \{(.*?)\} %s;" % (name, name), header, flags=re.S).group(1)
+        return sum(len(line.split(",")) for line in body.split(";") if line.strip())
+
+    assert pkg.ops.BLOCK_RECORD.size == 8 * fields("aeris_block")
+    assert pkg.ops.BLOCK_CONFIG.size == 8 * fields("aeris_block_config")
+    assert fields("aeris_modulation_layer") == 5
+
+
+def test_blocks_validation_needs_no_gpu(pkg):
+    lib, ops = pkg._lib.lib(), pkg.ops
+    fake = 0x1000
+    good = dict(B=1, H=16, W=16, dim=64, heads=1, head_dim=64, hidden=128, ws_y=16, ws_x=16, x_dtype=0, norm_dtype=0, norm_kind=0,
+                mod_order=0, mod_ways=0, mlp_act=1)
+    record = ops.BLOCK_RECORD.pack(*([fake] * 14), 0, 0, 0, 0, 0, 0)  # no modulation vector
+
+    def call(n=1, x=fake, out=fake, **change):
+        config = ops.BLOCK_CONFIG.pack(*{**good, **change}.values(), 1e-5, 0.125)
+        return lib.aeris_blocks_fwd(config, record, n, x, out, fake, fake, fake, fake, None, None)
+
+    for bad in (dict(n=0), dict(x=None), dict(out=None), dict(B=0), dict(hidden=-64), dict(mod_ways=1), dict(mlp_act=0), dict(mod_ways=2)):
+        assert call(**bad) == -1, bad
+    assert lib.aeris_modulation_layers_fwd(None, 1, 1, 64, 1, 0, None) == -1
+    assert lib.aeris_modulation_layers_fwd(b"\0" * 40, 1, 1, 64, 1, 0, None) == -1
+    assert lib.aeris_heun_update_fwd(fake, fake, None, fake, 1.0, fake, 0, None) == -1
+    assert lib.aeris_heun_update_fwd(fake + 4, fake, None, fake, 1.0, fake, 4, None) == -1
+
+
 def test_ops_refuse_cpu_tensors(pkg):
     x = torch.zeros(1, 4, 64, dtype=torch.bfloat16)
     with pytest.raises(RuntimeError, match="GPU"):

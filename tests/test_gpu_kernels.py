@@ -108,6 +108,21 @@ GEMM_EDGE_CASES = [
 ]
 
 
+@pytest.mark.parametrize("M,N", [(70, 68), (4096, 3072)])  # a 64x64-tile problem; 192 tiles of 256 rows (erf GELU as well)
+def test_gemm_gelu_of_infinite_and_huge_values(pkg, cuda, M, N):
+    """GELU of a pre-activation that overflowed is its limit, inf or 0, and NaN stays NaN."""
+    a, w = torch.zeros(M, 128), torch.zeros(N, 128)
+    a[:, 0] = 1.0
+    a[1, 0], a[2, 0], a[3, 0], a[M - 1, 0] = float("inf"), 3e38, float("nan"), float("inf")
+    w[:, 0] = 1.0
+    w[1::2, 0] = -1.0
+    out = pkg.ops.gemm(a.to(cuda, torch.bfloat16), w.to(cuda, torch.bfloat16), None, act="gelu").float().cpu()
+    for r in (1, M - 1):
+        assert bool((out[r, ::2] == float("inf")).all()) and bool((out[r, 1::2] == 0).all())
+    assert bool((out[2, ::2] > 2.9e38).all()) and bool((out[2, 1::2] == 0).all())
+    assert bool(out[3].isnan().all())
+
+
 @pytest.mark.parametrize("case", GEMM_EDGE_CASES, ids=lambda c: f"M{c[0]}_N{c[1]}_K{c[2]}_{c[3]}_g{c[5]}")
 def test_gemm_tile_edges(pkg, cuda, case):
     """Every form rounds its result once.  That alone is at most 2^-7 / sqrt(12) = 2.3e-3 of the result in the 2-norm for

@@ -523,6 +523,14 @@ def _block_events(fused, x, T, n, d, inner, hidden, window_size, mod_ways, mlp):
     return struct.pack(f"={len(handles)}Q", *handles)
 
 
+def heun_update_supported(x: torch.Tensor, f0: torch.Tensor, f1: Optional[torch.Tensor], times: torch.Tensor) -> bool:
+    """Whether ``heun_update`` takes these: f32 on one GPU, contiguous, one shape, 16-byte aligned (times: any alignment)."""
+    if not (times.is_cuda and times.dtype is torch.float32 and times.is_contiguous() and times.device == x.device):
+        return False
+    return all(v is None or (v.dtype is torch.float32 and v.is_cuda and v.device == x.device and v.is_contiguous() and
+                             v.shape == x.shape and v.data_ptr() % 16 == 0) for v in (x, f0, f1))
+
+
 def heun_update(x: torch.Tensor, f0: torch.Tensor, f1: Optional[torch.Tensor], times: torch.Tensor, i: int, sigma_data: float):
     """x + h f0, or with f1 x + (0.5 h) (f0 + f1), h = (times[i + 1] - times[i]) * sigma_data read on the device; f32, new tensor."""
     _dev(x, "x", torch.float32)

@@ -126,9 +126,10 @@ class TrigFlowSampler:
     def _advance(self, x, F_s, F_t, i):
         """x + h F_s, or x + (h / 2) (F_s + F_t), h = (t[i + 1] - t[i]) sigma_data  (inference.py:160-178)."""
         ts, sd = self.t_steps, self.sigma_data
-        if all(v is None or (v.dtype is torch.float32 and v.is_cuda and v.is_contiguous()) for v in (x, F_s, F_t, ts)):
+        if ops.heun_update_supported(x, F_s, F_t, ts):
             return ops.heun_update(x, F_s, F_t, ts, i, sd)
-        step = (ts[i + 1:i + 2] - ts[i:i + 1]) * sd  # another type, or a layout of the caller's own: the result has the promoted type
+        # a model of the caller's own may return another type or layout, or an output that broadcasts over the members
+        step = (ts[i + 1:i + 2] - ts[i:i + 1]) * sd
         return x + step * F_s if F_t is None else x + (0.5 * step) * (F_s + F_t)
 
     @torch.no_grad()

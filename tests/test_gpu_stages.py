@@ -354,3 +354,19 @@ def test_first_call_inside_a_capture_is_refused():
     """ % ROOT)
     r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=150)
     assert "CHILD_OK" in r.stdout, (r.stdout[-2000:], r.stderr[-2000:])
+
+
+def test_sampler_takes_what_the_update_kernel_does_not(pkg, cuda):
+    """A model of the caller's own: an output that broadcasts over the members, one that is not 16-byte aligned, a wider type."""
+    g = torch.Generator(device="cuda").manual_seed(5)
+    lat, cond = torch.randn(2, 33, 5, generator=g, device=cuda), torch.randn(2, 33, 3, generator=g, device=cuda)
+    flat = torch.randn(1 + 2 * 33 * 5, generator=g, device=cuda)
+    for out in (torch.randn(1, 33, 5, generator=g, device=cuda), flat[1:].view(2, 33, 5), flat[1:].view(2, 33, 5).double()):
+        s = pkg.TrigFlowSampler(lambda x, t, cond=None, x_div=1.0: out * t.to(out.dtype) if out.dtype == torch.float64 else out, n_steps=3, device=cuda)
+        x, ts = lat * s.sigma_data, s.t_steps
+        for i in range(3):
+            f = [out * t.double() if out.dtype == torch.float64 else out for t in (ts[i:i + 1], ts[i + 1:i + 2])]
+            step = (ts[i + 1:i + 2] - ts[i:i + 1]) * s.sigma_data
+            x = x + (0.5 * step) * (f[0] + f[1]) if i < 2 else x + step * f[0]
+        got = s.sample(cond, lat)
+        assert got.dtype == x.dtype and torch.equal(got, x)

@@ -18,7 +18,7 @@ from __future__ import annotations
 import math
 import os
 from dataclasses import dataclass
-from typing import Optional, Tuple
+from typing import NamedTuple, Optional, Tuple
 
 import torch
 import torch.nn as nn
@@ -282,11 +282,6 @@ def _weight_bias(module):
     return module.weight, getattr(module, "bias", None)
 
 
-def _mlp_params(modulation: nn.Sequential):
-    l0, _, l2 = modulation._modules.values()
-    return *_weight_bias(l0), *_weight_bias(l2)
-
-
 def _mat_ptr(w, rows, cols):
     """Address of a bf16 weight matrix [rows, cols] on the GPU, checked."""
     if not (w.is_cuda and w.dtype is torch.bfloat16 and w.is_contiguous() and w.shape[0] == rows and w.shape[1] == cols):
@@ -303,6 +298,46 @@ def _vec_ptr(v, n, dtype=torch.bfloat16):
         ops._dev(v, "bias / gain", dtype)
         raise RuntimeError(f"bias / gain must have {n} elements, got {v.numel()}")
     return v.data_ptr()
+
+
+class BlockCall(NamedTuple):
+    """One Swin block as ``ops.swin_blocks`` takes it."""
+    record: bytes  # packed addresses and options
+    fused: bool  # whether it runs the one-kernel attention
+    config: tuple  # what blocks of one call have in common
+    keep: tuple  # the tensors whose addresses the record holds
+
+
+def _run_blocks(calls, x, out):
+    """The blocks of ``calls``: x -> out (may be x), then in place; blocks of one configuration go in one native call.
+    Returns the last call's scratch buffers (attention output, MLP hidden)."""
+    i, scratch = 0, None
+    while i < len(calls):
+        j = i + 1
+        while j < len(calls) and calls[j].config == calls[i].config:
+            j += 1
+        scratch = ops.swin_blocks([c.record for c in calls[i:j]], x, out, *calls[i].config, shapes=[c.fused for c in calls[i:j]])
+        x, i = out, j
+    return scratch
+
+
+def _mlp_params(modulation: nn.Sequential):
+    l0, _, l2 = modulation._modules.values()
+    return *_weight_bias(l0), *_weight_bias(l2)
+
+
+def _modulation_vectors(modules, dt, extra=()):
+    """f32 [1 | b, N_i] of each modulation module on the noise-level embedding dt, and of the MLPs ``extra`` (parameter
+    tuples): two launches for all of them, but what a caller has hooked or put in a module's place is called as a module."""
+    plain = [type(m) is ModulationLinear and not m._forward_hooks and not m._forward_pre_hooks for m in modules]
+    mlps = [_mlp_params(m.modulation) for m, p in zip(modules, plain) if p] + list(extra)
+    got = iter(ops.modulation_mlps(dt.float().contiguous(), mlps) if mlps else ())
+    return [next(got) if p else m(dt) for m, p in zip(modules, plain)] + list(got)
+
+
+def _own_blocks(layer):
+    """Whether the layer's blocks are SwinLayer's: a caller may have replaced ``block_forward``."""
+    return getattr(type(layer), "block_forward", None) is SwinLayer.block_forward and "block_forward" not in layer.__dict__
 
 
 class SwinLayer(nn.Module):
@@ -344,24 +379,17 @@ class SwinLayer(nn.Module):
         return (0, 0)
 
     def modulations(self):
-        """The parameters (w0, b0, w2, b2) of every block's modulation MLP, for ops.modulation_mlps."""
+        """Every block's modulation module, for ``_modulation_vectors``."""
         if not self.opts.mod_ways:
             return []
-        return [_mlp_params(block._modules["4"].modulation) for block in self.modulelist._modules.values()]
+        return [block._modules["4"] for block in self.modulelist._modules.values()]
 
-    def norm_dtype(self):
-        return self.modulelist[0][0].weight.dtype
+    def block_calls(self, x, mods, shift):
+        """What ``_run_blocks`` needs of all blocks; ``mods``: their modulation vectors, f32 [1 | b, 2*ways*d]."""
+        blocks = self.modulelist._modules.values()
+        return [self._block_call(block, x, mods[j] if mods else None, shift) for j, block in enumerate(blocks)]
 
-    def block_records(self, x, mods, shift, norm_dtype):
-        """(records, one-kernel flags) of all blocks for ``run_blocks``; ``mods``: their modulation vectors, f32 [1 | b, 2*ways*d]."""
-        records, fused = [], []
-        for j, block in enumerate(self.modulelist._modules.values()):
-            r, f = self._record(block, x, mods[j] if mods else None, shift, norm_dtype)
-            records.append(r)
-            fused.append(f)
-        return records, fused
-
-    def _record(self, block, x, m, shift, norm_dtype):
+    def _block_call(self, block, x, m, shift):
         o = self.opts
         n1, attn, n2, ff = list(block._modules.values())[:4]
         b, _, d = x.shape
@@ -378,6 +406,10 @@ class SwinLayer(nn.Module):
         sub = attn._modules
         (qkv_w, qkv_b), (wo_w, wo_b) = _weight_bias(sub["to_qkv"]), _weight_bias(sub["wo"])
         (n1_w, n1_b), (n2_w, n2_b) = _weight_bias(n1), _weight_bias(n2)
+        norm_dtype = n1_w.dtype
+        if n2_w.dtype is not norm_dtype:  # the call takes one type for both: the wider holds either exactly
+            norm_dtype = torch.float32
+            n1_w, n1_b, n2_w, n2_b = (None if v is None else v.float() for v in (n1_w, n1_b, n2_w, n2_b))
         hid = dn_w.shape[1]
         up_rows = 2 * hid if swiglu else hid
         fused = attn.fuse_qkv and ops.qkv_attention_supported(d, attn.heads, attn.head_dim, attn.window_size, attn.image_shape)
@@ -385,7 +417,8 @@ class SwinLayer(nn.Module):
         table = attn.relative_position_bias_table
         if table is not None:  # the one-kernel attention takes the table in its own form, the attention kernel as it is
             if fused:
-                b4_ptr = attn._bias4().data_ptr()
+                table = attn._bias4()
+                b4_ptr = table.data_ptr()
             else:
                 table_ptr = _vec_ptr(table, attn.table_rows * attn.heads)
         rec = ops.BLOCK_RECORD.pack(
@@ -393,17 +426,10 @@ class SwinLayer(nn.Module):
             _mat_ptr(qkv_w, 3 * inner, d), _vec_ptr(qkv_b, 3 * inner), _mat_ptr(wo_w, d, inner), _vec_ptr(wo_b, d),
             _mat_ptr(up_w, up_rows, d), _vec_ptr(up_b, up_rows), _mat_ptr(dn_w, d, hid), _vec_ptr(dn_b, d), table_ptr, b4_ptr, mod_ptr,
             mod_stride, shift[0], shift[1], attn.shift_mask and (shift[0] > 0 or shift[1] > 0), fused)
-        return rec, fused
-
-    def run_blocks(self, records, fused, norm_dtype, x, out):
-        """The blocks of ``records`` (this layer's, or several like layers') in one call: x -> out, then in place."""
-        o = self.opts
-        block = next(iter(self.modulelist._modules.values()))
-        _, attn, _, ff = list(block._modules.values())[:4]
-        hid = ff._modules["w2" if o.mlp == "swiglu" else "fc2"].weight.shape[1]
-        return ops.swin_blocks(records, x, out, self.image_shape, attn.heads, attn.head_dim, hid, self.window_size,
-                               norm_dtype=norm_dtype, norm=o.norm, mod_order=o.mod_order, mod_ways=o.mod_ways, mlp=o.mlp,
-                               eps=o.norm_eps, scale=attn.scale, shapes=fused)
+        config = (attn.image_shape, attn.heads, attn.head_dim, hid, attn.window_size, norm_dtype, o.norm, o.mod_order, o.mod_ways, o.mlp,
+                  o.norm_eps, attn.scale)
+        # a reparametrised module computes its weight at the access above: the call holds it until the kernels are launched
+        return BlockCall(rec, fused, config, (n1_w, n1_b, n2_w, n2_b, qkv_w, qkv_b, wo_w, wo_b, up_w, up_b, dn_w, dn_b, table, m))
 
     def block_forward(self, j, x, dt, shift, out=None, tap=None):
         """One block.  x is not modified; the result is written to ``out`` (allocated if None; may be x).
@@ -413,12 +439,11 @@ class SwinLayer(nn.Module):
         of shared scratch that the next block overwrites.
         """
         block = self.modulelist[j]
-        m = ops.modulation_mlps(dt.float().contiguous(), [_mlp_params(block[4].modulation)])[0] if self.opts.mod_ways else None
-        nd = self.norm_dtype()
-        rec, fused = self._record(block, x, m, shift, nd)
+        m = _modulation_vectors([block[4]], dt)[0] if self.opts.mod_ways else None
+        call = self._block_call(block, x, m, shift)
         if out is None:
             out = torch.empty_like(x)
-        a, h = self.run_blocks([rec], [fused], nd, x, out)
+        a, h = _run_blocks([call], x, out)
         if tap is not None:
             tap("attn", a, block)
             tap("hidden", h, block)
@@ -431,16 +456,15 @@ class SwinLayer(nn.Module):
         if x.dtype not in (torch.bfloat16, torch.float32):
             raise TypeError("x must be bf16 or f32")
         x = x.contiguous()
-        if tap is not None:
+        if tap is not None or not _own_blocks(self):
             for j in range(self.sublayers):
                 x = self.block_forward(j, x, dt, shift, tap=tap)
             return x
         if self.sublayers == 0:
             return x
-        mods = ops.modulation_mlps(dt.float().contiguous(), self.modulations()) if self.opts.mod_ways else None
+        calls = self.block_calls(x, _modulation_vectors(self.modulations(), dt), shift)
         out = torch.empty_like(x)
-        nd = self.norm_dtype()
-        self.run_blocks(*self.block_records(x, mods, shift, nd), nd, x, out)
+        _run_blocks(calls, x, out)
         return out
 
 
@@ -601,26 +625,35 @@ class LocalAERIS(nn.Module):
         tok, t = self.input_stage(x, dt, out_dtype=self.residual_dtype, cond=cond, x_div=x_div)
         if block_hook is not None:
             block_hook(0, tok)
-        # every modulation MLP of the model depends on the noise level alone: two launches for all of them
-        mods = ops.modulation_mlps(t, [p for layer in self.layers for p in layer.modulations()] +
-                                   [_mlp_params(self.output_stage.modulation)])
+        layers = list(self.layers)
         half = (self.window_size[0] // 2, self.window_size[1] // 2)
-        records, fused, k = [], [], 0
-        nd = self.layers[0].norm_dtype() if len(self.layers) and self.layers[0].sublayers else None
-        for i, layer in enumerate(self.layers):
-            shift = half if i % 2 == 1 else (0, 0)  # model.py:471-475, folded into the attention kernel
-            n_mod = layer.sublayers if self.opts.mod_ways else 0
-            r, f = layer.block_records(tok, mods[k:k + n_mod], shift, nd)
-            k += n_mod
-            records += r
-            fused += f
-        if records and block_hook is None:
-            self.layers[0].run_blocks(records, fused, nd, tok, tok)
-        elif records:
-            for j in range(len(records)):
-                self.layers[0].run_blocks(records[j:j + 1], fused[j:j + 1], nd, tok, tok)
-                block_hook(j + 1, tok)
-        out = self.output_stage(tok, t, mods[-1])
+        shifts = [half if i % 2 == 1 else (0, 0) for i in range(len(layers))]  # model.py:471-475, folded into the attention kernel
+        if all(map(_own_blocks, layers)):
+            # every modulation MLP of the model depends on the noise level alone: two launches for all of them
+            modules = [m for layer in layers for m in layer.modulations()]
+            own_end = type(self.output_stage) is OutputStage
+            mods = _modulation_vectors(modules, t, [_mlp_params(self.output_stage.modulation)] if own_end else [])
+            calls, k = [], 0
+            for layer, shift in zip(layers, shifts):
+                n_mod = len(layer.modulations())
+                calls += layer.block_calls(tok, mods[k:k + n_mod], shift)
+                k += n_mod
+            if block_hook is None:
+                _run_blocks(calls, tok, tok)
+            else:
+                for j, call in enumerate(calls):
+                    _run_blocks([call], tok, tok)
+                    block_hook(j + 1, tok)
+            out = self.output_stage(tok, t, m=mods[-1]) if own_end else self.output_stage(tok, t)
+        else:
+            k = 0
+            for layer, shift in zip(layers, shifts):
+                for j in range(layer.sublayers):
+                    tok = layer.block_forward(j, tok, t, shift)
+                    k += 1
+                    if block_hook is not None:
+                        block_hook(k, tok)
+            out = self.output_stage(tok, t)
         return (out, tok) if return_hidden else out
 
 

@@ -469,8 +469,8 @@ BLOCK_RECORD = struct.Struct("=15Q5q")  # struct aeris_block of include/aeris_hi
 BLOCK_CONFIG = struct.Struct("=15q2d")  # struct aeris_block_config
 
 
-def swin_blocks(records, x: torch.Tensor, out: torch.Tensor, image_shape, heads: int, head_dim: int, hidden: int, window_size, *,
-                norm_dtype, norm: str, mod_order: str, mod_ways: int, mlp: str, eps: float, scale: float, shapes):
+def swin_blocks(records, x: torch.Tensor, out: torch.Tensor, image_shape, heads: int, head_dim: int, hidden: int, window_size,
+                norm_dtype, norm: str, mod_order: str, mod_ways: int, mlp: str, eps: float, scale: float, *, shapes):
     """n Swin blocks in one call (aeris_blocks_fwd): x [B, n, d] (bf16 | f32) -> out (may be x; same shape and dtype).
     ``records``: one packed BLOCK_RECORD per block; ``shapes``: per block whether it runs the one-kernel attention (what the
     scratch buffers and the timing records follow)."""

@@ -8,6 +8,7 @@ import math
 
 import pytest
 import torch
+import torch.nn.utils.parametrize
 
 import oracle
 from oracle import OracleConfig
@@ -393,3 +394,51 @@ def test_bench_json_contract_on_a_small_workload(pkg, cuda, monkeypatch, capsys)
         assert rf["bound"] in ("hbm", "mfma") and abs(rf["frac"] - rf["achieved"] / rf["peak"]) < 1e-9
     for k in r["kernels"].values():
         assert k["launches_per_step"] >= 1 and k["avg_ms"] > 0
+
+
+class _Copy(torch.nn.Module):
+    def forward(self, w):
+        return w.clone()
+
+
+def test_block_call_follows_the_modules_it_is_made_of(pkg, cuda):
+    """One native call for a layer's blocks reads what every block's own modules say: weights that a parametrisation computes
+    at the access, a softmax scale of one block, gains of another type than their neighbours', a hooked or replaced
+    modulation, an overridden block_forward."""
+    cfg = OracleConfig.ref(**CONFIG0, sublayers=2)
+    g = torch.Generator().manual_seed(3)
+    x, t = torch.randn(1, 2048, 128, generator=g).to(cuda), torch.randn(1, 128, generator=g).to(cuda)
+
+    def layer(cls=pkg.SwinLayer, sublayers=2):
+        torch.manual_seed(1)
+        return cls(None, cfg.dim, cfg.heads, cfg.head_dim, cfg.mlp_dim, cfg.window_size, cfg.image_shape, False, 10_000,
+                   sublayers=sublayers).to(torch.bfloat16).to(cuda)
+
+    want = layer()(x, t)
+    p = layer()
+    for block in p.modulelist:
+        for mod in (block[1].to_qkv, block[1].wo, block[3].w1, block[3].w2):
+            torch.nn.utils.parametrize.register_parametrization(mod, "weight", _Copy())
+    assert torch.equal(p(x, t), want)
+    p = layer()
+    p.modulelist[0][2].float()
+    p.modulelist[1][0].float()
+    assert torch.equal(p(x, t), want)
+    # one block with a scale of its own: as block by block
+    p = layer()
+    p.modulelist[1][1].scale *= 2.0
+    one = p.block_forward(0, x, t, (0, 0))
+    assert torch.equal(p(x, t), p.block_forward(1, one, t, (0, 0))) and not torch.equal(p(x, t), want)
+    p = layer()
+    p.modulelist[1][4].register_forward_hook(lambda mod, args, out: out * 0)
+    q = layer()
+    q.modulelist[1][4].modulation[2].weight.data.zero_()
+    q.modulelist[1][4].modulation[2].bias.data.zero_()
+    assert torch.equal(p(x, t), q(x, t)) and not torch.equal(p(x, t), want)
+
+    class Doubled(pkg.SwinLayer):
+        def block_forward(self, *args, **kw):
+            return 2 * super().block_forward(*args, **kw)
+
+    one = 2 * layer().block_forward(0, x, t, (0, 0))
+    assert torch.equal(layer(Doubled)(x, t), 2 * layer().block_forward(1, one, t, (0, 0)))

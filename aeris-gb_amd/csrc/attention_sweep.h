@@ -82,26 +82,33 @@ struct LoadVPlain {
 // Start values and mask of the logits of one query group.  The bias table lies in LDS as fp32 4-vectors
 // R4[s] = (R[s..s+3]), R reversed and multiplied by log2 e, so that the biases of 4 consecutive keys are one
 // ds_read_b128 at index sp(query) + qt(first key), read straight into the accumulators of K Q^T before its MFMAs:
-// the bias costs neither an add nor a zero-fill.  The cyclic-shift mask is computed from the window position (only
-// windows on the wrapped border of a shifted grid carry more than one region; -100 across regions); keys past the
-// window (windows whose token count is not a multiple of 32) get -inf.
+// the bias costs neither an add nor a zero-fill.  The index is a part of the lane's own plus a part that is a constant once kb
+// is one (the unrolled sweep): a per-lane base address and an immediate offset, no arithmetic per key group.  (Per-lane key
+// divisions instead, and whole padded key blocks below: 12x12 windows, 64800 tokens x 8 heads of 64 64.9 us, shifted 72.0; so
+// 62.5 and 65.1.  8 heads of 32 49.7 -> 42.5 us, 51840 tokens x 5 heads of 64 37.5 -> 35.0 us.)
+// The cyclic-shift mask is computed from the window position (only windows on the wrapped border of a shifted grid carry
+// more than one region; -100 across regions); keys past the window (windows whose token count is not a multiple of 32)
+// get -inf.
 template <int WS_Y, int WS_X, bool HAS_BIAS>
 struct WindowLogits {
   static constexpr int L = WS_Y * WS_X, LPAD = (L + 31) / 32 * 32, TBL = (2 * WS_Y - 1) * (2 * WS_X - 1);
   static constexpr float MASK_NEG = -100.0f * 1.4426950408889634f;  // the additive -100, in the exp2 domain
-  const unsigned char* sB;
-  const unsigned char* sB_lane;  // sB + (sp + 4 hi) * 16: the lane's part of every bias vector address
-  int sp, hi;
+  static_assert(WS_X % 4 == 0 && L % 16 == 0, "4 consecutive keys lie in one window row, 8 and 16 inside or outside the window");
+  // the lane's part of a bias vector's address: its upper half's keys are 4 further on, in the same window row or at the
+  // start of the next one (table rows are 2 WS_X - 1 entries: WS_X + 3 further)
+  const unsigned char *sB_same, *sB_next;
+  int hi;
   bool my, mx;
   int ry_q, rx_q, sy, sx;
 
   // qpos: the lane's query position in the window (already clamped to L - 1); my / mx: the window lies on the wrapped
   // border in y / x and the mask is on
   __device__ __forceinline__ WindowLogits(const unsigned char* bias_lds, int qpos, int hi_, bool my_, bool mx_, int sy_, int sx_)
-      : sB(bias_lds), hi(hi_), my(my_), mx(mx_), sy(sy_), sx(sx_) {
+      : hi(hi_), my(my_), mx(mx_), sy(sy_), sx(sx_) {
     const int qiy = qpos / WS_X, qix = qpos % WS_X;
-    sp = (TBL - 1) - (qiy + WS_Y - 1) * (2 * WS_X - 1) - qix - (WS_X - 1);
-    sB_lane = sB + (sp + 4 * hi) * 16;
+    const int sp = (TBL - 1) - (qiy + WS_Y - 1) * (2 * WS_X - 1) - qix - (WS_X - 1);
+    sB_same = bias_lds + (sp + 4 * hi) * 16;
+    sB_next = bias_lds + (sp + (WS_X + 3) * hi) * 16;
     ry_q = my ? (qiy < WS_Y - sy ? 1 : 2) : 0;
     rx_q = mx ? (qix < WS_X - sx ? 1 : 2) : 0;
   }
@@ -109,20 +116,10 @@ struct WindowLogits {
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       f32x4 bv = {0.f, 0.f, 0.f, 0.f};
-      if (HAS_BIAS) {
-        if (WS_X % 8 == 0 && LPAD == L) {
-          // the lane's 4 keys start at column (8-aligned part) + 4 hi of their window row and never cross into the next
-          // row: the index is the lane's own part, sp + 4 hi, plus a part that is a constant once kb is one (the
-          // unrolled sweep): a per-lane base address and an immediate offset, no arithmetic per key group
-          const int base = kb * 32 + g * 8;
-          const int qt0 = (base / WS_X) * (2 * WS_X - 1) + (base % WS_X);
-          bv = *reinterpret_cast<const f32x4*>(sB_lane + qt0 * 16);
-        } else {
-          const int key0 = kb * 32 + g * 8 + hi * 4;
-          const int kk = ((LPAD == L) || key0 < L) ? key0 : 0;
-          const int qt = (kk / WS_X) * (2 * WS_X - 1) + (kk % WS_X);
-          bv = *reinterpret_cast<const f32x4*>(sB + (sp + qt) * 16);
-        }
+      const int base = kb * 32 + g * 8;
+      if (HAS_BIAS && (LPAD == L || base < L)) {
+        const int qt0 = (base / WS_X) * (2 * WS_X - 1) + (base % WS_X);
+        bv = *reinterpret_cast<const f32x4*>((base % WS_X + 4 < WS_X ? sB_same : sB_next) + qt0 * 16);
       }
 #pragma unroll
       for (int i = 0; i < 4; ++i) a[g * 4 + i] = bv[i];
@@ -130,38 +127,26 @@ struct WindowLogits {
   }
   __device__ __forceinline__ void mask_block(int kb, f32x16& a) const {
     if (my || mx) {
-      if (WS_X % 8 == 0 && LPAD == L) {
-        // as in init_acc: the lane's 4 keys of a group lie in one window row, whose number is a constant once kb is; what
-        // depends on the lane is whether column (8-aligned part) + 4 hi + i has wrapped around, one compare per key
-        const int h4 = 4 * hi;
+      // as in init_acc: the lane's 4 keys of a group lie in one window row; where and in which row its upper half's lie is
+      // known once kb is.  What depends on the lane is whether column (first key's) + i has wrapped around.
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const int base = kb * 32 + g * 8;
-          const int kiy = base / WS_X, cx0 = base % WS_X;
-          const bool ydiff = my && ((kiy < WS_Y - sy) != (ry_q == 1));
+      for (int g = 0; g < 4; ++g) {
+        const int base = kb * 32 + g * 8, cx0 = base % WS_X;
+        if (LPAD != L && base >= L) break;
+        const bool next = cx0 + 4 >= WS_X;
+        const int kiy = base / WS_X + (next ? hi : 0), dx = next ? -cx0 * hi : 4 * hi;
+        const bool ydiff = my && ((kiy < WS_Y - sy) != (ry_q == 1));
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const bool xdiff = mx && ((h4 < WS_X - sx - i - cx0) != (rx_q == 1));
-            if (ydiff || xdiff) a[g * 4 + i] += MASK_NEG;
-          }
+        for (int i = 0; i < 4; ++i) {
+          const bool xdiff = mx && ((dx < WS_X - sx - i - cx0) != (rx_q == 1));
+          if (ydiff || xdiff) a[g * 4 + i] += MASK_NEG;
         }
-      } else {
-#pragma unroll
-        for (int g = 0; g < 4; ++g)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int key = kb * 32 + g * 8 + hi * 4 + i;
-            const int kiy = key / WS_X, kix = key % WS_X;
-            const int ry_k = my ? (kiy < WS_Y - sy ? 1 : 2) : 0;
-            const int rx_k = mx ? (kix < WS_X - sx ? 1 : 2) : 0;
-            if (ry_k != ry_q || rx_k != rx_q) a[g * 4 + i] += MASK_NEG;
-          }
       }
     }
     if (LPAD != L) {
 #pragma unroll
       for (int g = 0; g < 4; ++g)
-        if (kb * 32 + g * 8 + hi * 4 >= L) {
+        if (kb * 32 + g * 8 >= L) {
 #pragma unroll
           for (int i = 0; i < 4; ++i) a[g * 4 + i] = -INFINITY;
         }
@@ -192,9 +177,12 @@ __device__ __forceinline__ void build_bias_lds(unsigned char* sB, const uint16_t
 // from LDS two blocks ahead, V^T fragments one block ahead.  Without a bias the first MFMA of an S^T block takes a
 // literal zero as its C operand, and so does the first one of O^T: no accumulator is zero-filled by the VALU.
 // `mid(kb)` is called at the start of key block kb (a hook for work a kernel wants issued inside the sweep).
+// Of a last key block that is half outside the window only the half inside is exponentiated and multiplied by V (whose tile
+// then needs no rows past the window; K rows past it may hold anything).
 template <int NQ, int KS, int DB, bool HAS_BIAS, class Logits, class LoadK, class LoadV, class Mid>
 __device__ __forceinline__ void attention_sweep(const Logits& lg, const LoadK& load_k, const LoadV& load_v, const Mid& mid,
                                                 const bf16x8 (&qf)[KS], f32x16 (&o)[DB], float& sum) {
+  constexpr int L = Logits::L;
   {
     const f32x16 zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     f32x16 acc2[2];
@@ -225,8 +213,9 @@ __device__ __forceinline__ void attention_sweep(const Logits& lg, const LoadK& l
       // falls where only reads issued a block ago are outstanding, not on top of the V^T reads just issued
       if (kb + 1 < NQ) qk_block(acc2[(kb + 1) & 1], kf[(kb + 1) & 1]);
       __builtin_amdgcn_sched_barrier(0);
+      const bool both = kb * 32 + 16 < L;  // whether the block's upper 16 keys are inside the window
       load_v(2 * kb, vraw[0]);
-      load_v(2 * kb + 1, vraw[1]);
+      if (both) load_v(2 * kb + 1, vraw[1]);
       // Keep every accumulator of the S^T block just issued live across these reads.  Where the compiler can prove part
       // of it unused (keys past the window become -inf whatever the MFMA wrote) it would hand those registers to the
       // V^T reads, and it places no wait between an MFMA still writing a register and an assembly read returning into
@@ -236,18 +225,19 @@ __device__ __forceinline__ void attention_sweep(const Logits& lg, const LoadK& l
       if (kb + 2 < NQ) load_k(kb + 2, kf[kb & 1]);
       lg.mask_block(kb, a);
 #pragma unroll
-      for (int h = 0; h < 8; ++h) {
+      for (int h = 0; h < (both ? 8 : 4); ++h) {
         const float e0 = __builtin_amdgcn_exp2f(a[2 * h]);
         const float e1 = __builtin_amdgcn_exp2f(a[2 * h + 1]);
         pk[h] = pack_bf16x2(e0, e1);
         sum = dot2_ones(pk[h], sum);  // the row sum of what PV multiplies: the rounded values
       }
       __builtin_amdgcn_sched_barrier(0);
-      load_v.ready(vraw[0], vraw[1], vf[0], vf[1]);
+      if (both) load_v.ready(vraw[0], vraw[1], vf[0], vf[1]);
+      else load_v.ready(vraw[0], vf[0]);
       // the accumulators of block kb are consumed: the bias of block kb + 2 goes straight into them
       if (HAS_BIAS && kb + 2 < NQ) lg.init_acc(kb + 2, a);
 #pragma unroll
-      for (int t2 = 0; t2 < 2; ++t2) {
+      for (int t2 = 0; t2 < (both ? 2 : 1); ++t2) {
         const u32x4 pw = {pk[4 * t2], pk[4 * t2 + 1], pk[4 * t2 + 2], pk[4 * t2 + 3]};
         const bf16x8 pf = __builtin_bit_cast(bf16x8, pw);
 #pragma unroll
@@ -286,6 +276,7 @@ __device__ __forceinline__ void attention_sweep(const Logits& lg, const LoadK& l
         } else {
 #pragma unroll
           for (int t2 = 0; t2 < 2; ++t2) {
+            if (L % 32 != 0 && kb * 32 + 16 * t2 >= L) break;
             bf16x8 vf[DB];
             typename LoadV::Raw vraw[DB];
             load_v(2 * kb + t2, vraw);

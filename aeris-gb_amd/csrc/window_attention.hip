@@ -428,7 +428,7 @@ struct AttnPersistCfg {
   static constexpr int LPAD = NQ * 32;
   static constexpr int NT = NQ * 64;  // one wave per query group
   static constexpr int TBL = (2 * WS_Y - 1) * (2 * WS_X - 1);
-  static constexpr int KV_BYTES = LPAD * 128;
+  static constexpr int KV_BYTES = L * 128;  // a last key block that reaches past the K tile reads the V tile behind it
   static constexpr int SMEM = 4 * KV_BYTES + (HAS_BIAS ? TBL * 16 : 0);
 };
 
@@ -439,10 +439,11 @@ __global__ void __launch_bounds__(attn_persist_threads(WS_Y, WS_X))
 window_attention_persist_kernel(AttnParams p, int n_units) {
   using Cfg = AttnPersistCfg<WS_Y, WS_X, HAS_BIAS>;
   constexpr int HD = 64, KS = 4, DB = 2;
-  constexpr int L = Cfg::L, NQ = Cfg::NQ, LPAD = Cfg::LPAD, NT = Cfg::NT, TBL = Cfg::TBL, KVB = Cfg::KV_BYTES;
+  constexpr int L = Cfg::L, NQ = Cfg::NQ, NT = Cfg::NT, TBL = Cfg::TBL, KVB = Cfg::KV_BYTES;
   static_assert(WS_X % 4 == 0, "groups of 4 consecutive keys must stay inside one window row");
   constexpr float LOG2E = 1.4426950408889634f;
-  constexpr int DMA_PER_WAVE = (LPAD / 8 + NQ - 1) / NQ;  // instruction pairs (K, V) per wave and unit
+  static_assert(L % 8 == 0, "a load instruction fills 8 rows");
+  constexpr int DMA_PAIRS = L / 8, DMA_PER_WAVE = (DMA_PAIRS + NQ - 1) / NQ;  // instruction pairs (K, V) of a unit, of a wave
   typedef __attribute__((address_space(3))) void* lds_ptr;
   typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4_t;
   typedef __attribute__((address_space(3))) bf16x4_t* lds_bf16x4_ptr;
@@ -543,12 +544,12 @@ window_attention_persist_kernel(AttnParams p, int n_units) {
   // load number idx of the prepared unit -> buffer set `set`: pair idx / 2 (rows 8 ii .. 8 ii + 7), K for even idx, V for odd
   auto kv_issue = [&](int idx, int set) {
     const int j = idx >> 1, is_v = idx & 1;
-    const int ii = wave + j * NQ;  // the pairs divide evenly among the waves for every window built here
+    const int ii = wave + j * NQ;
+    if (DMA_PAIRS % NQ != 0 && ii >= DMA_PAIRS) return;  // wave-uniform
     const int key = ii * 8 + rsub;
     uint32_t off = kv_base + (is_v ? kv_relv[j] : kv_relk[j]);
     if (kv_wraps)  // wave-uniform: windows on the wrapped border of a shifted grid
-      off = token_row(kv_unit, key < L ? key : 0) * (ld_qkv * 2u) + (uint32_t)((pc ^ (is_v ? 2 * (key & 3) : (key >> 1) & 7)) << 4);
-    if (LPAD != L && key >= L) off = 0xFFFFFFF0u;  // outside the descriptor: arrives as zeros
+      off = token_row(kv_unit, key) * (ld_qkv * 2u) + (uint32_t)((pc ^ (is_v ? 2 * (key & 3) : (key >> 1) & 7)) << 4);
     unsigned char* dst = smem + set * 2 * KVB + is_v * KVB + ii * 1024;
     __builtin_amdgcn_raw_ptr_buffer_load_lds(is_v ? kv_rs_v : kv_rs_k, (lds_ptr)dst, 16, off, 0, 0, 0);
   };
@@ -569,7 +570,6 @@ window_attention_persist_kernel(AttnParams p, int n_units) {
   };
 
   const float cq = p.scale * LOG2E;
-  constexpr float MASK_NEG = -100.0f * LOG2E;
 
   // A load instruction holds its wave until the CU's one address unit has taken its 64 addresses, and with all waves
   // issuing their share of the next unit together right after the barrier nothing computes meanwhile.  The upper half
@@ -584,7 +584,6 @@ window_attention_persist_kernel(AttnParams p, int n_units) {
   int bias_head = cur.head;
   bf16x8 q_cur[KS], q_nxt[KS];
   uint32_t tok_cur, tok_nxt = 0;
-  static_assert((LPAD / 8) % NQ == 0, "the load pairs must divide evenly among the waves");
   load_q(cur, q_cur, tok_cur);
   kv_prepare(cur);
 #pragma unroll

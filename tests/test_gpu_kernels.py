@@ -521,6 +521,8 @@ NONFINITE_CASES = [
     ("one_unit_dma", 3, 32, 48, 2, 64, 16, 8, True, True),
     ("register_staged_rows", 1, 48, 64, 3, 64, 16, 8, True, False),
     ("register_staged_hd32", 1, 32, 64, 4, 32, 8, 4, True, True),
+    ("persistent_half_block", 2, 96, 96, 8, 64, 12, 6, True, True),  # 144 keys: half of the last key block is outside the window
+    ("one_unit_dma_half_block", 1, 36, 60, 4, 64, 12, 6, True, True),
     ("streaming_rows", 2, 40, 60, 3, 64, 20, 10, False, False),
     ("streaming_planes_hd128", 1, 120, 120, 2, 128, 60, 30, False, True),
 ]
@@ -576,7 +578,7 @@ def test_window_attention_streaming_rejects_bias_and_mask(pkg, cuda):
     assert e.value.code == -2
 
 
-@pytest.mark.parametrize("geo", [(2, 32, 64, 8, 4), (1, 36, 60, 12, 6), (1, 48, 80, 16, 8), (1, 32, 32, 16, 0)])
+@pytest.mark.parametrize("geo", [(2, 32, 64, 8, 4), (1, 36, 60, 12, 6), (4, 96, 108, 12, 6), (1, 48, 80, 16, 8), (1, 32, 32, 16, 0)])
 @pytest.mark.parametrize("disp", [(0, 0), (0, -1), (1, 0), (-2, 3)])
 def test_attention_index_map_bit_exact(pkg, cuda, geo, disp):
     """q = k = 0 and a bias table that is 0 at one displacement and -30000 elsewhere make every query copy the

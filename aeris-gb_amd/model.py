@@ -326,10 +326,15 @@ def _mlp_params(modulation: nn.Sequential):
     return *_weight_bias(l0), *_weight_bias(l2)
 
 
+def _plain(module, cls):
+    """Whether the module is ``cls`` as it is: no forward of its own, nothing hooked to its inputs or results."""
+    return type(module) is cls and "forward" not in module.__dict__ and not (module._forward_hooks or module._forward_pre_hooks)
+
+
 def _modulation_vectors(modules, dt, extra=()):
     """f32 [1 | b, N_i] of each modulation module on the noise-level embedding dt, and of the MLPs ``extra`` (parameter
     tuples): two launches for all of them, but what a caller has hooked or put in a module's place is called as a module."""
-    plain = [type(m) is ModulationLinear and not m._forward_hooks and not m._forward_pre_hooks for m in modules]
+    plain = [_plain(m, ModulationLinear) for m in modules]
     mlps = [_mlp_params(m.modulation) for m, p in zip(modules, plain) if p] + list(extra)
     got = iter(ops.modulation_mlps(dt.float().contiguous(), mlps) if mlps else ())
     return [next(got) if p else m(dt) for m, p in zip(modules, plain)] + list(got)
@@ -631,7 +636,7 @@ class LocalAERIS(nn.Module):
         if all(map(_own_blocks, layers)):
             # every modulation MLP of the model depends on the noise level alone: two launches for all of them
             modules = [m for layer in layers for m in layer.modulations()]
-            own_end = type(self.output_stage) is OutputStage
+            own_end = _plain(self.output_stage, OutputStage)
             mods = _modulation_vectors(modules, t, [_mlp_params(self.output_stage.modulation)] if own_end else [])
             calls, k = [], 0
             for layer, shift in zip(layers, shifts):

@@ -181,6 +181,23 @@ def test_output_stage_alone(pkg, cuda, preset, x_dtype):
     assert e <= 2e-5, e
 
 
+def test_model_calls_a_hooked_or_replaced_output_stage(pkg, cuda):
+    """The model computes the output stage's modulation with its blocks' only where the stage is as the package makes it: a
+    noise-level embedding changed by a hook, or a forward of the caller's, is what counts otherwise."""
+    cfg, sd, model = _stage_model(pkg, cuda, "ref")
+    g = torch.Generator().manual_seed(6)
+    x, t = torch.randn(1, 32 * 64, 138, generator=g).to(cuda), torch.tensor([0.4], device=cuda)
+    seen = []
+    stage = model.output_stage
+    with stage.register_forward_pre_hook(lambda mod, args: (args[0], args[1] * 0)):
+        got = model(x, t)
+    plain = stage.forward
+    stage.forward = lambda tok, dt: seen.append(1) or plain(tok, dt * 0)
+    assert torch.equal(model(x, t), got) and seen
+    del stage.forward
+    assert not torch.equal(model(x, t), got)
+
+
 @pytest.mark.parametrize("case", [
     # B, S, d, N, kind, x dtype, modulation rows, row mean
     (1, 1000, 1536, 69, "layernorm", torch.float32, 1, 0.0),    # ragged row count (1000 = 15 tiles + 40 rows)

@@ -21,7 +21,7 @@
 //                 wave has its Q fragments.  K must be even for that (the last k-tile then uses A1).
 //   bias          the head's relative-position bias as fp32 4-vectors (WindowLogits), prepared once per parameter value
 //                 by qkv_attention_bias_kernel, brought in by the load unit during the main loop
-// Units are walked in groups of 4 windows x all heads, so that a window's token rows and a head's weight rows are
+// Units are walked in groups of 4 (2, 1: few windows, see the launch) windows x all heads, so that a window's token rows and a head's weight rows are
 // shared in one XCD's L2; the groups are dealt to the 8 XCDs in turn (group g to XCD g % 8) and the units of an XCD's
 // groups to its workgroups in turn, which spreads the windows on the wrapped border of a shifted grid - a whole
 // window row, slower than the others by their mask arithmetic - evenly over XCDs and workgroups.
@@ -47,7 +47,7 @@ constexpr int QA_TBL = (2 * QA_WS - 1) * (2 * QA_WS - 1);
 constexpr int QA_BIAS_BYTES = 16384;                 // 961 x 16 B = 15 376, rounded up to whole 1 KB load instructions
 constexpr int QA_SPARE_OFF = QA_BIAS_OFF + QA_BIAS_BYTES;
 constexpr int QA_SMEM = QA_SPARE_OFF + 8192;         // 160 KB
-constexpr int QA_GM = 4;                             // windows per L2 group
+constexpr int QA_GM_SHIFT = 2;                       // log2 of the windows per L2 group, at most
 static_assert(QA_SMEM == 160 * 1024, "the layout fills the CU's LDS exactly");
 static_assert(QA_TBL * 16 <= QA_BIAS_BYTES, "bias table fits its slot");
 
@@ -63,6 +63,7 @@ struct QkvAttnParams {
   int use_mask;
   float q_scale;          // softmax scale times log2(e)
   int n_win, bpx;         // windows (B * nWy * nWx); workgroups per XCD
+  int gm_shift;           // log2 of the windows per L2 group
   // ceil(2^40 / d) for d = units per group, windows per image, windows per row: n / d = (n * m) >> 40 for n < 2^24.
   // A unit is decoded several times per unit and wave; as true divisions that was 40 % of the kernel's vector ALU work.
   uint64_t m_gsz, m_wpi, m_nwx;
@@ -97,13 +98,13 @@ __global__ void __launch_bounds__(QA_NT) qkv_window_attention_kernel(QkvAttnPara
 
   // ---- this workgroup's unit list: XCD x (workgroup id & 7: consecutive workgroups go to consecutive XCDs) owns the
   // groups x, x + 8, ...; its workgroup `slot` takes the units slot, slot + bpx, ... of those groups laid end to end.
-  // Only the very last group can be short (fewer than QA_GM windows) and it ends its XCD's sequence.
+  // Only the very last group can be short (fewer windows than the others) and it ends its XCD's sequence.
   const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-  const int gsz = QA_GM * p.heads;
-  const int n_groups = (p.n_win + QA_GM - 1) / QA_GM;
+  const int full = 1 << p.gm_shift, gsz = p.heads << p.gm_shift;
+  const int n_groups = (p.n_win + full - 1) >> p.gm_shift;
   const int my_groups = n_groups > xcd ? (n_groups - xcd + 7) / 8 : 0;
   int seq_len = my_groups * gsz;
-  if (my_groups > 0 && (my_groups - 1) * 8 + xcd == n_groups - 1) seq_len -= (n_groups * QA_GM - p.n_win) * p.heads;
+  if (my_groups > 0 && (my_groups - 1) * 8 + xcd == n_groups - 1) seq_len -= ((n_groups << p.gm_shift) - p.n_win) * p.heads;
   const int n_my = seq_len > slot ? (seq_len - slot + p.bpx - 1) / p.bpx : 0;
   if (n_my == 0) return;
   struct Unit { int head, b, wy, wx; };
@@ -111,12 +112,11 @@ __global__ void __launch_bounds__(QA_NT) qkv_window_attention_kernel(QkvAttnPara
     const int t = r * p.bpx + slot;
     const int lg = div_by_magic(t, p.m_gsz), within = t - lg * gsz;
     const int g = lg * 8 + xcd;
-    int gm = p.n_win - g * QA_GM;
-    if (gm > QA_GM) gm = QA_GM;
+    int gm = p.n_win - (g << p.gm_shift);
+    if (gm > full) gm = full;
     Unit u;
-    static_assert(QA_GM == 4, "the shift below");
-    u.head = gm == QA_GM ? within >> 2 : within / gm;  // only the very last group can be short
-    const int win = g * QA_GM + (within - u.head * gm);
+    u.head = gm == full ? within >> p.gm_shift : within / gm;  // only the very last group can be short
+    const int win = (g << p.gm_shift) + (within - u.head * gm);
     const int wpi = p.nWy * p.nWx;
     u.b = div_by_magic(win, p.m_wpi);
     const int wrem = win - u.b * wpi;
@@ -547,10 +547,22 @@ hipError_t qkv_attention_launch(const void* y, const void* w, const void* bias, 
   p.use_mask = use_mask;
   p.q_scale = scale * 1.4426950408889634f;
   p.n_win = B * p.nWy * p.nWx;
-  const int max_seq = ((p.n_win + QA_GM - 1) / QA_GM + 7) / 8 * QA_GM * heads;  // units of the XCD with the most groups
   if ((int64_t)p.n_win * heads >= (1 << 24)) return hipErrorInvalidValue;  // the range of div_by_magic
+  // Whole groups go to an XCD: with few of them the XCD with one more than the others works on alone.  Groups of 2 windows or
+  // of 1 where its 32 CUs then have at least a sixteenth fewer rounds of units; 4, which read the least into L2, otherwise.
+  // Groups of 4 -> by this rule, 24 heads, K 1536: 12 windows 98 -> 64 us, 72 windows 278 -> 237, 100 windows 364 -> 328; 36
+  // windows x 16 heads, K 1024: 92 -> 76, 39 windows 92 -> 78.  (1000 windows, 96 rounds -> 94 with groups of 1: 3138 -> 3184 us, hence the sixteenth.)
+  auto units = [&](int shift) {  // of the XCD with the most windows: the short last group counts where it alone is one more
+    const int groups = (p.n_win + (1 << shift) - 1) >> shift, most = (groups + 7) / 8;
+    return ((most << shift) - (groups % 8 == 1 ? (groups << shift) - p.n_win : 0)) * heads;
+  };
+  auto rounds = [&](int shift) { return (units(shift) + 31) / 32; };
+  p.gm_shift = QA_GM_SHIFT;
+  for (int shift = QA_GM_SHIFT - 1; shift >= 0; --shift)
+    if (rounds(shift) * 16 <= rounds(p.gm_shift) * 15) p.gm_shift = shift;
+  const int max_seq = units(p.gm_shift);
   auto magic = [](int d) { return (((uint64_t)1 << 40) + (uint64_t)d - 1) / (uint64_t)d; };
-  p.m_gsz = magic(QA_GM * heads);
+  p.m_gsz = magic(heads << p.gm_shift);
   p.m_wpi = magic(p.nWy * p.nWx);
   p.m_nwx = magic(p.nWx);
   p.bpx = max_seq < 32 ? max_seq : 32;

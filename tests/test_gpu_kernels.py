@@ -459,6 +459,8 @@ FUSED_CASES = [
     (2, 96, 160, 6, 384, 8, True, False),      # two batch entries, 120 windows x 6 heads
     (1, 48, 80, 3, 256, 8, True, True),        # 15 windows (the last group of 4 is short), 4 k-tiles (the fewest), 45 units < 256 workgroups
     (1, 32, 32, 2, 640, 8, True, True),        # every window on the wrapped border; 8 units
+    (1, 48, 208, 16, 256, 8, True, True),      # 39 windows: groups of 2 (3 rounds of units on the busiest XCD instead of 4), the last one short
+    (1, 96, 192, 24, 256, 8, True, False),     # 72 windows: groups of 1 (7 rounds instead of 9)
 ]
 
 

@@ -477,6 +477,8 @@ def swin_blocks(records, x: torch.Tensor, out: torch.Tensor, image_shape, heads:
     _dev(x, "x")
     _dev(out, "out", x.dtype)
     B, n, d = x.shape
+    if n != image_shape[0] * image_shape[1]:  # the native call takes its sizes from B, H and W alone
+        raise RuntimeError(f"x has {n} tokens per batch entry, expected {image_shape[0]}*{image_shape[1]}")
     T, inner, dev = B * n, heads * head_dim, x.device
     requests = [("norm", (B, n, d), torch.bfloat16), ("attn", (T, inner), torch.bfloat16), ("hidden", (B, n, hidden), torch.bfloat16)]
     if not all(shapes):

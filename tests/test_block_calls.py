@@ -1,0 +1,50 @@
+"""What the Python side of the blocks hands to the native library, recorded on the CPU: nothing is launched, so the calls
+that must be refused ahead of a launch can be made here."""
+import pytest
+import torch
+
+
+class Calls(list):
+    """The native calls made, as (name, arguments)."""
+
+    def names(self):
+        return [c[0] for c in self]
+
+
+@pytest.fixture
+def calls(pkg, monkeypatch):
+    """CPU tensors pass for GPU tensors and native calls are recorded instead of made."""
+    seen = Calls()
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True)
+    monkeypatch.setattr(pkg._lib, "call", lambda name, *args: seen.append((name, args)))
+    monkeypatch.setattr(pkg.ops, "_stream", lambda: 0)
+    monkeypatch.setattr(pkg.ops, "workspaces", lambda device, *req: [torch.empty(s, dtype=t) for _, s, t in req])
+    return seen
+
+
+def layer_of(pkg, preset="ref", cls=None, **kw):
+    torch.manual_seed(1)
+    return (cls or pkg.SwinLayer)(None, 128, 2, 64, 256, (8, 8), (16, 32), False, 10_000, preset=preset, **kw).to(torch.bfloat16)
+
+
+def inputs(pkg, n=512, b=1, dtype=torch.float32, rows=1):
+    return torch.randn(b, n, 128).to(dtype), torch.randn(rows, 128)
+
+
+def model_of(pkg, layers=2, **kw):
+    return pkg.LocalAERIS(None, 2, 128, 64, 256, (8, 8), (16, 32), n_layers=layers + 2, model_in_channels=10, model_out_channels=4, **kw)
+
+
+@pytest.mark.parametrize("preset", ["ref", "spec"])
+@pytest.mark.parametrize("n", [64, 511, 513, 1024])
+def test_another_token_count_than_the_grid_is_refused(pkg, calls, preset, n):
+    layer = layer_of(pkg, preset)
+    x, t = inputs(pkg, n)
+    for run in (lambda: layer(x, t), lambda: layer.block_forward(0, x, t, (0, 0)), lambda: layer.block_forward(0, x, t, (0, 0), out=x.clone())):
+        with pytest.raises(RuntimeError, match="tokens"):
+            run()
+    with pytest.raises(RuntimeError, match="tokens"):
+        model_of(pkg)(torch.randn(1, n, 10), torch.zeros(1))
+    assert "aeris_blocks_fwd" not in calls.names()
+    layer(*inputs(pkg))
+    assert calls.names()[-1] == "aeris_blocks_fwd"

@@ -399,11 +399,7 @@ class SwinLayer(nn.Module):
         n1, attn, n2, ff = list(block._modules.values())[:4]
         b, _, d = x.shape
         inner = attn.heads * attn.head_dim
-        mod_ptr = mod_stride = 0
-        if m is not None:
-            if m.shape[1] != 2 * o.mod_ways * d or m.shape[0] not in (1, b):
-                raise RuntimeError(f"modulation must be [1 | {b}, {2 * o.mod_ways * d}], got {tuple(m.shape)}")
-            mod_ptr, mod_stride = m.data_ptr(), m.shape[1] if m.shape[0] > 1 else 0
+        mod_ptr, mod_stride = (0, 0) if m is None else ops._rowvec(m, "modulation", 2 * o.mod_ways * d, b)
         sub = ff._modules
         swiglu = o.mlp == "swiglu"
         (up_w, up_b), (dn_w, dn_b) = (_weight_bias(sub["w1"]), _weight_bias(sub["w2"])) if swiglu else (

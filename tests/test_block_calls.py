@@ -48,3 +48,41 @@ def test_another_token_count_than_the_grid_is_refused(pkg, calls, preset, n):
     assert "aeris_blocks_fwd" not in calls.names()
     layer(*inputs(pkg))
     assert calls.names()[-1] == "aeris_blocks_fwd"
+
+
+def modulation_of(pkg, calls, make):
+    """Address and row stride that the native call gets for a hooked modulation's result ``make(vectors)``, and that result."""
+    layer, kept = layer_of(pkg), []
+
+    def hook(module, args, out):
+        kept.append(make(out))
+        return kept[-1]
+    layer.modulelist[0][4].register_forward_hook(hook)
+    layer(*inputs(pkg, b=3, rows=3))
+    record = pkg.ops.BLOCK_RECORD.unpack(calls[-1][1][1])
+    return record[14:16], kept[0]
+
+
+@pytest.mark.parametrize("name,make", [
+    ("as_it_is", lambda m: m),
+    ("one_row", lambda m: m[:1].clone()),
+    ("row_expanded", lambda m: m[:1].expand(3, -1)),
+    ("columns_of_a_wider_matrix", lambda m: torch.randn(3, 1000)[:, 100:868]),
+    ("every_other_row", lambda m: torch.randn(6, 768)[::2]),
+])
+def test_modulation_is_read_with_its_own_rows(pkg, calls, name, make):
+    got, m = modulation_of(pkg, calls, make)
+    assert got == (m.data_ptr(), 0 if m.shape[0] == 1 else m.stride(0))
+
+
+@pytest.mark.parametrize("name,make", [
+    ("bf16", lambda m: m.to(torch.bfloat16)),
+    ("f64", lambda m: m.double()),
+    ("too_few_columns", lambda m: m[:, :640]),
+    ("two_rows_of_three", lambda m: m[:2]),
+    ("columns_strided", lambda m: torch.randn(3, 1536)[:, ::2]),
+])
+def test_modulation_of_another_form_is_refused(pkg, calls, name, make):
+    with pytest.raises(RuntimeError, match="modulation"):
+        modulation_of(pkg, calls, make)
+    assert "aeris_blocks_fwd" not in calls.names()

@@ -442,3 +442,26 @@ def test_block_call_follows_the_modules_it_is_made_of(pkg, cuda):
 
     one = 2 * layer().block_forward(0, x, t, (0, 0))
     assert torch.equal(layer(Doubled)(x, t), 2 * layer().block_forward(1, one, t, (0, 0)))
+
+
+def test_modulation_of_a_hook_with_other_strides(pkg, cuda):
+    """A hooked modulation's result counts as it lies in memory: an expanded row and rows or columns of a wider matrix give the
+    bits of their contiguous copies; a bf16 result and one in host memory are refused."""
+    cfg = OracleConfig.ref(**CONFIG0)
+    g = torch.Generator().manual_seed(3)
+    x, t = torch.randn(3, 2048, 128, generator=g).to(cuda), torch.randn(3, 128, generator=g).to(cuda)
+    torch.manual_seed(1)
+    layer = pkg.SwinLayer(None, cfg.dim, cfg.heads, cfg.head_dim, cfg.mlp_dim, cfg.window_size, cfg.image_shape, False,
+                          10_000).to(torch.bfloat16).to(cuda)
+    wide = torch.randn(6, 900, generator=g).to(cuda)
+    result = []
+    layer.modulelist[0][4].register_forward_hook(lambda mod, args, out: result[0])
+    for m in (wide[:1, :768].expand(3, -1), wide[:3, 100:868], wide[::2, 1:769], wide[2:3, 4:772]):
+        result[:] = [m]
+        got = layer(x, t)
+        result[:] = [m.contiguous()]
+        assert torch.equal(got, layer(x, t)) and torch.isfinite(got).all()
+    for m in (wide[:3, :768].to(torch.bfloat16), wide[:3, :768].cpu()):
+        result[:] = [m]
+        with pytest.raises(RuntimeError, match="modulation"):
+            layer(x, t)

@@ -456,7 +456,7 @@ def test_modulation_of_a_hook_with_other_strides(pkg, cuda):
     wide = torch.randn(6, 900, generator=g).to(cuda)
     result = []
     layer.modulelist[0][4].register_forward_hook(lambda mod, args, out: result[0])
-    for m in (wide[:1, :768].expand(3, -1), wide[:3, 100:868], wide[::2, 1:769], wide[2:3, 4:772]):
+    for m in (wide[:1, :768].expand(3, -1), wide[:3, 100:868], wide[::2, 4:772], wide[2:3, 8:776]):
         result[:] = [m]
         got = layer(x, t)
         result[:] = [m.contiguous()]

@@ -479,6 +479,8 @@ def swin_blocks(records, x: torch.Tensor, out: torch.Tensor, image_shape, heads:
     B, n, d = x.shape
     if n != image_shape[0] * image_shape[1]:  # the native call takes its sizes from B, H and W alone
         raise RuntimeError(f"x has {n} tokens per batch entry, expected {image_shape[0]}*{image_shape[1]}")
+    if out.numel() != x.numel() or out.device != x.device:
+        raise RuntimeError(f"out has the wrong size or device: {tuple(out.shape)} on {out.device}, x {tuple(x.shape)} on {x.device}")
     T, inner, dev = B * n, heads * head_dim, x.device
     requests = [("norm", (B, n, d), torch.bfloat16), ("attn", (T, inner), torch.bfloat16), ("hidden", (B, n, hidden), torch.bfloat16)]
     if not all(shapes):

@@ -86,3 +86,12 @@ def test_modulation_of_another_form_is_refused(pkg, calls, name, make):
     with pytest.raises(RuntimeError, match="modulation"):
         modulation_of(pkg, calls, make)
     assert "aeris_blocks_fwd" not in calls.names()
+
+
+@pytest.mark.parametrize("tokens", [0, 1, 511, 513])
+def test_a_result_of_another_size_is_refused(pkg, calls, tokens):
+    layer = layer_of(pkg)
+    x, t = inputs(pkg)
+    with pytest.raises(RuntimeError, match="out has the wrong size"):
+        layer.block_forward(0, x, t, (0, 0), out=torch.empty(1, tokens, 128))
+    assert "aeris_blocks_fwd" not in calls.names()

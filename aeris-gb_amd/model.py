@@ -417,6 +417,8 @@ class SwinLayer(nn.Module):
         table_ptr = b4_ptr = 0
         table = attn.relative_position_bias_table
         if table is not None:  # the one-kernel attention takes the table in its own form, the attention kernel as it is
+            if tuple(table.shape) != (attn.table_rows, attn.heads):
+                raise RuntimeError(f"bias table must be [{attn.table_rows}, {attn.heads}], got {tuple(table.shape)}")
             if fused:
                 table = attn._bias4()
                 b4_ptr = table.data_ptr()

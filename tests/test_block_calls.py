@@ -95,3 +95,19 @@ def test_a_result_of_another_size_is_refused(pkg, calls, tokens):
     with pytest.raises(RuntimeError, match="out has the wrong size"):
         layer.block_forward(0, x, t, (0, 0), out=torch.empty(1, tokens, 128))
     assert "aeris_blocks_fwd" not in calls.names()
+
+
+@pytest.mark.parametrize("window", [8, 16])  # the attention kernel's table; the one-kernel attention's
+def test_a_bias_table_of_another_shape_is_refused(pkg, calls, window):
+    torch.manual_seed(1)
+    layer = pkg.SwinLayer(None, 256, 4, 64, 512, (window, window), (16, 32), False, 10_000, preset="spec", mod_ways=0).to(torch.bfloat16)
+    x = torch.randn(1, 512, 256)
+    layer(x)
+    attn = layer.modulelist[0][1]
+    good = attn.relative_position_bias_table
+    for shape in (good.shape[::-1], (good.numel(), 1), (good.shape[0], 2), (good.shape[0] - 1, 4)):
+        attn.relative_position_bias_table = torch.nn.Parameter(torch.zeros(shape, dtype=torch.bfloat16))
+        del calls[:]
+        with pytest.raises(RuntimeError, match="table"):
+            layer(x)
+        assert "aeris_blocks_fwd" not in calls.names()

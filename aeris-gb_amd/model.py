@@ -192,7 +192,6 @@ class Attention(nn.Module):
         self.rope = RoPE2D(**{k: v for k, v in rope_kwargs.items() if k in ("window_size", "rope_dim", "rope_base")})
         self.to_qkv = nn.Linear(dim, inner * 3, bias=bias)
         self.wo = nn.Linear(inner, dim, bias=bias)
-        self.table_rows = (2 * self.window_size[0] - 1) * (2 * self.window_size[1] - 1)
         if rel_pos_bias:
             wy, wx = self.window_size
             self.relative_position_bias_table = nn.Parameter(torch.zeros((2 * wy - 1) * (2 * wx - 1), heads))
@@ -417,13 +416,14 @@ class SwinLayer(nn.Module):
         table_ptr = b4_ptr = 0
         table = attn.relative_position_bias_table
         if table is not None:  # the one-kernel attention takes the table in its own form, the attention kernel as it is
-            if tuple(table.shape) != (attn.table_rows, attn.heads):
-                raise RuntimeError(f"bias table must be [{attn.table_rows}, {attn.heads}], got {tuple(table.shape)}")
+            rows = (2 * attn.window_size[0] - 1) * (2 * attn.window_size[1] - 1)
+            if tuple(table.shape) != (rows, attn.heads):
+                raise RuntimeError(f"bias table must be [{rows}, {attn.heads}], got {tuple(table.shape)}")
             if fused:
                 table = attn._bias4()
                 b4_ptr = table.data_ptr()
             else:
-                table_ptr = _vec_ptr(table, attn.table_rows * attn.heads)
+                table_ptr = _vec_ptr(table, rows * attn.heads)
         rec = ops.BLOCK_RECORD.pack(
             _vec_ptr(n1_w, d, norm_dtype), _vec_ptr(n1_b, d, norm_dtype), _vec_ptr(n2_w, d, norm_dtype), _vec_ptr(n2_b, d, norm_dtype),
             _mat_ptr(qkv_w, 3 * inner, d), _vec_ptr(qkv_b, 3 * inner), _mat_ptr(wo_w, d, inner), _vec_ptr(wo_b, d),

@@ -111,3 +111,14 @@ def test_a_bias_table_of_another_shape_is_refused(pkg, calls, window):
         with pytest.raises(RuntimeError, match="table"):
             layer(x)
         assert "aeris_blocks_fwd" not in calls.names()
+
+
+def test_a_module_saved_whole_by_an_earlier_version_still_runs(pkg, calls):
+    """A pickled module brings the attributes it was saved with: those of the attention module as it has always been made."""
+    layer = layer_of(pkg, "spec", mod_ways=0)
+    known = {"training", "heads", "head_dim", "window_size", "image_shape", "scale", "shift_mask", "fuse_qkv", "_b4cache"}
+    for name in [k for k in vars(layer.modulelist[0][1]) if k not in known and not k.startswith(("_parameters", "_buffers", "_modules",
+                 "_non_persistent", "_backward", "_is_full", "_forward", "_state_dict", "_load_state"))]:
+        del layer.modulelist[0][1].__dict__[name]
+    layer(inputs(pkg)[0])
+    assert calls.names()[-1] == "aeris_blocks_fwd"

@@ -339,9 +339,19 @@ def _modulation_vectors(modules, dt, extra=()):
     return [next(got) if p else m(dt) for m, p in zip(modules, plain)] + list(got)
 
 
+def _own(module, cls, method):
+    """Whether the module's ``method`` is that of ``cls``, neither overridden by its class nor replaced on the module itself."""
+    return getattr(type(module), method, None) is getattr(cls, method) and method not in module.__dict__
+
+
+def _own_block(block):
+    """Whether the native call does what the block's modules say: attention's ``core`` is a method that a caller may override."""
+    return _own(block._modules["1"], Attention, "core")
+
+
 def _own_blocks(layer):
-    """Whether the layer's blocks are SwinLayer's: a caller may have replaced ``block_forward``."""
-    return getattr(type(layer), "block_forward", None) is SwinLayer.block_forward and "block_forward" not in layer.__dict__
+    """Whether all of the layer's blocks can go in native calls: a caller may also have replaced ``block_forward``."""
+    return _own(layer, SwinLayer, "block_forward") and all(map(_own_block, layer.modulelist._modules.values()))
 
 
 class SwinLayer(nn.Module):
@@ -434,6 +444,36 @@ class SwinLayer(nn.Module):
         # a reparametrised module computes its weight at the access above: the call holds it until the kernels are launched
         return BlockCall(rec, fused, config, (n1_w, n1_b, n2_w, n2_b, qkv_w, qkv_b, wo_w, wo_b, up_w, up_b, dn_w, dn_b, table, m))
 
+    def _block_by_ops(self, block, x, m, shift, out):
+        """One block from the single operations, in the order of aeris_blocks_fwd."""
+        o = self.opts
+        n1, attn, n2, ff = list(block._modules.values())[:4]
+        b, n, d = x.shape
+        s1 = c1 = g1 = s2 = c2 = g2 = None
+        if o.mod_ways == 3:
+            s1, c1, g1, s2, c2, g2 = m.chunk(6, dim=1)  # model.py:399
+        elif o.mod_ways:
+            s1, c1, s2, c2 = m.chunk(4, dim=1)
+
+        def norm(module, x, shift, scale, out):
+            return ops.norm_modulate(x, module.weight, getattr(module, "bias", None), shift, scale, kind=o.norm, order=o.mod_order,
+                                     eps=o.norm_eps, out=out)
+
+        # intermediates live in shared scratch buffers (ops.workspace); only `out` is returned
+        y = norm(n1, x, s1, c1, ops.workspace("norm", (b, n, d), torch.bfloat16, x.device))
+        a = attn.core(y, shift, out=ops.workspace("attn", (b * n, attn.wo.weight.shape[1]), torch.bfloat16, x.device))
+        if out is None:
+            out = torch.empty_like(x)
+        ops.gemm(a, attn.wo.weight, attn.wo.bias, gate=g1, residual=x, rows_per_batch=n, out=out)
+        z = norm(n2, out, s2, c2, y)
+        swiglu = o.mlp == "swiglu"
+        up, down = (ff.w1, ff.w2) if swiglu else (ff.fc1, ff.fc2)
+        w, w_dn = up.weight, down.weight
+        h = ops.gemm(z, w, up.bias, act="swiglu" if swiglu else "gelu",
+                     out=ops.workspace("hidden", (b, n, w_dn.shape[1]), torch.bfloat16, x.device))
+        ops.gemm(h, w_dn, down.bias, gate=g2, residual=out, rows_per_batch=n, out=out)  # in place: out += gate * mlp
+        return out
+
     def block_forward(self, j, x, dt, shift, out=None, tap=None):
         """One block.  x is not modified; the result is written to ``out`` (allocated if None; may be x).
 
@@ -443,6 +483,8 @@ class SwinLayer(nn.Module):
         """
         block = self.modulelist[j]
         m = _modulation_vectors([block[4]], dt)[0] if self.opts.mod_ways else None
+        if not _own_block(block):
+            return self._block_by_ops(block, x, m, shift, out)
         call = self._block_call(block, x, m, shift)
         if out is None:
             out = torch.empty_like(x)

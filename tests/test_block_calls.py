@@ -122,3 +122,45 @@ def test_a_module_saved_whole_by_an_earlier_version_still_runs(pkg, calls):
         del layer.modulelist[0][1].__dict__[name]
     layer(inputs(pkg)[0])
     assert calls.names()[-1] == "aeris_blocks_fwd"
+
+
+def core_users(pkg, seen):
+    """Layers whose attention is computed by a ``core`` of the caller's: an attention module of a subclass, one with a ``core``
+    of its own, one that is no ``Attention`` at all."""
+    class Mine(pkg.Attention):
+        def core(self, y, shift=(0, 0), out=None):
+            seen.append(("subclass", shift))
+            return super().core(y, shift, out=out)
+
+    class Other(torch.nn.Module):
+        def __init__(self, wo):
+            super().__init__()
+            self.wo = wo
+
+        def core(self, y, shift, out=None):
+            seen.append(("module", shift))
+            return out.zero_()
+
+    a, b, c = layer_of(pkg, sublayers=2), layer_of(pkg, sublayers=2), layer_of(pkg, sublayers=2)
+    a.modulelist[1][1].__class__ = Mine
+    attn = b.modulelist[1][1]
+    attn.core = lambda y, shift, out=None: seen.append(("instance", shift)) or pkg.Attention.core(attn, y, shift, out=out)
+    c.modulelist[1][1] = Other(c.modulelist[1][1].wo)
+    return {"subclass": a, "instance": b, "module": c}
+
+
+def test_an_attention_core_of_the_callers_is_called(pkg, calls):
+    x, t = inputs(pkg)
+    seen = []
+    for name, layer in core_users(pkg, seen).items():
+        del seen[:], calls[:]
+        layer(x, t, shift=(4, 4))
+        assert seen == [(name, (4, 4))]
+        # the other block goes in one call; this one step by step, both norms, the two MLP projections and the output projection
+        assert calls.names().count("aeris_blocks_fwd") == 1 and calls.names().count("aeris_norm_modulate_fwd") == 2
+        assert calls.names().count("aeris_gemm_fwd") == 3
+        model = model_of(pkg, layers=1)
+        model.layers[0] = layer
+        del seen[:]
+        model(torch.randn(1, 512, 10), torch.zeros(1))
+        assert seen == [(name, (0, 0))]

@@ -465,3 +465,23 @@ def test_modulation_of_a_hook_with_other_strides(pkg, cuda):
         result[:] = [m]
         with pytest.raises(RuntimeError, match="modulation"):
             layer(x, t)
+
+
+@pytest.mark.parametrize("preset", ["ref", "spec"])
+def test_block_with_a_core_of_the_callers(pkg, cuda, preset):
+    """A block whose attention has a ``core`` of its own runs from the single operations: the bits of the native call where that
+    core is the package's, and what the core says where it is not."""
+    mk = OracleConfig.ref if preset == "ref" else (lambda **kw: OracleConfig.spec(mod_ways=2, **kw))
+    cfg = mk(n_layers=4, in_channels=20, out_channels=8, sublayers=2, **SMALL16)
+    model = make_model(pkg, cfg, oracle.init_model_weights(cfg, 2, nontrivial=True), cuda, torch.float32, preset)
+    g = torch.Generator().manual_seed(4)
+    x, t = torch.randn(2, 32 * 48, 20, generator=g).to(cuda), torch.tensor([0.3, 1.2], device=cuda)
+    want = model(x, t)
+    attn, seen = model.layers[1].modulelist[0][1], []
+    attn.core = lambda y, shift, out=None: seen.append(shift) or pkg.Attention.core(attn, y, shift, out=out)
+    assert torch.equal(model(x, t), want) and seen == [(8, 8)]
+    attn.core = lambda y, shift, out=None: out.zero_()
+    none = model(x, t)
+    del attn.core
+    attn.wo.weight.data.zero_()
+    assert torch.equal(none, model(x, t)) and not torch.equal(none, want)

@@ -528,8 +528,10 @@ def _block_events(fused, x, T, n, d, inner, hidden, window_size, mod_ways, mlp):
 
 
 def heun_update_supported(x: torch.Tensor, f0: torch.Tensor, f1: Optional[torch.Tensor], times: torch.Tensor) -> bool:
-    """Whether ``heun_update`` takes these: f32 on one GPU, contiguous, one shape, 16-byte aligned (times: any alignment)."""
-    if not (times.is_cuda and times.dtype is torch.float32 and times.is_contiguous() and times.device == x.device):
+    """Whether ``heun_update`` takes these: f32 on the current GPU (whose stream it is launched on), contiguous, one shape,
+    16-byte aligned (times: any alignment)."""
+    if not (times.is_cuda and times.dtype is torch.float32 and times.is_contiguous() and times.device == x.device and
+            x.device.index == torch._C._cuda_getDevice()):
         return False
     return all(v is None or (v.dtype is torch.float32 and v.is_cuda and v.device == x.device and v.is_contiguous() and
                              v.shape == x.shape and v.data_ptr() % 16 == 0) for v in (x, f0, f1))

@@ -164,3 +164,13 @@ def test_an_attention_core_of_the_callers_is_called(pkg, calls):
         del seen[:]
         model(torch.randn(1, 512, 10), torch.zeros(1))
         assert seen == [(name, (0, 0))]
+
+
+@pytest.mark.parametrize("current", [0, 1])
+def test_sampler_update_stays_on_the_tensors_device(pkg, calls, monkeypatch, current):
+    """The kernel goes to the current device's stream: a caller's own model on another device keeps the element-wise route."""
+    x, f, t = torch.randn(1, 8, 4), torch.randn(1, 8, 4), torch.linspace(1, 0, 3)
+    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: current)
+    monkeypatch.setattr(torch.Tensor, "device", torch.device("cuda:1"))
+    assert pkg.ops.heun_update_supported(x, f, None, t) == (current == 1)
+    assert pkg.ops.heun_update_supported(x, f, f, t) == (current == 1)

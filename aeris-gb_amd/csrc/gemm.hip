@@ -245,7 +245,8 @@ __global__ void __launch_bounds__(NT, 2) gemm_bf16_nt_tile_kernel(GemmParams p) 
     for (int e = 0; e < 4; ++e) {
       float x = acc[i][j][e];
       if (SWIGLU) x = silu_f(x) * acc[i][j + NJ][e];
-      else if (ACT == AERIS_ACT_GELU) x = OUT_F32 ? gelu_erf_f(x) : gelu_erf_bf16_f(x);
+      else if (ACT == GEMM_ACT_GELU_ERF) x = gelu_erf_bf16_f(x);
+      else if (ACT == AERIS_ACT_GELU) x = OUT_F32 ? gelu_erf_f(x) : gelu_bf16_f(x);
       else if (ACT == AERIS_ACT_SILU) x = silu_f(x);
       v[e] = x;
     }
@@ -339,7 +340,10 @@ hipError_t launch_tile_act(const GemmParams& p, hipStream_t stream) {
                                 : launch_tile<BM, BN, STAGES, A, false, VEC>(p, stream)
   switch (p.act) {
     case AERIS_ACT_GELU:
-    case GEMM_ACT_GELU_ERF: GO(AERIS_ACT_GELU);
+      if (p.c_dtype == AERIS_F32) return launch_tile<BM, BN, STAGES, AERIS_ACT_GELU, true, VEC>(p, stream);
+      // the polynomial: only as the last rows of a problem whose other rows take it, which are given to 64 x 64 tiles
+      return launch_tile<BM, BN, STAGES, BM == 64 ? AERIS_ACT_GELU : GEMM_ACT_GELU_ERF, false, VEC>(p, stream);
+    case GEMM_ACT_GELU_ERF: return launch_tile<BM, BN, STAGES, GEMM_ACT_GELU_ERF, false, VEC>(p, stream);
     case AERIS_ACT_SWIGLU: GO(AERIS_ACT_SWIGLU);
     case AERIS_ACT_SILU: GO(AERIS_ACT_SILU);
     default: GO(AERIS_ACT_NONE);
@@ -347,19 +351,22 @@ hipError_t launch_tile_act(const GemmParams& p, hipStream_t stream) {
 #undef GO
 }
 
+template <int BM, int BN, int STAGES, bool VEC, int ACT, bool OUT_F32>
+hipError_t configure_tile_kernel() {
+  return hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_bf16_nt_tile_kernel<BM, BN, STAGES, ACT, OUT_F32, VEC>),
+                             hipFuncAttributeMaxDynamicSharedMemorySize, STAGES * (BM + BN) * BK * 2);
+}
 template <int BM, int BN, int STAGES, bool VEC, int ACT>
 hipError_t configure_tile_act() {
-  constexpr int smem = STAGES * (BM + BN) * BK * 2;
-  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_bf16_nt_tile_kernel<BM, BN, STAGES, ACT, false, VEC>),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, smem);
-  if (e != hipSuccess) return e;
-  return hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_bf16_nt_tile_kernel<BM, BN, STAGES, ACT, true, VEC>),
-                             hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+  const hipError_t e = configure_tile_kernel<BM, BN, STAGES, VEC, ACT, false>();
+  return e != hipSuccess ? e : configure_tile_kernel<BM, BN, STAGES, VEC, ACT, true>();
 }
 template <int BM, int BN, int STAGES, bool VEC>
 hipError_t configure_tile() {
   hipError_t e = configure_tile_act<BM, BN, STAGES, VEC, AERIS_ACT_NONE>();
-  if (e == hipSuccess) e = configure_tile_act<BM, BN, STAGES, VEC, AERIS_ACT_GELU>();
+  if (e == hipSuccess) e = configure_tile_kernel<BM, BN, STAGES, VEC, AERIS_ACT_GELU, true>();
+  if (e == hipSuccess) e = configure_tile_kernel<BM, BN, STAGES, VEC, BM == 64 ? AERIS_ACT_GELU : GEMM_ACT_GELU_ERF, false>();
+  if (e == hipSuccess) e = configure_tile_kernel<BM, BN, STAGES, VEC, GEMM_ACT_GELU_ERF, false>();
   if (e == hipSuccess) e = configure_tile_act<BM, BN, STAGES, VEC, AERIS_ACT_SWIGLU>();
   if (e == hipSuccess) e = configure_tile_act<BM, BN, STAGES, VEC, AERIS_ACT_SILU>();
   return e;
@@ -468,7 +475,8 @@ hipError_t gemm_launch(const void* A, const void* W, void* C, const void* bias, 
   p.gate_batch_stride = gate_batch_stride;
   p.rows_per_batch = rows_per_batch > 0 ? rows_per_batch : M;
   p.tiles_n = 0;
-  p.act = act;
+  // GELU of bf16 results: by erf, but for the problems below that have a chip's worth of large tiles
+  p.act = act == AERIS_ACT_GELU && c_dtype == AERIS_BF16 ? GEMM_ACT_GELU_ERF : act;
   p.res_dtype = residual ? res_dtype : -1;
   p.c_dtype = c_dtype;
   // vector epilogue: 8 / 16-byte accesses to C and the residual (4-element alignment of every row), to bias and gate rows
@@ -478,16 +486,18 @@ hipError_t gemm_launch(const void* A, const void* W, void* C, const void* bias, 
   // what the persistent kernel cannot take: it addresses W through one buffer descriptor (31-bit size), forms row offsets
   // with 24-bit multiplies, row numbers, gate row offsets and batch numbers in 32 bits, numbers its tiles in 24 bits and
   // scales whole 64-column wave blocks of the query part
-  Shape s = {M, N, K / BK, act, c_dtype == AERIS_F32, residual != nullptr};
+  Shape s = {M, N, K / BK, p.act, c_dtype == AERIS_F32, residual != nullptr};
   bool persistent_ok = act != AERIS_ACT_SILU && (int64_t)(act == AERIS_ACT_SWIGLU ? 2 : 1) * N * K * 2 < (int64_t(1) << 31) &&
                              ldc < (1 << 23) && split < (1 << 23) && gate_batch_stride < (int64_t(1) << 31) &&
                              (rows_per_batch <= 0 || M / rows_per_batch < (int64_t(1) << 31)) && M + 512 < (int64_t(1) << 31) &&
                              tiles_of(s, 128, 256) < (int64_t(1) << 24) && q_cols % 64 == 0 && N >= 64;
-  // GELU: the polynomial where there is a chip's worth of 256 x 256 tiles, erf otherwise (whatever the tiles are)
-  if (act == AERIS_ACT_GELU && c_dtype == AERIS_BF16 &&
-      !(M >= 256 && (N % 256 == 0 || N >= 1024) && tiles_of(s, 256, 256) >= 256)) {
-    p.act = s.act = GEMM_ACT_GELU_ERF;
-    persistent_ok = persistent_ok && !gate && !residual;
+  // The polynomial where there is a chip's worth of 256 x 256 tiles, erf otherwise: one of them for all rows of a call, whatever
+  // tiles they are given to (equal rows, the members of a batch say, have equal results wherever they stand)
+  if (p.act == GEMM_ACT_GELU_ERF) {
+    if (persistent_ok && M >= 256 && (N % 256 == 0 || N >= 1024) && tiles_of(s, 256, 256) >= 256)
+      p.act = s.act = AERIS_ACT_GELU;
+    else
+      persistent_ok = persistent_ok && !gate && !residual;
   }
   if (!persistent_ok)
     return tiles_of(s, 128, 128) < 128 ? launch_tile_act<64, 64, 3, true>(p, stream) : launch_tile_act<128, 128, 2, true>(p, stream);

@@ -173,10 +173,9 @@ int aeris_output_stage_noalloc_fwd(const void* x, int x_dtype, const void* gamma
  * AERIS_ACT_GELU is the erf form, evaluated to the accuracy of the output type.  bf16 C where the problem has a chip's
  * worth of 256x256 tiles (M >= 256 and at least 256 tiles, N a multiple of 256 or >= 1024): a polynomial on the
  * clamp [-3.5, 3.5], |error| <= 2.0e-4 |x| for x >= -3.5 (a tenth of half a bf16 ulp) and the constant -8.1e-4 below
- * -3.5, where the exact value lies between -8.1e-4 and 0 (rows of a last, partly filled round of tiles may get the finer
- * form below).  Every other case: erf to 1.5e-7 absolute (f32 C), or GELU to 3e-7 |x| before the rounding (bf16 C).  The
- * forms agree to within one bf16 ulp of the result for x >= -1; which one runs depends on the shape only, never on the
- * data. */
+ * -3.5, where the exact value lies between -8.1e-4 and 0.  Every other case: erf to 1.5e-7 absolute (f32 C), or GELU to
+ * 3e-7 |x| before the rounding (bf16 C).  The forms agree to within one bf16 ulp of the result for x >= -1; all rows of a call
+ * take the same one, and which one that is depends on the shape and alignment only, never on the data. */
 int aeris_gemm_fwd(const void* A, const void* W, void* C, const void* bias, const float* gate,
                    const void* residual, int64_t M, int N, int K, int64_t ldc, int act, int res_dtype,
                    int c_dtype, int64_t gate_batch_stride, int64_t rows_per_batch, void* stream);

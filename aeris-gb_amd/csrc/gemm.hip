@@ -262,15 +262,16 @@ __global__ void __launch_bounds__(NT, 2) gemm_bf16_nt_tile_kernel(GemmParams p) 
       activated(i, j, v[j]);
       const int n = n_w + j * 16 + q * 4;
       if (VEC) {
-        if (p.gate) {
-          const f32x4 g = *reinterpret_cast<const f32x4*>(gr + (n < N ? n : N - 4));
-#pragma unroll
-          for (int e = 0; e < 4; ++e) v[j][e] *= g[e];
-        }
+        f32x4 g = {1.f, 1.f, 1.f, 1.f};
+        if (p.gate) g = *reinterpret_cast<const f32x4*>(gr + (n < N ? n : N - 4));
         if (p.res_dtype >= 0) {
+          // rounded once, as in the persistent kernel, which may have the other rows of the same call
           const u32x4 x = res[VEC ? i : 0][VEC ? j : 0];
 #pragma unroll
-          for (int e = 0; e < 4; ++e) v[j][e] += __uint_as_float(x[e]);
+          for (int e = 0; e < 4; ++e) v[j][e] = fmaf(v[j][e], g[e], __uint_as_float(x[e]));
+        } else if (p.gate) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[j][e] *= g[e];
         }
       } else {
         const int64_t off = (m0 + r) * rs + c_col_off(p, n);

@@ -653,12 +653,15 @@ __global__ void __launch_bounds__(NT) gemm_bf16_nt_persistent_kernel(GemmParams 
             if (n >= N) n = N - 4;
             gt[j] = *reinterpret_cast<const f32x4*>(gate_row_of(i * 32 + row) + n);
           }
-          if (p.gate) o *= gt[j];
-          if (p.res_dtype == AERIS_BF16) {
-            o.x += bf16_lo(rq[it].x); o.y += bf16_hi(rq[it].x); o.z += bf16_lo(rq[it].y); o.w += bf16_hi(rq[it].y);
-          } else if (p.res_dtype == AERIS_F32) {
+          // (gate and residual with one rounding, as on the interior path: equal rows have equal results)
+          if (p.res_dtype >= 0) {
+            const f32x4 x = p.res_dtype == AERIS_BF16
+                                ? f32x4{bf16_lo(rq[it].x), bf16_hi(rq[it].x), bf16_lo(rq[it].y), bf16_hi(rq[it].y)}
+                                : __builtin_bit_cast(f32x4, rq[it]);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) o[e] += __uint_as_float(rq[it][e]);
+            for (int e = 0; e < 4; ++e) o[e] = fmaf(o[e], gt[j][e], x[e]);
+          } else if (p.gate) {
+            o *= gt[j];
           }
           out[it] = o;
         }

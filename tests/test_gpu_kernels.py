@@ -173,6 +173,22 @@ def test_gemm_gelu_is_one_function_of_the_value(pkg, cuda, M, N, K):
     assert other == 0, other
 
 
+@pytest.mark.parametrize("M,N,K", [(14404, 1536, 1536), (4500, 4096, 1024), (8200, 1024, 512), (9000, 4096, 512), (8190, 1020, 512)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_gemm_gate_and_residual_of_equal_rows(pkg, cuda, M, N, K, dtype):
+    """Equal rows, gates and residuals give equal results wherever the rows stand, bit for bit: at the edge of a tile, in the
+    rows that are left to another kernel, on both sides of a batch boundary inside a tile."""
+    g = torch.Generator().manual_seed(M)
+    a = bf(torch.randn(1, K, generator=g)).to(cuda).expand(M, K).contiguous()
+    w = bf(torch.randn(N, K, generator=g) / math.sqrt(K)).to(cuda)
+    res = torch.randn(1, N, generator=g).to(dtype).to(cuda).expand(M, N).contiguous()
+    gate = torch.randn(1, N, generator=g).to(cuda)
+    for gates in (gate, gate.expand(2, N).contiguous()):
+        out = pkg.ops.gemm(a, w, None, gate=gates, residual=res, rows_per_batch=M // gates.shape[0], out_dtype=dtype)
+        other = (out != out[:1]).any(dim=1).sum().item()
+        assert other == 0, other
+
+
 def test_gemm_gelu_epilogue_pointwise(pkg, cuda):
     """The GELU of the GEMM epilogue, value by value: with one non-zero column in A and ones in W every output is
     GELU(x) for a chosen x.  Against the erf form in float64: the epilogue's polynomial is within 2.1e-4 |x| (a tenth of

@@ -308,16 +308,14 @@ class BlockCall(NamedTuple):
 
 
 def _run_blocks(calls, x, out):
-    """The blocks of ``calls``: x -> out (may be x), then in place; blocks of one configuration go in one native call.
-    Returns the last call's scratch buffers (attention output, MLP hidden)."""
-    i, scratch = 0, None
+    """The blocks of ``calls``: x -> out (may be x), then in place; blocks of one configuration go in one native call."""
+    i = 0
     while i < len(calls):
         j = i + 1
         while j < len(calls) and calls[j].config == calls[i].config:
             j += 1
-        scratch = ops.swin_blocks([c.record for c in calls[i:j]], x, out, *calls[i].config, shapes=[c.fused for c in calls[i:j]])
+        ops.swin_blocks([c.record for c in calls[i:j]], x, out, *calls[i].config, shapes=[c.fused for c in calls[i:j]])
         x, i = out, j
-    return scratch
 
 
 def _mlp_params(modulation: nn.Sequential):
@@ -444,7 +442,7 @@ class SwinLayer(nn.Module):
         # a reparametrised module computes its weight at the access above: the call holds it until the kernels are launched
         return BlockCall(rec, fused, config, (n1_w, n1_b, n2_w, n2_b, qkv_w, qkv_b, wo_w, wo_b, up_w, up_b, dn_w, dn_b, table, m))
 
-    def _block_by_ops(self, block, x, m, shift, out):
+    def _block_by_ops(self, block, x, m, shift, out, tap):
         """One block from the single operations, in the order of aeris_blocks_fwd."""
         o = self.opts
         n1, attn, n2, ff = list(block._modules.values())[:4]
@@ -462,6 +460,8 @@ class SwinLayer(nn.Module):
         # intermediates live in shared scratch buffers (ops.workspace); only `out` is returned
         y = norm(n1, x, s1, c1, ops.workspace("norm", (b, n, d), torch.bfloat16, x.device))
         a = attn.core(y, shift, out=ops.workspace("attn", (b * n, attn.wo.weight.shape[1]), torch.bfloat16, x.device))
+        if tap is not None:
+            tap("attn", a, block)
         if out is None:
             out = torch.empty_like(x)
         ops.gemm(a, attn.wo.weight, attn.wo.bias, gate=g1, residual=x, rows_per_batch=n, out=out)
@@ -471,27 +471,26 @@ class SwinLayer(nn.Module):
         w, w_dn = up.weight, down.weight
         h = ops.gemm(z, w, up.bias, act="swiglu" if swiglu else "gelu",
                      out=ops.workspace("hidden", (b, n, w_dn.shape[1]), torch.bfloat16, x.device))
+        if tap is not None:
+            tap("hidden", h, block)
         ops.gemm(h, w_dn, down.bias, gate=g2, residual=out, rows_per_batch=n, out=out)  # in place: out += gate * mlp
         return out
 
     def block_forward(self, j, x, dt, shift, out=None, tap=None):
         """One block.  x is not modified; the result is written to ``out`` (allocated if None; may be x).
 
-        ``tap(name, tensor, block)``, if given, is shown the two intermediates the block holds anyway: "attn" (attention
-        output ahead of the wo projection) and "hidden" (activated MLP hidden ahead of the down projection), both as views
-        of shared scratch that the next block overwrites.
+        ``tap(name, tensor, block)``, if given, is shown the two intermediates the block holds anyway before they are
+        consumed: "attn" (attention output ahead of the wo projection) and "hidden" (activated MLP hidden ahead of the
+        down projection), both as views of shared scratch that the next kernel overwrites.
         """
         block = self.modulelist[j]
         m = _modulation_vectors([block[4]], dt)[0] if self.opts.mod_ways else None
-        if not _own_block(block):
-            return self._block_by_ops(block, x, m, shift, out)
+        if tap is not None or not _own_block(block):
+            return self._block_by_ops(block, x, m, shift, out, tap)
         call = self._block_call(block, x, m, shift)
         if out is None:
             out = torch.empty_like(x)
-        a, h = _run_blocks([call], x, out)
-        if tap is not None:
-            tap("attn", a, block)
-            tap("hidden", h, block)
+        _run_blocks([call], x, out)
         return out
 
     def forward(self, x, dt=None, shift=None, tap=None):

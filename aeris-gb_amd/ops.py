@@ -493,7 +493,6 @@ def swin_blocks(records, x: torch.Tensor, out: torch.Tensor, image_shape, heads:
     events = _block_events(shapes, x, T, n, d, inner, hidden, window_size, mod_ways, mlp) if _profile is not None else None
     L.call("aeris_blocks_fwd", config, b"".join(records), len(records), x.data_ptr(), out.data_ptr(), ws[0].data_ptr(),
            ws[3].data_ptr() if len(ws) > 3 else None, ws[1].data_ptr(), ws[2].data_ptr(), events, _stream())
-    return ws[1], ws[2]
 
 
 def _block_events(fused, x, T, n, d, inner, hidden, window_size, mod_ways, mlp):

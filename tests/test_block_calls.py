@@ -174,3 +174,18 @@ def test_sampler_update_stays_on_the_tensors_device(pkg, calls, monkeypatch, cur
     monkeypatch.setattr(torch.Tensor, "device", torch.device("cuda:1"))
     assert pkg.ops.heun_update_supported(x, f, None, t) == (current == 1)
     assert pkg.ops.heun_update_supported(x, f, f, t) == (current == 1)
+
+
+@pytest.mark.parametrize("preset", ["ref", "spec"])
+def test_a_tap_sees_the_intermediates_before_they_are_used(pkg, calls, preset):
+    """``tap`` may change what it is shown: it is called between the operation that writes the tensor and the one that reads it."""
+    layer = layer_of(pkg, preset)
+    x, t = inputs(pkg)
+    seen = []
+    layer(x, t, tap=lambda name, tensor, block: seen.append((name, tensor, block, len(calls))))
+    assert [s[0] for s in seen] == ["attn", "hidden"] and all(s[2] is layer.modulelist[0] for s in seen)
+    (_, attn, _, at_attn), (_, hidden, _, at_hidden) = seen
+    assert attn.shape == (512, 128) and hidden.shape == (1, 512, 256)
+    wo, down = calls[at_attn], calls[at_hidden]
+    assert (wo[0], wo[1][0]) == ("aeris_gemm_fwd", attn.data_ptr()) and calls[at_attn - 1][0] == "aeris_window_attention_heads_fwd"
+    assert (down[0], down[1][0]) == ("aeris_gemm_fwd", hidden.data_ptr()) and at_hidden == len(calls) - 1

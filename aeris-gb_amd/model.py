@@ -477,7 +477,8 @@ class SwinLayer(nn.Module):
         return out
 
     def block_forward(self, j, x, dt, shift, out=None, tap=None):
-        """One block.  x is not modified; the result is written to ``out`` (allocated if None; may be x).
+        """One block.  x is not modified; the result is written to ``out`` (allocated if None; may be x; bf16 or f32, whatever
+        x is).
 
         ``tap(name, tensor, block)``, if given, is shown the two intermediates the block holds anyway before they are
         consumed: "attn" (attention output ahead of the wo projection) and "hidden" (activated MLP hidden ahead of the
@@ -485,7 +486,7 @@ class SwinLayer(nn.Module):
         """
         block = self.modulelist[j]
         m = _modulation_vectors([block[4]], dt)[0] if self.opts.mod_ways else None
-        if tap is not None or not _own_block(block):
+        if tap is not None or not _own_block(block) or (out is not None and out.dtype != x.dtype):
             return self._block_by_ops(block, x, m, shift, out, tap)
         call = self._block_call(block, x, m, shift)
         if out is None:

@@ -189,3 +189,14 @@ def test_a_tap_sees_the_intermediates_before_they_are_used(pkg, calls, preset):
     wo, down = calls[at_attn], calls[at_hidden]
     assert (wo[0], wo[1][0]) == ("aeris_gemm_fwd", attn.data_ptr()) and calls[at_attn - 1][0] == "aeris_window_attention_heads_fwd"
     assert (down[0], down[1][0]) == ("aeris_gemm_fwd", hidden.data_ptr()) and at_hidden == len(calls) - 1
+
+
+@pytest.mark.parametrize("x_dtype,out_dtype", [(torch.bfloat16, torch.float32), (torch.float32, torch.bfloat16)])
+def test_a_result_of_another_type_than_x(pkg, calls, x_dtype, out_dtype):
+    x, t = inputs(pkg, dtype=x_dtype)
+    out = torch.empty(1, 512, 128, dtype=out_dtype)
+    assert layer_of(pkg).block_forward(0, x, t, (0, 0), out=out) is out
+    code = pkg.ops._DT
+    wo, down = [a for name, a in calls if name == "aeris_gemm_fwd" and a[2] == out.data_ptr()]
+    assert (wo[5], wo[11], wo[12]) == (x.data_ptr(), code[x_dtype], code[out_dtype])  # residual, its type, the result's
+    assert (down[5], down[11], down[12]) == (out.data_ptr(), code[out_dtype], code[out_dtype])

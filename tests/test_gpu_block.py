@@ -485,3 +485,16 @@ def test_block_with_a_core_of_the_callers(pkg, cuda, preset):
     del attn.core
     attn.wo.weight.data.zero_()
     assert torch.equal(none, model(x, t)) and not torch.equal(none, want)
+
+
+def test_block_result_of_another_type_than_the_stream(pkg, cuda):
+    """An f32 result of a bf16 stream, and a bf16 result of an f32 stream, against the oracle."""
+    cfg = OracleConfig.ref(**CONFIG0)
+    sd = oracle.init_block_weights(cfg, 5, nontrivial=True)
+    layer = make_layer(pkg, cfg, sd, cuda)
+    g = torch.Generator().manual_seed(6)
+    x, t = torch.randn(1, 2048, 128, generator=g), torch.randn(1, 128, generator=g)
+    for x_dtype, out_dtype in ((torch.bfloat16, torch.float32), (torch.float32, torch.bfloat16)):
+        out = torch.empty(1, 2048, 128, dtype=out_dtype, device=cuda)
+        layer.block_forward(0, x.to(x_dtype).to(cuda), t.to(cuda), (0, 0), out=out)
+        assert rel_l2(out, oracle.block_forward(cfg, sd, x.to(x_dtype).float(), t, (0, 0))) <= 1e-2

@@ -673,7 +673,7 @@ class LocalAERIS(nn.Module):
         layers = list(self.layers)
         half = (self.window_size[0] // 2, self.window_size[1] // 2)
         shifts = [half if i % 2 == 1 else (0, 0) for i in range(len(layers))]  # model.py:471-475, folded into the attention kernel
-        if all(map(_own_blocks, layers)):
+        if block_hook is None and all(map(_own_blocks, layers)):
             # every modulation MLP of the model depends on the noise level alone: two launches for all of them
             modules = [m for layer in layers for m in layer.modulations()]
             own_end = _plain(self.output_stage, OutputStage)
@@ -683,18 +683,17 @@ class LocalAERIS(nn.Module):
                 n_mod = len(layer.modulations())
                 calls += layer.block_calls(tok, mods[k:k + n_mod], shift)
                 k += n_mod
-            if block_hook is None:
-                _run_blocks(calls, tok, tok)
-            else:
-                for j, call in enumerate(calls):
-                    _run_blocks([call], tok, tok)
-                    block_hook(j + 1, tok)
+            _run_blocks(calls, tok, tok)
             out = self.output_stage(tok, t, m=mods[-1]) if own_end else self.output_stage(tok, t)
         else:
-            k = 0
+            # block by block between two buffers: a hook may bring in the next block's weights, and looks at the stream
+            k, spare = 0, None
             for layer, shift in zip(layers, shifts):
                 for j in range(layer.sublayers):
-                    tok = layer.block_forward(j, tok, t, shift)
+                    if spare is None:
+                        spare = torch.empty_like(tok)
+                    res = layer.block_forward(j, tok, t, shift, out=spare)
+                    tok, spare = res, tok
                     k += 1
                     if block_hook is not None:
                         block_hook(k, tok)

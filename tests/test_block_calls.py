@@ -200,3 +200,27 @@ def test_a_result_of_another_type_than_x(pkg, calls, x_dtype, out_dtype):
     wo, down = [a for name, a in calls if name == "aeris_gemm_fwd" and a[2] == out.data_ptr()]
     assert (wo[5], wo[11], wo[12]) == (x.data_ptr(), code[x_dtype], code[out_dtype])  # residual, its type, the result's
     assert (down[5], down[11], down[12]) == (out.data_ptr(), code[out_dtype], code[out_dtype])
+
+
+def test_a_block_hook_may_change_the_blocks_to_come(pkg, calls):
+    """Weights brought in by the hook ahead of their block: the block runs with what its modules hold when its turn comes, and the
+    stream after the block before it stays whole until the block after it has run."""
+    model = model_of(pkg, layers=3)
+    blocks = [layer.modulelist[0] for layer in model.layers]
+    new = {}
+    states = []
+
+    def hook(k, hidden):
+        states.append(hidden.data_ptr())
+        if k in (1, 2):
+            for linear in (blocks[k][1].wo, blocks[k][4].modulation[2]):
+                linear.weight = torch.nn.Parameter(linear.weight.detach().clone())
+            new[k] = (blocks[k][1].wo.weight.data_ptr(), blocks[k][4].modulation[2].weight.data_ptr())
+
+    model(torch.randn(1, 512, 10), torch.zeros(1), block_hook=hook)
+    records = [pkg.ops.BLOCK_RECORD.unpack(a[1]) for name, a in calls if name == "aeris_blocks_fwd"]
+    read = [c for c in calls if c[0] in ("aeris_modulation_linear_fwd", "aeris_modulation_layers_fwd")]
+    assert [r[6] for r in records[1:]] == [new[1][0], new[2][0]]
+    for k in (1, 2):
+        assert any(new[k][1] in a or new[k][1].to_bytes(8, "little") in (a[0] if isinstance(a[0], bytes) else b"") for _, a in read)
+    assert len(states) == 4 and all(a != b for a, b in zip(states, states[1:]))

@@ -329,12 +329,10 @@ def _plain(module, cls):
 
 
 def _modulation_vectors(modules, dt, extra=()):
-    """f32 [1 | b, N_i] of each modulation module on the noise-level embedding dt, and of the MLPs ``extra`` (parameter
-    tuples): two launches for all of them, but what a caller has hooked or put in a module's place is called as a module."""
-    plain = [_plain(m, ModulationLinear) for m in modules]
-    mlps = [_mlp_params(m.modulation) for m, p in zip(modules, plain) if p] + list(extra)
-    got = iter(ops.modulation_mlps(dt.float().contiguous(), mlps) if mlps else ())
-    return [next(got) if p else m(dt) for m, p in zip(modules, plain)] + list(got)
+    """f32 [1 | b, N_i] of each ``ModulationLinear`` on the noise-level embedding dt, and of the MLPs ``extra`` (parameter
+    tuples): two launches for all of them."""
+    mlps = [_mlp_params(m.modulation) for m in modules] + list(extra)
+    return ops.modulation_mlps(dt.float().contiguous(), mlps) if mlps else []
 
 
 def _own(module, cls, method):
@@ -348,8 +346,10 @@ def _own_block(block):
 
 
 def _own_blocks(layer):
-    """Whether all of the layer's blocks can go in native calls: a caller may also have replaced ``block_forward``."""
-    return _own(layer, SwinLayer, "block_forward") and all(map(_own_block, layer.modulelist._modules.values()))
+    """Whether all of the layer's blocks can go in native calls, their modulation vectors computed ahead of the first: a caller
+    may have replaced ``block_forward`` or a modulation module, or hooked one (which is then called when its block is due)."""
+    return (_own(layer, SwinLayer, "block_forward") and all(map(_own_block, layer.modulelist._modules.values())) and
+            all(_plain(m, ModulationLinear) for m in layer.modulations()))
 
 
 class SwinLayer(nn.Module):
@@ -485,7 +485,7 @@ class SwinLayer(nn.Module):
         down projection), both as views of shared scratch that the next kernel overwrites.
         """
         block = self.modulelist[j]
-        m = _modulation_vectors([block[4]], dt)[0] if self.opts.mod_ways else None
+        m = block[4](dt) if self.opts.mod_ways else None  # f32 [1|b, 2*ways*d]
         if tap is not None or not _own_block(block) or (out is not None and out.dtype != x.dtype):
             return self._block_by_ops(block, x, m, shift, out, tap)
         call = self._block_call(block, x, m, shift)

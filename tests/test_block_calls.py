@@ -224,3 +224,29 @@ def test_a_block_hook_may_change_the_blocks_to_come(pkg, calls):
     for k in (1, 2):
         assert any(new[k][1] in a or new[k][1].to_bytes(8, "little") in (a[0] if isinstance(a[0], bytes) else b"") for _, a in read)
     assert len(states) == 4 and all(a != b for a, b in zip(states, states[1:]))
+
+
+@pytest.mark.parametrize("whole_model", [False, True])
+def test_a_hooked_modulation_is_called_when_its_block_is_due(pkg, calls, whole_model):
+    """A hook on a block's modulation may bring in that block's weights: it runs after the blocks before it are launched, and
+    its block's weights are read after it."""
+    if whole_model:
+        run = model_of(pkg, layers=3)
+        blocks = [layer.modulelist[0] for layer in run.layers]
+    else:
+        run = layer_of(pkg, sublayers=3)
+        blocks = list(run.modulelist)
+    new = []
+
+    def bring_in(module, args):
+        assert calls.names().count("aeris_blocks_fwd") == 2
+        linear = blocks[2][1].wo
+        linear.weight = torch.nn.Parameter(linear.weight.detach().clone())
+        new.append(linear.weight.data_ptr())
+    blocks[2][4].register_forward_pre_hook(bring_in)
+    if whole_model:
+        run(torch.randn(1, 512, 10), torch.zeros(1))
+    else:
+        run(*inputs(pkg))
+    records = [a[1] for name, a in calls if name == "aeris_blocks_fwd"]
+    assert len(new) == 1 and pkg.ops.BLOCK_RECORD.unpack(records[2])[6] == new[0]

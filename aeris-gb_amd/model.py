@@ -319,7 +319,7 @@ def _run_blocks(calls, x, out):
 
 
 def _mlp_params(modulation: nn.Sequential):
-    l0, _, l2 = modulation._modules.values()
+    l0, _, l2 = list(modulation._modules.values())[:3]
     return *_weight_bias(l0), *_weight_bias(l2)
 
 

@@ -250,3 +250,15 @@ def test_a_hooked_modulation_is_called_when_its_block_is_due(pkg, calls, whole_m
         run(*inputs(pkg))
     records = [a[1] for name, a in calls if name == "aeris_blocks_fwd"]
     assert len(new) == 1 and pkg.ops.BLOCK_RECORD.unpack(records[2])[6] == new[0]
+
+
+def test_a_modulation_mlp_with_more_in_its_sequence(pkg, calls):
+    """The first and third module of a modulation's sequence are its Linears, whatever follows them."""
+    model = model_of(pkg)
+    model(torch.randn(1, 512, 10), torch.zeros(1))
+    want = calls.names()
+    del calls[:]
+    for seq in (model.layers[0].modulelist[0][4].modulation, model.output_stage.modulation):
+        seq.append(torch.nn.Identity())
+    model(torch.randn(1, 512, 10), torch.zeros(1))
+    assert calls.names() == want

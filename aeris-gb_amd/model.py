@@ -15,6 +15,7 @@ Two presets of the one parameterised block:
 """
 from __future__ import annotations
 
+import itertools
 import math
 import os
 from dataclasses import dataclass
@@ -299,23 +300,32 @@ def _vec_ptr(v, n, dtype=torch.bfloat16):
     return v.data_ptr()
 
 
+_STORED = {nn.Parameter, type(None)}  # types of a module's weight and bias that are not computed at the access
+
+
 class BlockCall(NamedTuple):
     """One Swin block as ``ops.swin_blocks`` takes it."""
     record: bytes  # packed addresses and options
     fused: bool  # whether it runs the one-kernel attention
     config: tuple  # what blocks of one call have in common
     keep: tuple  # the tensors whose addresses the record holds
+    computed: bool  # whether some of them are made for this call alone (a reparametrised module's weight)
 
 
 def _run_blocks(calls, x, out):
-    """The blocks of ``calls``: x -> out (may be x), then in place; blocks of one configuration go in one native call."""
-    i = 0
-    while i < len(calls):
-        j = i + 1
-        while j < len(calls) and calls[j].config == calls[i].config:
-            j += 1
-        ops.swin_blocks([c.record for c in calls[i:j]], x, out, *calls[i].config, shapes=[c.fused for c in calls[i:j]])
-        x, i = out, j
+    """The blocks of ``calls`` (an iterable, drawn from as it goes): x -> out (may be x), then in place.  Blocks of one
+    configuration go in one native call; one with computed weights goes alone, before the next one's are made."""
+    group = []
+    for call in calls:
+        if group and (call.computed or call.config != group[0].config):
+            ops.swin_blocks([c.record for c in group], x, out, *group[0].config, shapes=[c.fused for c in group])
+            x, group = out, []
+        group.append(call)
+        if call.computed:
+            ops.swin_blocks([call.record], x, out, *call.config, shapes=[call.fused])
+            x, group, call = out, [], None
+    if group:
+        ops.swin_blocks([c.record for c in group], x, out, *group[0].config, shapes=[c.fused for c in group])
 
 
 def _mlp_params(modulation: nn.Sequential):
@@ -324,8 +334,12 @@ def _mlp_params(modulation: nn.Sequential):
 
 
 def _plain(module, cls):
-    """Whether the module is ``cls`` as it is: no forward of its own, nothing hooked to its inputs or results."""
-    return type(module) is cls and "forward" not in module.__dict__ and not (module._forward_hooks or module._forward_pre_hooks)
+    """Whether the module is ``cls`` as it is: no forward of its own, nothing hooked to its inputs or results, its modulation's
+    weights parameters and not computed at the access."""
+    if type(module) is not cls or "forward" in module.__dict__ or module._forward_hooks or module._forward_pre_hooks:
+        return False
+    l0, _, l2 = list(module.modulation._modules.values())[:3]
+    return "weight" in l0._parameters and "weight" in l2._parameters
 
 
 def _modulation_vectors(modules, dt, extra=()):
@@ -335,21 +349,22 @@ def _modulation_vectors(modules, dt, extra=()):
     return ops.modulation_mlps(dt.float().contiguous(), mlps) if mlps else []
 
 
-def _own(module, cls, method):
-    """Whether the module's ``method`` is that of ``cls``, neither overridden by its class nor replaced on the module itself."""
-    return getattr(type(module), method, None) is getattr(cls, method) and method not in module.__dict__
-
-
 def _own_block(block):
     """Whether the native call does what the block's modules say: attention's ``core`` is a method that a caller may override."""
-    return _own(block._modules["1"], Attention, "core")
+    attn = block._modules["1"]
+    return getattr(type(attn), "core", None) is Attention.core and "core" not in attn.__dict__
 
 
 def _own_blocks(layer):
     """Whether all of the layer's blocks can go in native calls, their modulation vectors computed ahead of the first: a caller
     may have replaced ``block_forward`` or a modulation module, or hooked one (which is then called when its block is due)."""
-    return (_own(layer, SwinLayer, "block_forward") and all(map(_own_block, layer.modulelist._modules.values())) and
-            all(_plain(m, ModulationLinear) for m in layer.modulations()))
+    if getattr(type(layer), "block_forward", None) is not SwinLayer.block_forward or "block_forward" in layer.__dict__:
+        return False
+    modulated = layer.opts.mod_ways
+    for block in layer.modulelist._modules.values():
+        if not _own_block(block) or (modulated and not _plain(block._modules["4"], ModulationLinear)):
+            return False
+    return True
 
 
 class SwinLayer(nn.Module):
@@ -397,9 +412,10 @@ class SwinLayer(nn.Module):
         return [block._modules["4"] for block in self.modulelist._modules.values()]
 
     def block_calls(self, x, mods, shift):
-        """What ``_run_blocks`` needs of all blocks; ``mods``: their modulation vectors, f32 [1 | b, 2*ways*d]."""
+        """What ``_run_blocks`` needs of each block, made as it is asked for; ``mods``: their modulation vectors, f32
+        [1 | b, 2*ways*d]."""
         blocks = self.modulelist._modules.values()
-        return [self._block_call(block, x, mods[j] if mods else None, shift) for j, block in enumerate(blocks)]
+        return (self._block_call(block, x, mods[j] if mods else None, shift) for j, block in enumerate(blocks))
 
     def _block_call(self, block, x, m, shift):
         o = self.opts
@@ -440,7 +456,8 @@ class SwinLayer(nn.Module):
         config = (attn.image_shape, attn.heads, attn.head_dim, hid, attn.window_size, norm_dtype, o.norm, o.mod_order, o.mod_ways, o.mlp,
                   o.norm_eps, attn.scale)
         # a reparametrised module computes its weight at the access above: the call holds it until the kernels are launched
-        return BlockCall(rec, fused, config, (n1_w, n1_b, n2_w, n2_b, qkv_w, qkv_b, wo_w, wo_b, up_w, up_b, dn_w, dn_b, table, m))
+        keep = (n1_w, n1_b, n2_w, n2_b, qkv_w, qkv_b, wo_w, wo_b, up_w, up_b, dn_w, dn_b)
+        return BlockCall(rec, fused, config, (*keep, table, m), not _STORED.issuperset(map(type, keep)))
 
     def _block_by_ops(self, block, x, m, shift, out, tap):
         """One block from the single operations, in the order of aeris_blocks_fwd."""
@@ -675,15 +692,15 @@ class LocalAERIS(nn.Module):
         shifts = [half if i % 2 == 1 else (0, 0) for i in range(len(layers))]  # model.py:471-475, folded into the attention kernel
         if block_hook is None and all(map(_own_blocks, layers)):
             # every modulation MLP of the model depends on the noise level alone: two launches for all of them
-            modules = [m for layer in layers for m in layer.modulations()]
+            modules = [layer.modulations() for layer in layers]
             own_end = _plain(self.output_stage, OutputStage)
-            mods = _modulation_vectors(modules, t, [_mlp_params(self.output_stage.modulation)] if own_end else [])
+            mods = _modulation_vectors(list(itertools.chain.from_iterable(modules)), t,
+                                       [_mlp_params(self.output_stage.modulation)] if own_end else [])
             calls, k = [], 0
-            for layer, shift in zip(layers, shifts):
-                n_mod = len(layer.modulations())
-                calls += layer.block_calls(tok, mods[k:k + n_mod], shift)
-                k += n_mod
-            _run_blocks(calls, tok, tok)
+            for layer, shift, own in zip(layers, shifts, modules):
+                calls.append(layer.block_calls(tok, mods[k:k + len(own)], shift))
+                k += len(own)
+            _run_blocks(itertools.chain.from_iterable(calls), tok, tok)
             out = self.output_stage(tok, t, m=mods[-1]) if own_end else self.output_stage(tok, t)
         else:
             # block by block between two buffers: a hook may bring in the next block's weights, and looks at the stream

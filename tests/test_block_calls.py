@@ -264,3 +264,38 @@ def test_a_modulation_mlp_with_more_in_its_sequence(pkg, calls):
         seq.append(torch.nn.Identity())
     model(torch.randn(1, 512, 10), torch.zeros(1))
     assert calls.names() == want
+
+
+@pytest.mark.parametrize("whole_model", [False, True])
+def test_computed_weights_live_one_block_at_a_time(pkg, calls, monkeypatch, whole_model):
+    """Weights that a parametrisation computes at the access exist for their own block only, not for all blocks of a call."""
+    import weakref
+
+    import torch.nn.utils.parametrize as parametrize
+    made, most = [], []
+
+    class Computed(torch.nn.Module):
+        def forward(self, w):
+            made.append(weakref.ref(w2 := w.clone()))
+            return w2
+
+    if whole_model:
+        run = model_of(pkg, layers=3)
+        blocks = [layer.modulelist[0] for layer in run.layers]
+    else:
+        run = layer_of(pkg, sublayers=3)
+        blocks = list(run.modulelist)
+    for b in blocks:
+        for linear in (b[1].to_qkv, b[1].wo, b[3].w1, b[3].w2, b[4].modulation[0], b[4].modulation[2]):
+            parametrize.register_parametrization(linear, "weight", Computed())
+    del made[:]
+
+    def call(name, *args):
+        calls.append((name, args))
+        most.append(sum(r() is not None for r in made))
+    monkeypatch.setattr(pkg._lib, "call", call)
+    if whole_model:
+        run(torch.randn(1, 512, 10), torch.zeros(1))
+    else:
+        run(*inputs(pkg))
+    assert len(made) == 18 and max(most) == 4, (len(made), most)

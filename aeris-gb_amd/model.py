@@ -336,7 +336,8 @@ def _mlp_params(modulation: nn.Sequential):
 def _plain(module, cls):
     """Whether the module is ``cls`` as it is: no forward of its own, nothing hooked to its inputs or results, its modulation's
     weights parameters and not computed at the access."""
-    if type(module) is not cls or "forward" in module.__dict__ or module._forward_hooks or module._forward_pre_hooks:
+    if (type(module) is not cls or "forward" in module.__dict__ or cls.forward is not _AS_DEFINED[cls] or module._forward_hooks or
+            module._forward_pre_hooks):
         return False
     l0, _, l2 = list(module.modulation._modules.values())[:3]
     return "weight" in l0._parameters and "weight" in l2._parameters
@@ -352,13 +353,13 @@ def _modulation_vectors(modules, dt, extra=()):
 def _own_block(block):
     """Whether the native call does what the block's modules say: attention's ``core`` is a method that a caller may override."""
     attn = block._modules["1"]
-    return getattr(type(attn), "core", None) is Attention.core and "core" not in attn.__dict__
+    return getattr(type(attn), "core", None) is _AS_DEFINED[Attention] and "core" not in attn.__dict__
 
 
 def _own_blocks(layer):
     """Whether all of the layer's blocks can go in native calls, their modulation vectors computed ahead of the first: a caller
     may have replaced ``block_forward`` or a modulation module, or hooked one (which is then called when its block is due)."""
-    if getattr(type(layer), "block_forward", None) is not SwinLayer.block_forward or "block_forward" in layer.__dict__:
+    if getattr(type(layer), "block_forward", None) is not _AS_DEFINED[SwinLayer] or "block_forward" in layer.__dict__:
         return False
     modulated = layer.opts.mod_ways
     for block in layer.modulelist._modules.values():
@@ -638,6 +639,11 @@ class OutputStage(nn.Module):
         y = ops.norm_modulate(x.contiguous(), self.norm.weight, beta, shift, scale, kind=self.norm_kind,
                               order="norm_then_mod", eps=self.norm_eps)
         return ops.gemm(y, self._head_weight(), out_dtype=torch.float32).view(b, n, -1)
+
+
+# the methods that native calls of several blocks stand in for, as this file defines them
+_AS_DEFINED = {Attention: Attention.core, SwinLayer: SwinLayer.block_forward, ModulationLinear: ModulationLinear.forward,
+               OutputStage: OutputStage.forward}
 
 
 class LocalAERIS(nn.Module):

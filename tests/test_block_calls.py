@@ -299,3 +299,14 @@ def test_computed_weights_live_one_block_at_a_time(pkg, calls, monkeypatch, whol
     else:
         run(*inputs(pkg))
     assert len(made) == 18 and max(most) == 4, (len(made), most)
+
+
+@pytest.mark.parametrize("cls,method", [("Attention", "core"), ("SwinLayer", "block_forward"), ("ModulationLinear", "forward"),
+                                        ("OutputStage", "forward")])
+def test_a_method_wrapped_on_the_class_is_called(pkg, calls, monkeypatch, cls, method):
+    """A profiler's or a patch's wrapper around a class's own method counts like an override on a module."""
+    cls, seen = getattr(pkg.model, cls), []
+    plain = getattr(cls, method)
+    monkeypatch.setattr(cls, method, lambda self, *args, **kw: seen.append(args) or plain(self, *args, **kw))
+    model_of(pkg, layers=2)(torch.randn(1, 512, 10), torch.zeros(1))
+    assert len(seen) == (1 if cls is pkg.model.OutputStage else 2)

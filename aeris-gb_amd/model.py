@@ -337,7 +337,7 @@ def _plain(module, cls):
     """Whether the module is ``cls`` as it is: no forward of its own, nothing hooked to its inputs or results, its modulation's
     weights parameters and not computed at the access."""
     if (type(module) is not cls or "forward" in module.__dict__ or cls.forward is not _AS_DEFINED[cls] or module._forward_hooks or
-            module._forward_pre_hooks):
+            module._forward_pre_hooks or torch.nn.modules.module._has_any_global_hook()):
         return False
     l0, _, l2 = list(module.modulation._modules.values())[:3]
     return "weight" in l0._parameters and "weight" in l2._parameters

@@ -310,3 +310,19 @@ def test_a_method_wrapped_on_the_class_is_called(pkg, calls, monkeypatch, cls, m
     monkeypatch.setattr(cls, method, lambda self, *args, **kw: seen.append(args) or plain(self, *args, **kw))
     model_of(pkg, layers=2)(torch.randn(1, 512, 10), torch.zeros(1))
     assert len(seen) == (1 if cls is pkg.model.OutputStage else 2)
+
+
+def test_hooks_on_all_modules_see_the_modulation_modules(pkg, calls):
+    """Hooks registered for every module (torch.nn.modules.module.register_module_forward_hook) see what they always saw: each
+    block's modulation, and the output stage with the arguments that count."""
+    model = model_of(pkg, layers=2)
+    hooks, seen = torch.nn.modules.module, []
+    with hooks.register_module_forward_hook(lambda module, args, out: seen.append((type(module).__name__, len(args)))):
+        model(torch.randn(1, 512, 10), torch.zeros(1))
+    assert [s for s in seen if s[0] == "ModulationLinear"] == [("ModulationLinear", 1)] * 2
+    given = []
+    with hooks.register_module_forward_pre_hook(lambda m, args: given.append(args) if isinstance(m, pkg.model.OutputStage) else None):
+        model.forward(torch.randn(1, 512, 10), torch.zeros(1))
+    with model.output_stage.register_forward_pre_hook(lambda m, args, kw: given.append(kw), with_kwargs=True):
+        model.forward(torch.randn(1, 512, 10), torch.zeros(1))
+    assert len(given) == 2 and len(given[0]) == 2 and given[1] == {}

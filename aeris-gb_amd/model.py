@@ -706,7 +706,10 @@ class LocalAERIS(nn.Module):
             for layer, shift, own in zip(layers, shifts, modules):
                 calls.append(layer.block_calls(tok, mods[k:k + len(own)], shift))
                 k += len(own)
-            _run_blocks(itertools.chain.from_iterable(calls), tok, tok)
+            # (in place but for a model of one block, which leaves the embedding whole)
+            hidden = torch.empty_like(tok) if sum(layer.sublayers for layer in layers) == 1 else tok
+            _run_blocks(itertools.chain.from_iterable(calls), tok, hidden)
+            tok = hidden
             out = self.output_stage(tok, t, m=mods[-1]) if own_end else self.output_stage(tok, t)
         else:
             # block by block between two buffers: a hook may bring in the next block's weights, and looks at the stream

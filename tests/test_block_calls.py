@@ -326,3 +326,12 @@ def test_hooks_on_all_modules_see_the_modulation_modules(pkg, calls):
     with model.output_stage.register_forward_pre_hook(lambda m, args, kw: given.append(kw), with_kwargs=True):
         model.forward(torch.randn(1, 512, 10), torch.zeros(1))
     assert len(given) == 2 and len(given[0]) == 2 and given[1] == {}
+
+
+@pytest.mark.parametrize("layers", [0, 1, 2])
+def test_the_embedding_survives_a_model_of_one_block(pkg, calls, layers):
+    """What the input stage returns is overwritten from the second block on, not by the first."""
+    model, tok = model_of(pkg, layers=layers), []
+    model.input_stage.register_forward_hook(lambda m, args, out: tok.append(out[0].data_ptr()))
+    _, hidden = model(torch.randn(1, 512, 10), torch.zeros(1), return_hidden=True)
+    assert (hidden.data_ptr() == tok[0]) == (layers != 1)

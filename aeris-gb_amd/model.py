@@ -339,14 +339,14 @@ def _plain(module, cls):
     if (type(module) is not cls or "forward" in module.__dict__ or cls.forward is not _AS_DEFINED[cls] or module._forward_hooks or
             module._forward_pre_hooks or torch.nn.modules.module._has_any_global_hook()):
         return False
-    l0, _, l2 = list(module.modulation._modules.values())[:3]
+    l0, _, l2 = list(module._modules["modulation"]._modules.values())[:3]
     return "weight" in l0._parameters and "weight" in l2._parameters
 
 
 def _modulation_vectors(modules, dt, extra=()):
     """f32 [1 | b, N_i] of each ``ModulationLinear`` on the noise-level embedding dt, and of the MLPs ``extra`` (parameter
     tuples): two launches for all of them."""
-    mlps = [_mlp_params(m.modulation) for m in modules] + list(extra)
+    mlps = [_mlp_params(m._modules["modulation"]) for m in modules] + list(extra)
     return ops.modulation_mlps(dt.float().contiguous(), mlps) if mlps else []
 
 
@@ -362,7 +362,7 @@ def _own_blocks(layer):
     if getattr(type(layer), "block_forward", None) is not _AS_DEFINED[SwinLayer] or "block_forward" in layer.__dict__:
         return False
     modulated = layer.opts.mod_ways
-    for block in layer.modulelist._modules.values():
+    for block in layer._modules["modulelist"]._modules.values():
         if not _own_block(block) or (modulated and not _plain(block._modules["4"], ModulationLinear)):
             return False
     return True
@@ -410,7 +410,7 @@ class SwinLayer(nn.Module):
         """Every block's modulation module, for ``_modulation_vectors``."""
         if not self.opts.mod_ways:
             return []
-        return [block._modules["4"] for block in self.modulelist._modules.values()]
+        return [block._modules["4"] for block in self._modules["modulelist"]._modules.values()]
 
     def block_calls(self, x, mods, shift):
         """What ``_run_blocks`` needs of each block, made as it is asked for; ``mods``: their modulation vectors, f32

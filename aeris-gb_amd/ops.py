@@ -526,9 +526,19 @@ def _block_events(fused, x, T, n, d, inner, hidden, window_size, mod_ways, mlp):
     return struct.pack(f"={len(handles)}Q", *handles)
 
 
+def _ordinary(*tensors) -> bool:
+    """Whether a native call may read and write these by their address: none of a subclass, wrapped by a transform (vmap, jvp,
+    grad) or with its sign pending, and nothing that follows tensors through operations is at work (forward-mode derivatives, tracing, dispatch modes)."""
+    return not (torch.jit.is_tracing() or torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() or
+                torch.autograd.forward_ad._current_level >= 0 or
+                any(type(t) is not torch.Tensor or torch._C._functorch.is_functorch_wrapped_tensor(t) or t.is_neg() for t in tensors))
+
+
 def heun_update_supported(x: torch.Tensor, f0: torch.Tensor, f1: Optional[torch.Tensor], times: torch.Tensor) -> bool:
     """Whether ``heun_update`` takes these: f32 on the current GPU (whose stream it is launched on), contiguous, one shape,
-    16-byte aligned (times: any alignment)."""
+    16-byte aligned (times: any alignment), in ordinary execution."""
+    if not _ordinary(*((x, f0, times) if f1 is None else (x, f0, f1, times))):
+        return False
     if not (times.is_cuda and times.dtype is torch.float32 and times.is_contiguous() and times.device == x.device and
             x.device.index == torch._C._cuda_getDevice()):
         return False

@@ -335,3 +335,50 @@ def test_the_embedding_survives_a_model_of_one_block(pkg, calls, layers):
     model.input_stage.register_forward_hook(lambda m, args, out: tok.append(out[0].data_ptr()))
     _, hidden = model(torch.randn(1, 512, 10), torch.zeros(1), return_hidden=True)
     assert (hidden.data_ptr() == tok[0]) == (layers != 1)
+
+
+@pytest.mark.parametrize("how", ["vmap", "jvp", "dual", "jit_trace", "make_fx", "subclass", "negated_view"])
+def test_sampler_update_under_transforms_and_tracing(pkg, calls, monkeypatch, how):
+    """With a model of the caller's own the sampler is ordinary tensor code: what follows tensors through it (vmap, forward-mode
+    derivatives, tracing, tensor subclasses) meets element-wise operations and no native call."""
+    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: None)
+    s = pkg.TrigFlowSampler(lambda x, t, cond=None, x_div=1.0: torch.sin(x) * t + cond, n_steps=2, device="cpu")
+    cond, lat, tangent = torch.randn(3, 5, 4), torch.randn(3, 5, 4), torch.randn(3, 5, 4)
+
+    def chain(x):
+        ts = s.t_steps
+        f0 = torch.sin(x) * ts[0] + cond
+        f1 = torch.sin(x + (ts[1] - ts[0]) * f0) * ts[1] + cond
+        x = x + (0.5 * (ts[1] - ts[0])) * (f0 + f1)
+        return x + (ts[2] - ts[1]) * (torch.sin(x) * ts[1] + cond)
+
+    def run(x):
+        return s.sample(cond, x)
+    del calls[:]
+    if how == "vmap":
+        got, want = torch.vmap(s.sample)(cond, lat), chain(lat)
+    elif how == "jvp":
+        got, want = torch.func.jvp(run, (lat,), (tangent,))[1], torch.func.jvp(chain, (lat,), (tangent,))[1]
+    elif how == "dual":
+        import torch.autograd.forward_ad as fw
+        with fw.dual_level():
+            got, want = (fw.unpack_dual(f(fw.make_dual(lat, tangent))).tangent for f in (run, chain))
+    elif how == "jit_trace":
+        got, want = torch.jit.trace(run, (torch.zeros_like(lat),), check_trace=False)(lat), chain(lat)
+    elif how == "make_fx":
+        from torch.fx.experimental.proxy_tensor import make_fx
+        got, want = make_fx(run)(torch.zeros_like(lat))(lat), chain(lat)
+    elif how == "negated_view":
+        plain = s.model
+        s.model = lambda x, t, cond=None, x_div=1.0: torch._neg_view(-plain(x, t, cond))
+        got, want = run(lat), chain(lat)
+        s.model = plain
+    else:
+        class Mine(torch.Tensor):
+            pass
+        got = run(lat.as_subclass(Mine))
+        assert type(got) is Mine
+        want = chain(lat)
+    assert torch.allclose(got.as_subclass(torch.Tensor), want, rtol=1e-5, atol=1e-5) and not calls
+    run(lat)
+    assert calls.names() == ["aeris_heun_update_fwd"] * 3

@@ -527,11 +527,15 @@ def _block_events(fused, x, T, n, d, inner, hidden, window_size, mod_ways, mlp):
 
 
 def _ordinary(*tensors) -> bool:
-    """Whether a native call may read and write these by their address: none of a subclass, wrapped by a transform (vmap, jvp,
-    grad) or with its sign pending, and nothing that follows tensors through operations is at work (forward-mode derivatives, tracing, dispatch modes)."""
-    return not (torch.jit.is_tracing() or torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() or
-                torch.autograd.forward_ad._current_level >= 0 or
-                any(type(t) is not torch.Tensor or torch._C._functorch.is_functorch_wrapped_tensor(t) or t.is_neg() for t in tensors))
+    """Whether a native call may read and write these by their address: none of a subclass or with its sign pending, and nothing
+    that follows tensors through operations is at work (vmap, jvp and the like, forward-mode derivatives, tracing, dispatch modes)."""
+    if (torch._C._is_tracing() or torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() or
+            torch.autograd.forward_ad._current_level >= 0 or torch._C._functorch.maybe_current_level() is not None):
+        return False
+    for t in tensors:
+        if type(t) is not torch.Tensor or t.is_neg():
+            return False
+    return True
 
 
 def heun_update_supported(x: torch.Tensor, f0: torch.Tensor, f1: Optional[torch.Tensor], times: torch.Tensor) -> bool:

@@ -273,11 +273,14 @@ def _norm_module(opts: BlockOptions, dim):
     return nn.RMSNorm(dim, eps=opts.eps)
 
 
+_AS_TORCH = {nn.Linear, nn.LayerNorm, nn.RMSNorm}  # modules whose weight and bias are what their parameter table holds
+
+
 def _weight_bias(module):
     """A module's weight and bias (None if it has none).  Straight from the parameter table where they are plain parameters:
     a forward looks up a dozen of these per block, and nn.Module's attribute protocol is most of what that costs."""
     p = module._parameters
-    if "weight" in p and ("bias" in p or not hasattr(module, "bias")):
+    if type(module) in _AS_TORCH and "weight" in p and ("bias" in p or not hasattr(module, "bias")):
         return p["weight"], p.get("bias")
     return module.weight, getattr(module, "bias", None)
 
@@ -340,7 +343,7 @@ def _plain(module, cls):
             module._forward_pre_hooks or torch.nn.modules.module._has_any_global_hook()):
         return False
     l0, _, l2 = list(module._modules["modulation"]._modules.values())[:3]
-    return "weight" in l0._parameters and "weight" in l2._parameters
+    return type(l0) is type(l2) is nn.Linear and "weight" in l0._parameters and "weight" in l2._parameters
 
 
 def _modulation_vectors(modules, dt, extra=()):

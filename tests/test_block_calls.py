@@ -382,3 +382,21 @@ def test_sampler_update_under_transforms_and_tracing(pkg, calls, monkeypatch, ho
     assert torch.allclose(got.as_subclass(torch.Tensor), want, rtol=1e-5, atol=1e-5) and not calls
     run(lat)
     assert calls.names() == ["aeris_heun_update_fwd"] * 3
+
+
+def test_a_weight_that_a_subclass_works_out(pkg, calls):
+    """A Linear whose class answers ``weight`` with something else than the parameter it stores: that is what the block takes."""
+    layer, made = layer_of(pkg), []
+
+    class Doubled(torch.nn.Linear):
+        @property
+        def weight(self):
+            made.append(2 * self._parameters["weight"])
+            return made[-1]
+    layer.modulelist[0][1].wo.__class__ = Doubled
+    layer(*inputs(pkg))
+    assert pkg.ops.BLOCK_RECORD.unpack(calls[-1][1][1])[6] == made[-1].data_ptr()
+    mod = layer.modulelist[0][4].modulation[2]
+    mod.__class__ = Doubled
+    layer(*inputs(pkg))
+    assert any(made_.data_ptr() in args for made_ in made for name, args in calls if name == "aeris_modulation_linear_fwd")

@@ -285,6 +285,11 @@ def _weight_bias(module):
     return module.weight, getattr(module, "bias", None)
 
 
+def _part(module, name):
+    """``module.name``, without the attribute protocol where it is a module of its own."""
+    return module._modules.get(name) or getattr(module, name)
+
+
 def _mat_ptr(w, rows, cols):
     """Address of a bf16 weight matrix [rows, cols] on the GPU, checked."""
     if not (w.is_cuda and w.dtype is torch.bfloat16 and w.is_contiguous() and w.shape[0] == rows and w.shape[1] == cols):
@@ -427,12 +432,10 @@ class SwinLayer(nn.Module):
         b, _, d = x.shape
         inner = attn.heads * attn.head_dim
         mod_ptr, mod_stride = (0, 0) if m is None else ops._rowvec(m, "modulation", 2 * o.mod_ways * d, b)
-        sub = ff._modules
         swiglu = o.mlp == "swiglu"
-        (up_w, up_b), (dn_w, dn_b) = (_weight_bias(sub["w1"]), _weight_bias(sub["w2"])) if swiglu else (
-            _weight_bias(sub["fc1"]), _weight_bias(sub["fc2"]))
-        sub = attn._modules
-        (qkv_w, qkv_b), (wo_w, wo_b) = _weight_bias(sub["to_qkv"]), _weight_bias(sub["wo"])
+        up, down = ("w1", "w2") if swiglu else ("fc1", "fc2")
+        (up_w, up_b), (dn_w, dn_b) = _weight_bias(_part(ff, up)), _weight_bias(_part(ff, down))
+        (qkv_w, qkv_b), (wo_w, wo_b) = _weight_bias(_part(attn, "to_qkv")), _weight_bias(_part(attn, "wo"))
         (n1_w, n1_b), (n2_w, n2_b) = _weight_bias(n1), _weight_bias(n2)
         norm_dtype = n1_w.dtype
         if n2_w.dtype is not norm_dtype:  # the call takes one type for both: the wider holds either exactly

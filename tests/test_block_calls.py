@@ -400,3 +400,19 @@ def test_a_weight_that_a_subclass_works_out(pkg, calls):
     mod.__class__ = Doubled
     layer(*inputs(pkg))
     assert any(made_.data_ptr() in args for made_ in made for name, args in calls if name == "aeris_modulation_linear_fwd")
+
+
+def test_an_mlp_that_passes_its_parts_through(pkg, calls):
+    """A wrapper in the MLP's place whose w1 and w2 are attributes but not modules of its own."""
+    class Around(torch.nn.Module):
+        def __init__(self, inner):
+            super().__init__()
+            self.inner = inner
+
+        w1 = property(lambda self: self.inner.w1)
+        w2 = property(lambda self: self.inner.w2)
+    layer = layer_of(pkg)
+    ff = layer.modulelist[0][3]
+    layer.modulelist[0][3] = Around(ff)
+    layer(*inputs(pkg))
+    assert pkg.ops.BLOCK_RECORD.unpack(calls[-1][1][1])[8:12:2] == (ff.w1.weight.data_ptr(), ff.w2.weight.data_ptr())

@@ -447,14 +447,15 @@ class SwinLayer(nn.Module):
         table_ptr = b4_ptr = 0
         table = attn.relative_position_bias_table
         if table is not None:  # the one-kernel attention takes the table in its own form, the attention kernel as it is
-            rows = (2 * attn.window_size[0] - 1) * (2 * attn.window_size[1] - 1)
-            if tuple(table.shape) != (rows, attn.heads):
-                raise RuntimeError(f"bias table must be [{rows}, {attn.heads}], got {tuple(table.shape)}")
+            wy, wx = attn.window_size
+            rows, cols = table.shape
+            if rows != (2 * wy - 1) * (2 * wx - 1) or cols != attn.heads:
+                raise RuntimeError(f"bias table must be [{(2 * wy - 1) * (2 * wx - 1)}, {attn.heads}], got {tuple(table.shape)}")
             if fused:
                 table = attn._bias4()
                 b4_ptr = table.data_ptr()
             else:
-                table_ptr = _vec_ptr(table, rows * attn.heads)
+                table_ptr = _vec_ptr(table, rows * cols)
         rec = ops.BLOCK_RECORD.pack(
             _vec_ptr(n1_w, d, norm_dtype), _vec_ptr(n1_b, d, norm_dtype), _vec_ptr(n2_w, d, norm_dtype), _vec_ptr(n2_b, d, norm_dtype),
             _mat_ptr(qkv_w, 3 * inner, d), _vec_ptr(qkv_b, 3 * inner), _mat_ptr(wo_w, d, inner), _vec_ptr(wo_b, d),
@@ -464,7 +465,7 @@ class SwinLayer(nn.Module):
                   o.norm_eps, attn.scale)
         # a reparametrised module computes its weight at the access above: the call holds it until the kernels are launched
         keep = (n1_w, n1_b, n2_w, n2_b, qkv_w, qkv_b, wo_w, wo_b, up_w, up_b, dn_w, dn_b)
-        return BlockCall(rec, fused, config, (*keep, table, m), not _STORED.issuperset(map(type, keep)))
+        return BlockCall(rec, fused, config, (keep, table, m), not _STORED.issuperset(map(type, keep)))
 
     def _block_by_ops(self, block, x, m, shift, out, tap):
         """One block from the single operations, in the order of aeris_blocks_fwd."""

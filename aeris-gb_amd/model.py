@@ -280,7 +280,7 @@ def _weight_bias(module):
     """A module's weight and bias (None if it has none).  Straight from the parameter table where they are plain parameters:
     a forward looks up a dozen of these per block, and nn.Module's attribute protocol is most of what that costs."""
     p = module._parameters
-    if type(module) in _AS_TORCH and "weight" in p and ("bias" in p or not hasattr(module, "bias")):
+    if type(module) in _AS_TORCH and "weight" in p and ("bias" in p or not ("bias" in module.__dict__ or "bias" in module._buffers)):
         return p["weight"], p.get("bias")
     return module.weight, getattr(module, "bias", None)
 
@@ -292,7 +292,8 @@ def _part(module, name):
 
 def _mat_ptr(w, rows, cols):
     """Address of a bf16 weight matrix [rows, cols] on the GPU, checked."""
-    if not (w.is_cuda and w.dtype is torch.bfloat16 and w.is_contiguous() and w.shape[0] == rows and w.shape[1] == cols):
+    shape = w.shape
+    if not (w.is_cuda and w.dtype is torch.bfloat16 and w.is_contiguous() and shape[0] == rows and shape[1] == cols):
         ops._dev(w, "w", torch.bfloat16)
         raise RuntimeError(f"w must be [{rows}, {cols}], got {tuple(w.shape)}")
     return w.data_ptr()
@@ -532,7 +533,7 @@ class SwinLayer(nn.Module):
             return x
         if self.sublayers == 0:
             return x
-        calls = self.block_calls(x, _modulation_vectors(self.modulations(), dt), shift)
+        calls = self.block_calls(x, _modulation_vectors(self.modulations(), dt) if self.opts.mod_ways else [], shift)
         out = torch.empty_like(x)
         _run_blocks(calls, x, out)
         return out

@@ -256,9 +256,10 @@ def _rowvec(t: Optional[torch.Tensor], name: str, d: int, B: int):
         return None, 0
     if not t.is_cuda or t.dtype != torch.float32:
         raise RuntimeError(f"{name} must be a float32 GPU tensor")
-    if t.dim() != 2 or t.shape[1] != d or t.stride(1) != 1 or t.shape[0] not in (1, B):
-        raise RuntimeError(f"{name} must be [1, {d}] or [{B}, {d}] with unit column stride, got {tuple(t.shape)}")
-    return t.data_ptr(), (t.stride(0) if t.shape[0] > 1 else 0)
+    shape = t.shape
+    if len(shape) != 2 or shape[1] != d or t.stride(1) != 1 or shape[0] not in (1, B):
+        raise RuntimeError(f"{name} must be [1, {d}] or [{B}, {d}] with unit column stride, got {tuple(shape)}")
+    return t.data_ptr(), (t.stride(0) if shape[0] > 1 else 0)
 
 
 def norm_modulate(x: torch.Tensor, gamma: torch.Tensor, beta: Optional[torch.Tensor] = None,
@@ -479,7 +480,7 @@ def swin_blocks(records, x: torch.Tensor, out: torch.Tensor, image_shape, heads:
     B, n, d = x.shape
     if n != image_shape[0] * image_shape[1]:  # the native call takes its sizes from B, H and W alone
         raise RuntimeError(f"x has {n} tokens per batch entry, expected {image_shape[0]}*{image_shape[1]}")
-    if out.numel() != x.numel() or out.device != x.device:
+    if out is not x and (out.numel() != x.numel() or out.device != x.device):
         raise RuntimeError(f"out has the wrong size or device: {tuple(out.shape)} on {out.device}, x {tuple(x.shape)} on {x.device}")
     T, inner, dev = B * n, heads * head_dim, x.device
     requests = [("norm", (B, n, d), torch.bfloat16), ("attn", (T, inner), torch.bfloat16), ("hidden", (B, n, hidden), torch.bfloat16)]
@@ -526,28 +527,25 @@ def _block_events(fused, x, T, n, d, inner, hidden, window_size, mod_ways, mlp):
     return struct.pack(f"={len(handles)}Q", *handles)
 
 
-def _ordinary(*tensors) -> bool:
-    """Whether a native call may read and write these by their address: none of a subclass or with its sign pending, and nothing
-    that follows tensors through operations is at work (vmap, jvp and the like, forward-mode derivatives, tracing, dispatch modes)."""
-    if (torch._C._is_tracing() or torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() or
-            torch.autograd.forward_ad._current_level >= 0 or torch._C._functorch.maybe_current_level() is not None):
-        return False
-    for t in tensors:
-        if type(t) is not torch.Tensor or t.is_neg():
-            return False
-    return True
+def _ordinary_execution() -> bool:
+    """Whether nothing is at work that follows tensors through operations and would miss a native call: vmap, jvp and the like,
+    forward-mode derivatives, tracing, dispatch modes."""
+    return not (torch._C._is_tracing() or torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() or
+                torch.autograd.forward_ad._current_level >= 0 or torch._C._functorch.maybe_current_level() is not None)
 
 
 def heun_update_supported(x: torch.Tensor, f0: torch.Tensor, f1: Optional[torch.Tensor], times: torch.Tensor) -> bool:
-    """Whether ``heun_update`` takes these: f32 on the current GPU (whose stream it is launched on), contiguous, one shape,
-    16-byte aligned (times: any alignment), in ordinary execution."""
-    if not _ordinary(*((x, f0, times) if f1 is None else (x, f0, f1, times))):
+    """Whether ``heun_update`` takes these: ordinary tensors (of no subclass, no sign pending) in ordinary execution, f32 on the
+    current GPU (whose stream it is launched on), contiguous, one shape, 16-byte aligned (times: any alignment)."""
+    device, shape = x.device, x.shape
+    if not (_ordinary_execution() and device.index == torch._C._cuda_getDevice()):
         return False
-    if not (times.is_cuda and times.dtype is torch.float32 and times.is_contiguous() and times.device == x.device and
-            x.device.index == torch._C._cuda_getDevice()):
-        return False
-    return all(v is None or (v.dtype is torch.float32 and v.is_cuda and v.device == x.device and v.is_contiguous() and
-                             v.shape == x.shape and v.data_ptr() % 16 == 0) for v in (x, f0, f1))
+    for v in (x, f0, f1, times):
+        if v is not None and not (type(v) is torch.Tensor and v.is_cuda and v.dtype is torch.float32 and v.device == device and
+                                  v.is_contiguous() and not v.is_neg() and
+                                  (v is times or (v.shape == shape and v.data_ptr() % 16 == 0))):
+            return False
+    return True
 
 
 def heun_update(x: torch.Tensor, f0: torch.Tensor, f1: Optional[torch.Tensor], times: torch.Tensor, i: int, sigma_data: float):

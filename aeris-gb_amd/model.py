@@ -446,7 +446,8 @@ class SwinLayer(nn.Module):
         up_rows = 2 * hid if swiglu else hid
         fused = attn.fuse_qkv and ops.qkv_attention_supported(d, attn.heads, attn.head_dim, attn.window_size, attn.image_shape)
         table_ptr = b4_ptr = 0
-        table = attn.relative_position_bias_table
+        stored = attn._parameters if type(attn) is Attention else {}
+        table = stored["relative_position_bias_table"] if "relative_position_bias_table" in stored else attn.relative_position_bias_table
         if table is not None:  # the one-kernel attention takes the table in its own form, the attention kernel as it is
             wy, wx = attn.window_size
             rows, cols = table.shape

@@ -475,20 +475,23 @@ def swin_blocks(records, x: torch.Tensor, out: torch.Tensor, image_shape, heads:
     """n Swin blocks in one call (aeris_blocks_fwd): x [B, n, d] (bf16 | f32) -> out (may be x; same shape and dtype).
     ``records``: one packed BLOCK_RECORD per block; ``shapes``: per block whether it runs the one-kernel attention (what the
     scratch buffers and the timing records follow)."""
-    _dev(x, "x")
-    _dev(out, "out", x.dtype)
+    dtype, dev = x.dtype, x.device
     B, n, d = x.shape
-    if n != image_shape[0] * image_shape[1]:  # the native call takes its sizes from B, H and W alone
-        raise RuntimeError(f"x has {n} tokens per batch entry, expected {image_shape[0]}*{image_shape[1]}")
-    if out is not x and (out.numel() != x.numel() or out.device != x.device):
-        raise RuntimeError(f"out has the wrong size or device: {tuple(out.shape)} on {out.device}, x {tuple(x.shape)} on {x.device}")
-    T, inner, dev = B * n, heads * head_dim, x.device
+    # (the native call takes its sizes from B, H and W alone)
+    if not (x.is_cuda and x.is_contiguous() and n == image_shape[0] * image_shape[1] and
+            (out is x or (out.dtype is dtype and out.is_contiguous() and out.device == dev and out.numel() == x.numel()))):
+        _dev(x, "x")
+        _dev(out, "out", dtype)
+        if n != image_shape[0] * image_shape[1]:
+            raise RuntimeError(f"x has {n} tokens per batch entry, expected {image_shape[0]}*{image_shape[1]}")
+        raise RuntimeError(f"out has the wrong size or device: {tuple(out.shape)} on {out.device}, x {tuple(x.shape)} on {dev}")
+    T, inner = B * n, heads * head_dim
     requests = [("norm", (B, n, d), torch.bfloat16), ("attn", (T, inner), torch.bfloat16), ("hidden", (B, n, hidden), torch.bfloat16)]
     if not all(shapes):
         requests.append(("qkv", (3 * heads, T, head_dim), torch.bfloat16))
     ws = workspaces(dev, *requests)
     config = BLOCK_CONFIG.pack(B, image_shape[0], image_shape[1], d, heads, head_dim, hidden, window_size[0], window_size[1],
-                               _DT[x.dtype], _DT[norm_dtype], L.NORM_LAYER if norm == "layernorm" else L.NORM_RMS,
+                               _DT[dtype], _DT[norm_dtype], L.NORM_LAYER if norm == "layernorm" else L.NORM_RMS,
                                L.NORM_THEN_MOD if mod_order == "norm_then_mod" else L.MOD_THEN_NORM, mod_ways,
                                L.ACT_SWIGLU if mlp == "swiglu" else L.ACT_GELU, eps, scale)
     events = _block_events(shapes, x, T, n, d, inner, hidden, window_size, mod_ways, mlp) if _profile is not None else None

@@ -121,7 +121,7 @@ __device__ __forceinline__ float heun_one(float x, float f0, float f1, bool two,
   const float hf = h * f;
   return x + hf;
 }
-__global__ void __launch_bounds__(256) heun_update_kernel(const float* __restrict__ x, const float* __restrict__ f0,
+__global__ void __launch_bounds__(256) heun_update_kernel(const float* x, const float* __restrict__ f0,
                                                          const float* __restrict__ f1, const float* __restrict__ t,
                                                          float sigma_data, float* out, int64_t n) {
   const float step = (t[1] - t[0]) * sigma_data;

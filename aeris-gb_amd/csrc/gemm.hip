@@ -86,7 +86,8 @@ __global__ void __launch_bounds__(NT, 2) gemm_bf16_nt_tile_kernel(GemmParams p) 
   // ---- loads: a wave brings in BM / 4 rows of A and BN / 4 rows of W per k-tile.  Rows past the end of A or W are
   // outside the descriptors (size in bytes: whole rows) and arrive as zeros; they feed only what is never stored.
   constexpr int AR = BM / 4, BR = BN / 4;
-  // The row part of an offset is in the per-lane offset, which is what the range check looks at; the k part is not.
+  // (The range check covers both parts of an offset, the per-lane one and the k-tile's: a byte k < 2 K of row r is at 2 K r + k, past
+  // the end exactly for the rows past the end.)
   constexpr int LD_MAX = A_LD > B_LD ? A_LD : B_LD;
   uint32_t ld_voff[LD_MAX];  // lane part of the source offset, per 8-row block
   {

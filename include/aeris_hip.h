@@ -174,7 +174,7 @@ int aeris_output_stage_noalloc_fwd(const void* x, int x_dtype, const void* gamma
  * worth of 256x256 tiles (M >= 256 and at least 256 tiles, N a multiple of 256 or >= 1024): a polynomial on the
  * clamp [-3.5, 3.5], |error| <= 2.0e-4 |x| for x >= -3.5 (a tenth of half a bf16 ulp) and the constant -8.1e-4 below
  * -3.5, where the exact value lies between -8.1e-4 and 0.  Every other case: erf to 1.5e-7 absolute (f32 C), or GELU to
- * 3e-7 |x| before the rounding (bf16 C).  The forms agree to within one bf16 ulp of the result for x >= -1; all rows of a call
+ * 4.1e-7 |x| before the rounding (bf16 C).  The forms agree to within one bf16 ulp of the result for x >= -1; all rows of a call
  * take the same one, and which one that is depends on the shape and alignment only, never on the data. */
 int aeris_gemm_fwd(const void* A, const void* W, void* C, const void* bias, const float* gate,
                    const void* residual, int64_t M, int N, int K, int64_t ldc, int act, int res_dtype,
@@ -247,7 +247,7 @@ int aeris_input_stage_fwd(const float* x0, int C0, float div0, const float* x1, 
  *   norm1 (+ modulation) -> to_qkv + window attention -> wo (* gate + residual) -> norm2 (+ modulation) -> MLP up -> MLP
  *   down (* gate + residual)
  * for each block, from one call: for small token counts the host's share of a block is otherwise longer than the GPU's.
- * Block 0 reads x and writes out (which may be x); the blocks after it work in place on out.  Nothing is kept between calls.
+ * x and out hold B*H*W rows of dim; block 0 reads x and writes out (which may be x); the blocks after it work in place on out.  Nothing is kept between calls.
  *   mod_ways 0 | 2 | 3 per branch: modulation f32 [B_mod, 2*mod_ways*dim] = (shift, scale[, gate]) of the attention branch,
  *   then of the MLP branch (model.py:399); modulation_stride 0: one row for the whole batch, else the rows' distance.
  *   Scratch (bf16, 16-byte aligned, borrowed): norm_scratch [T, dim], qkv_scratch [3*heads][T, head_dim] (NULL if every block

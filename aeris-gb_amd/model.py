@@ -436,6 +436,8 @@ class SwinLayer(nn.Module):
         swiglu = o.mlp == "swiglu"
         up, down = ("w1", "w2") if swiglu else ("fc1", "fc2")
         (up_w, up_b), (dn_w, dn_b) = _weight_bias(_part(ff, up)), _weight_bias(_part(ff, down))
+        if swiglu:  # a SwiGLU MLP has no biases, whatever its Linears hold (FeedForward)
+            up_b = dn_b = None
         (qkv_w, qkv_b), (wo_w, wo_b) = _weight_bias(_part(attn, "to_qkv")), _weight_bias(_part(attn, "wo"))
         (n1_w, n1_b), (n2_w, n2_b) = _weight_bias(n1), _weight_bias(n2)
         norm_dtype = n1_w.dtype
@@ -494,13 +496,15 @@ class SwinLayer(nn.Module):
         ops.gemm(a, attn.wo.weight, attn.wo.bias, gate=g1, residual=x, rows_per_batch=n, out=out)
         z = norm(n2, out, s2, c2, y)
         swiglu = o.mlp == "swiglu"
-        up, down = (ff.w1, ff.w2) if swiglu else (ff.fc1, ff.fc2)
-        w, w_dn = up.weight, down.weight
-        h = ops.gemm(z, w, up.bias, act="swiglu" if swiglu else "gelu",
+        if swiglu:  # no biases, whatever its Linears hold (FeedForward)
+            w, w_dn, bias, bias_dn = ff.w1.weight, ff.w2.weight, None, None
+        else:
+            w, w_dn, bias, bias_dn = ff.fc1.weight, ff.fc2.weight, ff.fc1.bias, ff.fc2.bias
+        h = ops.gemm(z, w, bias, act="swiglu" if swiglu else "gelu",
                      out=ops.workspace("hidden", (b, n, w_dn.shape[1]), torch.bfloat16, x.device))
         if tap is not None:
             tap("hidden", h, block)
-        ops.gemm(h, w_dn, down.bias, gate=g2, residual=out, rows_per_batch=n, out=out)  # in place: out += gate * mlp
+        ops.gemm(h, w_dn, bias_dn, gate=g2, residual=out, rows_per_batch=n, out=out)  # in place: out += gate * mlp
         return out
 
     def block_forward(self, j, x, dt, shift, out=None, tap=None):

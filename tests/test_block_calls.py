@@ -416,3 +416,23 @@ def test_an_mlp_that_passes_its_parts_through(pkg, calls):
     layer.modulelist[0][3] = Around(ff)
     layer(*inputs(pkg))
     assert pkg.ops.BLOCK_RECORD.unpack(calls[-1][1][1])[8:12:2] == (ff.w1.weight.data_ptr(), ff.w2.weight.data_ptr())
+
+
+def test_a_swiglu_mlp_has_no_biases(pkg, calls):
+    """FeedForward multiplies by its two weights: a bias that one of its Linears holds counts neither there nor in a block, and
+    what stands in a Linear's place needs none."""
+    layer = layer_of(pkg)
+    ff = layer.modulelist[0][3]
+    ff.w1.bias, ff.w2.bias = (torch.nn.Parameter(torch.ones(n, dtype=torch.bfloat16)) for n in (512, 128))
+    layer(*inputs(pkg))
+    assert pkg.ops.BLOCK_RECORD.unpack(calls[-1][1][1])[9:12:2] == (0, 0)
+    layer(*inputs(pkg), tap=lambda *a: None)
+    assert [args[3] for name, args in calls if name == "aeris_gemm_fwd"] == [None] * 3
+
+    class Weight(torch.nn.Module):
+        def __init__(self, weight):
+            super().__init__()
+            self.weight = weight
+    ff.w1, ff.w2 = Weight(ff.w1.weight), Weight(ff.w2.weight)
+    layer(*inputs(pkg))
+    layer(*inputs(pkg), tap=lambda *a: None)

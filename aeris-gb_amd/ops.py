@@ -539,9 +539,9 @@ def _ordinary_execution() -> bool:
 
 def heun_update_supported(x: torch.Tensor, f0: torch.Tensor, f1: Optional[torch.Tensor], times: torch.Tensor) -> bool:
     """Whether ``heun_update`` takes these: ordinary tensors (of no subclass, no sign pending) in ordinary execution, f32 on the
-    current GPU (whose stream it is launched on), contiguous, one shape, 16-byte aligned (times: any alignment)."""
+    current GPU (whose stream it is launched on), contiguous, not empty, one shape, 16-byte aligned (times: any alignment)."""
     device, shape = x.device, x.shape
-    if not (_ordinary_execution() and device.index == torch._C._cuda_getDevice()):
+    if not (_ordinary_execution() and device.index == torch._C._cuda_getDevice() and x.numel()):
         return False
     for v in (x, f0, f1, times):
         if v is not None and not (type(v) is torch.Tensor and v.is_cuda and v.dtype is torch.float32 and v.device == device and

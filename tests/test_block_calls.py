@@ -176,6 +176,15 @@ def test_sampler_update_stays_on_the_tensors_device(pkg, calls, monkeypatch, cur
     assert pkg.ops.heun_update_supported(x, f, f, t) == (current == 1)
 
 
+@pytest.mark.parametrize("shape", [(0, 8, 4), (2, 0, 4)])
+def test_sampler_update_of_nothing(pkg, calls, monkeypatch, shape):
+    """No members, or no tokens: an empty result, and no launch (the native call refuses a size of 0)."""
+    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: None)
+    s = pkg.TrigFlowSampler(lambda x, t, cond=None, x_div=1.0: torch.sin(x) * t, n_steps=2, device="cpu")
+    del calls[:]
+    assert s.sample(torch.zeros(shape), torch.zeros(shape)).shape == shape and not calls
+
+
 @pytest.mark.parametrize("preset", ["ref", "spec"])
 def test_a_tap_sees_the_intermediates_before_they_are_used(pkg, calls, preset):
     """``tap`` may change what it is shown: it is called between the operation that writes the tensor and the one that reads it."""

@@ -532,8 +532,9 @@ def _block_events(fused, x, T, n, d, inner, hidden, window_size, mod_ways, mlp):
 
 def _ordinary_execution() -> bool:
     """Whether nothing is at work that follows tensors through operations and would miss a native call: vmap, jvp and the like,
-    forward-mode derivatives, tracing, dispatch modes."""
+    forward-mode derivatives, tracing, function and dispatch modes."""
     return not (torch._C._is_tracing() or torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() or
+                torch._C._len_torch_function_stack() or
                 torch.autograd.forward_ad._current_level >= 0 or torch._C._functorch.maybe_current_level() is not None)
 
 

@@ -346,7 +346,7 @@ def test_the_embedding_survives_a_model_of_one_block(pkg, calls, layers):
     assert (hidden.data_ptr() == tok[0]) == (layers != 1)
 
 
-@pytest.mark.parametrize("how", ["vmap", "jvp", "dual", "jit_trace", "make_fx", "subclass", "negated_view"])
+@pytest.mark.parametrize("how", ["vmap", "jvp", "dual", "jit_trace", "make_fx", "function_mode", "subclass", "negated_view"])
 def test_sampler_update_under_transforms_and_tracing(pkg, calls, monkeypatch, how):
     """With a model of the caller's own the sampler is ordinary tensor code: what follows tensors through it (vmap, forward-mode
     derivatives, tracing, tensor subclasses) meets element-wise operations and no native call."""
@@ -377,6 +377,16 @@ def test_sampler_update_under_transforms_and_tracing(pkg, calls, monkeypatch, ho
     elif how == "make_fx":
         from torch.fx.experimental.proxy_tensor import make_fx
         got, want = make_fx(run)(torch.zeros_like(lat))(lat), chain(lat)
+    elif how == "function_mode":
+        class Counts(torch.overrides.TorchFunctionMode):
+            updates = 0
+
+            def __torch_function__(self, func, types, args=(), kwargs=None):
+                self.updates += func in (torch.add, torch.Tensor.add)
+                return func(*args, **(kwargs or {}))
+        with Counts() as mode:
+            got, want = run(lat), chain(lat)
+        assert mode.updates == 2 * (3 + 1 + 3)  # the model's own, F_s + F_t, the updates
     elif how == "negated_view":
         plain = s.model
         s.model = lambda x, t, cond=None, x_div=1.0: torch._neg_view(-plain(x, t, cond))

@@ -34,6 +34,13 @@ constexpr int BK = 64;
 constexpr int NT = 256;
 constexpr int GM = 8;  // row panels per L2 group
 
+// a b + c with both results rounded
+__device__ __forceinline__ float mul_add_rounded(float a, float b, float c) {
+#pragma clang fp contract(off)
+  const float ab = a * b;
+  return ab + c;
+}
+
 // ends a wave's use of a k-tile: its LDS reads have returned, all but its n newest loads have arrived, then the barrier
 // (one asm statement: nothing the compiler schedules may come between, and no LDS access may cross it)
 template <int N>
@@ -266,10 +273,14 @@ __global__ void __launch_bounds__(NT, 2) gemm_bf16_nt_tile_kernel(GemmParams p) 
         f32x4 g = {1.f, 1.f, 1.f, 1.f};
         if (p.gate) g = *reinterpret_cast<const f32x4*>(gr + (n < N ? n : N - 4));
         if (p.res_dtype >= 0) {
-          // rounded once, as in the persistent kernel, which may have the other rows of the same call
           const u32x4 x = res[VEC ? i : 0][VEC ? j : 0];
+          if (p.row0) {  // the last rows of a call whose others have the persistent kernel: rounded once, as there
 #pragma unroll
-          for (int e = 0; e < 4; ++e) v[j][e] = fmaf(v[j][e], g[e], __uint_as_float(x[e]));
+            for (int e = 0; e < 4; ++e) v[j][e] = fmaf(v[j][e], g[e], __uint_as_float(x[e]));
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[j][e] = mul_add_rounded(v[j][e], g[e], __uint_as_float(x[e]));
+          }
         } else if (p.gate) {
 #pragma unroll
           for (int e = 0; e < 4; ++e) v[j][e] *= g[e];

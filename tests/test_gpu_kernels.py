@@ -189,6 +189,18 @@ def test_gemm_gate_and_residual_of_equal_rows(pkg, cuda, M, N, K, dtype):
         assert other == 0, other
 
 
+@pytest.mark.parametrize("M,N,K", [(200, 64, 128), (2048, 128, 512), (2047, 260, 256)])
+def test_gemm_gate_and_residual_of_a_small_problem_round_apart(pkg, cuda, M, N, K):
+    """A call that the 64 x 64 tiles have to themselves: value times gate rounded, the sum rounded, as element-wise operations on
+    the plain product do it, bit for bit (f32 results)."""
+    g = torch.Generator().manual_seed(M)
+    a, w = bf(torch.randn(M, K, generator=g)).to(cuda), bf(torch.randn(N, K, generator=g) / math.sqrt(K)).to(cuda)
+    gate, res = torch.randn(1, N, generator=g).to(cuda), torch.randn(M, N, generator=g).to(cuda)
+    plain = pkg.ops.gemm(a, w, None, out_dtype=torch.float32)
+    scaled = plain * gate
+    assert torch.equal(pkg.ops.gemm(a, w, None, gate=gate, residual=res, out_dtype=torch.float32), scaled + res)
+
+
 def test_gemm_gelu_epilogue_pointwise(pkg, cuda):
     """The GELU of the GEMM epilogue, value by value: with one non-zero column in A and ones in W every output is
     GELU(x) for a chosen x.  Against the erf form in float64: the epilogue's polynomial is within 2.1e-4 |x| (a tenth of

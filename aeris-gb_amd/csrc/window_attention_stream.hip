@@ -1,12 +1,18 @@
 // Windowed multi-head self-attention for gfx950, streaming variant: windows of any size up to 4096 tokens
 // (the reference's 60 x 60) and head_dim 64 or 128, no relative-position bias, no shift mask (model.py:289-293).
 //
-// One workgroup = 256 queries of one (window, head): 8 waves x 32 queries, one workgroup per CU (with 128 queries per
-// workgroup and two workgroups per CU every K / V chunk was loaded, transposed and stored twice as often per query:
-// 6-7 % slower).  The keys of the window are streamed
-// through LDS in chunks of 64 (four buffers: the global loads of chunk j+2 are in flight while chunk j is
-// being consumed, and are written to LDS at its end) with an online softmax (running row max m and row sum l, output rescaled only when a max
-// moves).  Window partition, window reverse and the cyclic shift are address arithmetic exactly as in the
+// One workgroup = a block of queries of one (window, head), 32 per wave; the keys of the window are streamed through LDS in
+// chunks of 64 with an online softmax.  How many waves and chunk buffers a workgroup has follows the window (the rule
+// stands at the launch):
+//   8 waves, 4 buffers   windows of more than 2048 tokens with head_dim 128: one workgroup per CU, a barrier per two chunks
+//   4 waves, 2 buffers   the others: two workgroups per CU (head_dim 64: three), so that one's start - token table, Q, the first
+//                        chunk - and its output stores run beside another's sweep, and windows whose size is no multiple of
+//                        256 leave fewer waves without queries
+//   2 waves, 1 buffer    windows of up to 64 tokens: a single chunk, nothing to prefetch
+// (8 waves for all windows, before -> now: 280 x 570 tokens in 10 x 38 windows with 4 heads x 64 156 -> 97 us,
+// 6 x 6 windows on 360 x 720 with 6 x 64 535 -> 193 us, two members of 60 x 104 with 12 x 8 windows and 3 x 128 16.1 -> 11.8 us.)
+// The global loads of the next chunks are in flight while a chunk is consumed; with a running row max m and row sum l the
+// output is rescaled only when a max moves).  Window partition, window reverse and the cyclic shift are address arithmetic exactly as in the
 // one-window-per-workgroup kernel (window_attention.hip); the token row of every window position is computed once
 // per workgroup into an LDS table, so the streaming loop needs no integer division.
 //
@@ -40,12 +46,7 @@ struct StreamParams {
 };
 
 constexpr int KC = 64;    // keys per chunk
-constexpr int NWAVE = 8;         // waves per workgroup (two per SIMD, one workgroup per CU)
-constexpr int QB = 32 * NWAVE;   // queries per workgroup
 constexpr int MAX_L = 4096;
-// K / V chunk buffers in LDS.  With four, chunk j + 2 is written while chunk j is consumed and the workgroup needs a
-// barrier only after every second chunk (2 buffers, one barrier per chunk: 2.5 % slower).
-constexpr int NBUF = 4;
 
 // byte offset of 16-byte chunk `chunk` of row `row` in a tile with 128-byte rows (8 chunks), swizzled over double rows
 __device__ __forceinline__ uint32_t off128(int row, int chunk) {
@@ -65,7 +66,7 @@ __device__ __forceinline__ uint32_t vt_off(int d, int chunk) {
 // the same for 256-byte rows (16 chunks)
 __device__ __forceinline__ uint32_t off256(int row, int chunk) { return (uint32_t)(row * 256 + ((chunk ^ (row & 15)) << 4)); }
 
-template <int HD>
+template <int HD, int NBUF>
 struct StreamCfg {
   static constexpr int K_BYTES = KC * HD * 2;
   static constexpr int V_BYTES = HD * KC * 2;
@@ -78,19 +79,22 @@ struct StreamCfg {
 
 }  // namespace
 
-// DMA (head_dim 128): K and V chunks go into LDS by the load unit itself (buffer_load ... lds: no staging registers,
-// no ds_write, no transposing VALU work) and V stays row-major; the V^T fragments of P V then come from
-// ds_read_b64_tr_b16, the LDS read that transposes on the way out (within 16 lanes, source lane 4e + a reads 4
-// consecutive elements and result lane 4a + b receives element b of source lanes a, 4 + a, 8 + a, 12 + a).  Rows of
-// 256 B, 16-byte chunks XOR-swizzled: K by row & 15 (conflict-free ds_read_b128 fragments), V by 4 (row & 3) (the 4
-// keys x 4 column groups that the two 16-lane halves of a transposing read's 32-lane pass gather - 16 pieces of 16
-// bytes - land on the 16 distinct slots of a 256-byte bank period; with 2 (row & 3) the two halves shared eight).  Needs every byte offset
-// inside an image's k / v plane to fit 32 bits (span_bytes; checked by the launcher).
-template <int HD, bool DMA>
+// DMA: K and V chunks go into LDS by the load unit itself (buffer_load ... lds: no staging registers, no ds_write, no
+// transposing VALU work) and V stays row-major; the V^T fragments of P V then come from ds_read_b64_tr_b16, the LDS read that
+// transposes on the way out (within 16 lanes, source lane 4e + a reads 4 consecutive elements and result lane 4a + b
+// receives element b of source lanes a, 4 + a, 8 + a, 12 + a).  The 16-byte chunks of a row are XOR-swizzled.  head_dim 128,
+// rows of 256 B: K by row & 15 (conflict-free ds_read_b128 fragments), V by 4 (row & 3) (the 4 keys x 4 column groups that the
+// two 16-lane halves of a transposing read's 32-lane pass gather - 16 pieces of 16 bytes - land on the 16 distinct slots of a
+// 256-byte bank period; with 2 (row & 3) the two halves shared eight).  head_dim 64, rows of 128 B: K over double rows
+// (off128()), V by 2 (row & 3), as in the one-window kernels.  Needs every byte offset inside an image's k / v plane to fit 32
+// bits (span_bytes; checked by the launcher); the register form, eight waves, takes what does not.  (head_dim 64, eight waves
+// either way: 360 x 720 tokens in 60 x 60 windows with 8 heads 2168 -> 2076 us; with 4 waves and 2 buffers 1978.)
+template <int HD, bool DMA, int NWAVE, int NBUF>
 __global__ void __launch_bounds__(64 * NWAVE) __attribute__((amdgpu_waves_per_eu(2)))
 window_attention_stream_kernel(StreamParams p) {
-  static_assert(!DMA || HD == 128, "the DMA form is built for head_dim 128");
-  using Cfg = StreamCfg<HD>;
+  static_assert(DMA ? (NWAVE == 8 && NBUF == 4) || (NWAVE == 4 && NBUF == 2) || (NWAVE == 2 && NBUF == 1) : NWAVE == 8 && NBUF == 4, "forms that exist");
+  using Cfg = StreamCfg<HD, NBUF>;
+  constexpr int QB = 32 * NWAVE;  // queries per workgroup
   constexpr int CH = HD / 8;   // 16-byte chunks per head row
   constexpr int KS = HD / 16;  // k16 steps of QK^T
   constexpr int DB = HD / 32;  // 32-row blocks of O^T
@@ -226,14 +230,29 @@ window_attention_stream_kernel(StreamParams p) {
   typedef __attribute__((address_space(3))) void* lds_vptr;
   const __amdgpu_buffer_rsrc_t rs_k = __builtin_amdgcn_make_buffer_rsrc((void*)kbase, 0, (int)p.span_bytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t rs_v = __builtin_amdgcn_make_buffer_rsrc((void*)vbase, 0, (int)p.span_bytes, 0x00020000);
+  constexpr int RPI = 1024 / (HD * 2);                           // rows per instruction: 4 (head_dim 128) or 8
+  constexpr int CHUNK_LOADS = DMA ? 2 * KC / (RPI * NWAVE) : 0;  // load instructions of a wave per chunk
+  static_assert(NBUF != 2 || CHUNK_LOADS < 16, "the counted wait below");
   auto issue_chunk = [&](int j, int buf) {
-    const int rsub = lane >> 4, pc = lane & 15;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int ii = wave + NWAVE * i;  // 0..15
-      const int row = 4 * ii + rsub, key = j * KC + row;
-      const uint32_t rowoff = key < L ? (uint32_t)tok[key < L ? key : 0] * (ld_qkv * 2u) : 0xFFFFF000u;
-      const uint32_t ok = rowoff + (uint32_t)((pc ^ (row & 15)) << 4), ov = rowoff + (uint32_t)((pc ^ (4 * rsub)) << 4);
+    for (int i = 0; i < KC / (RPI * NWAVE); ++i) {
+      const int ii = wave + NWAVE * i;
+      auto row_offset = [&](int row) {
+        const int key = j * KC + row;
+        return key < L ? (uint32_t)tok[key < L ? key : 0] * (ld_qkv * 2u) : 0xFFFFF000u;
+      };
+      uint32_t ok, ov;
+      if constexpr (HD == 128) {
+        const int rsub = lane >> 4, pc = lane & 15, row = 4 * ii + rsub;
+        const uint32_t rowoff = row_offset(row);
+        ok = rowoff + (uint32_t)((pc ^ (row & 15)) << 4);
+        ov = rowoff + (uint32_t)((pc ^ (4 * rsub)) << 4);
+      } else {
+        const int pair = 4 * ii + (lane >> 4), logical = (lane & 15) ^ (pair & 7);  // K: off128(), double rows
+        const int row_v = 8 * ii + (lane >> 3);
+        ok = row_offset(2 * pair + (logical >> 3)) + (uint32_t)((logical & 7) << 4);
+        ov = row_offset(row_v) + (uint32_t)(((lane & 7) ^ (2 * (row_v & 3))) << 4);
+      }
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_k, (lds_vptr)(smem + buf * Cfg::K_BYTES + ii * 1024), 16, ok, 0, 0, 0);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_v, (lds_vptr)(smem + Cfg::V_BASE + buf * Cfg::V_BYTES + ii * 1024), 16, ov, 0, 0, 0);
     }
@@ -247,7 +266,7 @@ window_attention_stream_kernel(StreamParams p) {
     const int jb = lane >> 4, e = (lane >> 2) & 3, a = lane & 3;
 #pragma unroll
     for (int db = 0; db < DB; ++db) {
-      const int chunk = (4 * db + 2 * (jb & 1) + (a >> 1)) ^ (4 * e);
+      const int chunk = (4 * db + 2 * (jb & 1) + (a >> 1)) ^ (HD == 128 ? 4 * e : 2 * e);
       v_tr[db] = (uint32_t)(Cfg::V_BASE + (4 * (jb >> 1) + e) * (HD * 2) + (chunk << 4) + (a & 1) * 8);
       asm volatile("" : "+v"(v_tr[db]));
     }
@@ -293,8 +312,10 @@ window_attention_stream_kernel(StreamParams p) {
 
   if (DMA) {
     issue_chunk(0, 0);
-    if (nch > 1) issue_chunk(1, 1);
-    __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0): this wave's loads into LDS have landed
+    if (NBUF > 1 && nch > 1) issue_chunk(1, 1);
+    // lgkmcnt(0), and this wave's loads into LDS have landed (two buffers: those of chunk 0, chunk 1 is awaited when it is due)
+    if (NBUF == 2 && nch > 1) __builtin_amdgcn_s_waitcnt(0x0070 | CHUNK_LOADS);
+    else __builtin_amdgcn_s_waitcnt(0x0070);
   } else {
     load_chunk(0);
     store_chunk(0);
@@ -315,7 +336,9 @@ window_attention_stream_kernel(StreamParams p) {
     if (DMA) {
       // both chunks of the next pair are requested at the start of this pair (the buffers were last read before the
       // barrier that ended the pair before), and awaited at the barrier that ends this pair
-      if ((u & 1) == 0) {
+      if (NBUF == 2) {
+        if (j > 0 && j + 1 < nch) issue_chunk(j + 1, (u + 1) & 1);  // (chunk 1 was requested with chunk 0)
+      } else if (NBUF == 4 && (u & 1) == 0) {
         if (j + LEAD < nch) issue_chunk(j + LEAD, (u + LEAD) & (NBUF - 1));
         if (j + LEAD + 1 < nch) issue_chunk(j + LEAD + 1, (u + LEAD + 1) & (NBUF - 1));
       }
@@ -380,8 +403,8 @@ window_attention_stream_kernel(StreamParams p) {
     };
     auto v_ready = [&](int slot) {
       if (DMA) {
-        static_assert(!DMA || DB == 4, "the DMA form is built for head_dim 128");
-        lds_tr_wait(vtr[slot][0], vtr[slot][DMA ? 1 : 0], vtr[slot][DMA ? 2 : 0], vtr[slot][DMA ? 3 : 0]);
+        if constexpr (DB == 4) lds_tr_wait(vtr[slot][0], vtr[slot][DMA ? 1 : 0], vtr[slot][DMA ? 2 : 0], vtr[slot][DMA ? 3 : 0]);
+        else lds_tr_wait(vtr[slot][0], vtr[slot][DMA ? 1 : 0]);
 #pragma unroll
         for (int db = 0; db < DB; ++db) vfb[slot][db] = tr_frag_value(vtr[slot][DMA ? db : 0]);
       }
@@ -441,7 +464,7 @@ window_attention_stream_kernel(StreamParams p) {
     }  // wave_active
 
     if (!DMA && j + LEAD < nch) store_chunk((u + LEAD) & (NBUF - 1));
-    if (NBUF == 2 || (u & 1)) {
+    if (NBUF == 2 || (NBUF == 4 && (u & 1))) {
       if (DMA) __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the next pair's chunks, requested two chunks ago
       __syncthreads();
     }
@@ -479,22 +502,38 @@ window_attention_stream_kernel(StreamParams p) {
 
 // ---------------------------------------------------------------------------------------------
 
-static int stream_smem(int head_dim, int L) { return NBUF * (KC * head_dim * 2 + head_dim * KC * 2) + ((L * 4 + 15) / 16) * 16 + 16; }
+static int stream_smem(int head_dim, int L, int nbuf) { return nbuf * (KC * head_dim * 2 + head_dim * KC * 2) + ((L * 4 + 15) / 16) * 16 + 16; }
 
 bool attention_stream_supported(int ws_y, int ws_x, int head_dim, bool has_bias, bool use_mask) {
   const int64_t L = (int64_t)ws_y * ws_x;
   return (head_dim == 64 || head_dim == 128) && L >= 1 && L <= MAX_L && !has_bias && !use_mask;
 }
 
+namespace {
+template <int HD, bool DMA, int NWAVE, int NBUF>
+hipError_t configure_one() {
+  return hipFuncSetAttribute(reinterpret_cast<const void*>(window_attention_stream_kernel<HD, DMA, NWAVE, NBUF>),
+                             hipFuncAttributeMaxDynamicSharedMemorySize, stream_smem(HD, MAX_L, NBUF));
+}
+template <int HD, bool DMA, int NWAVE, int NBUF>
+hipError_t launch_one(StreamParams p, int L, hipStream_t stream) {
+  p.qblks = (L + 32 * NWAVE - 1) / (32 * NWAVE);
+  const int64_t grid = (int64_t)((p.n_units + 7) / 8) * 8 * p.qblks;
+  hipLaunchKernelGGL((window_attention_stream_kernel<HD, DMA, NWAVE, NBUF>), dim3((unsigned)grid), dim3(64 * NWAVE),
+                     stream_smem(HD, L, NBUF), stream, p);
+  return hipGetLastError();
+}
+}  // namespace
+
 hipError_t attention_stream_configure_all() {
-  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(window_attention_stream_kernel<64, false>),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, stream_smem(64, MAX_L));
-  if (e != hipSuccess) return e;
-  e = hipFuncSetAttribute(reinterpret_cast<const void*>(window_attention_stream_kernel<128, false>),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, stream_smem(128, MAX_L));
-  if (e != hipSuccess) return e;
-  return hipFuncSetAttribute(reinterpret_cast<const void*>(window_attention_stream_kernel<128, true>),
-                             hipFuncAttributeMaxDynamicSharedMemorySize, stream_smem(128, MAX_L));
+  hipError_t e = configure_one<64, false, 8, 4>();
+  if (e == hipSuccess) e = configure_one<128, false, 8, 4>();
+  if (e == hipSuccess) e = configure_one<64, true, 2, 1>();
+  if (e == hipSuccess) e = configure_one<128, true, 2, 1>();
+  if (e == hipSuccess) e = configure_one<64, true, 4, 2>();
+  if (e == hipSuccess) e = configure_one<128, true, 8, 4>();
+  if (e == hipSuccess) e = configure_one<128, true, 4, 2>();
+  return e;
 }
 
 hipError_t attention_stream_launch(const void* qkv, void* out, int B, int H, int W, int heads, int head_dim, int ws_y,
@@ -511,19 +550,20 @@ hipError_t attention_stream_launch(const void* qkv, void* out, int B, int H, int
   p.scale = scale;
   const int L = ws_y * ws_x;
   p.n_units = B * p.nWy * p.nWx * heads;
-  p.qblks = (L + QB - 1) / QB;
-  const int64_t grid = (int64_t)((p.n_units + 7) / 8) * 8 * p.qblks;
-  const int smem = stream_smem(head_dim, L);
   // bytes of an image's k (or v) plane that a token offset can reach; the DMA form addresses them with 32 bits
   const int64_t span = ((int64_t)H * W - 1) * tok_stride * 2 + (int64_t)head_dim * 2;
   p.span_bytes = span < ((int64_t)1 << 32) - 4096 ? (uint32_t)span : 0u;
-  if (head_dim == 64)
-    hipLaunchKernelGGL((window_attention_stream_kernel<64, false>), dim3((unsigned)grid), dim3(64 * NWAVE), smem, stream, p);
-  else if (p.span_bytes != 0 && tok_stride > 0)
-    hipLaunchKernelGGL((window_attention_stream_kernel<128, true>), dim3((unsigned)grid), dim3(64 * NWAVE), smem, stream, p);
-  else
-    hipLaunchKernelGGL((window_attention_stream_kernel<128, false>), dim3((unsigned)grid), dim3(64 * NWAVE), smem, stream, p);
-  return hipGetLastError();
+  const bool dma = p.span_bytes != 0 && tok_stride > 0;
+  // Windows above 2048 tokens with head_dim 128: 8 waves where few workgroups share the chip (4 windows of 3600 with 12 heads:
+  // 308 us against 315), the same on a full grid (360 x 720: 5389, 5372).  Below, 4 waves: L = 1395 1152 -> 1093 us, 400
+  // 361 -> 352, 192 140 -> 127, 128 139 -> 108 (but 960 528 -> 539).  head_dim 64 always has the smaller workgroups.
+  if (head_dim == 64) {
+    if (!dma) return launch_one<64, false, 8, 4>(p, L, stream);
+    return L <= KC ? launch_one<64, true, 2, 1>(p, L, stream) : launch_one<64, true, 4, 2>(p, L, stream);
+  }
+  if (!dma) return launch_one<128, false, 8, 4>(p, L, stream);
+  return L <= KC ? launch_one<128, true, 2, 1>(p, L, stream)
+                 : L <= 2048 ? launch_one<128, true, 4, 2>(p, L, stream) : launch_one<128, true, 8, 4>(p, L, stream);
 }
 
 }  // namespace aeris

@@ -435,6 +435,46 @@ def test_window_attention_streaming_wide_rows_match_compact(pkg, cuda):
     assert bool(torch.isfinite(out_small.float()).all()) and float(out_small.float().abs().mean()) > 1e-3
 
 
+@pytest.mark.parametrize("case", [
+    # B, H, W, heads, head_dim, ws_y, ws_x, shift_y, shift_x: at the edges between the kernel's workgroup sizes
+    (1, 4, 6, 2, 64, 1, 1, 0, 0),            # L = 1
+    (2, 14, 18, 3, 64, 7, 9, 3, 4),          # L = 63: one chunk, two waves
+    (1, 24, 16, 2, 128, 8, 8, 4, 4),         # L = 64, full
+    (1, 26, 10, 2, 64, 13, 5, 6, 2),         # L = 65: a second chunk with one key
+    (1, 13, 10, 3, 128, 13, 5, 6, 2),
+    (1, 16, 32, 2, 128, 8, 16, 4, 8),        # L = 128: one query block, full
+    (1, 26, 20, 2, 64, 13, 10, 6, 5),        # L = 130: a second block with two queries, a third chunk with two keys
+    (1, 39, 15, 2, 128, 13, 15, 6, 0),       # L = 195
+    (1, 64, 64, 1, 128, 32, 64, 16, 32),     # L = 2048: the largest of four waves with head_dim 128
+    (1, 33, 126, 1, 128, 33, 63, 0, 31),     # L = 2079: eight waves
+    (1, 33, 63, 1, 64, 33, 63, 16, 31),
+], ids=lambda c: f"B{c[0]}_{c[1]}x{c[2]}_h{c[3]}x{c[4]}_ws{c[5]}x{c[6]}_s{c[7]}x{c[8]}")
+def test_window_attention_streaming_workgroup_sizes(pkg, cuda, case):
+    """Same oracle and tolerance as the other streaming cases."""
+    test_window_attention_streaming_parity(pkg, cuda, case)
+
+
+def test_window_attention_streaming_wide_rows_match_compact_hd64(pkg, cuda):
+    """head_dim 64: rows of a [S, 3 * inner] matrix too wide for 32-bit offsets go through registers, a compact copy of
+    some of its heads straight into LDS, bit for bit the same (the key order and the arithmetic per wave are)."""
+    H, W, heads, hd, ws = 80, 90, 1600, 64, 10
+    S, inner = H * W, heads * hd
+    assert (S - 1) * 3 * inner * 2 >= 2 ** 32
+    g = torch.Generator(device=cuda).manual_seed(12)
+    qkv = torch.empty(S, 3 * inner, dtype=torch.bfloat16, device=cuda)
+    for c0 in range(0, 3 * inner, 32768):
+        c1 = min(c0 + 32768, 3 * inner)
+        qkv[:, c0:c1] = torch.randn(S, c1 - c0, generator=g, device=cuda).to(torch.bfloat16)
+    out = pkg.ops.window_attention(qkv, 1, (H, W), heads, hd, (ws, ws), (5, 5), None, False)
+    pick = [0, 803, 1599]
+    cols = torch.cat([torch.arange(c * inner + h * hd, c * inner + (h + 1) * hd) for c in range(3) for h in pick]).to(cuda)
+    out_small = pkg.ops.window_attention(qkv.index_select(1, cols).contiguous(), 1, (H, W), len(pick), hd, (ws, ws), (5, 5), None, False)
+    torch.cuda.synchronize()
+    for i, h in enumerate(pick):
+        assert torch.equal(out[:, h * hd:(h + 1) * hd], out_small[:, i * hd:(i + 1) * hd]), h
+    assert float(out_small.float().abs().mean()) > 1e-3
+
+
 HEAD_PLANE_CASES = [
     # B, H, W, heads, hd, ws_y, ws_x, shift, bias, mask -- one-window kernel (small and large grids) and streaming kernel
     (1, 48, 64, 3, 64, 16, 16, 8, True, True),

@@ -89,7 +89,7 @@ struct LoadVPlain {
 // The cyclic-shift mask is computed from the window position (only windows on the wrapped border of a shifted grid carry
 // more than one region; -100 across regions); keys past the window (windows whose token count is not a multiple of 32)
 // get -inf.
-template <int WS_Y, int WS_X, bool HAS_BIAS>
+template <int WS_Y, int WS_X, bool HAS_BIAS, int PITCH = 2 * WS_X - 1>
 struct WindowLogits {
   static constexpr int L = WS_Y * WS_X, LPAD = (L + 31) / 32 * 32, TBL = (2 * WS_Y - 1) * (2 * WS_X - 1);
   static constexpr float MASK_NEG = -100.0f * 1.4426950408889634f;  // the additive -100, in the exp2 domain
@@ -106,9 +106,9 @@ struct WindowLogits {
   __device__ __forceinline__ WindowLogits(const unsigned char* bias_lds, int qpos, int hi_, bool my_, bool mx_, int sy_, int sx_)
       : hi(hi_), my(my_), mx(mx_), sy(sy_), sx(sx_) {
     const int qiy = qpos / WS_X, qix = qpos % WS_X;
-    const int sp = (TBL - 1) - (qiy + WS_Y - 1) * (2 * WS_X - 1) - qix - (WS_X - 1);
+    const int sp = (WS_Y - 1 - qiy) * PITCH + (WS_X - 1 - qix);
     sB_same = bias_lds + (sp + 4 * hi) * 16;
-    sB_next = bias_lds + (sp + (WS_X + 3) * hi) * 16;
+    sB_next = bias_lds + (sp + (PITCH - WS_X + 4) * hi) * 16;
     ry_q = my ? (qiy < WS_Y - sy ? 1 : 2) : 0;
     rx_q = mx ? (qix < WS_X - sx ? 1 : 2) : 0;
   }
@@ -118,7 +118,7 @@ struct WindowLogits {
       f32x4 bv = {0.f, 0.f, 0.f, 0.f};
       const int base = kb * 32 + g * 8;
       if (HAS_BIAS && (LPAD == L || base < L)) {
-        const int qt0 = (base / WS_X) * (2 * WS_X - 1) + (base % WS_X);
+        const int qt0 = (base / WS_X) * PITCH + (base % WS_X);
         bv = *reinterpret_cast<const f32x4*>((base % WS_X + 4 < WS_X ? sB_same : sB_next) + qt0 * 16);
       }
 #pragma unroll
@@ -164,6 +164,21 @@ __device__ __forceinline__ void build_bias_lds(unsigned char* sB, const uint16_t
 #pragma unroll
     for (int e = 0; e < 4; ++e)
       if (j - e >= 0) sBf[(j - e) * 4 + e] = r;
+  }
+}
+
+// The same with rows of PITCH = 2 WS_X - 4 vectors: those that start in a row's first 2 WS_X - 4 columns are all that a key
+// group (whose first column is a multiple of 4) reads.
+template <int WS_Y, int WS_X>
+__device__ __forceinline__ void build_bias_rows_lds(unsigned char* sB, const uint16_t* table, int heads, int head, int tid, int nt) {
+  constexpr int ROW = 2 * WS_X - 1, PITCH = 2 * WS_X - 4, TBL = (2 * WS_Y - 1) * ROW;
+  float* sBf = reinterpret_cast<float*>(sB);
+  for (int j = tid; j < TBL; j += nt) {
+    const int y = j / ROW, x = j - y * ROW;
+    const float r = bf16_bits_to_f32(table[(int64_t)(TBL - 1 - j) * heads + head]) * 1.4426950408889634f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (x - e >= 0 && x - e < PITCH) sBf[(y * PITCH + x - e) * 4 + e] = r;
   }
 }
 

@@ -665,6 +665,117 @@ window_attention_persist_kernel(AttnParams p, int n_units) {
 }
 
 // ---------------------------------------------------------------------------------------------
+// Units of one window and head with one K / V tile in LDS, several workgroups per CU: what a workgroup waits for (its tile, its
+// stores) runs under the others' sweeps, where the persistent kernel above has the next unit's loads in flight instead and
+// one workgroup per CU.  For 8x8 windows, whose two waves leave a persistent workgroup's CU nearly empty: six workgroups per CU
+// (33792 tokens x 12 heads of 64 53.4 -> 34.6 us, 115200 x 8 97 -> 99, 179968 x 9 169.5 -> 173.8 (four per CU: 37.4, 97.5, 172.4;
+// eight: 36.8, 106, 193), 2048 x 4 5.9 -> 4.8 us), and for 12x12 windows too few to walk (4608 tokens x 4 heads 9.0 -> 7.9 us; at 3600 units
+// five waves beside five others do not spread over four SIMDs: 85 us, the persistent kernel 65.5).
+// What follows from the lane is worked out per unit: kept across units it filled the registers of a third wave per SIMD.  The bias
+// table holds only the vectors that a key group can start at (build_bias_rows_lds).
+template <int WS_Y, int WS_X, bool HAS_BIAS>
+struct AttnWalkCfg {
+  static constexpr int L = WS_Y * WS_X;
+  static constexpr int NQ = (L + 31) / 32;
+  static constexpr int NT = NQ * 64;  // one wave per query group
+  static constexpr int PITCH = 2 * WS_X - 4;
+  static constexpr int KV_BYTES = L * 128;
+  static constexpr int SMEM = 2 * KV_BYTES + (HAS_BIAS ? (2 * WS_Y - 1) * PITCH * 16 : 0);
+};
+
+template <int WS_Y, int WS_X, bool HAS_BIAS>
+__global__ void __launch_bounds__(attn_persist_threads(WS_Y, WS_X)) __attribute__((amdgpu_waves_per_eu(3)))
+window_attention_walk_kernel(AttnParams p, int n_units) {
+  using Cfg = AttnWalkCfg<WS_Y, WS_X, HAS_BIAS>;
+  constexpr int HD = 64, KS = 4, DB = 2;
+  constexpr int L = Cfg::L, NQ = Cfg::NQ, NT = Cfg::NT, KVB = Cfg::KV_BYTES;
+  constexpr float LOG2E = 1.4426950408889634f;
+  static_assert(L % 8 == 0 && WS_X % 4 == 0, "a load instruction fills 8 rows; 4 keys lie in one window row");
+  constexpr int PAIRS = L / 8;  // load instruction pairs (K, V) of a unit
+  typedef __attribute__((address_space(3))) void* lds_ptr;
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  unsigned char *const sK = smem, *const sV = smem + KVB, *const sB = smem + 2 * KVB;
+
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int H = p.H, W = p.W, inner = p.heads * HD;
+  const uint32_t ld_qkv = (uint32_t)p.tok_stride;
+  const int wpi = p.nWy * p.nWx, n_win = p.B * wpi;
+  const uint32_t plane_bytes = (uint32_t)p.B * (uint32_t)(H * W) * ld_qkv * 2u;  // < 2^32, checked by the caller
+  const float cq = p.scale * LOG2E;
+  int bias_head = -1;
+
+  for (int u = blockIdx.x; u < n_units; u += gridDim.x) {
+    int lane = tid & 63;
+    asm volatile("" : "+v"(lane));  // what follows from the lane is worked out per unit and not kept in registers across units
+    const int l31 = lane & 31, hi = lane >> 5, rsub = lane >> 3, pc = lane & 7;
+    const int head = u / n_win, win = u - head * n_win;
+    const int b = win / wpi, wrem = win - b * wpi;
+    const int wy = wrem / p.nWx, wx = wrem - wy * p.nWx;
+    const int y0 = wy * WS_Y + p.sy, x0 = wx * WS_X + p.sx;
+    const uint32_t img_base = (uint32_t)b * (uint32_t)(H * W);
+    auto token_row = [&](int pos) -> uint32_t {
+      int Y = y0 + pos / WS_X, X = x0 + pos % WS_X;
+      if (Y >= H) Y -= H;
+      if (X >= W) X -= W;
+      return img_base + (uint32_t)Y * (uint32_t)W + (uint32_t)X;
+    };
+    if (u != (int)blockIdx.x) __builtin_amdgcn_s_barrier();  // every wave has read what it needs of the unit before
+    __builtin_amdgcn_sched_barrier(0);
+    const uint16_t* const base = p.qkv + head * p.head_stride;
+    int qpos = wave * 32 + l31;
+    const bool q_valid = qpos < L;
+    if (!q_valid) qpos = L - 1;
+    const uint32_t q_tok = token_row(qpos);
+    bf16x8 qf[KS];
+#pragma unroll
+    for (int s2 = 0; s2 < KS; ++s2) qf[s2] = *reinterpret_cast<const bf16x8*>(base + (uint64_t)q_tok * ld_qkv + hi * 8 + s2 * 16);
+    const __amdgpu_buffer_rsrc_t rs_k = __builtin_amdgcn_make_buffer_rsrc((void*)(base + p.part_stride), 0, (int)plane_bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rs_v = __builtin_amdgcn_make_buffer_rsrc((void*)(base + 2 * p.part_stride), 0, (int)plane_bytes, 0x00020000);
+#pragma unroll
+    for (int j = 0; j < (PAIRS + NQ - 1) / NQ; ++j) {
+      const int ii = wave + j * NQ;
+      if (PAIRS % NQ == 0 || ii < PAIRS) {  // wave-uniform
+        const int key = ii * 8 + rsub;
+        const uint32_t off = token_row(key) * (ld_qkv * 2u);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_k, (lds_ptr)(sK + ii * 1024), 16, off + (uint32_t)((pc ^ ((key >> 1) & 7)) << 4), 0, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_v, (lds_ptr)(sV + ii * 1024), 16, off + (uint32_t)((pc ^ (2 * (key & 3))) << 4), 0, 0, 0);
+      }
+    }
+    if (HAS_BIAS && head != bias_head) {
+      build_bias_rows_lds<WS_Y, WS_X>(sB, p.table, p.heads, head, tid, NT);
+      bias_head = head;
+    }
+    if (!p.q_prescaled) {
+#pragma unroll
+      for (int s2 = 0; s2 < KS; ++s2) {
+        u32x4 w = __builtin_bit_cast(u32x4, qf[s2]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) w[e] = pack_bf16x2(bf16_lo(w[e]) * cq, bf16_hi(w[e]) * cq);
+        qf[s2] = __builtin_bit_cast(bf16x8, w);
+      }
+    }
+    __builtin_amdgcn_s_waitcnt(0x0070);  // this wave's loads into LDS and its bias writes have landed
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    const bool my = p.use_mask && p.sy > 0 && wy == p.nWy - 1;
+    const bool mx = p.use_mask && p.sx > 0 && wx == p.nWx - 1;
+    auto load_k = [&](int kb, bf16x8 (&f)[KS]) {
+#pragma unroll
+      for (int s2 = 0; s2 < KS; ++s2) f[s2] = *reinterpret_cast<const bf16x8*>(sK + k_off<64>(kb * 32 + l31, s2 * 2 + hi));
+    };
+    const uint32_t v_addr = lds_byte_address(sV);
+    auto v_step = [&](int step) { return v_addr + (uint32_t)step * 2048u; };
+    const LoadVTransposed<DB, decltype(v_step)> load_v(lane, v_step);
+    const WindowLogits<WS_Y, WS_X, HAS_BIAS, Cfg::PITCH> logits(sB, qpos, hi, my, mx, p.sy, p.sx);
+    f32x16 o[DB];
+    float sum;
+    attention_sweep<NQ, KS, DB, HAS_BIAS>(logits, load_k, load_v, [](int) {}, qf, o, sum);
+    store_attention_rows<DB>(p.out + (uint64_t)q_tok * (uint32_t)inner + head * HD + hi * 8, o, sum, q_valid);
+  }
+}
+
+// ---------------------------------------------------------------------------------------------
 
 #define AERIS_ATTN_SHAPES(X) X(8, 8, 32) X(8, 8, 64) X(12, 12, 32) X(12, 12, 64) X(16, 16, 32) X(16, 16, 64)
 
@@ -691,13 +802,13 @@ hipError_t attention_configure_all() {
   e = hipFuncSetAttribute(reinterpret_cast<const void*>(window_attention_dma_kernel<Y, Xx, Bi>),                \
                           hipFuncAttributeMaxDynamicSharedMemorySize, AttnDmaCfg<Y, Xx, Bi>::SMEM);             \
   if (e != hipSuccess) return e;
-  CFGD(8, 8, true) CFGD(8, 8, false) CFGD(12, 12, true) CFGD(12, 12, false) CFGD(16, 16, true) CFGD(16, 16, false)
+  CFGD(16, 16, true) CFGD(16, 16, false)
 #undef CFGD
 #define CFGP(Y, Xx, Bi)                                                                                        \
   e = hipFuncSetAttribute(reinterpret_cast<const void*>(window_attention_persist_kernel<Y, Xx, Bi>),            \
                           hipFuncAttributeMaxDynamicSharedMemorySize, AttnPersistCfg<Y, Xx, Bi>::SMEM);         \
   if (e != hipSuccess) return e;
-  CFGP(8, 8, true) CFGP(8, 8, false) CFGP(12, 12, true) CFGP(12, 12, false) CFGP(16, 16, true) CFGP(16, 16, false)
+  CFGP(12, 12, true) CFGP(12, 12, false) CFGP(16, 16, true) CFGP(16, 16, false)
 #undef CFGP
   {
     int dev = 0, cus = 0;
@@ -715,16 +826,30 @@ static hipError_t launch_attn(const AttnParams& p, hipStream_t stream) {
   // head_dim 64 with every offset inside a q / k / v plane below 2^32 bytes: K and V straight into LDS
   if (HD == 64 && p.head_stride >= (int64_t)p.B * p.H * p.W * p.tok_stride &&
       (int64_t)p.B * p.H * p.W * p.tok_stride * 2 < (int64_t)0xFFFFFFF0u) {
-    if (grid >= 2 * (int64_t)g_attn_cus) {  // enough units for every CU to stream a few: the persistent form
-      using P = AttnPersistCfg<WS_Y, WS_X, HAS_BIAS>;
-      hipLaunchKernelGGL((window_attention_persist_kernel<WS_Y, WS_X, HAS_BIAS>), dim3((unsigned)g_attn_cus), dim3(P::NT), P::SMEM,
-                         stream, p, (int)grid);
+    if constexpr (WS_X < 16) {
+      constexpr int PER_CU = 6;
+      if (WS_X == 8 || grid < 2 * (int64_t)g_attn_cus) {
+        using P = AttnWalkCfg<WS_Y, WS_X, HAS_BIAS>;
+        const int64_t most = (int64_t)PER_CU * g_attn_cus;
+        hipLaunchKernelGGL((window_attention_walk_kernel<WS_Y, WS_X, HAS_BIAS>), dim3((unsigned)(grid < most ? grid : most)), dim3(P::NT),
+                           P::SMEM, stream, p, (int)grid);
+        return hipGetLastError();
+      }
+    }
+    if constexpr (WS_X > 8) {
+      if (grid >= 2 * (int64_t)g_attn_cus) {  // enough units for every CU to stream a few: the persistent form
+        using P = AttnPersistCfg<WS_Y, WS_X, HAS_BIAS>;
+        hipLaunchKernelGGL((window_attention_persist_kernel<WS_Y, WS_X, HAS_BIAS>), dim3((unsigned)g_attn_cus), dim3(P::NT), P::SMEM,
+                           stream, p, (int)grid);
+        return hipGetLastError();
+      }
+    }
+    if constexpr (WS_X == 16) {
+      using D = AttnDmaCfg<WS_Y, WS_X, HAS_BIAS>;
+      hipLaunchKernelGGL((window_attention_dma_kernel<WS_Y, WS_X, HAS_BIAS>), dim3((unsigned)grid), dim3(D::NT), D::SMEM,
+                         stream, p);
       return hipGetLastError();
     }
-    using D = AttnDmaCfg<WS_Y, WS_X, HAS_BIAS>;
-    hipLaunchKernelGGL((window_attention_dma_kernel<WS_Y, WS_X, HAS_BIAS>), dim3((unsigned)grid), dim3(D::NT), D::SMEM,
-                       stream, p);
-    return hipGetLastError();
   }
   hipLaunchKernelGGL((window_attention_kernel<WS_Y, WS_X, HD, HAS_BIAS>), dim3((unsigned)grid), dim3(Cfg::NT),
                      Cfg::SMEM, stream, p);

@@ -336,6 +336,22 @@ def test_window_attention_planes_parity(pkg, cuda, case, prescaled):
         assert (out.float().cpu().view(B, H * W, inner) - ref).abs().max() < 0.06
 
 
+@pytest.mark.parametrize("prescaled", [True, False], ids=["qscaled", "qraw"])
+@pytest.mark.parametrize("case", [
+    (1, 8, 8, 1, 64, 8, 4, True, True, 1.0),        # one unit, every border region in it
+    (1, 64, 256, 8, 64, 8, 4, True, True, 1.0),     # 2048 units: more than run at once, workgroups cross from head to head
+    (2, 64, 64, 13, 64, 8, 0, False, False, 1.0),   # 1664 units, no bias
+    (1, 64, 256, 7, 64, 8, 4, True, True, 6.0),     # two-pass form, 1792 units
+    (1, 12, 12, 1, 64, 12, 6, True, True, 1.0),
+    (2, 24, 24, 63, 64, 12, 6, True, True, 1.0),    # 504 units: the largest below the persistent form
+    (2, 24, 24, 64, 64, 12, 6, True, True, 1.0),    # 512: the smallest of the persistent form
+    (2, 24, 24, 9, 64, 12, 6, True, True, 6.0),
+], ids=lambda c: f"B{c[0]}_{c[1]}x{c[2]}_h{c[3]}_ws{c[5]}_s{c[6]}_b{int(c[7])}m{int(c[8])}_x{c[9]:g}")
+def test_window_attention_several_workgroups_per_cu(pkg, cuda, case, prescaled):
+    """8x8 windows, and 12x12 ones with few units: same oracle and tolerance as the other head-plane cases."""
+    test_window_attention_planes_parity(pkg, cuda, case, prescaled)
+
+
 STREAM_CASES = [
     # B, H, W, heads, head_dim, ws_y, ws_x, shift_y, shift_x  -- shapes only the streaming kernel takes
     (1, 120, 120, 2, 128, 60, 60, 30, 30),   # the reference's window: 3600 tokens, head_dim 128 (model.py:22-27), shifted

@@ -176,26 +176,43 @@ __global__ void __launch_bounds__(256) norm_modulate_kernel(NormParams p) {
   }
 }
 
+// sum over the 64 / SUB lanes of a row, the same value in each of them, in wave_sum's order (lanes without elements add zeros)
+template <int SUB>
+__device__ __forceinline__ float lanes_sum(float v) {
+  if (SUB == 1) return wave_sum(v);
+  v = dpp_add<0xB1, 0xF>(v);   // quad_perm [1,0,3,2]
+  v = dpp_add<0x4E, 0xF>(v);   // quad_perm [2,3,0,1]
+  v = dpp_add<0x141, 0xF>(v);  // row_half_mirror
+  v = dpp_add<0x140, 0xF>(v);  // row_mirror: every lane holds the sum of its 16
+  if (SUB == 2) {              // + that of the other 16 of the 32
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  }
+  return v;
+}
+
 // Rows of up to 2048 elements: a kernel without a loop.  A block of four waves takes 4 * ROWS consecutive rows of one
-// batch entry (wave w the rows w, w + 4, ...), requests all of them first, folds the per-column parameters once into
+// batch entry (wave w the rows w, w + 4, ...; SUB rows side by side in a wave's lanes count as so many waves), requests all of them first, folds the per-column parameters once into
 // LDS while the rows are in flight (as fp32, the first and second four columns of a lane's eight in separate arrays so
 // that the 16-byte reads of neighbouring lanes do not share banks), and then normalises row by row.  Short-lived waves
 // with few registers (eight waves per SIMD) keep more bytes in flight and mix loads and stores more evenly than waves
 // that walk down the matrix: a plain copy reaches 5.85 TB/s this way against 5.3 TB/s with the persistent structure.
-template <int NV, bool X_F32, bool PRE, bool FULL, int ROWS>
+template <int NV, bool X_F32, bool PRE, bool FULL, int ROWS, int SUB>
 __global__ void __launch_bounds__(256) norm_modulate_block_kernel(NormParams p, int64_t blocks_per_batch) {
-  constexpr int GROUPS = NV * 64;  // column groups of 8 that the LDS arrays hold
+  static_assert(SUB == 1 || NV == 1, "several rows in a wave's lanes: rows of one column group per lane");
+  constexpr int LPR = 64 / SUB;  // lanes of a row
+  constexpr int GROUPS = NV * LPR;  // column groups of 8 that the LDS arrays hold
   __shared__ f32x4 sG[2][GROUPS], sB[2][GROUPS];
   __shared__ f32x4 sP1[PRE ? 2 : 1][PRE ? GROUPS : 1], sP0[PRE ? 2 : 1][PRE ? GROUPS : 1];
   typedef __attribute__((address_space(1))) const unsigned char* gc_ptr;
   typedef __attribute__((address_space(1))) unsigned char* g_ptr;
   const gc_ptr xg = (gc_ptr)p.x;
   const g_ptr yg = (g_ptr)p.y;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int lane = threadIdx.x & (LPR - 1), w = threadIdx.x / LPR;  // lane within the row's lanes; row slot of the block
   const int d = p.d;
   const float inv_d = 1.0f / (float)d;
   const int64_t b = (int64_t)blockIdx.x / blocks_per_batch;
-  const int64_t first = b * p.rows_per_batch + ((int64_t)blockIdx.x - b * blocks_per_batch) * (4 * ROWS);
+  const int64_t first = b * p.rows_per_batch + ((int64_t)blockIdx.x - b * blocks_per_batch) * (4 * SUB * ROWS);
   int64_t end = (b + 1) * p.rows_per_batch;  // rows of this batch entry end here
   if (end > p.rows) end = p.rows;
 
@@ -203,11 +220,11 @@ __global__ void __launch_bounds__(256) norm_modulate_block_kernel(NormParams p, 
   Raw raw[ROWS][NV];
 #pragma unroll
   for (int j = 0; j < ROWS; ++j) {
-    int64_t row = first + j * 4 + w;
+    int64_t row = first + j * (4 * SUB) + w;
     if (row > end - 1) row = end - 1;  // past the end: the last row again, never stored
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
-      const int col = (v * 64 + lane) * 8;
+      const int col = (v * LPR + lane) * 8;
       raw[j][v].a = u32x4{0u, 0u, 0u, 0u};
       raw[j][v].b = u32x4{0u, 0u, 0u, 0u};
       if (FULL || col < d) {
@@ -281,12 +298,12 @@ __global__ void __launch_bounds__(256) norm_modulate_block_kernel(NormParams p, 
 
 #pragma unroll
   for (int j = 0; j < ROWS; ++j) {
-    const int64_t row = first + j * 4 + w;
+    const int64_t row = first + j * (4 * SUB) + w;
     float u[NV][8];
     float s = 0.f;
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
-      const int g = v * 64 + lane;
+      const int g = v * LPR + lane;
       const bool act = FULL || g * 8 < d;
       if (X_F32) {
 #pragma unroll
@@ -312,7 +329,7 @@ __global__ void __launch_bounds__(256) norm_modulate_block_kernel(NormParams p, 
 #pragma unroll
       for (int e = 0; e < 8; ++e) s += (p.kind == AERIS_NORM_RMS) ? u[v][e] * u[v][e] : u[v][e];
     }
-    s = wave_sum(s);
+    s = lanes_sum<SUB>(s);
     float mean = 0.f, rstd;
     if (p.kind == AERIS_NORM_RMS) {
       rstd = rsqrtf(s * inv_d + p.eps);
@@ -321,20 +338,20 @@ __global__ void __launch_bounds__(256) norm_modulate_block_kernel(NormParams p, 
       float qs = 0.f;
 #pragma unroll
       for (int v = 0; v < NV; ++v) {
-        const bool act = FULL || (v * 64 + lane) * 8 < d;
+        const bool act = FULL || (v * LPR + lane) * 8 < d;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           const float c = act ? u[v][e] - mean : 0.f;
           qs += c * c;
         }
       }
-      qs = wave_sum(qs);
+      qs = lanes_sum<SUB>(qs);
       rstd = rsqrtf(qs * inv_d + p.eps);
     }
     if (row < end) {
 #pragma unroll
       for (int v = 0; v < NV; ++v) {
-        const int g = v * 64 + lane;
+        const int g = v * LPR + lane;
         if (!(FULL || g * 8 < d)) continue;
         const f32x4 ga = sG[0][g], gb = sG[1][g], ba = sB[0][g], bb = sB[1][g];
         float o[8];
@@ -358,36 +375,50 @@ __global__ void __launch_bounds__(256) norm_modulate_block_kernel(NormParams p, 
 
 bool norm_supported(int d) { return d > 0 && d % 8 == 0 && d <= 12 * 512; }
 
+template <int NV, int ROWS, int SUB>
+static hipError_t launch_rows(NormParams p, bool x_f32, bool pre, hipStream_t stream) {
+  constexpr int BLOCK = 4 * SUB * ROWS;  // rows of a block, all of one batch entry
+  if (!p.mod_batch_stride) p.rows_per_batch = p.rows;
+  const int64_t batches = (p.rows + p.rows_per_batch - 1) / p.rows_per_batch, bpb = (p.rows_per_batch + BLOCK - 1) / BLOCK;
+  if (batches * bpb >= (int64_t(1) << 31)) return hipErrorInvalidValue;
+  const dim3 grid((unsigned)(batches * bpb)), block(256);
+#define AERIS_NORM_BLK(XF, PR)                                                                                            \
+  do {                                                                                                                    \
+    if (p.d == NV * 512 / SUB)                                                                                            \
+      hipLaunchKernelGGL((norm_modulate_block_kernel<NV, XF, PR, true, ROWS, SUB>), grid, block, 0, stream, p, bpb);      \
+    else                                                                                                                  \
+      hipLaunchKernelGGL((norm_modulate_block_kernel<NV, XF, PR, false, ROWS, SUB>), grid, block, 0, stream, p, bpb);     \
+  } while (0)
+  if (x_f32) {
+    if (pre) AERIS_NORM_BLK(true, true);
+    else AERIS_NORM_BLK(true, false);
+  } else {
+    if (pre) AERIS_NORM_BLK(false, true);
+    else AERIS_NORM_BLK(false, false);
+  }
+#undef AERIS_NORM_BLK
+  return hipGetLastError();
+}
+
+// Four rows per wave and lane group (1, 2, 3: 2-4 % slower on 1 036 800 rows of 1536), one where that leaves a CU with no more than
+// two blocks: 2048 x 128 bf16 3.8 -> 2.8 us, 2048 x 512 f32 4.9 -> 3.7, 4704 x 640 7.0 -> 5.8, 8192 x 1536 16.3 -> 15.6; at 728
+// blocks (23296 x 192) 6.7 against 7.3.
+template <int NV, int SUB>
+static hipError_t launch_few_or_many(const NormParams& p, bool x_f32, bool pre, hipStream_t stream) {
+  return p.rows <= (int64_t)512 * 16 * SUB ? launch_rows<NV, 1, SUB>(p, x_f32, pre, stream) : launch_rows<NV, 4, SUB>(p, x_f32, pre, stream);
+}
+
 template <int NV>
 static hipError_t launch_norm(const NormParams& p, bool x_f32, bool pre, hipStream_t stream) {
   if constexpr (NV <= 4) {
-    // rows of up to 2048 elements: blocks of 4 waves x 4 rows that never straddle a batch entry (1, 2, 3 rows per wave: 2-4 % slower)
-    constexpr int ROWS = 4;
-    const int64_t rpb = p.mod_batch_stride ? p.rows_per_batch : p.rows;
-    const int64_t batches = (p.rows + rpb - 1) / rpb;
-    const int64_t bpb = (rpb + 4 * ROWS - 1) / (4 * ROWS);
-    if (batches * bpb >= (int64_t(1) << 31)) return hipErrorInvalidValue;
-    {
-      NormParams q = p;
-      q.rows_per_batch = rpb;
-      dim3 grid((unsigned)(batches * bpb)), block(256);
-#define AERIS_NORM_BLK(XF, PR)                                                                                           \
-  do {                                                                                                                   \
-    if (p.d == NV * 512)                                                                                                   \
-      hipLaunchKernelGGL((norm_modulate_block_kernel<NV, XF, PR, true, ROWS>), grid, block, 0, stream, q, bpb);                  \
-    else                                                                                                                   \
-      hipLaunchKernelGGL((norm_modulate_block_kernel<NV, XF, PR, false, ROWS>), grid, block, 0, stream, q, bpb);                 \
-  } while (0)
-      if (x_f32) {
-        if (pre) AERIS_NORM_BLK(true, true);
-        else AERIS_NORM_BLK(true, false);
-      } else {
-        if (pre) AERIS_NORM_BLK(false, true);
-        else AERIS_NORM_BLK(false, false);
-      }
-#undef AERIS_NORM_BLK
-      return hipGetLastError();
+    // Rows of up to 2048 elements: blocks of four waves that never straddle a batch entry.  Rows of up to 256 (128) elements lie in
+    // half (a quarter) of a wave's lanes, two (four) beside each other: 500 000 x 128 f32 104.7 -> 65.9 us, 500 000 x 256 bf16
+    // 109.8 -> 83.7, 23296 x 192 f32 9.3 -> 6.7.
+    if constexpr (NV == 1) {
+      if (p.d <= 128) return launch_few_or_many<NV, 4>(p, x_f32, pre, stream);
+      if (p.d <= 256) return launch_few_or_many<NV, 2>(p, x_f32, pre, stream);
     }
+    return launch_few_or_many<NV, 1>(p, x_f32, pre, stream);
   } else {
   // enough waves to cover HBM latency, few enough that parameter folding is amortised over many rows
   int64_t blocks = (p.rows + 3) / 4;

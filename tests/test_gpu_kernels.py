@@ -777,6 +777,27 @@ def test_norm_modulate_parity(pkg, cuda, d, kind, order, xdt):
     assert rel_l2(out32, ref) <= 1e-5
 
 
+@pytest.mark.parametrize("d", [8, 120, 128, 136, 192, 256, 264])  # one, two or four rows in a wave's lanes, full and not
+@pytest.mark.parametrize("B,S", [(3, 333), (1, 1), (2, 17), (2, 17000)])  # one row per wave and lane group, or (34000 rows) four
+@pytest.mark.parametrize("kind,order", [("layernorm", "norm_then_mod"), ("rmsnorm", "mod_then_norm")])
+def test_norm_modulate_short_rows(pkg, cuda, d, B, S, kind, order):
+    g = torch.Generator().manual_seed(d + S)
+    x = 1.5 * torch.randn(B, S, d, generator=g) + 0.3
+    gamma, beta = 1 + 0.2 * torch.randn(d, generator=g), 0.2 * torch.randn(d, generator=g) if kind == "layernorm" else None
+    mods = 0.3 * torch.randn(B, 2 * d, generator=g)
+    shift, scale = mods[:, :d], mods[:, d:]
+
+    def norm(v):
+        return oracle.layer_norm(v, gamma, beta, 1e-5) if kind == "layernorm" else oracle.rms_norm(v, gamma, 1e-5)
+
+    ref = norm(oracle.modulate(x, shift, scale)) if order == "mod_then_norm" else oracle.modulate(norm(x), shift, scale)
+    md = mods.to(cuda)
+    out = pkg.ops.norm_modulate(x.to(cuda), gamma.to(cuda), None if beta is None else beta.to(cuda), md[:, :d], md[:, d:], kind=kind,
+                                order=order, eps=1e-5, out_dtype=torch.float32)
+    torch.cuda.synchronize()
+    assert rel_l2(out, ref) <= 1e-5  # f32 sums of at most 264 terms
+
+
 def test_norm_modulate_variants(pkg, cuda):
     d, B, S = 512, 2, 50
     g = torch.Generator().manual_seed(1)

@@ -18,7 +18,7 @@ from concurrent.futures import ThreadPoolExecutor
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(CSRC, "libaeris_hip.so")
-SOURCES = ["api.hip", "gemm.hip", "gemm_persistent.hip", "window_attention.hip", "qkv_window_attention.hip", "window_attention_stream.hip", "norm_modulate.hip", "small_ops.hip", "output_stage.hip", "input_stage.hip"]
+SOURCES = ["api.hip", "gemm.hip", "gemm_persistent.hip", "gemm_norm.hip", "window_attention.hip", "qkv_window_attention.hip", "window_attention_stream.hip", "norm_modulate.hip", "small_ops.hip", "output_stage.hip", "input_stage.hip"]
 HEADERS = ["common.h", "kernels.h", "gemm_common.h", "attention_sweep.h", os.path.join("..", "..", "include", "aeris_hip.h")]
 # sources whose transposing LDS reads are inline assembly: their device assembly is checked after every compile
 # (asm_check.py says for what); the compile keeps its temporaries for that, in a scratch directory

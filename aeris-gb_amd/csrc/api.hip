@@ -499,6 +499,35 @@ int aeris_input_stage_fwd(const float* x0, int C0, float div0, const float* x1, 
 // the layouts callers build without this header (ctypes / struct.pack): 8-byte fields, no padding
 static_assert(sizeof(aeris_block) == 20 * 8 && sizeof(aeris_block_config) == 17 * 8 && sizeof(aeris_modulation_layer) == 5 * 8, "ABI");
 
+namespace {
+// The norm of a block and the projection behind it as one kernel (split > 0: into head planes, the first q_cols columns scaled),
+// for arguments that aeris_norm_modulate_fwd and the aeris_gemm_fwd or aeris_gemm_heads_fwd call behind it would both take: what
+// those refuse is left to them.  `y`, their intermediate, is not written.
+int norm_gemm_fwd(const aeris_block_config* c, int64_t mod_stride, const void* x, const void* y, const void* gamma, const void* beta,
+                  const float* shift, const float* scale, const void* W, const void* bias, void* C, int64_t N, int act, int split,
+                  float q_scale, int64_t q_cols, void* stream, bool* taken) {
+  *taken = false;
+  const int64_t B = c->B, rows = c->H * c->W;
+  for (const void* p : {x, y, gamma, W, static_cast<const void*>(C)})
+    if (!p || !aligned16(p)) return AERIS_OK;
+  if (!aligned16(beta) || !aligned16(shift) || !aligned16(scale) || (shift && (mod_stride < 0 || (mod_stride & 3)))) return AERIS_OK;
+  if ((c->x_dtype != AERIS_BF16 && c->x_dtype != AERIS_F32) || (c->norm_dtype != AERIS_BF16 && c->norm_dtype != AERIS_F32) ||
+      (c->norm_kind != AERIS_NORM_LAYER && c->norm_kind != AERIS_NORM_RMS) ||
+      (c->mod_order != AERIS_NORM_THEN_MOD && c->mod_order != AERIS_MOD_THEN_NORM) || !((float)c->eps >= 0.f) || split % 8 ||
+      !(q_scale > 0.f && q_scale < 3.0e38f) || N > 0x7fffffffLL || rows > 0x7fffffffLL / B)
+    return AERIS_OK;
+  if (!aeris::norm_gemm_takes(B * rows, (int)N, (int)c->dim, bias, shift != nullptr, mod_stride, B, rows, act == AERIS_ACT_SWIGLU))
+    return AERIS_OK;
+  if (int rc = ensure_init(stream, true)) return rc;
+  *taken = true;
+  const hipError_t e = aeris::norm_gemm_launch(x, (int)c->x_dtype, gamma, beta, (int)c->norm_dtype, shift, scale, mod_stride, rows,
+                                               (int)c->norm_kind, (int)c->mod_order, (float)c->eps, W, C, bias, B * rows, (int)N,
+                                               (int)c->dim, N, act, split, B * rows * split, q_scale, (int)q_cols,
+                                               reinterpret_cast<hipStream_t>(stream));
+  return e == hipSuccess ? AERIS_OK : hip_fail(e, "aeris_blocks_fwd: norm and projection launch");
+}
+}  // namespace
+
 int aeris_blocks_fwd(const aeris_block_config* c, const aeris_block* blocks, int n, const void* x, void* out,
                      void* norm_scratch, void* qkv_scratch, void* attn_scratch, void* hidden_scratch, void* const* events,
                      void* stream) {
@@ -542,25 +571,41 @@ int aeris_blocks_fwd(const aeris_block_config* c, const aeris_block* blocks, int
     }
     const void* in = i == 0 ? x : out;
     const int sy = (int)b.shift_y, sx = (int)b.shift_x;
-    STEP(aeris_norm_modulate_fwd(in, xdt, norm_scratch, AERIS_BF16, b.norm1_weight, b.norm1_bias, (int)c->norm_dtype, shift1, scale1,
-                                 b.modulation_stride, B, rows, d, (int)c->norm_kind, (int)c->mod_order, eps, stream));
-    if (b.fuse_qkv && aeris::qkv_attention_supported(wy, wx, hd, d, rows) && 3 * inner * d * 2 < (int64_t(1) << 31)) {
+    const bool one_kernel_attention =
+        b.fuse_qkv && aeris::qkv_attention_supported(wy, wx, hd, d, rows) && 3 * inner * d * 2 < (int64_t(1) << 31);
+    constexpr float LOG2E = 1.4426950408889634f;
+    bool done = false;  // the norm and the projection behind it, in one kernel (not where each call is timed by itself)
+    if (!events && !one_kernel_attention)
+      if (int rc = norm_gemm_fwd(c, b.modulation_stride, in, norm_scratch, b.norm1_weight, b.norm1_bias, shift1, scale1, b.qkv_weight,
+                                 b.qkv_bias, qkv_scratch, 3 * inner, AERIS_ACT_NONE, hd, scale * LOG2E, inner, stream, &done))
+        return rc;
+    if (!done)
+      STEP(aeris_norm_modulate_fwd(in, xdt, norm_scratch, AERIS_BF16, b.norm1_weight, b.norm1_bias, (int)c->norm_dtype, shift1, scale1,
+                                   b.modulation_stride, B, rows, d, (int)c->norm_kind, (int)c->mod_order, eps, stream));
+    if (one_kernel_attention) {
       STEP(aeris_qkv_window_attention_fwd(norm_scratch, b.qkv_weight, b.qkv_bias, b.bias4, attn_scratch, B, H, W, heads, hd, d, wy, wx,
                                           sy, sx, (int)b.use_mask, scale, stream));
     } else {
       if (!qkv_scratch) return fail(AERIS_EINVAL, "%s: block %d needs qkv_scratch", who, i);
-      constexpr float LOG2E = 1.4426950408889634f;
-      STEP(aeris_gemm_heads_fwd(norm_scratch, b.qkv_weight, qkv_scratch, b.qkv_bias, T, (int)(3 * inner), d, hd, T * hd, scale * LOG2E,
-                                heads, stream));
+      if (!done)
+        STEP(aeris_gemm_heads_fwd(norm_scratch, b.qkv_weight, qkv_scratch, b.qkv_bias, T, (int)(3 * inner), d, hd, T * hd, scale * LOG2E,
+                                  heads, stream));
       STEP(aeris_window_attention_heads_fwd(qkv_scratch, attn_scratch, b.bias_table, B, H, W, heads, hd, wy, wx, sy, sx,
                                             (int)b.use_mask, scale, 1, T * hd, stream));
     }
     STEP(aeris_gemm_fwd(attn_scratch, b.wo_weight, out, b.wo_bias, gate1, in, T, d, (int)inner, d, AERIS_ACT_NONE, xdt, xdt,
                         gate1 ? b.modulation_stride : 0, rows, stream));
-    STEP(aeris_norm_modulate_fwd(out, xdt, norm_scratch, AERIS_BF16, b.norm2_weight, b.norm2_bias, (int)c->norm_dtype, shift2, scale2,
-                                 b.modulation_stride, B, rows, d, (int)c->norm_kind, (int)c->mod_order, eps, stream));
-    STEP(aeris_gemm_fwd(norm_scratch, b.up_weight, hidden_scratch, b.up_bias, nullptr, nullptr, T, hidden, d, hidden, (int)c->mlp_act, 0,
-                        AERIS_BF16, 0, T, stream));
+    done = false;
+    if (!events)
+      if (int rc = norm_gemm_fwd(c, b.modulation_stride, out, norm_scratch, b.norm2_weight, b.norm2_bias, shift2, scale2, b.up_weight,
+                                 b.up_bias, hidden_scratch, hidden, (int)c->mlp_act, 0, 1.0f, 0, stream, &done))
+        return rc;
+    if (!done) {
+      STEP(aeris_norm_modulate_fwd(out, xdt, norm_scratch, AERIS_BF16, b.norm2_weight, b.norm2_bias, (int)c->norm_dtype, shift2, scale2,
+                                   b.modulation_stride, B, rows, d, (int)c->norm_kind, (int)c->mod_order, eps, stream));
+      STEP(aeris_gemm_fwd(norm_scratch, b.up_weight, hidden_scratch, b.up_bias, nullptr, nullptr, T, hidden, d, hidden, (int)c->mlp_act, 0,
+                          AERIS_BF16, 0, T, stream));
+    }
     STEP(aeris_gemm_fwd(hidden_scratch, b.down_weight, out, b.down_bias, gate2, out, T, d, hidden, d, AERIS_ACT_NONE, xdt, xdt,
                         gate2 ? b.modulation_stride : 0, rows, stream));
   }

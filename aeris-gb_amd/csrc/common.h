@@ -48,6 +48,21 @@ __device__ __forceinline__ float wave_sum(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
 }
 
+// sum over the 64 / SUB lanes of a row, the same value in each of them, in wave_sum's order (lanes without elements add zeros)
+template <int SUB>
+__device__ __forceinline__ float lanes_sum(float v) {
+  if (SUB == 1) return wave_sum(v);
+  v = dpp_add<0xB1, 0xF>(v);   // quad_perm [1,0,3,2]
+  v = dpp_add<0x4E, 0xF>(v);   // quad_perm [2,3,0,1]
+  v = dpp_add<0x141, 0xF>(v);  // row_half_mirror
+  v = dpp_add<0x140, 0xF>(v);  // row_mirror: every lane holds the sum of its 16
+  if (SUB == 2) {              // + that of the other 16 of the 32
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  }
+  return v;
+}
+
 // ---- buffer_load_dwordx4 ... lds (16 bytes per lane from global memory straight into LDS, lane l at LDS byte
 // m0 + 16 l) as inline assembly.  The compiler's builtin form makes every later LDS access a possible alias of the load
 // in the compiler's eyes: it then guards LDS reads with s_waitcnt vmcnt(0) wherever it cannot count the operations in

@@ -15,6 +15,15 @@ hipError_t gemm_launch(const void* A, const void* W, void* C, const void* bias, 
                        int c_dtype, int64_t gate_batch_stride, int64_t rows_per_batch, int split, int64_t plane_stride,
                        float q_scale, int q_cols, hipStream_t stream);
 
+// norm, modulation and the projection behind them in one kernel (gemm_norm.hip), for what norm_gemm_takes says; act is
+// AERIS_ACT_NONE (bf16 C, `split` as above), _GELU or _SWIGLU
+bool norm_gemm_takes(int64_t M, int N, int K, const void* bias, bool modulated, int64_t mod_batch_stride, int64_t B,
+                     int64_t rows_per_batch, bool swiglu);
+hipError_t norm_gemm_launch(const void* x, int x_dtype, const void* gamma, const void* beta, int param_dtype, const float* shift,
+                            const float* scale, int64_t mod_batch_stride, int64_t rows_per_batch, int kind, int order, float eps,
+                            const void* W, void* C, const void* bias, int64_t M, int N, int K, int64_t ldc, int act, int split,
+                            int64_t plane_stride, float q_scale, int q_cols, hipStream_t stream);
+
 // returns hipErrorInvalidValue when (ws_y, ws_x, head_dim) has no instantiation.  q / k / v of (token, head) start at
 // part * part_stride + head * head_stride + token * tok_stride (elements) for part = 0, 1, 2
 bool attention_supported(int ws_y, int ws_x, int head_dim);

@@ -176,21 +176,6 @@ __global__ void __launch_bounds__(256) norm_modulate_kernel(NormParams p) {
   }
 }
 
-// sum over the 64 / SUB lanes of a row, the same value in each of them, in wave_sum's order (lanes without elements add zeros)
-template <int SUB>
-__device__ __forceinline__ float lanes_sum(float v) {
-  if (SUB == 1) return wave_sum(v);
-  v = dpp_add<0xB1, 0xF>(v);   // quad_perm [1,0,3,2]
-  v = dpp_add<0x4E, 0xF>(v);   // quad_perm [2,3,0,1]
-  v = dpp_add<0x141, 0xF>(v);  // row_half_mirror
-  v = dpp_add<0x140, 0xF>(v);  // row_mirror: every lane holds the sum of its 16
-  if (SUB == 2) {              // + that of the other 16 of the 32
-    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
-  }
-  return v;
-}
-
 // Rows of up to 2048 elements: a kernel without a loop.  A block of four waves takes 4 * ROWS consecutive rows of one
 // batch entry (wave w the rows w, w + 4, ...; SUB rows side by side in a wave's lanes count as so many waves), requests all of them first, folds the per-column parameters once into
 // LDS while the rows are in flight (as fp32, the first and second four columns of a lane's eight in separate arrays so

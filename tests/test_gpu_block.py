@@ -498,3 +498,37 @@ def test_block_result_of_another_type_than_the_stream(pkg, cuda):
         out = torch.empty(1, 2048, 128, dtype=out_dtype, device=cuda)
         layer.block_forward(0, x.to(x_dtype).to(cuda), t.to(cuda), (0, 0), out=out)
         assert rel_l2(out, oracle.block_forward(cfg, sd, x.to(x_dtype).float(), t, (0, 0))) <= 1e-2
+
+
+@pytest.mark.parametrize("B,image,window,dim,heads,hd,hidden,form,x_dtype", [
+    (1, (8, 8), (8, 8), 64, 2, 32, 192, "spec0", torch.bfloat16),       # one row tile
+    (1, (5, 13), (5, 13), 128, 1, 128, 64, "ref", torch.float32),       # 65 rows: one past a tile; one tile of w1's columns
+    (3, (8, 8), (8, 8), 128, 4, 32, 128, "ref", torch.float32),         # a modulation row per tile
+    (2, (12, 36), (12, 12), 64, 1, 64, 64, "spec3", torch.float32),     # ... which 432 rows refuse: two kernels
+    (1, (12, 36), (12, 12), 128, 2, 32, 320, "swiglu", torch.bfloat16),
+    (1, (168, 256), (8, 8), 128, 2, 64, 512, "swiglu", torch.float32),  # more row tiles than workgroups wanted (GELU would be the polynomial in the call by itself)
+])
+def test_block_norm_and_projection_in_one_kernel(pkg, cuda, B, image, window, dim, heads, hd, hidden, form, x_dtype):
+    """dim <= 128: the block's norms run inside the projections behind them, but not while each call is timed: same bits, and
+    both within the block's bar of the fp32 oracle."""
+    geo = dict(dim=dim, heads=heads, head_dim=hd, mlp_dim=hidden, window_size=window, image_shape=image)
+    mk = {"spec0": lambda: OracleConfig.spec(mod_ways=0, **geo), "spec3": lambda: OracleConfig.spec(mod_ways=3, **geo),
+          "ref": lambda: OracleConfig.ref(**geo),
+          "swiglu": lambda: OracleConfig.spec(norm="rmsnorm", mlp="swiglu", bias=False, mod_ways=3, **geo)}
+    cfg = mk[form]()
+    sd = oracle.init_block_weights(cfg, 11, nontrivial=True)
+    g = torch.Generator().manual_seed(12)
+    x = (torch.randn(B, image[0] * image[1], dim, generator=g) * 2 + 0.5).to(x_dtype)
+    t = torch.randn(B, dim, generator=g) if cfg.mod_ways else None
+    layer = make_layer(pkg, cfg, sd, cuda)
+    xg, tg = x.to(cuda), None if t is None else t.to(cuda)
+    with torch.no_grad():
+        out = layer(xg, tg)
+        pkg.ops.profile_begin()
+        try:
+            timed = layer(xg, tg)
+        finally:
+            pkg.ops.profile_end()
+    assert torch.equal(out, timed)
+    if image[0] * image[1] <= 4096:
+        assert rel_l2(out, oracle.block_forward(cfg, sd, x.float(), t, (0, 0))) <= 1e-2

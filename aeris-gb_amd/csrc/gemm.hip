@@ -6,14 +6,14 @@
 // other, so one's first loads and epilogue fall under another's main loop), three k-tiles in flight, every epilogue
 // operand requested ahead of the main loop, and little code (fetched cold: the kernel before this one, 128 x 128
 // register-staged with every epilogue option in one body, took 18-24 us for what takes 4-5 us here).  Measured before -> after:
-// 2048 x 128 x 128 17.9 -> 3.8 us, 2048 x 128 x 512 22.1 -> 5.3 us, 2048 x 256 x 1024 32.1 -> 8.3 us, 8192 x 256 x 256 25.0 ->
-// 7.0 us.  128 x 128 tiles of the same kernel take what neither this size nor the persistent kernel can (odd N, unaligned
+// 2048 x 128 x 128 17.9 -> 3.8 us, 2048 x 128 x 512 22.1 -> 5.0 us, 2048 x 256 x 1024 32.1 -> 7.1 us, 8192 x 256 x 256 25.0 ->
+// 6.8 us.  128 x 128 tiles of the same kernel take what neither this size nor the persistent kernel can (odd N, unaligned
 // rows, W of 2 GiB and more, SiLU).
 //   - global loads go straight into LDS (buffer_load ... lds, 16 bytes per lane); a load instruction of a wave fetches
 //     8 rows x 128 B and the lane -> chunk map is the inverse of the LDS swizzle (swz_off), so fragment reads are
 //     conflict-free ds_read_b128 and nothing is staged through registers
 //   - STAGES k-tiles of 64 in LDS, one barrier per k-tile: the loads of k-tile j + STAGES - 1 are issued right behind the
-//     barrier that ends the reading of k-tile j - 1, and waited for with a counted vmcnt
+//     barrier that ends the reading of k-tile j - 1 and the fragment reads of k-tile j, and waited for with a counted vmcnt
 //   - v_mfma_f32_16x16x32_bf16 with the weight fragment first and accumulators that start at the bias: the same
 //     arithmetic in the same order as the persistent kernel, bit for bit
 //   - the epilogue works on the accumulators where they are: a lane holds 4 consecutive n of one row; for bf16 C two column
@@ -202,21 +202,27 @@ __global__ void __launch_bounds__(NT, 2) gemm_bf16_nt_tile_kernel(GemmParams p) 
     if (STAGES > 2 && behind >= STAGES - 2) wait_barrier<(STAGES - 2) * LPT>();
     else if (STAGES > 3 && behind == 1) wait_barrier<LPT>();
     else wait_barrier<0>();
-    if (behind >= STAGES - 1) issue(kt + STAGES - 1, wr);
     const unsigned char* st = smem + rd * STAGE;
+    bf16x8 af[2][FM], bf[2][FN];
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
-      bf16x8 af[FM], bf[FN];
 #pragma unroll
-      for (int i = 0; i < FM; ++i) af[i] = *reinterpret_cast<const bf16x8*>(st + a_roff[ks] + i * 16 * 128);
+      for (int i = 0; i < FM; ++i) af[ks][i] = *reinterpret_cast<const bf16x8*>(st + a_roff[ks] + i * 16 * 128);
 #pragma unroll
-      for (int j = 0; j < FN; ++j) bf[j] = *reinterpret_cast<const bf16x8*>(st + b_roff[ks] + j * 16 * 128);
+      for (int j = 0; j < FN; ++j) bf[ks][j] = *reinterpret_cast<const bf16x8*>(st + b_roff[ks] + j * 16 * 128);
+    }
+    // The loads come behind the fragment reads: each holds the wave for 70-95 cycles, in which the fragments arrive.  (The serial chain
+    // of a k-tile, not the latency of its loads, is what a small problem waits for: four, six or nine k-tiles in flight instead of
+    // three measured the same or slower.  Loads first -> reads first: 2048 x 256 x 1024 8.0 -> 7.1 us, 2048 x 512 x 2048 13.0 ->
+    // 10.9, 3000 x 3072 x 1024 33.3 -> 29.4; 2048 x 128 x 128 the same.)
+    if (behind >= STAGES - 1) issue(kt + STAGES - 1, wr);
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
       for (int i = 0; i < FM; ++i)
 #pragma unroll
         for (int j = 0; j < FN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[j], af[i], acc[i][j], 0, 0, 0);
-    }
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[ks][j], af[ks][i], acc[i][j], 0, 0, 0);
     if (++rd == STAGES) rd = 0;
     if (++wr == STAGES) wr = 0;
   }

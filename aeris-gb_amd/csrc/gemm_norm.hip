@@ -250,21 +250,23 @@ __global__ void __launch_bounds__(NT, 2) norm_gemm_kernel(NormGemmParams p) {
     for (int kt = 0; kt < KT; ++kt, ++done) {
       // (the first wait also ends the writing of y)
       wait_k_tile<STAGES - 2>(total - 1 - done);
-      if (done + STAGES - 1 < total) issue();
       const unsigned char *sa = smem + kt * STAGE, *sb = sW + rd * STAGE;
+      bf16x8 af[2][FM], bf[2][FN];
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks) {
-        bf16x8 af[FM], bf[FN];
 #pragma unroll
-        for (int i = 0; i < FM; ++i) af[i] = *reinterpret_cast<const bf16x8*>(sa + a_roff[ks] + i * 16 * 128);
+        for (int i = 0; i < FM; ++i) af[ks][i] = *reinterpret_cast<const bf16x8*>(sa + a_roff[ks] + i * 16 * 128);
 #pragma unroll
-        for (int j = 0; j < FN; ++j) bf[j] = *reinterpret_cast<const bf16x8*>(sb + b_roff[ks] + j * 16 * 128);
+        for (int j = 0; j < FN; ++j) bf[ks][j] = *reinterpret_cast<const bf16x8*>(sb + b_roff[ks] + j * 16 * 128);
+      }
+      if (done + STAGES - 1 < total) issue();  // behind the fragment reads, as in gemm_bf16_nt_tile_kernel
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
         for (int i = 0; i < FM; ++i)
 #pragma unroll
           for (int j = 0; j < FN; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[j], af[i], acc[i][j], 0, 0, 0);
-      }
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[ks][j], af[ks][i], acc[i][j], 0, 0, 0);
       if (++rd == STAGES) rd = 0;
     }
     // ---- epilogue: a lane holds 4 consecutive n of one row

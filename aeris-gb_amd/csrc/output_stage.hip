@@ -134,7 +134,12 @@ __global__ void __launch_bounds__(OS_THREADS) output_stage_kernel(OutStageParams
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   constexpr int NFC = NF * 16;
   constexpr int CHUNK_BYTES = 2 * 2 * NF * 1024;  // two k-steps of 32 x (hi, lo) x NF fragments of 1 KB
-  float* const stg = reinterpret_cast<float*>(smem + 2 * CHUNK_BYTES);  // [64][N] results of the tile
+  // [64][N] results of the tile, over the weight's stages once the last chunk has been read.  40 KB of LDS for 80 columns leave
+  // registers as the limit, three or four workgroups per CU; with an area of its own (58 KB for 69 columns) there were two, too few
+  // loads in flight.  Both folds in one launch included: 259 200 x 512 f32 -> 69 168.6 -> 156.9 us (3.8 TB/s), 51 840 x 320
+  // bf16 30.3 -> 24.6, 8192 x 1536 47.3 -> 43.9, 2048 x 256 14.6 -> 11.8.
+  float* const stg = reinterpret_cast<float*>(smem);
+  static_assert(OS_ROWS * NFC * 4 <= 2 * CHUNK_BYTES, "results of a tile");
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l15 = lane & 15, q = lane >> 4;
   const int64_t m0 = (int64_t)blockIdx.x * OS_ROWS;
@@ -276,7 +281,7 @@ __global__ void __launch_bounds__(OS_THREADS) output_stage_kernel(OutStageParams
 template <int NF>
 hipError_t launch_main(const OutStageParams& p, bool xf, bool ln, hipStream_t stream) {
   const dim3 grid((unsigned)((p.M + OS_ROWS - 1) / OS_ROWS)), block(OS_THREADS);
-  const size_t lds = 2 * (2 * 2 * NF * 1024) + (((size_t)OS_ROWS * p.N * 4 + 15) & ~(size_t)15);
+  const size_t lds = 2 * (2 * 2 * NF * 1024);
 #define GO(XF, LNV) hipLaunchKernelGGL((output_stage_kernel<NF, XF, LNV>), grid, block, lds, stream, p)
   if (xf) { if (ln) GO(true, true); else GO(true, false); }
   else { if (ln) GO(false, true); else GO(false, false); }

@@ -463,6 +463,24 @@ hipError_t launch_kind(Kind kind, const GemmParams& p, hipStream_t stream) {
   return gemm_persistent_launch(p, kind == PERSISTENT256 ? 256 : 128, stream);
 }
 
+Shape shape_of(const GemmParams& p, int act) { return {p.M, p.N, p.K / BK, act, p.c_dtype == AERIS_F32, p.residual != nullptr}; }
+
+// vector epilogue: 8 / 16-byte accesses to C and the residual (4-element alignment of every row), to bias and gate rows
+bool vector_epilogue(const GemmParams& p) {
+  return (p.split || (p.ldc & 3) == 0) && (p.N & 3) == 0 && (reinterpret_cast<uintptr_t>(p.gate) & 15) == 0 &&
+         (p.gate_batch_stride & 3) == 0 && (reinterpret_cast<uintptr_t>(p.bias) & 7) == 0;
+}
+
+// what the persistent kernel cannot take: it addresses W through one buffer descriptor (31-bit size), forms row offsets
+// with 24-bit multiplies, row numbers, gate row offsets and batch numbers in 32 bits, numbers its tiles in 24 bits and
+// scales whole 64-column wave blocks of the query part
+bool persistent_takes(const GemmParams& p) {
+  return p.act != AERIS_ACT_SILU && (int64_t)(p.act == AERIS_ACT_SWIGLU ? 2 : 1) * p.N * p.K * 2 < (int64_t(1) << 31) &&
+         p.ldc < (1 << 23) && p.split < (1 << 23) && p.gate_batch_stride < (int64_t(1) << 31) &&
+         (p.rows_per_batch <= 0 || p.M / p.rows_per_batch < (int64_t(1) << 31)) && p.M + 512 < (int64_t(1) << 31) &&
+         tiles_of(shape_of(p, p.act), 128, 256) < (int64_t(1) << 24) && p.q_cols % 64 == 0 && p.N >= 64;
+}
+
 // the same problem from row `first` on, `rows` of them
 GemmParams rows_of(const GemmParams& p0, int64_t first, int64_t rows) {
   GemmParams p = p0;
@@ -476,6 +494,11 @@ GemmParams rows_of(const GemmParams& p0, int64_t first, int64_t rows) {
 }
 
 }  // namespace
+
+bool gemm_gelu_by_polynomial(const GemmParams& p) {
+  return vector_epilogue(p) && persistent_takes(p) && p.M >= 256 && (p.N % 256 == 0 || p.N >= 1024) &&
+         tiles_of(shape_of(p, AERIS_ACT_GELU), 256, 256) >= 256;
+}
 
 hipError_t gemm_launch(const void* A, const void* W, void* C, const void* bias, const float* gate,
                        const void* residual, int64_t M, int N, int K, int64_t ldc, int act, int res_dtype,
@@ -501,22 +524,13 @@ hipError_t gemm_launch(const void* A, const void* W, void* C, const void* bias, 
   p.act = act == AERIS_ACT_GELU && c_dtype == AERIS_BF16 ? GEMM_ACT_GELU_ERF : act;
   p.res_dtype = residual ? res_dtype : -1;
   p.c_dtype = c_dtype;
-  // vector epilogue: 8 / 16-byte accesses to C and the residual (4-element alignment of every row), to bias and gate rows
-  const bool vec = (split || (ldc & 3) == 0) && (N & 3) == 0 && (reinterpret_cast<uintptr_t>(gate) & 15) == 0 &&
-                   (gate_batch_stride & 3) == 0 && (reinterpret_cast<uintptr_t>(bias) & 7) == 0;
-  if (!vec) return launch_tile_act<128, 128, 2, false>(p, stream);
-  // what the persistent kernel cannot take: it addresses W through one buffer descriptor (31-bit size), forms row offsets
-  // with 24-bit multiplies, row numbers, gate row offsets and batch numbers in 32 bits, numbers its tiles in 24 bits and
-  // scales whole 64-column wave blocks of the query part
-  Shape s = {M, N, K / BK, p.act, c_dtype == AERIS_F32, residual != nullptr};
-  bool persistent_ok = act != AERIS_ACT_SILU && (int64_t)(act == AERIS_ACT_SWIGLU ? 2 : 1) * N * K * 2 < (int64_t(1) << 31) &&
-                             ldc < (1 << 23) && split < (1 << 23) && gate_batch_stride < (int64_t(1) << 31) &&
-                             (rows_per_batch <= 0 || M / rows_per_batch < (int64_t(1) << 31)) && M + 512 < (int64_t(1) << 31) &&
-                             tiles_of(s, 128, 256) < (int64_t(1) << 24) && q_cols % 64 == 0 && N >= 64;
+  if (!vector_epilogue(p)) return launch_tile_act<128, 128, 2, false>(p, stream);
+  Shape s = shape_of(p, p.act);
+  bool persistent_ok = persistent_takes(p);
   // The polynomial where there is a chip's worth of 256 x 256 tiles, erf otherwise: one of them for all rows of a call, whatever
   // tiles they are given to (equal rows, the members of a batch say, have equal results wherever they stand)
   if (p.act == GEMM_ACT_GELU_ERF) {
-    if (persistent_ok && M >= 256 && (N % 256 == 0 || N >= 1024) && tiles_of(s, 256, 256) >= 256)
+    if (gemm_gelu_by_polynomial(p))
       p.act = s.act = AERIS_ACT_GELU;
     else
       persistent_ok = persistent_ok && !gate && !residual;

@@ -62,6 +62,10 @@ __device__ __forceinline__ uint32_t swz_off(int row, int chunk) {
   return (uint32_t)((row >> 1) * 256 + (((((row & 1) << 3) | chunk) ^ ((row >> 1) & 7)) << 4));
 }
 
+// whether a GELU with bf16 C is evaluated by the polynomial (AERIS_ACT_GELU) and not by erf (GEMM_ACT_GELU_ERF): one answer
+// for the GEMM of this shape and alignment and for the kernel that has a norm ahead of it
+bool gemm_gelu_by_polynomial(const GemmParams& p);
+
 // persistent kernel (gemm_persistent.hip), tiles of tile_height (128 or 256) rows x 256 columns; needs N % 4 == 0 and ldc % 4 == 0
 hipError_t gemm_persistent_configure();
 hipError_t gemm_persistent_launch(const GemmParams& p, int tile_height, hipStream_t stream);

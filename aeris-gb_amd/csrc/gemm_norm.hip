@@ -292,6 +292,7 @@ __global__ void __launch_bounds__(NT, 2) norm_gemm_kernel(NormGemmParams p) {
           float x = acc[i][j][e];
           if (SWIGLU) x = silu_f(x) * acc[i][j + NJ][e];
           else if (ACT == GEMM_ACT_GELU_ERF) x = gelu_erf_bf16_f(x);
+          else if (ACT == AERIS_ACT_GELU) x = gelu_bf16_f(x);
           v[j][e] = x;
         }
       uint16_t* const c_row = reinterpret_cast<uint16_t*>(g.C) + (m0 + r) * rs;
@@ -354,6 +355,8 @@ hipError_t norm_gemm_launch(const void* x, int x_dtype, const void* gamma, const
   g.C = C;
   g.bias = reinterpret_cast<const uint16_t*>(bias);
   g.M = M; g.N = N; g.K = K; g.ldc = ldc;
+  g.rows_per_batch = M;
+  g.act = act; g.res_dtype = -1; g.c_dtype = AERIS_BF16;
   g.split = split; g.plane_stride = plane_stride;
   g.q_scale = q_scale; g.q_cols = q_cols;
   p.x = x; p.x_f32 = x_dtype == AERIS_F32;
@@ -373,6 +376,7 @@ hipError_t norm_gemm_launch(const void* x, int x_dtype, const void* gamma, const
   const dim3 grid((unsigned)(tiles_m * p.shares));
   const bool pre = order == AERIS_MOD_THEN_NORM && (shift || scale);
   if (act == AERIS_ACT_SWIGLU) launch_pre<AERIS_ACT_SWIGLU>(p, pre, grid, stream);
+  else if (act == AERIS_ACT_GELU && gemm_gelu_by_polynomial(g)) launch_pre<AERIS_ACT_GELU>(p, pre, grid, stream);
   else if (act == AERIS_ACT_GELU) launch_pre<GEMM_ACT_GELU_ERF>(p, pre, grid, stream);
   else launch_pre<AERIS_ACT_NONE>(p, pre, grid, stream);
   return hipGetLastError();

@@ -506,7 +506,8 @@ def test_block_result_of_another_type_than_the_stream(pkg, cuda):
     (3, (8, 8), (8, 8), 128, 4, 32, 128, "ref", torch.float32),         # a modulation row per tile
     (2, (12, 36), (12, 12), 64, 1, 64, 64, "spec3", torch.float32),     # ... which 432 rows refuse: two kernels
     (1, (12, 36), (12, 12), 128, 2, 32, 320, "swiglu", torch.bfloat16),
-    (1, (168, 256), (8, 8), 128, 2, 64, 512, "swiglu", torch.float32),  # more row tiles than workgroups wanted (GELU would be the polynomial in the call by itself)
+    (1, (168, 256), (8, 8), 128, 2, 64, 512, "swiglu", torch.float32),  # more row tiles than workgroups wanted
+    (1, (168, 256), (8, 8), 128, 2, 64, 512, "spec0", torch.float32),   # ... and 256 tiles of 256 x 256 and more: GELU by polynomial
 ])
 def test_block_norm_and_projection_in_one_kernel(pkg, cuda, B, image, window, dim, heads, hd, hidden, form, x_dtype):
     """dim <= 128: the block's norms run inside the projections behind them, but not while each call is timed: same bits, and

@@ -81,7 +81,7 @@ __global__ void __launch_bounds__(NT, 2) norm_gemm_kernel(NormGemmParams p) {
   const int n_tiles = (g.tiles_n - tn0 < p.col_tiles ? g.tiles_n - tn0 : p.col_tiles);
   const int total = n_tiles * KT;  // k-tiles of W, in order
 
-  // ---- W: a wave brings in 16 rows of a k-tile.  Rows past the end of W are outside the descriptor and arrive as zeros.
+  // ---- W: a wave brings in 16 rows of a k-tile
   uint32_t ld_voff[2];
   {
     const int dr = lane >> 4, pos = lane & 15;
@@ -228,7 +228,7 @@ __global__ void __launch_bounds__(NT, 2) norm_gemm_kernel(NormGemmParams p) {
   const int rows = (int)(g.M - m0 < BM ? g.M - m0 : BM);
   const int64_t rs = c_row_stride(g);
   const __amdgpu_buffer_rsrc_t rs_bias =
-      __builtin_amdgcn_make_buffer_rsrc((void*)g.bias, 0, g.bias ? (SWIGLU ? 4 : 2) * N : 0, 0x00020000);  // columns outside read 0
+      __builtin_amdgcn_make_buffer_rsrc((void*)g.bias, 0, g.bias ? (SWIGLU ? 4 : 2) * N : 0, 0x00020000);  // without a bias everything reads 0
   typedef uint32_t __attribute__((__vector_size__(2 * sizeof(uint32_t)))) raw2;
   int done = 0, rd = 0;
   for (int t = 0; t < n_tiles; ++t) {
@@ -298,18 +298,13 @@ __global__ void __launch_bounds__(NT, 2) norm_gemm_kernel(NormGemmParams p) {
       uint16_t* const c_row = reinterpret_cast<uint16_t*>(g.C) + (m0 + r) * rs;
       if (NJ == 1) {
         const int n = n_w + q * 4;
-        if (row_ok && n < N) *reinterpret_cast<u32x2*>(c_row + c_col_off(g, n)) = u32x2{pack_bf16x2(v[0][0], v[0][1]), pack_bf16x2(v[0][2], v[0][3])};
+        if (row_ok) *reinterpret_cast<u32x2*>(c_row + c_col_off(g, n)) = u32x2{pack_bf16x2(v[0][0], v[0][1]), pack_bf16x2(v[0][2], v[0][3])};
       } else {
         // lane (l15, q) of the swapped pair of column fragments holds the columns 16 (q & 1) + 8 (q >> 1) ..
         const auto x = __builtin_amdgcn_permlane16_swap(pack_bf16x2(v[0][0], v[0][1]), pack_bf16x2(v[NJ - 1][0], v[NJ - 1][1]), false, false);
         const auto y = __builtin_amdgcn_permlane16_swap(pack_bf16x2(v[0][2], v[0][3]), pack_bf16x2(v[NJ - 1][2], v[NJ - 1][3]), false, false);
         const int n = n_w + 16 * (q & 1) + 8 * (q >> 1);
-        if (row_ok && n < N) {
-          // N % 4 == 0: 8 columns are whole or exactly their first half is inside
-          uint16_t* const c = c_row + c_col_off(g, n);
-          if (n + 8 <= N) *reinterpret_cast<u32x4*>(c) = u32x4{x[0], y[0], x[1], y[1]};
-          else *reinterpret_cast<u32x2*>(c) = u32x2{x[0], y[0]};
-        }
+        if (row_ok) *reinterpret_cast<u32x4*>(c_row + c_col_off(g, n)) = u32x4{x[0], y[0], x[1], y[1]};
       }
     }
   }
@@ -336,13 +331,14 @@ void launch_pre(const NormGemmParams& p, bool pre, dim3 grid, hipStream_t stream
 //      131072    62.0 -> 48.7    73.5 -> 72.3     32.0 -> 24.4
 // (a block of dim 128 on a 32 x 64 grid 44.0 -> 38.5, on 180 x 360 406 -> 357)
 // From 192 on the norm that every share of the columns repeats costs more than the launch and the traffic that go.
-// The rest is what the vector epilogue and one descriptor over W need, and one modulation row per row tile.
+// The rest is whole column tiles (N is 3 * heads * head_dim or the hidden width, both multiples of 64 wherever the projection behind
+// them is taken), what the vector epilogue and one descriptor over W need, and one modulation row per row tile.
 bool norm_gemm_takes(int64_t M, int N, int K, const void* bias, bool modulated, int64_t mod_batch_stride, int64_t B,
                      int64_t rows_per_batch, bool swiglu) {
-  return K % BK == 0 && K <= MAX_K && (N & 3) == 0 && (reinterpret_cast<uintptr_t>(bias) & 7) == 0 &&
+  return K % BK == 0 && K <= MAX_K && N % BN == 0 && (reinterpret_cast<uintptr_t>(bias) & 7) == 0 &&
          (int64_t)(swiglu ? 2 : 1) * N * K * 2 < (int64_t(1) << 31) && M < (int64_t(1) << 31) &&
          (!modulated || mod_batch_stride == 0 || B == 1 || rows_per_batch % BM == 0) &&
-         (M + BM - 1) / BM * ((N + 31) / 32) < (int64_t(1) << 31);
+         (M + BM - 1) / BM * (N / 32) < (int64_t(1) << 31);
 }
 
 hipError_t norm_gemm_launch(const void* x, int x_dtype, const void* gamma, const void* beta, int param_dtype, const float* shift,
@@ -367,7 +363,7 @@ hipError_t norm_gemm_launch(const void* x, int x_dtype, const void* gamma, const
   p.kind = kind; p.eps = eps;
   const int bn_out = act == AERIS_ACT_SWIGLU ? BN / 2 : BN;
   const int64_t tiles_m = (M + BM - 1) / BM;
-  g.tiles_n = (N + bn_out - 1) / bn_out;
+  g.tiles_n = N / bn_out;
   // two workgroups per CU (three fit): one hides the other's norm (8192 x 128 -> 512: 11.5 us with one, 9.55 with two, 12.8 with
   // four, 2048 rows 6.4 with any)
   const int64_t want = (512 + tiles_m - 1) / tiles_m;

@@ -324,18 +324,38 @@ void launch_pre(const NormGemmParams& p, bool pre, dim3 grid, hipStream_t stream
 
 // Rows of 64 and 128 elements.  Two kernels -> this one, us (f32 rows, layer norm; calls replayed from a HIP graph):
 //        rows      128 -> 384     128 -> 512 GELU    64 -> 192     192 -> 576     256 -> 768     256 -> 1024 GELU
-//         256     6.5 ->  5.6     6.8 ->  6.0      6.3 ->  5.2     6.9 ->  7.5    7.1 ->  7.7     7.4 ->  8.2
-//        2048     7.0 ->  5.9     7.4 ->  6.4      6.5 ->  5.5     8.0 ->  9.0    8.6 ->  9.7     9.3 -> 10.5
-//        8192     9.4 ->  8.4    12.2 ->  9.6      7.5 ->  6.5    13.0 -> 13.2   14.5 -> 14.8    20.2 -> 19.1
-//       32768    23.0 -> 16.9    30.2 -> 25.6     13.3 ->  9.6    31.8 -> 26.7
-//      131072    62.0 -> 48.7    73.5 -> 72.3     32.0 -> 24.4
-// (a block of dim 128 on a 32 x 64 grid 44.0 -> 38.5, on 180 x 360 406 -> 357)
-// From 192 on the norm that every share of the columns repeats costs more than the launch and the traffic that go.
+//         256     6.2 ->  4.7     6.4 ->  5.2      5.9 ->  4.5     6.9 ->  7.5    7.1 ->  7.7     7.4 ->  8.2
+//        2048     6.6 ->  5.1     7.1 ->  5.8      6.2 ->  4.7     8.0 ->  9.0    8.6 ->  9.7     9.3 -> 10.5
+//        8192     8.6 ->  8.1    11.2 ->  9.2      7.2 ->  5.8    13.0 -> 13.2   14.5 -> 14.8    20.2 -> 19.1
+//       32768    20.0 -> 16.9    27.2 -> 22.8     13.4 ->  9.4    31.8 -> 26.7
+//      131072    61.2 -> 47.0    74.3 -> 63.1     31.1 -> 24.0
+// From 192 on the norm that every share of the columns repeats costs more than the launch and the traffic that go, until there are
+// many rows (not built for those).
+// A ceiling on the rows: a large plain product has tiles of 256, and the norm's launch and its traffic, half as much with a bf16 x,
+// come to less than what tiles of 64 cost; soonest with SwiGLU, which reads two rows of W per output column.  A block with two
+// kernels -> with one of them, the other the same in both, us:
+//        rows           to_qkv, f32 x   to_qkv, bf16 x    GELU, f32 x     GELU, bf16 x     SwiGLU, f32 x   SwiGLU, bf16 x
+//  dim 128, hidden 512
+//       24576            68.4 ->  64.9    61.5 ->  59.0   68.4 ->  63.0    61.5 ->  57.8    66.6 ->  64.1    59.5 ->  59.1
+//       32768            77.5 ->  76.5    68.2 ->  67.4   77.5 ->  74.7    68.2 ->  68.1    79.8 ->  82.4    70.0 ->  75.0
+//      131072           249   -> 246     221   -> 218    249   -> 235     221   -> 213     256   -> 258     228   -> 235
+//      524288           933   -> 883     814   -> 822    933   -> 921     814   -> 839     957   -> 984     862   -> 919
+//     1036800          1709   ->1647    1503   ->1541   1709   ->1700    1503   ->1575    1772   ->1838    1594   ->1742
+//  dim 64, hidden 256
+//       45056            65.3 ->  61.1    59.5 ->  55.3   65.3 ->  59.0    59.5 ->  55.4    61.9 ->  58.7    56.4 ->  55.0
+//      184320           162   -> 165     142   -> 137    162   -> 152     142   -> 138     168   -> 162     147   -> 147
+//      524288           446   -> 437     388   -> 400    446   -> 452     388   -> 397     456   -> 483     400   -> 422
 // The rest is whole column tiles (N is 3 * heads * head_dim or the hidden width, both multiples of 64 wherever the projection behind
 // them is taken), what the vector epilogue and one descriptor over W need, and one modulation row per row tile.
-bool norm_gemm_takes(int64_t M, int N, int K, const void* bias, bool modulated, int64_t mod_batch_stride, int64_t B,
+static int64_t most_rows(int N, int K, bool x_f32, bool swiglu) {
+  if (!swiglu) return x_f32 ? int64_t(1) << 31 : 196608;
+  if (x_f32) return N * (int64_t)K <= 256 * 128 ? 196608 : 28672;
+  return N * (int64_t)K <= 256 * 64 ? 49152 : 12288;
+}
+
+bool norm_gemm_takes(int64_t M, int N, int K, bool x_f32, const void* bias, bool modulated, int64_t mod_batch_stride, int64_t B,
                      int64_t rows_per_batch, bool swiglu) {
-  return K % BK == 0 && K <= MAX_K && N % BN == 0 && (reinterpret_cast<uintptr_t>(bias) & 7) == 0 &&
+  return M <= most_rows(N, K, x_f32, swiglu) && K % BK == 0 && K <= MAX_K && N % BN == 0 && (reinterpret_cast<uintptr_t>(bias) & 7) == 0 &&
          (int64_t)(swiglu ? 2 : 1) * N * K * 2 < (int64_t(1) << 31) && M < (int64_t(1) << 31) &&
          (!modulated || mod_batch_stride == 0 || B == 1 || rows_per_batch % BM == 0) &&
          (M + BM - 1) / BM * (N / 32) < (int64_t(1) << 31);

@@ -253,8 +253,8 @@ int aeris_input_stage_fwd(const float* x0, int C0, float div0, const float* x1, 
  *   Scratch (bf16, 16-byte aligned, borrowed): norm_scratch [T, dim], qkv_scratch [3*heads][T, head_dim] (NULL if every block
  *   takes the one-kernel attention: fuse_qkv and the shape supported), attn_scratch [T, heads*head_dim], hidden_scratch
  *   [T, hidden] with T = B*H*W.
- *   Without events, blocks of dim <= 128 run each norm and the projection behind it as one kernel and leave norm_scratch unwritten
- *   (it is needed all the same).
+ *   Without events, blocks of dim <= 128 run a norm and the projection behind it as one kernel where that is faster and then
+ *   leave norm_scratch unwritten (it is needed all the same).
  *   events: NULL, or 2 * (7 or, with one-kernel attention, 6) hipEvent_t per block, recorded on the stream before and after
  *   each of the calls. */
 typedef struct aeris_block {

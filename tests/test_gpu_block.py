@@ -533,3 +533,45 @@ def test_block_norm_and_projection_in_one_kernel(pkg, cuda, B, image, window, di
     assert torch.equal(out, timed)
     if image[0] * image[1] <= 4096:
         assert rel_l2(out, oracle.block_forward(cfg, sd, x.float(), t, (0, 0))) <= 1e-2
+
+
+@pytest.mark.parametrize("B,image,window,dim,heads,hd,hidden,form,x_dtype,one_kernel", [
+    (1, (32, 64), (8, 8), 128, 4, 32, 512, "spec0", torch.bfloat16, True),
+    (1, (64, 256), (8, 8), 64, 1, 64, 256, "spec0", torch.float32, True),    # 256 row tiles: several column tiles a workgroup, erf
+    (1, (168, 256), (8, 8), 128, 2, 64, 512, "spec0", torch.float32, True),  # ... and polynomial
+    (1, (112, 256), (8, 8), 128, 2, 64, 512, "swiglu", torch.float32, True),  # 28672 rows, the most
+    (1, (120, 256), (8, 8), 128, 2, 64, 512, "swiglu", torch.float32, False),
+    (2, (12, 36), (12, 12), 64, 1, 64, 64, "spec3", torch.float32, False),   # 432 rows a modulation row: no row tile's multiple
+    (1, (8, 8), (8, 8), 192, 3, 64, 192, "spec0", torch.float32, False),     # rows of 192 elements
+])
+def test_block_norm_and_projection_route(pkg, cuda, monkeypatch, B, image, window, dim, heads, hd, hidden, form, x_dtype, one_kernel):
+    """Which blocks run both norms inside the projections: what they would write to is as it was before the call.  Either way the
+    bits are those of the calls one by one."""
+    geo = dict(dim=dim, heads=heads, head_dim=hd, mlp_dim=hidden, window_size=window, image_shape=image)
+    mk = {"spec0": lambda: OracleConfig.spec(mod_ways=0, **geo), "spec3": lambda: OracleConfig.spec(mod_ways=3, **geo),
+          "swiglu": lambda: OracleConfig.spec(norm="rmsnorm", mlp="swiglu", bias=False, mod_ways=0, **geo)}
+    cfg = mk[form]()
+    sd = oracle.init_block_weights(cfg, 11, nontrivial=True)
+    g = torch.Generator().manual_seed(12)
+    x = (torch.randn(B, image[0] * image[1], dim, generator=g) * 2 + 0.5).to(x_dtype).to(cuda)
+    t = torch.randn(B, dim, generator=g).to(cuda) if cfg.mod_ways else None
+    layer = make_layer(pkg, cfg, sd, cuda)
+    normed, workspaces = [], pkg.ops.workspaces
+
+    def marked(device, *requests):
+        ws = workspaces(device, *requests)
+        assert requests[0][0] == "norm"
+        normed.append(ws[0].fill_(7.0))
+        return ws
+
+    with torch.no_grad():
+        with monkeypatch.context() as m:
+            m.setattr(pkg.ops, "workspaces", marked)
+            out = layer(x, t)
+        assert len(normed) == 1 and bool((normed[0] == 7.0).all()) == one_kernel
+        pkg.ops.profile_begin()
+        try:
+            timed = layer(x, t)
+        finally:
+            pkg.ops.profile_end()
+    assert torch.equal(out, timed)

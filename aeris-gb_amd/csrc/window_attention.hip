@@ -667,9 +667,9 @@ window_attention_persist_kernel(AttnParams p, int n_units) {
 // ---------------------------------------------------------------------------------------------
 // Units of one window and head with one K / V tile in LDS, several workgroups per CU: what a workgroup waits for (its tile, its
 // stores) runs under the others' sweeps, where the persistent kernel above has the next unit's loads in flight instead and
-// one workgroup per CU.  For 8x8 windows, whose two waves leave a persistent workgroup's CU nearly empty: six workgroups per CU
-// (33792 tokens x 12 heads of 64 53.4 -> 34.6 us, 115200 x 8 97 -> 99, 179968 x 9 169.5 -> 173.8 (four per CU: 37.4, 97.5, 172.4;
-// eight: 36.8, 106, 193), 2048 x 4 5.9 -> 4.8 us), and for 12x12 windows too few to walk (4608 tokens x 4 heads 9.0 -> 7.9 us; at 3600 units
+// one workgroup per CU.  For 8x8 windows up to the size of the last-level cache (walk_8x8), whose two waves leave a persistent
+// workgroup's CU nearly empty: six workgroups per CU (33792 tokens x 12 heads of 64 53.4 -> 34.6 us (four per CU: 37.4, eight: 36.8),
+// 2048 x 4 5.9 -> 4.8 us), and for 12x12 windows too few to walk (4608 tokens x 4 heads 9.0 -> 7.9 us; at 3600 units
 // five waves beside five others do not spread over four SIMDs: 85 us, the persistent kernel 65.5).
 // What follows from the lane is worked out per unit: kept across units it filled the registers of a third wave per SIMD.  The bias
 // table holds only the vectors that a key group can start at (build_bias_rows_lds).
@@ -808,7 +808,7 @@ hipError_t attention_configure_all() {
   e = hipFuncSetAttribute(reinterpret_cast<const void*>(window_attention_persist_kernel<Y, Xx, Bi>),            \
                           hipFuncAttributeMaxDynamicSharedMemorySize, AttnPersistCfg<Y, Xx, Bi>::SMEM);         \
   if (e != hipSuccess) return e;
-  CFGP(12, 12, true) CFGP(12, 12, false) CFGP(16, 16, true) CFGP(16, 16, false)
+  CFGP(8, 8, true) CFGP(8, 8, false) CFGP(12, 12, true) CFGP(12, 12, false) CFGP(16, 16, true) CFGP(16, 16, false)
 #undef CFGP
   {
     int dev = 0, cus = 0;
@@ -817,6 +817,19 @@ hipError_t attention_configure_all() {
       g_attn_cus = cus;
   }
   return hipSuccess;
+}
+
+// Whether 8x8 windows have several workgroups per CU: unless q, k, v and the output together go beyond the last-level cache (256 MB).
+// There memory is what both kernels wait for, and the one that always has the next unit's loads in flight is the faster one; with a
+// bias table only from four windows per CU and head on, since its workgroups rebuild the table whenever their units change the head.
+// Persistent -> several workgroups, us, by MiB of q, k, v and output:
+//   bias, 2772 windows and more    262: 56.7 -> 49.5   297: 64.9 -> 63.3   309: 66.8 -> 66.9   349: 75.3 -> 77.7   900: 182 -> 197   2700: 554 -> 611
+//   bias, 1800 windows             281: 64.3 -> 59.4   394: 88.4 -> 88.0   675: 147 -> 152     (1200 windows  600: 136 -> 133   900: 202 -> 207)
+//   bias, 528 windows              396: 103 -> 94      990: 251 -> 245
+//   no bias                        248: 48.1 -> 41.8   272: 54.6 -> 54.6   309: 61.5 -> 65.6   394: 80.1 -> 88.0
+static bool walk_8x8(const AttnParams& p, bool has_bias) {
+  const int64_t mib = (int64_t)p.B * p.H * p.W * p.heads * 64 * 8 >> 20, windows = (int64_t)p.B * p.nWy * p.nWx;
+  return mib <= (has_bias ? 312 : 272) || (has_bias && windows < 4 * (int64_t)g_attn_cus);
 }
 
 template <int WS_Y, int WS_X, int HD, bool HAS_BIAS>
@@ -828,7 +841,7 @@ static hipError_t launch_attn(const AttnParams& p, hipStream_t stream) {
       (int64_t)p.B * p.H * p.W * p.tok_stride * 2 < (int64_t)0xFFFFFFF0u) {
     if constexpr (WS_X < 16) {
       constexpr int PER_CU = 6;
-      if (WS_X == 8 || grid < 2 * (int64_t)g_attn_cus) {
+      if (WS_X == 8 ? walk_8x8(p, HAS_BIAS) : grid < 2 * (int64_t)g_attn_cus) {
         using P = AttnWalkCfg<WS_Y, WS_X, HAS_BIAS>;
         const int64_t most = (int64_t)PER_CU * g_attn_cus;
         hipLaunchKernelGGL((window_attention_walk_kernel<WS_Y, WS_X, HAS_BIAS>), dim3((unsigned)(grid < most ? grid : most)), dim3(P::NT),
@@ -836,13 +849,11 @@ static hipError_t launch_attn(const AttnParams& p, hipStream_t stream) {
         return hipGetLastError();
       }
     }
-    if constexpr (WS_X > 8) {
-      if (grid >= 2 * (int64_t)g_attn_cus) {  // enough units for every CU to stream a few: the persistent form
-        using P = AttnPersistCfg<WS_Y, WS_X, HAS_BIAS>;
-        hipLaunchKernelGGL((window_attention_persist_kernel<WS_Y, WS_X, HAS_BIAS>), dim3((unsigned)g_attn_cus), dim3(P::NT), P::SMEM,
-                           stream, p, (int)grid);
-        return hipGetLastError();
-      }
+    if (grid >= 2 * (int64_t)g_attn_cus) {  // enough units for every CU to stream a few: the persistent form
+      using P = AttnPersistCfg<WS_Y, WS_X, HAS_BIAS>;
+      hipLaunchKernelGGL((window_attention_persist_kernel<WS_Y, WS_X, HAS_BIAS>), dim3((unsigned)g_attn_cus), dim3(P::NT), P::SMEM,
+                         stream, p, (int)grid);
+      return hipGetLastError();
     }
     if constexpr (WS_X == 16) {
       using D = AttnDmaCfg<WS_Y, WS_X, HAS_BIAS>;

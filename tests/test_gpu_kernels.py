@@ -346,6 +346,9 @@ def test_window_attention_planes_parity(pkg, cuda, case, prescaled):
     (2, 24, 24, 63, 64, 12, 6, True, True, 1.0),    # 504 units: the largest below the persistent form
     (2, 24, 24, 64, 64, 12, 6, True, True, 1.0),    # 512: the smallest of the persistent form
     (2, 24, 24, 9, 64, 12, 6, True, True, 6.0),
+    (1, 256, 256, 10, 64, 8, 4, True, True, 1.0),    # 320 MiB of q, k, v and output: the persistent form ...
+    (1, 248, 256, 11, 64, 8, 4, True, True, 1.0),    # ... but not for 992 windows
+    (1, 256, 256, 9, 64, 8, 0, False, False, 1.0),   # 288 MiB, without a table
 ], ids=lambda c: f"B{c[0]}_{c[1]}x{c[2]}_h{c[3]}_ws{c[5]}_s{c[6]}_b{int(c[7])}m{int(c[8])}_x{c[9]:g}")
 def test_window_attention_several_workgroups_per_cu(pkg, cuda, case, prescaled):
     """8x8 windows, and 12x12 ones with few units: same oracle and tolerance as the other head-plane cases."""

@@ -669,8 +669,10 @@ window_attention_persist_kernel(AttnParams p, int n_units) {
 // stores) runs under the others' sweeps, where the persistent kernel above has the next unit's loads in flight instead and
 // one workgroup per CU.  For 8x8 windows up to the size of the last-level cache (walk_8x8), whose two waves leave a persistent
 // workgroup's CU nearly empty: six workgroups per CU (33792 tokens x 12 heads of 64 53.4 -> 34.6 us (four per CU: 37.4, eight: 36.8),
-// 2048 x 4 5.9 -> 4.8 us), and for 12x12 windows too few to walk (4608 tokens x 4 heads 9.0 -> 7.9 us; at 3600 units
-// five waves beside five others do not spread over four SIMDs: 85 us, the persistent kernel 65.5).
+// 2048 x 4 5.9 -> 4.8 us), and for 12x12 windows of which every CU gets one at most (4608 tokens x 4 heads 9.0 -> 7.9 us).  Five waves
+// beside five others do not spread over four SIMDs: 12x12 windows with more units than CUs have one workgroup of the kernel for
+// single units each (260 units 10.8 us, here 14.2; 480 12.7, here 15.6; without a table 288 units 8.4 and 9.5), from two per CU on the
+// persistent kernel (3600 units 65.5 us, here 85).
 // What follows from the lane is worked out per unit: kept across units it filled the registers of a third wave per SIMD.  The bias
 // table holds only the vectors that a key group can start at (build_bias_rows_lds).
 template <int WS_Y, int WS_X, bool HAS_BIAS>
@@ -802,7 +804,7 @@ hipError_t attention_configure_all() {
   e = hipFuncSetAttribute(reinterpret_cast<const void*>(window_attention_dma_kernel<Y, Xx, Bi>),                \
                           hipFuncAttributeMaxDynamicSharedMemorySize, AttnDmaCfg<Y, Xx, Bi>::SMEM);             \
   if (e != hipSuccess) return e;
-  CFGD(16, 16, true) CFGD(16, 16, false)
+  CFGD(12, 12, true) CFGD(12, 12, false) CFGD(16, 16, true) CFGD(16, 16, false)
 #undef CFGD
 #define CFGP(Y, Xx, Bi)                                                                                        \
   e = hipFuncSetAttribute(reinterpret_cast<const void*>(window_attention_persist_kernel<Y, Xx, Bi>),            \
@@ -841,7 +843,7 @@ static hipError_t launch_attn(const AttnParams& p, hipStream_t stream) {
       (int64_t)p.B * p.H * p.W * p.tok_stride * 2 < (int64_t)0xFFFFFFF0u) {
     if constexpr (WS_X < 16) {
       constexpr int PER_CU = 6;
-      if (WS_X == 8 ? walk_8x8(p, HAS_BIAS) : grid < 2 * (int64_t)g_attn_cus) {
+      if (WS_X == 8 ? walk_8x8(p, HAS_BIAS) : grid <= g_attn_cus) {
         using P = AttnWalkCfg<WS_Y, WS_X, HAS_BIAS>;
         const int64_t most = (int64_t)PER_CU * g_attn_cus;
         hipLaunchKernelGGL((window_attention_walk_kernel<WS_Y, WS_X, HAS_BIAS>), dim3((unsigned)(grid < most ? grid : most)), dim3(P::NT),
@@ -855,7 +857,7 @@ static hipError_t launch_attn(const AttnParams& p, hipStream_t stream) {
                          stream, p, (int)grid);
       return hipGetLastError();
     }
-    if constexpr (WS_X == 16) {
+    if constexpr (WS_X > 8) {
       using D = AttnDmaCfg<WS_Y, WS_X, HAS_BIAS>;
       hipLaunchKernelGGL((window_attention_dma_kernel<WS_Y, WS_X, HAS_BIAS>), dim3((unsigned)grid), dim3(D::NT), D::SMEM,
                          stream, p);

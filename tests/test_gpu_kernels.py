@@ -343,6 +343,9 @@ def test_window_attention_planes_parity(pkg, cuda, case, prescaled):
     (2, 64, 64, 13, 64, 8, 0, False, False, 1.0),   # 1664 units, no bias
     (1, 64, 256, 7, 64, 8, 4, True, True, 6.0),     # two-pass form, 1792 units
     (1, 12, 12, 1, 64, 12, 6, True, True, 1.0),
+    (2, 24, 24, 32, 64, 12, 6, True, True, 1.0),    # 256 units: the largest with one per CU
+    (2, 24, 24, 33, 64, 12, 6, True, True, 1.0),    # 264: one workgroup a unit
+    (2, 24, 24, 33, 64, 12, 6, False, False, 1.0),
     (2, 24, 24, 63, 64, 12, 6, True, True, 1.0),    # 504 units: the largest below the persistent form
     (2, 24, 24, 64, 64, 12, 6, True, True, 1.0),    # 512: the smallest of the persistent form
     (2, 24, 24, 9, 64, 12, 6, True, True, 6.0),

@@ -4,7 +4,8 @@
 // One workgroup = a block of queries of one (window, head), 32 per wave; the keys of the window are streamed through LDS in
 // chunks of 64 with an online softmax.  How many waves and chunk buffers a workgroup has follows the window (the rule
 // stands at the launch):
-//   8 waves, 4 buffers   windows of more than 2048 tokens with head_dim 128: one workgroup per CU, a barrier per two chunks
+//   8 waves, 4 buffers   windows of more than 2048 tokens with head_dim 128, and few windows: one workgroup per CU, a barrier
+//                        per two chunks
 //   4 waves, 2 buffers   the others: two workgroups per CU (head_dim 64: three), so that one's start - token table, Q, the first
 //                        chunk - and its output stores run beside another's sweep, and windows whose size is no multiple of
 //                        256 leave fewer waves without queries
@@ -555,15 +556,22 @@ hipError_t attention_stream_launch(const void* qkv, void* out, int B, int H, int
   p.span_bytes = span < ((int64_t)1 << 32) - 4096 ? (uint32_t)span : 0u;
   const bool dma = p.span_bytes != 0 && tok_stride > 0;
   // Windows above 2048 tokens with head_dim 128: 8 waves where few workgroups share the chip (4 windows of 3600 with 12 heads:
-  // 308 us against 315), the same on a full grid (360 x 720: 5389, 5372).  Below, 4 waves: L = 1395 1152 -> 1093 us, 400
-  // 361 -> 352, 192 140 -> 127, 128 139 -> 108 (but 960 528 -> 539).  head_dim 64 always has the smaller workgroups.
+  // 308 us against 315), the same on a full grid (360 x 720: 5389, 5372).  Below, 4 waves (500 000 tokens x 3 heads, 8 -> 4 waves:
+  // L = 1395 1319 -> 1160 us, 960 965 -> 868, 400 633 -> 570, 192 427 -> 387, 128 398 -> 306), head_dim 64 for any L (500 000 x 6:
+  // L = 1395 1630 -> 1250), except where 8 waves are one workgroup per CU and 4 waves would be up to two: the chip is as full
+  // either way, and the two load every K / V chunk twice (`lone`, per XCD of 32 CUs; 8 -> 4 waves):
+  //   head_dim 128, units of 130 tokens  144: 10.9 -> 12.0 us   240: 12.3 -> 12.8   (the second workgroup has two queries)   192 tokens  144: 12.1 -> 12.0
+  //     400 tokens  72: 19.5 -> 20.1   120: 22.0 -> 22.2      900 tokens  48: 31.8 -> 32.9      1395  32: 41.8 -> 43.4      2048  24: 57.6 -> 60.0
+  //   head_dim 64, register form with 8 waves   900 tokens  40: 21.1 -> 21.3   1395  24: 27.4 -> 28.0   2048  24: 37.7 -> 38.5   3600  16: 63.5 -> 67.5
+  const int64_t per_xcd = (p.n_units + 7) / 8, wgs4 = per_xcd * ((L + 127) / 128), wgs8 = per_xcd * ((L + 255) / 256);
+  const bool lone = wgs8 <= 32 && wgs4 > 32;
   if (head_dim == 64) {
-    if (!dma) return launch_one<64, false, 8, 4>(p, L, stream);
+    if (!dma || (lone && L > 1024)) return launch_one<64, false, 8, 4>(p, L, stream);
     return L <= KC ? launch_one<64, true, 2, 1>(p, L, stream) : launch_one<64, true, 4, 2>(p, L, stream);
   }
   if (!dma) return launch_one<128, false, 8, 4>(p, L, stream);
-  return L <= KC ? launch_one<128, true, 2, 1>(p, L, stream)
-                 : L <= 2048 ? launch_one<128, true, 4, 2>(p, L, stream) : launch_one<128, true, 8, 4>(p, L, stream);
+  if (L > 2048 || (lone && (L <= 160 || L > 512 || (L > 384 && wgs4 <= 48)))) return launch_one<128, true, 8, 4>(p, L, stream);
+  return L <= KC ? launch_one<128, true, 2, 1>(p, L, stream) : launch_one<128, true, 4, 2>(p, L, stream);
 }
 
 }  // namespace aeris

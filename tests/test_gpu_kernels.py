@@ -470,6 +470,11 @@ def test_window_attention_streaming_wide_rows_match_compact(pkg, cuda):
     (1, 64, 64, 1, 128, 32, 64, 16, 32),     # L = 2048: the largest of four waves with head_dim 128
     (1, 33, 126, 1, 128, 33, 63, 0, 31),     # L = 2079: eight waves
     (1, 33, 63, 1, 64, 33, 63, 16, 31),
+    # few windows, eight waves although four would do for the size
+    (2, 26, 100, 4, 128, 13, 10, 6, 5),      # L = 130, 160 units
+    (1, 120, 60, 4, 128, 20, 20, 10, 10),    # L = 400, 72 units
+    (1, 96, 128, 4, 128, 32, 64, 16, 0),     # L = 2048, 24 units
+    (1, 72, 64, 8, 64, 36, 32, 0, 16),       # L = 1152, 32 units, head_dim 64: through registers
 ], ids=lambda c: f"B{c[0]}_{c[1]}x{c[2]}_h{c[3]}x{c[4]}_ws{c[5]}x{c[6]}_s{c[7]}x{c[8]}")
 def test_window_attention_streaming_workgroup_sizes(pkg, cuda, case):
     """Same oracle and tolerance as the other streaming cases."""

@@ -106,7 +106,7 @@ struct WindowLogits {
   __device__ __forceinline__ WindowLogits(const unsigned char* bias_lds, int qpos, int hi_, bool my_, bool mx_, int sy_, int sx_)
       : hi(hi_), my(my_), mx(mx_), sy(sy_), sx(sx_) {
     const int qiy = qpos / WS_X, qix = qpos % WS_X;
-    const int sp = (WS_Y - 1 - qiy) * PITCH + (WS_X - 1 - qix);
+    const int sp = (2 * WS_Y - 2) * PITCH + 2 * WS_X - 2 - (qiy + WS_Y - 1) * PITCH - qix - (WS_X - 1);
     sB_same = bias_lds + (sp + 4 * hi) * 16;
     sB_next = bias_lds + (sp + (PITCH - WS_X + 4) * hi) * 16;
     ry_q = my ? (qiy < WS_Y - sy ? 1 : 2) : 0;

@@ -13,7 +13,8 @@
 //     8 rows x 128 B and the lane -> chunk map is the inverse of the LDS swizzle (swz_off), so fragment reads are
 //     conflict-free ds_read_b128 and nothing is staged through registers
 //   - STAGES k-tiles of 64 in LDS, one barrier per k-tile: the loads of k-tile j + STAGES - 1 are issued right behind the
-//     barrier that ends the reading of k-tile j - 1 and the fragment reads of k-tile j, and waited for with a counted vmcnt
+//     barrier that ends the reading of k-tile j - 1 (tiles of 64: and the fragment reads of k-tile j), and waited for with a
+//     counted vmcnt
 //   - v_mfma_f32_16x16x32_bf16 with the weight fragment first and accumulators that start at the bias: the same
 //     arithmetic in the same order as the persistent kernel, bit for bit
 //   - the epilogue works on the accumulators where they are: a lane holds 4 consecutive n of one row; for bf16 C two column
@@ -203,6 +204,14 @@ __global__ void __launch_bounds__(NT, 2) gemm_bf16_nt_tile_kernel(GemmParams p) 
     else if (STAGES > 3 && behind == 1) wait_barrier<LPT>();
     else wait_barrier<0>();
     const unsigned char* st = smem + rd * STAGE;
+    // Tiles of 64: the loads come behind the fragment reads: each holds the wave for 70-95 cycles, in which the fragments arrive.  (The
+    // serial chain of a k-tile, not the latency of its loads, is what a small problem waits for: four, six or nine k-tiles in flight
+    // instead of three measured the same or slower.  Loads first -> reads first: 2048 x 256 x 1024 8.0 -> 7.1 us, 2048 x 512 x 2048
+    // 13.0 -> 10.9; 2048 x 128 x 128 the same.)  With two stages, tiles of 128, the one k-tile ahead is requested at once: reads
+    // first, 2048 x 1538 x 1536 25.2 -> 26.6 us, 4096 x 4098 x 4096 167 -> 174, SiLU 3000 x 3072 x 1024 31.4 -> 33.4 (but
+    // 1000 x 1002 x 1024, 64 tiles in all, 17.1 -> 16.4).
+    constexpr bool READS_FIRST = STAGES > 2;
+    if (!READS_FIRST && behind >= STAGES - 1) issue(kt + STAGES - 1, wr);
     bf16x8 af[2][FM], bf[2][FN];
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
@@ -211,11 +220,7 @@ __global__ void __launch_bounds__(NT, 2) gemm_bf16_nt_tile_kernel(GemmParams p) 
 #pragma unroll
       for (int j = 0; j < FN; ++j) bf[ks][j] = *reinterpret_cast<const bf16x8*>(st + b_roff[ks] + j * 16 * 128);
     }
-    // The loads come behind the fragment reads: each holds the wave for 70-95 cycles, in which the fragments arrive.  (The serial chain
-    // of a k-tile, not the latency of its loads, is what a small problem waits for: four, six or nine k-tiles in flight instead of
-    // three measured the same or slower.  Loads first -> reads first: 2048 x 256 x 1024 8.0 -> 7.1 us, 2048 x 512 x 2048 13.0 ->
-    // 10.9, 3000 x 3072 x 1024 33.3 -> 29.4; 2048 x 128 x 128 the same.)
-    if (behind >= STAGES - 1) issue(kt + STAGES - 1, wr);
+    if (READS_FIRST && behind >= STAGES - 1) issue(kt + STAGES - 1, wr);
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks)
 #pragma unroll

@@ -809,6 +809,20 @@ def test_norm_modulate_short_rows(pkg, cuda, d, B, S, kind, order):
     assert rel_l2(out, ref) <= 1e-5  # f32 sums of at most 264 terms
 
 
+@pytest.mark.parametrize("rows,d,xdt", [
+    (3072, 1536, torch.float32), (3073, 1536, torch.float32), (4097, 1536, torch.float32),   # one row per wave, four, one
+    (7168, 640, torch.float32), (7169, 640, torch.float32), (5120, 1024, torch.bfloat16), (5121, 1024, torch.bfloat16),
+])
+def test_norm_modulate_rows_per_wave(pkg, cuda, rows, d, xdt):
+    g = torch.Generator().manual_seed(rows)
+    x = (1.5 * torch.randn(1, rows, d, generator=g) + 0.3).to(xdt)
+    gamma, beta = 1 + 0.2 * torch.randn(d, generator=g), 0.2 * torch.randn(d, generator=g)
+    out = pkg.ops.norm_modulate(x.to(cuda), gamma.to(cuda), beta.to(cuda), None, None, kind="layernorm", order="norm_then_mod", eps=1e-5,
+                                out_dtype=torch.float32)
+    torch.cuda.synchronize()
+    assert rel_l2(out, oracle.layer_norm(x.float(), gamma, beta, 1e-5)) <= 1e-5  # f32 sums of at most 1536 terms
+
+
 def test_norm_modulate_variants(pkg, cuda):
     d, B, S = 512, 2, 50
     g = torch.Generator().manual_seed(1)

@@ -4,8 +4,8 @@
 // One workgroup = a block of queries of one (window, head), 32 per wave; the keys of the window are streamed through LDS in
 // chunks of 64 with an online softmax.  How many waves and chunk buffers a workgroup has follows the window (the rule
 // stands at the launch):
-//   8 waves, 4 buffers   windows of more than 2048 tokens with head_dim 128, and few windows: one workgroup per CU, a barrier
-//                        per two chunks
+//   8 waves, 4 buffers   windows of more than 2048 tokens with head_dim 128, and few windows (head_dim 64: through registers): one
+//                        workgroup per CU, a barrier per two chunks
 //   4 waves, 2 buffers   the others: two workgroups per CU (head_dim 64: three), so that one's start - token table, Q, the first
 //                        chunk - and its output stores run beside another's sweep, and windows whose size is no multiple of
 //                        256 leave fewer waves without queries
@@ -225,15 +225,13 @@ window_attention_stream_kernel(StreamParams p) {
     }
   };
 
-  // DMA form: one instruction of a wave fills 1 KB = 4 rows of a chunk; wave w issues rows 4w.. and 32 + 4w.. of K and
-  // of V.  Lane = (row within the four, LDS chunk slot); it fetches the global chunk that the swizzle keeps there.
+  // DMA form: one instruction of a wave fills 1 KB = RPI rows of a chunk; wave w issues the pieces w, w + NWAVE, ... of K and of V.
+  // Lane = (row within the piece, LDS chunk slot); it fetches the global chunk that the swizzle keeps there.
   // Keys past the window get an offset outside the descriptor and arrive as zeros (their scores are masked).
   typedef __attribute__((address_space(3))) void* lds_vptr;
   const __amdgpu_buffer_rsrc_t rs_k = __builtin_amdgcn_make_buffer_rsrc((void*)kbase, 0, (int)p.span_bytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t rs_v = __builtin_amdgcn_make_buffer_rsrc((void*)vbase, 0, (int)p.span_bytes, 0x00020000);
-  constexpr int RPI = 1024 / (HD * 2);                           // rows per instruction: 4 (head_dim 128) or 8
-  constexpr int CHUNK_LOADS = DMA ? 2 * KC / (RPI * NWAVE) : 0;  // load instructions of a wave per chunk
-  static_assert(NBUF != 2 || CHUNK_LOADS < 16, "the counted wait below");
+  constexpr int RPI = 1024 / (HD * 2);  // rows per instruction: 4 (head_dim 128) or 8
   auto issue_chunk = [&](int j, int buf) {
 #pragma unroll
     for (int i = 0; i < KC / (RPI * NWAVE); ++i) {
@@ -314,9 +312,10 @@ window_attention_stream_kernel(StreamParams p) {
   if (DMA) {
     issue_chunk(0, 0);
     if (NBUF > 1 && nch > 1) issue_chunk(1, 1);
-    // lgkmcnt(0), and this wave's loads into LDS have landed (two buffers: those of chunk 0, chunk 1 is awaited when it is due)
-    if (NBUF == 2 && nch > 1) __builtin_amdgcn_s_waitcnt(0x0070 | CHUNK_LOADS);
-    else __builtin_amdgcn_s_waitcnt(0x0070);
+    // vmcnt(0) lgkmcnt(0): this wave's loads into LDS have landed.  (With two buffers chunk 1 need not have: a wait for chunk 0 alone,
+    // counted, and a barrier without the compiler's fence, which waits for everything.  Units of 128 and 256 tokens, head_dim 128:
+    // 3200 x 128 99 -> 89 us, 1600 x 256 74 -> 54 - 60; but 416 x 256, one round of workgroups, 16.9 -> 17.9.  Not taken here.)
+    __builtin_amdgcn_s_waitcnt(0x0070);
   } else {
     load_chunk(0);
     store_chunk(0);
@@ -335,8 +334,9 @@ window_attention_stream_kernel(StreamParams p) {
     if (j >= nch) break;
     constexpr int LEAD = NBUF / 2;  // chunk j + LEAD is loaded and written to LDS while chunk j is consumed
     if (DMA) {
-      // both chunks of the next pair are requested at the start of this pair (the buffers were last read before the
-      // barrier that ended the pair before), and awaited at the barrier that ends this pair
+      // Two buffers: the next chunk is requested at the start of this one and awaited at the barrier that ends this one.  Four: both
+      // chunks of the next pair at the start of this pair, awaited at the barrier that ends it.  (The buffers were last read before
+      // the barrier ahead of the request.)
       if (NBUF == 2) {
         if (j > 0 && j + 1 < nch) issue_chunk(j + 1, (u + 1) & 1);  // (chunk 1 was requested with chunk 0)
       } else if (NBUF == 4 && (u & 1) == 0) {
@@ -466,7 +466,7 @@ window_attention_stream_kernel(StreamParams p) {
 
     if (!DMA && j + LEAD < nch) store_chunk((u + LEAD) & (NBUF - 1));
     if (NBUF == 2 || (NBUF == 4 && (u & 1))) {
-      if (DMA) __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the next pair's chunks, requested two chunks ago
+      if (DMA) __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the next chunk or pair of chunks, requested at the start of this one
       __syncthreads();
     }
   }

@@ -387,22 +387,31 @@ static hipError_t launch_rows(NormParams p, bool x_f32, bool pre, hipStream_t st
 
 // Four rows per wave and lane group (1, 2, 3: 2-4 % slower on 1 036 800 rows of 1536), one where that leaves a CU with no more than
 // two blocks (SUB > 1: 2048 x 128 bf16 3.8 -> 2.8 us; at 728 blocks, 23296 x 192, 6.7 against 7.3) and the parameters, which every
-// block of four rows then reads again, do not outweigh the waves that it adds.  Four -> one row per wave, us:
-//   f32  d = 512:   4096 4.5 -> 3.7   7000 5.5 -> 5.3   8192 5.8 -> 7.0        768:  4096 6.2 -> 5.4   6000 8.1 -> 7.3   6500 8.3 -> 8.7
-//        d = 1024:  4096 7.2 -> 6.7   7000 11.3 -> 10.5   8192 11.7 -> 12.1    1536: 3000 8.3 -> 7.8   4096 8.7 -> 10.1   5000 14.6 -> 11.7   7000 15.6 -> 14.8
-//   bf16 d = 768:   4096 5.6 -> 4.6   8192 6.6 -> 6.2        1024: 4096 5.7 -> 5.2   5000 6.5 -> 5.3   5500 6.3 -> 6.6
-//        d = 1536:  4096 6.3 -> 5.9   5500 8.4 -> 8.2   6000 8.4 -> 9.3        2048: 3000 7.9 -> 6.2   3400 8.0 -> 8.1   5000 9.5 -> 9.9   8192 12.0 -> 15.6
-// (up to 4096 rows are one round of one block of sixteen per CU: above 1280 f32 elements the rows short of that keep it).  Rows that
-// fill the lanes (512, 1024, 1536, 2048) turn sooner than those around them; the limits are what 2000 to 8192 rows of 17 widths showed.
+// block of four rows then reads again, do not outweigh the waves that it adds.  Time with four over time with one row per wave, each
+// the mean of both orders of the two outputs in memory (which alone move it by up to a tenth):
+//   rows               3000   3400   4096   5000   6000   7000   8192
+//   f32   d =  512     1.26   1.26   1.24   1.32   1.18   1.17   0.96
+//              768     1.35   1.26   1.21   1.31   1.19   0.98   0.86
+//             1024     1.28   1.11   1.07   1.17   1.13   1.08   1.02
+//             1280     1.37   1.06   1.01   1.28   1.15   1.05   0.96
+//             1536     1.07   0.93   0.91   1.31   1.14   1.07   1.00
+//             2048     1.10   0.94   0.90   1.28   1.10   1.00   0.98
+//   bf16  d =  768     1.34   1.25   1.26   1.37   1.27   1.10   1.02
+//             1024     1.34   1.31   1.22   1.21   1.02   0.89   0.98
+//             1280     1.36   1.26   1.23   1.33   1.23   0.98   0.88
+//             1536     1.33   1.24   1.00   1.06   0.87   0.82   0.73
+//             1792     1.40   1.26   1.23   1.31   1.04   0.83   0.81
+//             2048     1.26   0.98   0.97   1.04   0.89   0.88   0.80
+// (4096 rows are one round of one block of sixteen per CU: wide f32 rows just short of that keep it.)
 static bool one_row_per_wave(int64_t rows, int d, bool x_f32, int sub) {
   if (sub > 1) return rows <= (int64_t)512 * 16 * sub;
-  static const struct { int d; int most_f32, most_bf16; } limits[] = {
-      {384, 8192, 8192},  {704, 7168, 8192},  {1016, 6144, 8192}, {1024, 7168, 5120}, {1280, 7168, 7168},
-      {1528, 6144, 6144}, {1536, 6144, 5120}, {2040, 6144, 5632}, {2048, 6144, 3072}};
-  if (x_f32 && d > 1280 && rows > 3072 && rows <= 4096) return false;
-  for (const auto& l : limits)
-    if (d <= l.d) return rows <= (x_f32 ? l.most_f32 : l.most_bf16);
-  return false;
+  if (x_f32) {
+    if (d > 1408 && rows > 3072 && rows <= 4096) return false;
+    return rows <= (d <= 384 || d >= 1536 ? 8192 : d <= 512 || d > 896 ? 7680 : d <= 704 ? 7168 : 6656);
+  }
+  if (d < 1024) return rows <= 8192;
+  if (d % 512 == 0) return rows <= (d == 1024 ? 6144 : d == 1536 ? 5120 : 3072);  // rows that fill the lanes
+  return rows <= (d <= 1280 ? 6656 : d < 1536 ? 6144 : 5632);
 }
 template <int NV, int SUB>
 static hipError_t launch_few_or_many(const NormParams& p, bool x_f32, bool pre, hipStream_t stream) {

@@ -516,7 +516,7 @@ int norm_gemm_fwd(const aeris_block_config* c, int64_t mod_stride, const void* x
       (c->mod_order != AERIS_NORM_THEN_MOD && c->mod_order != AERIS_MOD_THEN_NORM) || !((float)c->eps >= 0.f) || split % 8 ||
       !(q_scale > 0.f && q_scale < 3.0e38f) || N > 0x7fffffffLL || rows > 0x7fffffffLL / B)
     return AERIS_OK;
-  if (!aeris::norm_gemm_takes(B * rows, (int)N, (int)c->dim, c->x_dtype == AERIS_F32, bias, shift != nullptr, mod_stride, B, rows, act == AERIS_ACT_SWIGLU))
+  if (!aeris::norm_gemm_takes(B * rows, (int)N, (int)c->dim, c->x_dtype == AERIS_F32, act, bias, shift != nullptr, mod_stride, B, rows))
     return AERIS_OK;
   if (int rc = ensure_init(stream, true)) return rc;
   *taken = true;

@@ -331,32 +331,48 @@ void launch_pre(const NormGemmParams& p, bool pre, dim3 grid, hipStream_t stream
 //      131072    61.2 -> 47.0    74.3 -> 63.1     31.1 -> 24.0
 // From 192 on the norm that every share of the columns repeats costs more than the launch and the traffic that go, until there are
 // many rows (not built for those).
-// A ceiling on the rows: a large plain product has tiles of 256, and the norm's launch and its traffic, half as much with a bf16 x,
-// come to less than what tiles of 64 cost; soonest with SwiGLU, which reads two rows of W per output column.  A block with two
-// kernels -> with one of them, the other the same in both, us:
-//        rows           to_qkv, f32 x   to_qkv, bf16 x    GELU, f32 x     GELU, bf16 x     SwiGLU, f32 x   SwiGLU, bf16 x
-//  dim 128, hidden 512
-//       24576            68.4 ->  64.9    61.5 ->  59.0   68.4 ->  63.0    61.5 ->  57.8    66.6 ->  64.1    59.5 ->  59.1
-//       32768            77.5 ->  76.5    68.2 ->  67.4   77.5 ->  74.7    68.2 ->  68.1    79.8 ->  82.4    70.0 ->  75.0
-//      131072           249   -> 246     221   -> 218    249   -> 235     221   -> 213     256   -> 258     228   -> 235
-//      524288           933   -> 883     814   -> 822    933   -> 921     814   -> 839     957   -> 984     862   -> 919
-//     1036800          1709   ->1647    1503   ->1541   1709   ->1700    1503   ->1575    1772   ->1838    1594   ->1742
-//  dim 64, hidden 256
-//       45056            65.3 ->  61.1    59.5 ->  55.3   65.3 ->  59.0    59.5 ->  55.4    61.9 ->  58.7    56.4 ->  55.0
-//      184320           162   -> 165     142   -> 137    162   -> 152     142   -> 138     168   -> 162     147   -> 147
-//      524288           446   -> 437     388   -> 400    446   -> 452     388   -> 397     456   -> 483     400   -> 422
 // The rest is whole column tiles (N is 3 * heads * head_dim or the hidden width, both multiples of 64 wherever the projection behind
 // them is taken), what the vector epilogue and one descriptor over W need, and one modulation row per row tile.
-static int64_t most_rows(int N, int K, bool x_f32, bool swiglu) {
-  if (!swiglu) return x_f32 ? int64_t(1) << 31 : 196608;
-  if (x_f32) return N * (int64_t)K <= 256 * 128 ? 196608 : 28672;
-  return N * (int64_t)K <= 256 * 64 ? 49152 : 12288;
+//
+// A ceiling on the rows (rows_taken).  Once x and C are larger than the last-level cache (256 MB) the plain product with its tiles of
+// 256 waits for memory less than tiles of 64 do, more than the norm's pass costs, except where
+//   - x is f32 and not much smaller than C (N <= 4 K): the norm's pass is much of the traffic
+//   - the plain product's column tiles are partly empty: GELU with N % 256 != 0 and N < 1024 (and by erf), SwiGLU of 64 columns
+// SwiGLU reads two rows of W per output column; from 320 columns of 128 or 512 of 64 on its products lose sooner.  Time of the two
+// kernels over this one's, mean of both orders of the two results in memory:
+//            rows      8192  12288  16384  24576  32768  45056  65536  92160 131072 196608 259200 345600 524288 1036800
+//   none  K=128 N=384 f32   1.08   1.18   1.29   1.35   1.21   1.37   1.08   1.16   1.21   1.15   1.01   1.03   1.04   1.02
+//                    bf16   1.05   1.13   1.21   1.32   1.24   1.42   1.11   1.06   1.16   1.07   1.08   0.91   0.89   0.85
+//         K=64  N=192 bf16  1.19   1.14   1.19   1.34   1.42   1.46   1.35   1.38   1.39   1.15   1.21   1.23   1.15   0.83
+//         K=64  N=768 f32   1.13   1.07   1.05   1.17   1.04   1.22   1.13   1.06   1.10   0.84   0.85   0.87   0.83   0.82
+//   GELU  K=128 N=512 f32   1.26   1.03   1.22   1.37   1.15   1.29   1.07   1.13   1.13   0.96   1.01   1.01   1.01   0.99
+//                    bf16   1.21   1.00   1.21   1.35   1.20   1.26   1.16   1.06   1.09   1.03   0.93   0.94   0.88   0.88
+//         K=64  N=320 bf16  1.01   1.07   1.14   1.18   1.27   1.32   1.43   1.40   1.49   1.50   1.50   1.43   1.32   1.33
+//   SwiGLU K=64 N=64  bf16  1.27   1.29   1.35   1.32   1.71   1.54   1.79   1.57   1.80   1.61   1.56   1.53   1.59   1.49
+//         K=64  N=256 f32   1.26   1.12   1.14   1.16   1.12   1.17   1.17   1.08   1.10   1.10   1.12   1.09   0.88   0.89
+//         K=128 N=256 bf16  1.23   1.03   1.11   1.28   1.18   1.23   1.00   0.91   0.98   0.93   0.91   0.87   0.77   0.78
+//         K=128 N=384 f32   1.11   1.18   1.11   1.29   1.12   1.13   0.87   1.04   0.97   0.94   0.83   0.86   0.86   0.84
+//         K=128 N=512 f32   1.00   0.93   0.99   1.13   0.93   0.93   0.82   0.94   0.93   0.82   0.88   0.89   0.92   0.88
+//         K=64  N=1024 f32  0.93   0.85   0.87   0.85   0.80   0.86   0.93   0.92   0.84   0.90   0.86   0.84   0.87   0.85
+// (A block of dim 128, hidden 512, bf16, on 720 x 1440: SwiGLU 1885 -> 1703 us with two kernels again.)
+static bool rows_taken(int64_t M, int N, int K, bool x_f32, int act) {
+  const int64_t nk = (int64_t)N * K;
+  const bool cached = M * (K * (x_f32 ? 4 : 2) + N * (int64_t)2) <= 280000000;
+  if (act == AERIS_ACT_SWIGLU) {
+    if (N <= 64) return true;
+    if (N >= 1024) return M <= 4096;
+    if (N > 512 || nk > 49152) return M <= 10240;
+    if (nk > 40960) return M <= 49152;
+    return cached && (x_f32 || K < 128 || N < 256 || M <= 65536);
+  }
+  if (act == AERIS_ACT_GELU && N % 256 && N < 1024) return true;
+  return cached || (x_f32 && N <= 4 * K);
 }
 
-bool norm_gemm_takes(int64_t M, int N, int K, bool x_f32, const void* bias, bool modulated, int64_t mod_batch_stride, int64_t B,
-                     int64_t rows_per_batch, bool swiglu) {
-  return M <= most_rows(N, K, x_f32, swiglu) && K % BK == 0 && K <= MAX_K && N % BN == 0 && (reinterpret_cast<uintptr_t>(bias) & 7) == 0 &&
-         (int64_t)(swiglu ? 2 : 1) * N * K * 2 < (int64_t(1) << 31) && M < (int64_t(1) << 31) &&
+bool norm_gemm_takes(int64_t M, int N, int K, bool x_f32, int act, const void* bias, bool modulated, int64_t mod_batch_stride, int64_t B,
+                     int64_t rows_per_batch) {
+  return K % BK == 0 && K <= MAX_K && N % BN == 0 && (reinterpret_cast<uintptr_t>(bias) & 7) == 0 && M < (int64_t(1) << 31) &&
+         (int64_t)(act == AERIS_ACT_SWIGLU ? 2 : 1) * N * K * 2 < (int64_t(1) << 31) && rows_taken(M, N, K, x_f32, act) &&
          (!modulated || mod_batch_stride == 0 || B == 1 || rows_per_batch % BM == 0) &&
          (M + BM - 1) / BM * (N / 32) < (int64_t(1) << 31);
 }

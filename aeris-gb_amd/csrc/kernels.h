@@ -17,8 +17,8 @@ hipError_t gemm_launch(const void* A, const void* W, void* C, const void* bias, 
 
 // norm, modulation and the projection behind them in one kernel (gemm_norm.hip), for what norm_gemm_takes says; act is
 // AERIS_ACT_NONE (bf16 C, `split` as above), _GELU or _SWIGLU
-bool norm_gemm_takes(int64_t M, int N, int K, bool x_f32, const void* bias, bool modulated, int64_t mod_batch_stride, int64_t B,
-                     int64_t rows_per_batch, bool swiglu);
+bool norm_gemm_takes(int64_t M, int N, int K, bool x_f32, int act, const void* bias, bool modulated, int64_t mod_batch_stride, int64_t B,
+                     int64_t rows_per_batch);
 hipError_t norm_gemm_launch(const void* x, int x_dtype, const void* gamma, const void* beta, int param_dtype, const float* shift,
                             const float* scale, int64_t mod_batch_stride, int64_t rows_per_batch, int kind, int order, float eps,
                             const void* W, void* C, const void* bias, int64_t M, int N, int K, int64_t ldc, int act, int split,

@@ -539,8 +539,13 @@ def test_block_norm_and_projection_in_one_kernel(pkg, cuda, B, image, window, di
     (1, (32, 64), (8, 8), 128, 4, 32, 512, "spec0", torch.bfloat16, True),
     (1, (64, 256), (8, 8), 64, 1, 64, 256, "spec0", torch.float32, True),    # 256 row tiles: several column tiles a workgroup, erf
     (1, (168, 256), (8, 8), 128, 2, 64, 512, "spec0", torch.float32, True),  # ... and polynomial
-    (1, (112, 256), (8, 8), 128, 2, 64, 512, "swiglu", torch.float32, True),  # 28672 rows, the most
-    (1, (120, 256), (8, 8), 128, 2, 64, 512, "swiglu", torch.float32, False),
+    (1, (40, 256), (8, 8), 128, 2, 64, 512, "swiglu", torch.float32, True),  # 10240 rows, the most
+    (1, (48, 256), (8, 8), 128, 2, 64, 512, "swiglu", torch.float32, False),
+    (1, (256, 256), (8, 8), 128, 2, 64, 256, "swiglu", torch.bfloat16, True),  # 65536 rows, the most
+    (1, (264, 256), (8, 8), 128, 2, 64, 256, "swiglu", torch.bfloat16, False),
+    (1, (528, 512), (8, 8), 128, 2, 64, 320, "spec0", torch.bfloat16, True),   # 277 million bytes of x and q, k, v
+    (1, (544, 512), (8, 8), 128, 2, 64, 320, "spec0", torch.bfloat16, False),  # 285 million
+    (1, (544, 512), (8, 8), 128, 2, 64, 512, "spec0", torch.float32, True),    # more, but f32 rows
     (2, (12, 36), (12, 12), 64, 1, 64, 64, "spec3", torch.float32, False),   # 432 rows a modulation row: no row tile's multiple
     (1, (8, 8), (8, 8), 192, 3, 64, 192, "spec0", torch.float32, False),     # rows of 192 elements
 ])

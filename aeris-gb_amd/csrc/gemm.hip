@@ -211,34 +211,26 @@ __global__ void __launch_bounds__(NT, 2) gemm_bf16_nt_tile_kernel(GemmParams p) 
     // first, 2048 x 1538 x 1536 25.2 -> 26.6 us, 4096 x 4098 x 4096 167 -> 174, SiLU 3000 x 3072 x 1024 31.4 -> 33.4 (but
     // 1000 x 1002 x 1024, 64 tiles in all, 17.1 -> 16.4).
     constexpr bool READS_FIRST = STAGES > 2;
-    auto read = [&](int ks, bf16x8 (&af)[FM], bf16x8 (&bf)[FN]) {
+    constexpr int STEPS = READS_FIRST ? 2 : 1;  // k-steps of 32 whose fragments are held at once
+    if (!READS_FIRST && behind >= STAGES - 1) issue(kt + STAGES - 1, wr);
 #pragma unroll
-      for (int i = 0; i < FM; ++i) af[i] = *reinterpret_cast<const bf16x8*>(st + a_roff[ks] + i * 16 * 128);
+    for (int k0 = 0; k0 < 2; k0 += STEPS) {
+      bf16x8 af[STEPS][FM], bf[STEPS][FN];
 #pragma unroll
-      for (int j = 0; j < FN; ++j) bf[j] = *reinterpret_cast<const bf16x8*>(st + b_roff[ks] + j * 16 * 128);
-    };
-    auto multiply = [&](const bf16x8 (&af)[FM], const bf16x8 (&bf)[FN]) {
+      for (int ks = 0; ks < STEPS; ++ks) {
 #pragma unroll
-      for (int i = 0; i < FM; ++i)
+        for (int i = 0; i < FM; ++i) af[ks][i] = *reinterpret_cast<const bf16x8*>(st + a_roff[k0 + ks] + i * 16 * 128);
 #pragma unroll
-        for (int j = 0; j < FN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[j], af[i], acc[i][j], 0, 0, 0);
-    };
-    if constexpr (READS_FIRST) {
-      bf16x8 af[2][FM], bf[2][FN];
-#pragma unroll
-      for (int ks = 0; ks < 2; ++ks) read(ks, af[ks], bf[ks]);
-      if (behind >= STAGES - 1) issue(kt + STAGES - 1, wr);
-#pragma unroll
-      for (int ks = 0; ks < 2; ++ks) multiply(af[ks], bf[ks]);
-    } else {
-      if (behind >= STAGES - 1) issue(kt + STAGES - 1, wr);
-#pragma unroll
-      for (int ks = 0; ks < 2; ++ks) {
-        bf16x8 af[FM], bf[FN];
-        read(ks, af, bf);
-        multiply(af, bf);
+        for (int j = 0; j < FN; ++j) bf[ks][j] = *reinterpret_cast<const bf16x8*>(st + b_roff[k0 + ks] + j * 16 * 128);
       }
+      if (READS_FIRST && behind >= STAGES - 1) issue(kt + STAGES - 1, wr);
+#pragma unroll
+      for (int ks = 0; ks < STEPS; ++ks)
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+          for (int j = 0; j < FN; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[ks][j], af[ks][i], acc[i][j], 0, 0, 0);
     }
     if (++rd == STAGES) rd = 0;
     if (++wr == STAGES) wr = 0;

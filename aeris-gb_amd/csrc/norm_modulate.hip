@@ -390,13 +390,15 @@ static hipError_t launch_rows(NormParams p, bool x_f32, bool pre, hipStream_t st
 // block of four rows then reads again, do not outweigh the waves that it adds.  Time with four over time with one row per wave, each
 // the mean of both orders of the two outputs in memory (which alone move it by up to a tenth):
 //   rows               3000   3400   4096   5000   6000   7000   8192
-//   f32   d =  512     1.26   1.26   1.24   1.32   1.18   1.17   0.96
+//   f32   d =  448            1.18   1.16   1.34   1.21   1.11   1.00
+//              512     1.26   1.26   1.24   1.32   1.18   1.17   0.96
 //              768     1.35   1.26   1.21   1.31   1.19   0.98   0.86
 //             1024     1.28   1.11   1.07   1.17   1.13   1.08   1.02
 //             1280     1.37   1.06   1.01   1.28   1.15   1.05   0.96
 //             1536     1.07   0.93   0.91   1.31   1.14   1.07   1.00
 //             2048     1.10   0.94   0.90   1.28   1.10   1.00   0.98
-//   bf16  d =  768     1.34   1.25   1.26   1.37   1.27   1.10   1.02
+//   bf16  d =  448            1.18   1.15   1.18   1.12   1.09   0.93
+//              768     1.34   1.25   1.26   1.37   1.27   1.10   1.02
 //             1024     1.34   1.31   1.22   1.21   1.02   0.89   0.98
 //             1280     1.36   1.26   1.23   1.33   1.23   0.98   0.88
 //             1536     1.33   1.24   1.00   1.06   0.87   0.82   0.73
@@ -407,9 +409,9 @@ static bool one_row_per_wave(int64_t rows, int d, bool x_f32, int sub) {
   if (sub > 1) return rows <= (int64_t)512 * 16 * sub;
   if (x_f32) {
     if (d > 1408 && rows > 3072 && rows <= 4096) return false;
-    return rows <= (d <= 384 || d >= 1536 ? 8192 : d <= 512 || d > 896 ? 7680 : d <= 704 ? 7168 : 6656);
+    return rows <= (d < 512 || d >= 1536 ? 8192 : d == 512 || d > 896 ? 7680 : d <= 704 ? 7168 : 6656);
   }
-  if (d < 1024) return rows <= 8192;
+  if (d < 1024) return rows <= (d > 416 && d < 512 ? 7168 : 8192);
   if (d % 512 == 0) return rows <= (d == 1024 ? 6144 : d == 1536 ? 5120 : 3072);  // rows that fill the lanes
   return rows <= (d <= 1280 ? 6656 : d < 1536 ? 6144 : 5632);
 }

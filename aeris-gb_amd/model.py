@@ -18,6 +18,7 @@ from __future__ import annotations
 import itertools
 import math
 import os
+import struct
 from dataclasses import dataclass
 from typing import NamedTuple, Optional, Tuple
 
@@ -588,6 +589,10 @@ class InputStage(nn.Module):
     def forward(self, x, interval, out_dtype=None, cond=None, x_div=1.0):
         """x [b, n, Cin]; or x [b, n, C0] with cond [b, n, Cin - C0]: the embedding of cat([x / x_div, cond], 2)
         (inference.py:160) without building the concatenated tensor."""
+        tok = self._tokens(x, out_dtype, cond, x_div)
+        return tok, timestep_embedding(interval, tok.shape[-1], self.sinusoidal_emb_max_period)
+
+    def _tokens(self, x, out_dtype, cond, x_div):
         b, n, c = x.shape
         if cond is not None:
             c += cond.shape[-1]
@@ -604,16 +609,13 @@ class InputStage(nn.Module):
         x2 = x.reshape(b * n, -1).float().contiguous()
         c2 = None if cond is None else cond.reshape(b * n, -1).float().contiguous()
         if fused:
-            tok = ops.input_stage(x2, x_div if cond is not None else 1.0, c2, ape, wp, dim,
-                                  out_dtype=out_dtype or self.model_dtype).view(b, n, -1)
+            return ops.input_stage(x2, x_div if cond is not None else 1.0, c2, ape, wp, dim,
+                                   out_dtype=out_dtype or self.model_dtype).view(b, n, -1)
+        if cond is None:
+            a = ops.embed_prepare(x2, ape, k_pad, split=True)
         else:
-            if cond is None:
-                a = ops.embed_prepare(x2, ape, k_pad, split=True)
-            else:
-                a = ops.embed_concat(x2, x_div, c2, ape, k_pad, split=True)
-            tok = ops.gemm(a, wp, None, out_dtype=out_dtype or self.model_dtype).view(b, n, -1)
-        t = timestep_embedding(interval, tok.shape[-1], self.sinusoidal_emb_max_period)
-        return tok, t
+            a = ops.embed_concat(x2, x_div, c2, ape, k_pad, split=True)
+        return ops.gemm(a, wp, None, out_dtype=out_dtype or self.model_dtype).view(b, n, -1)
 
 
 class OutputStage(nn.Module):
@@ -738,6 +740,73 @@ class LocalAERIS(nn.Module):
                         block_hook(k, tok)
             out = self.output_stage(tok, t)
         return (out, tok) if return_hidden else out
+
+
+def _unhooked(module, cls):
+    """Whether the module is ``cls`` as it is, its forward called by nobody but this file: no forward of its own, no hook."""
+    return not (type(module) is not cls or "forward" in module.__dict__ or cls.forward is not _AS_DEFINED[cls] or module._forward_hooks or
+                module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks)
+
+
+_AS_DEFINED.update({LocalAERIS: LocalAERIS.forward, InputStage: InputStage.forward})
+
+
+class CallsAhead:
+    """The denoiser calls of one draw, made by the sampler one after the other without anything of the caller's in between: what
+    depends on the noise level alone, the modulation vectors, is computed for several levels at a time (the matrices are read
+    once for all of them, and a level that ends one step and begins the next is computed once), and what the blocks' modules
+    hold is looked up once.  Same kernels on the same values as ``LocalAERIS.forward``: the same bits.  Lives as long as the draw.
+    """
+    LEVELS = 8  # levels at a time: the rows that the modulation kernel takes in one pass over a matrix
+
+    def __init__(self, model, levels):
+        layers = list(model.layers)
+        half = (model.window_size[0] // 2, model.window_size[1] // 2)
+        self.model, self.levels = model, levels
+        self.layers = [(layer, half if i % 2 == 1 else (0, 0), layer.modulations()) for i, layer in enumerate(layers)]
+        self.first, self.vectors, self.calls = 0, None, None
+
+    def _modulations(self, i, dim):
+        """The modulation vectors of level i, f32 [1, N] each: those of the blocks, then the output stage's."""
+        if self.vectors is None or not self.first <= i < self.first + self.LEVELS:
+            t = timestep_embedding(self.levels[i:i + self.LEVELS], dim, self.model.input_stage.sinusoidal_emb_max_period)
+            modules = [m for _, _, own in self.layers for m in own]
+            self.first, self.vectors = i, _modulation_vectors(modules, t, [_mlp_params(self.model.output_stage.modulation)])
+        return [v[i - self.first:i - self.first + 1] for v in self.vectors]
+
+    def _block_calls(self, tok, mods):
+        k = 0
+        for layer, shift, own in self.layers:
+            yield from layer.block_calls(tok, mods[k:k + len(own)], shift)
+            k += len(own)
+
+    def __call__(self, x, cond, x_div, i):
+        """``LocalAERIS.forward(x, levels[i:i + 1], cond=cond, x_div=x_div)``."""
+        model = self.model
+        tok = model.input_stage._tokens(x, model.residual_dtype, cond, x_div)
+        mods = self._modulations(i, tok.shape[-1])
+        if self.calls is None:
+            self.calls = list(self._block_calls(tok, mods))
+        calls = self.calls
+        hidden = torch.empty_like(tok) if len(calls) == 1 else tok
+        if any(c.computed or c.config != calls[0].config for c in calls):
+            _run_blocks(self._block_calls(tok, mods), tok, hidden)
+        elif calls:
+            at = ops.BLOCK_MODULATION
+            records = [c.record for c in calls] if len(mods) == 1 else [
+                c.record[:at] + struct.pack("=Q", m.data_ptr()) + c.record[at + 8:] for c, m in zip(calls, mods)]
+            ops.swin_blocks(records, tok, hidden, *calls[0].config, shapes=[c.fused for c in calls])
+        return model.output_stage(hidden, None, m=mods[-1])
+
+
+def calls_ahead(model, levels):
+    """``CallsAhead`` for a draw with ``model`` at the noise levels f32 [n], None where each call has to look again at what the
+    model's modules are: a model of another class, one with hooks or methods of the caller's, weights that are computed."""
+    if not (_unhooked(model, LocalAERIS) and _unhooked(model._modules.get("input_stage"), InputStage) and
+            _unhooked(model._modules.get("output_stage"), OutputStage) and _plain(model.output_stage, OutputStage) and
+            all(type(layer) is SwinLayer and _own_blocks(layer) for layer in model.layers) and ops._ordinary_execution()):
+        return None
+    return CallsAhead(model, levels)
 
 
 def convert_inference_checkpoint(path, N, model, map_location="cpu"):

@@ -467,6 +467,7 @@ def modulation_mlps(x: torch.Tensor, mlps):
 
 
 BLOCK_RECORD = struct.Struct("=15Q5q")  # struct aeris_block of include/aeris_hip.h
+BLOCK_MODULATION = 14 * 8  # offset of its modulation address
 BLOCK_CONFIG = struct.Struct("=15q2d")  # struct aeris_block_config
 
 

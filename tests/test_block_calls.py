@@ -455,3 +455,82 @@ def test_a_swiglu_mlp_has_no_biases(pkg, calls):
     ff.w1, ff.w2 = Weight(ff.w1.weight), Weight(ff.w2.weight)
     layer(*inputs(pkg))
     layer(*inputs(pkg), tap=lambda *a: None)
+
+
+def draw_of(pkg, calls, monkeypatch, change=lambda sampler: None, steps=10, **kw):
+    """The native calls of one draw, by name, with a model of two blocks."""
+    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: None)
+    s = pkg.TrigFlowSampler(model_of(pkg, **kw), n_steps=steps, device="cpu")
+    change(s)
+    del calls[:]
+    s.sample(torch.randn(1, 512, 6), torch.randn(1, 512, 4))
+    return calls.names()
+
+
+@pytest.mark.parametrize("kw", [dict(preset="ref"), dict(preset="spec", mod_ways=2)])
+def test_a_draw_computes_the_modulation_of_several_levels_at_once(pkg, calls, monkeypatch, kw):
+    """Ten levels: two passes over the modulation matrices for nineteen denoiser calls, each with its own level's vectors."""
+    names = draw_of(pkg, calls, monkeypatch, **kw)
+    assert names.count("aeris_blocks_fwd") == 19 and names.count("aeris_modulation_layers_fwd") == 4
+    assert [c[1][2] for c in calls if c[0] == "aeris_modulation_layers_fwd"] == [8, 8, 2, 2]
+    records = [c[1][1] for c in calls if c[0] == "aeris_blocks_fwd"]
+    size = pkg.ops.BLOCK_RECORD.size
+    vectors = [[pkg.ops.BLOCK_RECORD.unpack(r[k:k + size])[14] for k in (0, size)] for r in records]
+    level = [0] + [k for i in range(1, 10) for k in (i, i)]
+    for k in range(2):  # consecutive rows within a pass
+        width = 4 * 128 * 2 * kw.get("mod_ways", 3)
+        for a, b, va, vb in zip(level, level[1:], vectors, vectors[1:]):
+            if a // 8 == b // 8:
+                assert vb[k] - va[k] == (b - a) * width
+
+
+@pytest.mark.parametrize("what", ["model_hook", "input_hook", "output_hook", "modulation_hook", "core", "model_class", "model_forward",
+                                  "sampler_class", "sampler_method", "advance"])
+def test_a_draw_with_parts_of_the_callers_looks_at_every_call(pkg, calls, monkeypatch, what):
+    seen = []
+
+    def change(s):
+        m = s.model
+        if what == "model_hook":
+            m.register_forward_hook(lambda *a: seen.append(1))
+        elif what == "input_hook":
+            m.input_stage.register_forward_hook(lambda *a: seen.append(1))
+        elif what == "output_hook":
+            m.output_stage.register_forward_pre_hook(lambda *a: seen.append(1))
+        elif what == "modulation_hook":
+            m.layers[0].modulelist[0][4].register_forward_hook(lambda *a: seen.append(1))
+        elif what == "core":
+            attn = m.layers[0].modulelist[0][1]
+            attn.core = lambda y, shift, out=None: seen.append(1) or pkg.Attention.core(attn, y, shift, out=out)
+        elif what == "model_class":
+            m.__class__ = type("Mine", (pkg.LocalAERIS,), {"forward": lambda self, *a, **kw: seen.append(1) or pkg.LocalAERIS.forward(self, *a, **kw)})
+        elif what == "model_forward":
+            m.forward = lambda *a, **kw: seen.append(1) or pkg.LocalAERIS.forward(m, *a, **kw)
+        elif what == "sampler_class":
+            s.__class__ = type("Mine", (pkg.TrigFlowSampler,), {"_denoise": lambda self, *a: seen.append(1) or pkg.TrigFlowSampler._denoise(self, *a)})
+        elif what == "sampler_method":
+            s._denoise = lambda *a: seen.append(1) or pkg.TrigFlowSampler._denoise(s, *a)
+        else:
+            s._advance = lambda *a: seen.append(1) or pkg.TrigFlowSampler._advance(s, *a)
+    draw_of(pkg, calls, monkeypatch, change, steps=2)
+    assert len(seen) == 3
+
+
+def test_a_draw_with_computed_weights_makes_them_at_every_call(pkg, calls, monkeypatch):
+    made = []
+
+    class Made(torch.nn.Module):
+        def forward(self, w):
+            made.append(1)
+            return w.clone()
+
+    def change(s):
+        torch.nn.utils.parametrize.register_parametrization(s.model.layers[1].modulelist[0][1].wo, "weight", Made())
+        del made[:]
+    names = draw_of(pkg, calls, monkeypatch, change, steps=2)
+    assert names.count("aeris_blocks_fwd") == 6 and len(made) >= 3
+
+
+def test_an_empty_model_draws(pkg, calls, monkeypatch):
+    names = draw_of(pkg, calls, monkeypatch, steps=2, layers=0)
+    assert names.count("aeris_output_stage_fwd") == 3 and "aeris_blocks_fwd" not in names

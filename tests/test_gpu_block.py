@@ -316,6 +316,25 @@ def test_full_grid_block_against_oracle_strips(pkg, cuda, name, geo):
             assert err <= 1e-2, (name, shifted, k, err)
 
 
+@pytest.mark.parametrize("form,B,steps", [("ref", 1, 10), ("spec2", 3, 9), ("spec0", 1, 2)])
+def test_a_draw_is_its_denoiser_calls_one_by_one(pkg, cuda, form, B, steps):
+    """What a draw computes ahead for several noise levels is what each call computes by itself, bit for bit."""
+    mk = OracleConfig.ref if form == "ref" else (lambda **kw: OracleConfig.spec(mod_ways=int(form[-1]), **kw))
+    cfg = mk(n_layers=4, in_channels=20, out_channels=8, sublayers=2, **SMALL16)
+    model = make_model(pkg, cfg, oracle.init_model_weights(cfg, 2, nontrivial=True), cuda, torch.float32, "ref" if form == "ref" else "spec")
+    g = torch.Generator().manual_seed(4)
+    cond, lat = torch.randn(B, 32 * 48, 12, generator=g).to(cuda), torch.randn(B, 32 * 48, 8, generator=g).to(cuda)
+    one_by_one = pkg.TrigFlowSampler(lambda x, t, cond=None, x_div=1.0: model(x, t, cond=cond, x_div=x_div), n_steps=steps, device=cuda)
+    s = pkg.TrigFlowSampler(model, n_steps=steps, device=cuda)
+    want = one_by_one.sample(cond, lat)
+    assert torch.equal(s.sample(cond, lat), want) and torch.isfinite(want).all()
+    s.capture(cond, lat)
+    for _ in range(3):
+        assert torch.equal(s.sample_graph(cond, lat), want)
+        model(torch.cat([lat, cond], 2), torch.zeros(1, device=cuda))
+        torch.cuda.synchronize()
+
+
 def test_full_grid_ensemble_batch_matches_single_members(pkg, cuda):
     """configs[4] shape: 4 ensemble members as batch 4 on the 720x1440 grid (4 147 200 rows through every kernel,
     per-member modulation vectors).  A member's rows of the batched result must be bit-identical to running that

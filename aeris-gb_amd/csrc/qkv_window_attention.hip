@@ -303,20 +303,6 @@ __global__ void __launch_bounds__(QA_NT) qkv_window_attention_kernel(QkvAttnPara
     const int l15 = lane_t & 15, q4 = lane_t >> 4, l31 = lane_t & 31, hi = lane_t >> 5;
     const int qpos = wave_u * 32 + l31;
     const uint32_t q_rel = (uint32_t)((qpos / QA_WS) * W + qpos % QA_WS);
-#if defined(QA_LAB) && QA_LAB == 2
-    {  // timing only: the main loop alone (the accumulators are folded into one store so that they stay live)
-      f32x4 t = {0.f, 0.f, 0.f, 0.f};
-      for (int i = 0; i < QA_FM; ++i) for (int j = 0; j < QA_FN; ++j) t += acc[i][j];
-      issue_a();
-      *reinterpret_cast<f32x4*>(p.out + ((uint64_t)un.b * (uint32_t)(H * W) + window_base(un) + q_rel) * (uint32_t)inner + un.head * QA_HD + hi * 8) = t;
-      u32x2 bq0[QA_FN];
-      for (int j = 0; j < QA_FN; ++j) bq0[j] = u32x2{0u, 0u};
-      init_acc(bq0);
-      __builtin_amdgcn_s_waitcnt(WAIT_ALL);
-      __builtin_amdgcn_s_barrier();
-      return;
-    }
-#endif
     unsigned char* const sQ = smem;                                   // A0: idle, its refill is issued below
     unsigned char* const sK = smem + QA_A_BYTES;                      // A1: the last k-tile's stage
     unsigned char* const sV0 = smem + QA_W_OFF + sw_last * QA_W_BYTES;  // the last k-tile's W stage: V rows 0..191
@@ -372,13 +358,8 @@ __global__ void __launch_bounds__(QA_NT) qkv_window_attention_kernel(QkvAttnPara
     __builtin_amdgcn_sched_barrier(0);
     // 3. the sweep
     // (wave-uniform, and said so: the mask arithmetic must stay behind a scalar branch that all but the border windows skip)
-#ifdef QA_LAB_MASK_EVERY  // timing experiment: every QA_LAB_MASK_EVERY-th unit of a workgroup takes the mask path
-    const bool my = __builtin_amdgcn_readfirstlane((int)(p.use_mask && (r_done % QA_LAB_MASK_EVERY) == 0)) != 0;
-    const bool mx = false;
-#else
     const bool my = __builtin_amdgcn_readfirstlane((int)(p.use_mask && p.sy > 0 && un.wy == p.nWy - 1)) != 0;
     const bool mx = __builtin_amdgcn_readfirstlane((int)(p.use_mask && p.sx > 0 && un.wx == p.nWx - 1)) != 0;
-#endif
     const WindowLogits<QA_WS, QA_WS, HAS_BIAS> logits(smem + QA_BIAS_OFF, qpos, hi, my, mx, p.sy, p.sx);
     auto load_k = [&](int kb, bf16x8 (&f)[KS]) {
 #pragma unroll
@@ -394,12 +375,7 @@ __global__ void __launch_bounds__(QA_NT) qkv_window_attention_kernel(QkvAttnPara
     const LoadVTransposed<DB, decltype(v_step)> load_v(lane_t, v_step);
     f32x16 o[DB];
     float sum;
-#if defined(QA_LAB) && QA_LAB >= 1
-    sum = 1.f;
-    for (int db = 0; db < DB; ++db) for (int e = 0; e < 16; ++e) o[db][e] = __builtin_bit_cast(float, __builtin_bit_cast(u32x4, qf[e & 3])[db]);
-#else
     attention_sweep<NQ, KS, DB, HAS_BIAS>(logits, load_k, load_v, [](int) {}, qf, o, sum);
-#endif
     const uint32_t tok = (uint32_t)un.b * (uint32_t)(H * W) + (window_wraps(un) ? token_in_image(un, qpos) : window_base(un) + q_rel);
     // the next unit's projection bias: requested ahead of the output stores (vector memory operations complete in order)
     u32x2 bq_next[QA_FN];

@@ -426,12 +426,21 @@ namespace {
 // (Over 487 shapes, M 1024 .. 51 840, N and K 192 .. 4096, every epilogue, all forms and the 128 x 128 tiles of the tile kernel
 // timed: the choice takes 0.2 % longer than the fastest form on average, 24 % at most, where the small tiles are kept one
 // size too long, 24 576 x 192 x 192: 10.8 us against 8.7.)
-enum Kind { TILE64, PERSISTENT128, PERSISTENT256 };
+//
+// Tiles of 192 columns take 0.85-0.95 of the time of those of 256 for three quarters of the work, so they pay only where they need
+// no more rounds: N just over a multiple of 256, or a last round that is mostly empty.  256 -> 192 columns, us:
+//   256 rows   8192 x 1536 x 1536 (f32 C and residual) 45.1 -> 42.6, x 6144 126 -> 119; 9000 x 1152 x 1152 34.6 -> 32.2; 14400 x 1536 x 1536
+//              82.1 -> 76.3; 30000 x 576 x 576 43.8 -> 39.8; 10000 x 2304 x 768 (planes) 39.7 -> 37.1; 51840 x 320 x 1280 (bf16) 57.6 -> 53.3
+//   128 rows   12480 x 384 x 384 (f32) 14.6 -> 12.4, x 1088 22.3 -> 20.0
+//   more rounds: 64800 x 1536 x 512 97.5 -> 106, 64800 x 512 x 2048 (bf16) 118 -> 140, 518400 x 1536 x 1536 (f32) 2402 -> 2595
+// A bf16 residual is read in 64-byte pieces there, which short products wait for (51840 x 320 x 320 25.3 -> 27.1, 128 rows 32768 x 192 x
+// 768 17.4 -> 18.5), and short plain ones in tiles of 128 rows gain nothing (32768 x 576 x 192 17.7 -> 18.3).
+enum Kind { TILE64, PERSISTENT128, PERSISTENT256, PERSISTENT128_192, PERSISTENT256_192 };
 
 struct Shape {
   int64_t M;
   int N, KT, act;
-  bool f32, res;
+  bool f32, res, w192;  // w192: tiles of 192 columns take the problem
 };
 
 float epilogue_us(const Shape& s) {  // of a 256 x 256 tile
@@ -450,6 +459,13 @@ float estimate_us(Kind kind, const Shape& s) {
     const float per_k = n <= 3.f ? 0.15f + 0.17f * n : 0.22f * n;
     return 3.0f + s.KT * per_k + n * (s.f32 ? 1.0f : 0.5f);
   }
+  if (kind == PERSISTENT128_192 || kind == PERSISTENT256_192) {
+    const bool tall = kind == PERSISTENT256_192;
+    const int bm = tall ? 256 : 128;
+    auto rounds = [&](int bn) { return ((tiles_of(s, bm, bn) + 7) / 8 + 31) / 32; };
+    if (!s.w192 || rounds(192) > rounds(256) || !(s.f32 || (tall && (!s.res || s.KT >= 16)))) return 1e30f;
+    return (s.f32 ? (tall ? 0.93f : 0.88f) : 0.95f) * estimate_us(tall ? PERSISTENT256 : PERSISTENT128, s);
+  }
   const int bm = kind == PERSISTENT256 ? 256 : 128;
   const int64_t per_xcd = (tiles_of(s, bm, 256) + 7) / 8;
   const float rounds = (float)((per_xcd + 31) / 32);
@@ -460,7 +476,7 @@ float estimate_us(Kind kind, const Shape& s) {
 Kind best_kind(const Shape& s, float* us) {
   Kind best = TILE64;
   *us = estimate_us(TILE64, s);
-  for (Kind k : {PERSISTENT128, PERSISTENT256}) {
+  for (Kind k : {PERSISTENT128, PERSISTENT256, PERSISTENT128_192, PERSISTENT256_192}) {
     const float t = estimate_us(k, s);
     if (t < *us) { *us = t; best = k; }
   }
@@ -469,10 +485,11 @@ Kind best_kind(const Shape& s, float* us) {
 
 hipError_t launch_kind(Kind kind, const GemmParams& p, hipStream_t stream) {
   if (kind == TILE64) return launch_tile_act<64, 64, 3, true>(p, stream);
-  return gemm_persistent_launch(p, kind == PERSISTENT256 ? 256 : 128, stream);
+  return gemm_persistent_launch(p, kind == PERSISTENT256 || kind == PERSISTENT256_192 ? 256 : 128,
+                                kind == PERSISTENT128_192 || kind == PERSISTENT256_192 ? 192 : 256, stream);
 }
 
-Shape shape_of(const GemmParams& p, int act) { return {p.M, p.N, p.K / BK, act, p.c_dtype == AERIS_F32, p.residual != nullptr}; }
+Shape shape_of(const GemmParams& p, int act) { return {p.M, p.N, p.K / BK, act, p.c_dtype == AERIS_F32, p.residual != nullptr, gemm_persistent_takes_192(p)}; }
 
 // vector epilogue: 8 / 16-byte accesses to C and the residual (4-element alignment of every row), to bias and gate rows
 bool vector_epilogue(const GemmParams& p) {
@@ -560,7 +577,8 @@ hipError_t gemm_launch(const void* A, const void* W, void* C, const void* bias, 
     rest.M = M - head.M;
     float t_rest = 0.f;
     const Kind rest_kind = best_kind(rest, &t_rest);
-    if (estimate_us(PERSISTENT256, head) + t_rest < 0.97f * one) {
+    // (against tiles of 192 the estimate of two launches is too low: 14400 x 1536 x 1536 82.1 us, x 6144 253, in one 76.3 and 247)
+    if (estimate_us(PERSISTENT256, head) + t_rest < (kind == PERSISTENT256_192 ? 0.90f : 0.97f) * one) {
       const hipError_t e = launch_kind(PERSISTENT256, rows_of(p, 0, head.M), stream);
       return e != hipSuccess ? e : launch_kind(rest_kind, rows_of(p, head.M, rest.M), stream);
     }

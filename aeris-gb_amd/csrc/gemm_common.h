@@ -66,8 +66,10 @@ __device__ __forceinline__ uint32_t swz_off(int row, int chunk) {
 // for the GEMM of this shape and alignment and for the kernel that has a norm ahead of it
 bool gemm_gelu_by_polynomial(const GemmParams& p);
 
-// persistent kernel (gemm_persistent.hip), tiles of tile_height (128 or 256) rows x 256 columns; needs N % 4 == 0 and ldc % 4 == 0
+// persistent kernel (gemm_persistent.hip), tiles of tile_height (128 or 256) rows x tile_width (256, or 192 where
+// gemm_persistent_takes_192) columns; needs N % 4 == 0 and ldc % 4 == 0
 hipError_t gemm_persistent_configure();
-hipError_t gemm_persistent_launch(const GemmParams& p, int tile_height, hipStream_t stream);
+bool gemm_persistent_takes_192(const GemmParams& p);
+hipError_t gemm_persistent_launch(const GemmParams& p, int tile_height, int tile_width, hipStream_t stream);
 
 }  // namespace aeris

@@ -1,4 +1,4 @@
-// Persistent bf16 MFMA GEMM for gfx950, 256x256 (or 128x256) output tiles, k-tiles of 64:  C[M,N] = epilogue(A[M,K] * W[N,K]^T)
+// Persistent bf16 MFMA GEMM for gfx950, output tiles of 256 or 128 rows x 256 or 192 columns, k-tiles of 64:  C[M,N] = epilogue(A[M,K] * W[N,K]^T)
 //
 // Same LDS swizzle as the plain tile kernel (gemm.hip), built around what bounds it on MI355X:
 //   - v_mfma_f32_16x16x32_bf16, not 32x32x16: same FLOP per cycle and the same LDS bytes per FLOP (a fragment is
@@ -16,6 +16,10 @@
 //     the MFMA stream if the computing wave issued it
 //   - tiles of 128 rows (same main loop, 16 MFMAs per slot instead of 32) where they fill the chip and 256-row tiles do not:
 //     8192 x 1024 x 1024 with f32 residual 29.8 -> 26 us, 12480 x 384 x 1088 27.8 -> 22 us; per FLOP they are 30 % slower
+//   - tiles of 192 columns (waves four by two, 64 or 32 rows x 96 columns each: 10 fragment reads for 24 MFMAs where two by four
+//     would need 11) where N or the last round leaves tiles of 256 partly empty: 8192 x 1536 x 6144 with f32 residual is 192 tiles on
+//     256 CUs, 126 -> 119 us as 256 of them; 12480 x 384 x 384 14.6 -> 12.4.  A tile takes 0.85 of a full one's time, which the choice of
+//     form (gemm.hip) weighs
 //   - tiles are ordered so that the workgroups resident on one XCD (blockIdx % 8) cover a contiguous chunk, 4 row
 //     panels x all column tiles at a time: few distinct A / W k-slices per step compete for that XCD's 4 MB L2
 //   - the epilogue stages through the idle A stage (wave-private 4 KB): fragments (4 consecutive n per lane) are
@@ -29,17 +33,15 @@
 namespace aeris {
 
 namespace {
-constexpr int BN = 256, BK = 64, WM = 2, WN = 4;
-constexpr int NT = WM * WN * 64;          // 512 threads
-constexpr int FN = BN / WN / 16;          // 4 fragments of 16 columns
-constexpr int B_BYTES = BN * BK * 2;      // 32 KB per stage of the W tile
+constexpr int BK = 64, WAVES = 8;
+constexpr int NT = WAVES * 64;            // 512 threads
 constexpr int A_STAGES = 2, B_STAGES = 3;
 constexpr int GM = 4;                     // row panels per L2 group
 constexpr int STG_BYTES = 4096;           // staging area of a wave in the epilogue
 // tile height 256: two A stages of 32 KB, the idle one doubles as the staging area (a wave's part of it is 4 KB); height
 // 128: two of 16 KB and a staging area of its own.  160 KB of LDS either way: all of the CU's.
-constexpr int smem_bytes(int bm) { return A_STAGES * bm * BK * 2 + B_STAGES * B_BYTES + (bm == 256 ? 0 : WM * WN * STG_BYTES); }
-static_assert(smem_bytes(256) == 160 * 1024 && smem_bytes(128) == 160 * 1024, "LDS of a CU");
+constexpr int smem_bytes(int bm, int bn) { return A_STAGES * bm * BK * 2 + B_STAGES * bn * BK * 2 + (bm == 256 ? 0 : WAVES * STG_BYTES); }
+static_assert(smem_bytes(256, 256) == 160 * 1024 && smem_bytes(128, 256) == 160 * 1024, "LDS of a CU");
 }  // namespace
 
 // PLAIN: no gate and no residual (qkv, fc1): the epilogue is compiled without those paths - about 2 % faster than
@@ -47,9 +49,12 @@ static_assert(smem_bytes(256) == 160 * 1024 && smem_bytes(128) == 160 * 1024, "L
 // fc2 on a bf16 residual stream), compiled as a kernel of its own so that its deeper residual prefetch does not
 // share registers with the general path.  RES_F32: the same for f32 C with an f32 residual (proj, fc2 on an f32
 // residual stream).
-template <int BM, int ACT, bool OUT_F32, bool PLAIN, bool RES_BF16 = false, bool RES_F32 = false>
+template <int BM, int BN, int ACT, bool OUT_F32, bool PLAIN, bool RES_BF16 = false, bool RES_F32 = false>
 __global__ void __launch_bounds__(NT) gemm_bf16_nt_persistent_kernel(GemmParams p_in) {
-  constexpr int FM = BM / WM / 16;          // 8 (4) fragments of 16 rows
+  constexpr int WM = BN == 256 ? 2 : 4, WN = WAVES / WM;  // waves over the tile: 128 (64) rows x 64 columns each, or 64 (32) x 96
+  constexpr int FM = BM / WM / 16, FN = BN / WN / 16;     // fragments of 16 rows, of 16 columns
+  constexpr int B_BYTES = BN * BK * 2;                    // 32 (24) KB per stage of the W tile
+  constexpr int W_LD = BN / 64;                           // load instructions of a wave per k-tile of W (8 rows each)
   constexpr int A_BYTES = BM * BK * 2;      // 32 (16) KB per stage of the A tile
   constexpr int A_LD = BM / 64;             // load instructions of a wave per k-tile of A (8 rows each); 4 for W
   constexpr int B_OFF = A_STAGES * A_BYTES;
@@ -97,11 +102,11 @@ __global__ void __launch_bounds__(NT) gemm_bf16_nt_persistent_kernel(GemmParams 
   // swizzled tile layout (swz_off), so the lane fetches the chunk which that layout keeps at its LDS slot (eight
   // consecutive lanes fetch the 128 contiguous bytes of one row).  Rows past the end of A or W are outside the
   // buffer descriptor and arrive as zeros; they only feed rows / columns of C that are never stored.
-  // Per k-tile a wave brings in 32 rows of A and 32 rows of W, 4 instructions each.  Waves 0-3 (group 0) load the
+  // Per k-tile a wave brings in 32 rows of A and 32 (24) rows of W, 4 (3) instructions.  Waves 0-3 (group 0) load the
   // rows of A that only group 0 reads, waves 4-7 those of group 1.  A and W are two independent streams over the
   // flat sequence (tile, k-tile): W runs one k-tile further ahead than A.
   const int wave_u = __builtin_amdgcn_readfirstlane(wave);
-  const int grp = wave_u / WN;
+  const int grp = wave_u / (WAVES / 2), wm_u = wave_u / WN;
   uint32_t ld_voff[2];  // lane part of the source offset, for even / odd 8-row blocks
   {
     const int dr = lane >> 4, pos = lane & 15;
@@ -128,7 +133,7 @@ __global__ void __launch_bounds__(NT) gemm_bf16_nt_persistent_kernel(GemmParams 
     if (rows > BM) rows = BM;
     rs_a = __builtin_amdgcn_make_buffer_rsrc((void*)(p.A + m0 * K), 0, (int)(rows * K * 2), 0x00020000);
   };
-  // Always 4 loads, also past the end of the list (into stages nobody reads any more, from a descriptor without
+  // Always all loads, also past the end of the list (into stages nobody reads any more, from a descriptor without
   // records): the number of loads in flight at any point of the k-loop is then the same for every k-tile, and no wait
   // has to be chosen at run time.
   auto issue_a = [&]() {
@@ -159,14 +164,14 @@ __global__ void __launch_bounds__(NT) gemm_bf16_nt_persistent_kernel(GemmParams 
     const int n0 = tile_n * BN_OUT;
     // SwiGLU: tile rows [64 c, 64 c + 64) are the gate rows, then the up rows, of 32 output columns
     if (SWIGLU) lw_row = (uint32_t)((wave_u & 1) * N + n0 + (wave_u >> 1) * 32);
-    else lw_row = (uint32_t)(n0 + wave_u * 32);
+    else lw_row = (uint32_t)(n0 + wave_u * (W_LD * 8));
   };
   auto issue_w = [&]() {
-    unsigned char* sd = smem + B_OFF + lw_stage * B_BYTES + wave_u * 4096;
+    unsigned char* sd = smem + B_OFF + lw_stage * B_BYTES + wave_u * (W_LD * 1024);
     const uint32_t so = lw_row * (uint32_t)(K * 2) + (uint32_t)lw_kt * (BK * 2);
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_wc, (lds_ptr)(sd + i * 1024), 16, ld_voff[i & 1],
+    for (int i = 0; i < W_LD; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_wc, (lds_ptr)(sd + i * 1024), 16, W_LD & 1 ? ld_voff[(wave_u + i) & 1] : ld_voff[i & 1],
                                                so + (uint32_t)(i * 8) * (uint32_t)(K * 2), 0, 0);
     if (++lw_stage == B_STAGES) lw_stage = 0;
     if (++lw_kt == KT) {
@@ -222,7 +227,8 @@ __global__ void __launch_bounds__(NT) gemm_bf16_nt_persistent_kernel(GemmParams 
   }
 
   // s_waitcnt immediates: vmcnt in bits 3:0 (and 15:14), expcnt in 6:4 (7 = no wait), lgkmcnt in 11:8 (15 = no wait)
-  constexpr int WAIT_LGKM0 = 0xC07F, WAIT_VM0 = 0x0F70, WAIT_VM4 = 0x0F74, WAIT_AW_LGKM0 = 0x0070 | (A_LD + 4);
+  constexpr int WAIT_LGKM0 = 0xC07F, WAIT_VM0 = 0x0F70, WAIT_VM4 = 0x0F74, WAIT_W = 0x0F70 | W_LD,
+                WAIT_AW_LGKM0 = 0x0070 | (A_LD + W_LD);
 
   // ---- epilogue of the tile whose accumulators are complete.
   // Vector memory operations of a wave complete in order, so a wait for a load also waits for every store issued
@@ -240,7 +246,7 @@ __global__ void __launch_bounds__(NT) gemm_bf16_nt_persistent_kernel(GemmParams 
     const int rrow = lane_t >> 3, rch = lane_t & 7;  // read-back mapping: row rrow + 8*it, 16-byte chunk rch
     int tile_m, tile_n;
     decode(r_done, tile_m, tile_n);
-    const int64_t m_base = (int64_t)tile_m * BM + grp * (BM / WM);
+    const int64_t m_base = (int64_t)tile_m * BM + wm_u * (BM / WM);
     // Row addressing: the first row of this wave group in C / the residual is a wave-uniform 64-bit base, a lane adds
     // its row r (0..127, relative) times the row stride as a 24-bit multiply (strides < 2^23, checked at launch)
     // instead of a 64 x 64-bit multiply per access.  rows_left <= 0: a group entirely below the matrix.
@@ -250,14 +256,15 @@ __global__ void __launch_bounds__(NT) gemm_bf16_nt_persistent_kernel(GemmParams 
     const int n_wave = tile_n * BN_OUT + (wave_u % WN) * (SWIGLU ? 32 : BN / WN);  // first output column of this wave
     u32x2 bq_next[FN];  // loaded ahead of the last block's stores, used after them
     // The query part of a qkv projection is multiplied by q_scale here, in fp32, before its only rounding.  Whole
-    // 64-column wave blocks lie inside or outside the query columns (q_cols % 64 == 0, checked at launch): a
-    // wave-uniform branch that two thirds of the tiles of such a projection skip.
+    // 64-column wave blocks (column fragments, of 96-column ones) lie inside or outside the query columns (q_cols % 64 == 0, checked
+    // at launch): a wave-uniform branch that two thirds of the tiles of such a projection skip.
     if (PLAIN && ACT == AERIS_ACT_NONE && !OUT_F32 && n_wave < p.q_cols) {
       const float qs = p.q_scale;
 #pragma unroll
       for (int i = 0; i < FM; ++i)
 #pragma unroll
-        for (int j = 0; j < FN; ++j) acc[i][j] *= qs;
+        for (int j = 0; j < FN; ++j)
+          if (BN == 256 || n_wave + j * 16 < p.q_cols) acc[i][j] *= qs;
     }
     // Staging area of this wave, 32 rows of 128 B: the A stage that the loader fills next is idle during the
     // epilogue, and the 4 KB of it that this wave's own loads will fill are written by nobody else (tile height 128: an
@@ -342,12 +349,34 @@ __global__ void __launch_bounds__(NT) gemm_bf16_nt_persistent_kernel(GemmParams 
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     };
 
+    // The same for 96 columns: a block is one row fragment, rows of 192 B in a pitch of 208, which sixteen rows' writes of one
+    // chunk then spread over the banks like the swizzle does; read back as 3 chunks a lane, C in row segments of 192 B.
+    constexpr int PITCH = NJ * 32 + 16, CPR = NJ * 2;  // bytes, chunks of a staged row
+    auto stage_rows_bf16 = [&](int i) {
+      u32x2 w2[NJ];
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        float v[4];
+        fragment(i, j, v);
+        w2[j] = u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+      }
+#pragma unroll
+      for (int mm = 0; mm < NJ / 2; ++mm) {
+        const auto rx = __builtin_amdgcn_permlane16_swap(w2[2 * mm].x, w2[2 * mm + 1].x, false, false);
+        const auto ry = __builtin_amdgcn_permlane16_swap(w2[2 * mm].y, w2[2 * mm + 1].y, false, false);
+        *reinterpret_cast<u32x4*>(stg + l15 * PITCH + (4 * mm + 2 * (q & 1) + (q >> 1)) * 16) = u32x4{rx[0], ry[0], rx[1], ry[1]};
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+
     // Interior tiles (every row and column of the group's 128 x 64 block inside the matrix, one gate row) take paths
     // without any per-lane condition where that gains (residual forms: +5 % on K = 1536; plain GELU: +1 %; plain without
     // activation measured 2 % slower this way and stays on the general path): straight-line code lets the compiler wait
     // for exactly the loads a block needs.
     const bool inside = rows_left == BM / WM && n_wave + BN_OUT / WN <= N && !gate_per_lane;
-    const bool interior = PLAIN && (ACT == AERIS_ACT_GELU || ACT == GEMM_ACT_GELU_ERF) && !OUT_F32 && inside;
+    const bool interior = BN == 256 && PLAIN && (ACT == AERIS_ACT_GELU || ACT == GEMM_ACT_GELU_ERF) && !OUT_F32 && inside;
     // Interior plain SwiGLU tiles skip the staging (in the read-back of the general path half of the lanes idle on
     // its 64-byte rows; +2 %).  For the other forms this was slower (qkv -4 %, proj -5 %: 64-byte row pieces).
     const bool interior_direct = SWIGLU && PLAIN && !OUT_F32 && inside;
@@ -358,7 +387,118 @@ __global__ void __launch_bounds__(NT) gemm_bf16_nt_persistent_kernel(GemmParams 
     // tile's bias) and leave those to drain under the first slots of the next tile, whose first counted wait (end of
     // M1(0)) covers them.  The wait has to stand inside the path: behind the join the compiler no longer knows that the
     // operations left outstanding are stores, and puts a wait for all of them into the k-loop.
-    if (interior_direct) {
+    if constexpr (BN == 192 && PLAIN && !OUT_F32) {
+      constexpr int ITS = CPR / 4;  // 16 rows x CPR chunks / 64 lanes
+      int row_of[ITS];
+      unsigned char* c_lane[ITS];
+      bool ok[ITS], full[ITS];
+#pragma unroll
+      for (int it = 0; it < ITS; ++it) {
+        const int id = it * 64 + lane_t;
+        row_of[it] = id / CPR;
+        const int n = n_wave + (id - row_of[it] * CPR) * 8;
+        ok[it] = n < N;
+        full[it] = n + 8 <= N;  // N % 4 == 0: a chunk is whole or exactly its first half is inside
+        c_lane[it] = reinterpret_cast<unsigned char*>(p.C) + (m_base * c_row_stride(p) + c_col_off(p, ok[it] ? n : 0)) * 2;
+      }
+#pragma unroll
+      for (int i = 0; i < FM; ++i) {
+        stage_rows_bf16(i);
+        u32x4 out[ITS];
+#pragma unroll
+        for (int it = 0; it < ITS; ++it) {
+          const int id = it * 64 + lane_t;
+          out[it] = *reinterpret_cast<const u32x4*>(stg + row_of[it] * PITCH + (id - row_of[it] * CPR) * 16);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (i + 1 == FM && r_done + 1 < n_my) load_bias(r_done + 1, bq_next, q);  // ahead of the stores below
+#pragma unroll
+        for (int it = 0; it < ITS; ++it) {
+          const int r = i * 16 + row_of[it];
+          if (ok[it] && r < rows_left) {
+            unsigned char* cp = c_lane[it] + (int64_t)__mul24(r, rs24) * 2;
+            if (full[it]) *reinterpret_cast<u32x4*>(cp) = out[it];
+            else *reinterpret_cast<u32x2*>(cp) = u32x2{out[it].x, out[it].y};
+          }
+        }
+      }
+      __builtin_amdgcn_s_waitcnt(WAIT_VM0);
+    } else if constexpr (BN == 192 && RES_BF16) {
+      // bf16 C and residual: units of 32 rows x 32 columns as in the f32 paths, staged as fp32; a lane has 8 columns of a row, four
+      // lanes the unit's 64 bytes of C.  Residual rows two units ahead, ahead of the stores.
+      constexpr int NU = FN / 2, UNITS = FM / 2 * NU;
+      const int urow = lane_t >> 2, uch = lane_t & 3;
+      auto unit_col = [&](int u) { return n_wave + (u % NU) * 32 + uch * 8; };
+      u32x4 rq[3][2];
+      auto load_res = [&](int u) {
+        const int n = unit_col(u), n_ld = n < N - 8 ? n : N - 8;  // 8 columns that exist; half a chunk: its 4 are the upper ones
+#pragma unroll
+        for (int it = 0; it < 2; ++it) {
+          int r = (u / NU) * 32 + urow + 16 * it;
+          if (r > rows_left - 1) r = rows_left - 1;
+          rq[u % 3][it] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint16_t*>(p.residual) + m_base * p.ldc + (int64_t)__mul24(r, ld24) + n_ld);
+        }
+      };
+      load_res(0);
+#pragma unroll
+      for (int u = 0; u < UNITS; ++u) {
+        const int i = u / NU, j = u % NU, n = unit_col(u);
+#pragma unroll
+        for (int ii = 0; ii < 2; ++ii)
+#pragma unroll
+          for (int jj = 0; jj < 2; ++jj) {
+            float v[4];
+            fragment(2 * i + ii, 2 * j + jj, v);
+            *reinterpret_cast<f32x4*>(stg + swz_off(ii * 16 + l15, jj * 4 + q)) = f32x4{v[0], v[1], v[2], v[3]};
+          }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        if (u == 0 && UNITS > 1) load_res(1);  // once the first unit's accumulators are staged and their registers free
+        f32x4 g0 = {1.f, 1.f, 1.f, 1.f}, g1 = g0;
+        const int n_g0 = n < N - 4 ? n : N - 4, n_g1 = n + 4 < N - 4 ? n + 4 : N - 4;
+        if (gate_tile) {
+          g0 = *reinterpret_cast<const f32x4*>(gate_tile + n_g0);
+          g1 = *reinterpret_cast<const f32x4*>(gate_tile + n_g1);
+        }
+        u32x4 out[2];
+#pragma unroll
+        for (int it = 0; it < 2; ++it) {
+          const int row = urow + 16 * it;
+          f32x4 o0 = *reinterpret_cast<const f32x4*>(stg + swz_off(row, 2 * uch));
+          f32x4 o1 = *reinterpret_cast<const f32x4*>(stg + swz_off(row, 2 * uch + 1));
+          if (gate_per_lane) {
+            const float* gr = gate_row_of(i * 32 + row);
+            g0 = *reinterpret_cast<const f32x4*>(gr + n_g0);
+            g1 = *reinterpret_cast<const f32x4*>(gr + n_g1);
+          }
+          u32x4 r4 = rq[u % 3][it];
+          if (n + 8 > N) { r4.x = r4.z; r4.y = r4.w; }
+          const f32x4 x0 = {bf16_lo(r4.x), bf16_hi(r4.x), bf16_lo(r4.y), bf16_hi(r4.y)}, x1 = {bf16_lo(r4.z), bf16_hi(r4.z), bf16_lo(r4.w), bf16_hi(r4.w)};
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            o0[e] = fmaf(o0[e], g0[e], x0[e]);
+            o1[e] = fmaf(o1[e], g1[e], x1[e]);
+          }
+          out[it] = u32x4{pack_bf16x2(o0[0], o0[1]), pack_bf16x2(o0[2], o0[3]), pack_bf16x2(o1[0], o1[1]), pack_bf16x2(o1[2], o1[3])};
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (u + 2 < UNITS) load_res(u + 2);  // ahead of the stores below
+        if (u + 1 == UNITS && r_done + 1 < n_my) load_bias(r_done + 1, bq_next, q);
+#pragma unroll
+        for (int it = 0; it < 2; ++it) {
+          const int r = i * 32 + urow + 16 * it;
+          if (n < N && r < rows_left) {
+            unsigned char* cp = reinterpret_cast<unsigned char*>(p.C) + (m_base * p.ldc + n + (int64_t)__mul24(r, ld24)) * 2;
+            if (n + 8 <= N) *reinterpret_cast<u32x4*>(cp) = out[it];
+            else *reinterpret_cast<u32x2*>(cp) = u32x2{out[it].x, out[it].y};
+          }
+        }
+      }
+      __builtin_amdgcn_s_waitcnt(WAIT_VM0);
+    } else if (interior_direct) {
       // No staging: after a swap between lane rows (v_permlane16_swap on the registers of column fragments 2m and
       // 2m + 1) lane (l15, q) owns 8 consecutive columns, 32 m + 16 (q & 1) + 8 (q >> 1) .., of row 16 i + l15: four
       // lanes cover 64 contiguous bytes of a row of C, a store instruction 16 rows.
@@ -687,7 +827,8 @@ __global__ void __launch_bounds__(NT) gemm_bf16_nt_persistent_kernel(GemmParams 
   };
 
   // ---- flat pipeline over (tile, k-tile), ping-pong between the two wave groups.
-  // Group 0 (wm = 0, one wave per SIMD) and group 1 (wm = 1, the other wave of each SIMD) run, per k-tile j, the
+  // (Counts for tiles of 256 x 256; 192 columns: 10 reads, 24 MFMAs, 3 loads of W.)
+  // Group 0 (waves 0-3, one per SIMD) and group 1 (waves 4-7, the other one of each SIMD) run, per k-tile j, the
   // slots  M0 | C0 | M1 | C1 : a memory slot reads the fragments of half a k-tile (12 ds_read_b128) and issues 4
   // loads, a compute slot issues the 32 MFMAs on those fragments.  Group 1 runs one slot behind group 0 and every
   // slot ends in a workgroup barrier: while one wave of a SIMD computes, the other one does its memory work.
@@ -748,7 +889,7 @@ __global__ void __launch_bounds__(NT) gemm_bf16_nt_persistent_kernel(GemmParams 
           for (int jn = 0; jn < FN; ++jn)
             acc[i][jn] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bfr[jn], af[i], acc[i][jn], 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
-        if (half == 1) __builtin_amdgcn_s_waitcnt(WAIT_VM4);
+        if (half == 1) __builtin_amdgcn_s_waitcnt(WAIT_W);
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -760,10 +901,10 @@ __global__ void __launch_bounds__(NT) gemm_bf16_nt_persistent_kernel(GemmParams 
 
 namespace {
 
-template <int BM, int ACT, bool OUT_F32, bool PLAIN, bool RES_BF16 = false, bool RES_F32 = false>
+template <int BM, int ACT, bool OUT_F32, bool PLAIN, bool RES_BF16 = false, bool RES_F32 = false, int BN = 256>
 hipError_t configure_one() {
-  return hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_bf16_nt_persistent_kernel<BM, ACT, OUT_F32, PLAIN, RES_BF16, RES_F32>),
-                             hipFuncAttributeMaxDynamicSharedMemorySize, smem_bytes(BM));
+  return hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_bf16_nt_persistent_kernel<BM, BN, ACT, OUT_F32, PLAIN, RES_BF16, RES_F32>),
+                             hipFuncAttributeMaxDynamicSharedMemorySize, smem_bytes(BM, BN));
 }
 template <int BM, int ACT>
 hipError_t configure_act() {
@@ -781,13 +922,18 @@ hipError_t configure_all() {
   if (e == hipSuccess) e = configure_act<BM, AERIS_ACT_SWIGLU>();
   if (e == hipSuccess) e = configure_one<BM, AERIS_ACT_NONE, true, false, false, true>();
   if (e == hipSuccess) e = configure_one<BM, GEMM_ACT_GELU_ERF, false, true>();
+  if (e == hipSuccess) e = configure_one<BM, AERIS_ACT_NONE, false, true, false, false, 192>();
+  if (e == hipSuccess) e = configure_one<BM, AERIS_ACT_GELU, false, true, false, false, 192>();
+  if (e == hipSuccess) e = configure_one<BM, GEMM_ACT_GELU_ERF, false, true, false, false, 192>();
+  if (e == hipSuccess) e = configure_one<BM, AERIS_ACT_NONE, false, false, true, false, 192>();
+  if (e == hipSuccess) e = configure_one<BM, AERIS_ACT_NONE, true, false, false, true, 192>();
   return e;
 }
 
 template <int BM, int ACT>
 void launch_act(const GemmParams& p, dim3 grid, hipStream_t stream) {
   const bool f32 = p.c_dtype == AERIS_F32, plain = !p.gate && p.res_dtype < 0;
-#define GO(...) hipLaunchKernelGGL((gemm_bf16_nt_persistent_kernel<BM, ACT, __VA_ARGS__>), grid, dim3(NT), smem_bytes(BM), stream, p)
+#define GO(...) hipLaunchKernelGGL((gemm_bf16_nt_persistent_kernel<BM, 256, ACT, __VA_ARGS__>), grid, dim3(NT), smem_bytes(BM, 256), stream, p)
   if constexpr (ACT == AERIS_ACT_NONE) {
     if (f32 && p.res_dtype == AERIS_F32 && !p.split) {
       GO(true, false, false, true);
@@ -803,8 +949,19 @@ void launch_act(const GemmParams& p, dim3 grid, hipStream_t stream) {
 }
 
 template <int BM>
-hipError_t launch_bm(GemmParams p, hipStream_t stream) {
-  const int bn_out = p.act == AERIS_ACT_SWIGLU ? BN / 2 : BN;
+void launch_192(const GemmParams& p, dim3 grid, hipStream_t stream) {
+#define GO(...) hipLaunchKernelGGL((gemm_bf16_nt_persistent_kernel<BM, 192, __VA_ARGS__>), grid, dim3(NT), smem_bytes(BM, 192), stream, p)
+  if (p.c_dtype == AERIS_F32) GO(AERIS_ACT_NONE, true, false, false, true);
+  else if (p.res_dtype >= 0) GO(AERIS_ACT_NONE, false, false, true);
+  else if (p.act == AERIS_ACT_GELU) GO(AERIS_ACT_GELU, false, true);
+  else if (p.act == GEMM_ACT_GELU_ERF) GO(GEMM_ACT_GELU_ERF, false, true);
+  else GO(AERIS_ACT_NONE, false, true);
+#undef GO
+}
+
+template <int BM>
+hipError_t launch_bm(GemmParams p, int bn, hipStream_t stream) {
+  const int bn_out = p.act == AERIS_ACT_SWIGLU ? bn / 2 : bn;
   p.tiles_m = (int)((p.M + BM - 1) / BM);
   p.tiles_n = (p.N + bn_out - 1) / bn_out;
   p.total_tiles = p.tiles_m * p.tiles_n;
@@ -822,9 +979,10 @@ hipError_t launch_bm(GemmParams p, hipStream_t stream) {
     p.rpb_magic = (uint32_t)((((uint64_t)1 << p.rpb_shift) + (uint64_t)p.rows_per_batch - 1) / (uint64_t)p.rows_per_batch);
   }
   const dim3 grid(8 * p.bpx);
-  if (p.act == AERIS_ACT_SWIGLU) launch_act<BM, AERIS_ACT_SWIGLU>(p, grid, stream);
+  if (bn == 192) launch_192<BM>(p, grid, stream);
+  else if (p.act == AERIS_ACT_SWIGLU) launch_act<BM, AERIS_ACT_SWIGLU>(p, grid, stream);
   else if (p.act == GEMM_ACT_GELU_ERF)
-    hipLaunchKernelGGL((gemm_bf16_nt_persistent_kernel<BM, GEMM_ACT_GELU_ERF, false, true>), grid, dim3(NT), smem_bytes(BM), stream, p);
+    hipLaunchKernelGGL((gemm_bf16_nt_persistent_kernel<BM, 256, GEMM_ACT_GELU_ERF, false, true>), grid, dim3(NT), smem_bytes(BM, 256), stream, p);
   else if (p.act == AERIS_ACT_GELU) launch_act<BM, AERIS_ACT_GELU>(p, grid, stream);
   else launch_act<BM, AERIS_ACT_NONE>(p, grid, stream);
   return hipGetLastError();
@@ -839,8 +997,15 @@ hipError_t gemm_persistent_configure() {
 }
 
 // p.act must be NONE, GELU, GELU_ERF (bf16 C without gate and residual) or SWIGLU; N % 4 == 0 and ldc % 4 == 0; bias / gate rows 8- / 16-byte aligned
-hipError_t gemm_persistent_launch(const GemmParams& p, int tile_height, hipStream_t stream) {
-  return tile_height == 128 ? launch_bm<128>(p, stream) : launch_bm<256>(p, stream);
+hipError_t gemm_persistent_launch(const GemmParams& p, int tile_height, int tile_width, hipStream_t stream) {
+  return tile_height == 128 ? launch_bm<128>(p, tile_width, stream) : launch_bm<256>(p, tile_width, stream);
+}
+
+bool gemm_persistent_takes_192(const GemmParams& p) {
+  if (p.act == AERIS_ACT_GELU || p.act == GEMM_ACT_GELU_ERF) return p.c_dtype == AERIS_BF16 && !p.gate && p.res_dtype < 0;
+  if (p.act != AERIS_ACT_NONE) return false;
+  if (p.c_dtype == AERIS_F32) return p.res_dtype == AERIS_F32 && !p.split;
+  return p.res_dtype == AERIS_BF16 || (p.res_dtype < 0 && !p.gate);
 }
 
 }  // namespace aeris

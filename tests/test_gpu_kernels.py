@@ -159,6 +159,35 @@ def test_gemm_tile_edges(pkg, cuda, case):
     assert bool((pad[0] == 7.0).all()) and bool((pad[-1] == 7.0).all())
 
 
+@pytest.mark.parametrize("case", [
+    (7990, 1156, 320, None, True, 2, torch.float32, torch.float32),     # 4 columns in the last tile, a batch boundary inside a tile
+    (16000, 580, 64, None, False, 0, torch.float32, torch.float32),     # one k-tile
+    (12480, 384, 384, None, True, 2, torch.float32, torch.float32),     # 128 rows, two tiles exactly
+    (6001, 1540, 1088, None, True, 0, torch.bfloat16, torch.bfloat16),  # half a 16-byte chunk, one row in the last tile's last block
+    (7002, 1540, 1088, None, False, 3, torch.bfloat16, torch.bfloat16),
+    (8551, 1280, 320, "gelu", True, 0, None, torch.bfloat16),           # by erf
+    (6100, 1540, 256, "gelu", False, 0, None, torch.bfloat16),
+    (6290, 3328, 832, "gelu", True, 0, None, torch.bfloat16),           # by polynomial
+    (8152, 4224, 1408, None, True, 0, None, torch.bfloat16),
+], ids=lambda c: f"M{c[0]}_N{c[1]}_K{c[2]}_{c[3]}_g{c[5]}")
+def test_gemm_tiles_of_192_columns(pkg, cuda, case):
+    """Shapes that need no more rounds of 192-column tiles than of 256, at the edges of those tiles; errors as for the others."""
+    test_gemm_tile_edges(pkg, cuda, case)
+
+
+def test_gemm_heads_query_columns_end_inside_a_wave_of_96(pkg, cuda):
+    """22 heads of 64: the query columns end in the fifteenth block of 96 columns.  Planes without a scale bit for bit, query planes
+    to the rounding of the scaled value (half a bf16 ulp) against the unrounded product."""
+    M, K, heads, hd = 8152, 1408, 22, 64
+    g = torch.Generator().manual_seed(3)
+    a, w = bf(torch.randn(M, K, generator=g)).to(cuda), bf(torch.randn(3 * heads * hd, K, generator=g) / math.sqrt(K)).to(cuda)
+    plain = pkg.ops.gemm_heads(a, w, None, hd)
+    scaled = pkg.ops.gemm_heads(a, w, None, hd, q_scale=0.18, q_planes=heads)
+    assert torch.equal(scaled[heads:], plain[heads:])
+    ref = ((a.float() @ w.float().T) * 0.18).view(M, 3 * heads, hd).permute(1, 0, 2)[:heads]
+    assert bool(((scaled[:heads].float() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-5).all())
+
+
 @pytest.mark.parametrize("M,N,K", [(9000, 4096, 512), (5500, 3072, 768), (3000, 6144, 1536), (13500, 1280, 320), (8200, 1024, 512)])
 def test_gemm_gelu_is_one_function_of_the_value(pkg, cuda, M, N, K):
     """Equal rows give equal results wherever they stand: also where the rows of the last, partly filled round of tiles are left to

@@ -404,6 +404,7 @@ hipError_t configure_tile() {
 // touch every instantiation so that attribute set-up never happens inside a captured region
 hipError_t gemm_configure_all() {
   hipError_t e = configure_tile<64, 64, 3, true>();
+  if (e == hipSuccess) e = configure_tile<64, 64, 2, true>();
   if (e == hipSuccess) e = configure_tile<128, 128, 2, true>();
   if (e == hipSuccess) e = configure_tile<128, 128, 2, false>();
   if (e == hipSuccess) e = gemm_persistent_configure();
@@ -483,13 +484,23 @@ Kind best_kind(const Shape& s, float* us) {
   return best;
 }
 
+Shape shape_of(const GemmParams& p, int act) { return {p.M, p.N, p.K / BK, act, p.c_dtype == AERIS_F32, p.residual != nullptr, gemm_persistent_takes_192(p)}; }
+
 hipError_t launch_kind(Kind kind, const GemmParams& p, hipStream_t stream) {
-  if (kind == TILE64) return launch_tile_act<64, 64, 3, true>(p, stream);
+  if (kind == TILE64) {
+    // Three stages are 48 KB: three workgroups per CU.  Of four per CU the last would have the chip nearly to itself: with two stages
+    // (32 KB) all four run at once.  Three stages -> two, us, plain bf16: 3000 x 1152 x 384 (846 tiles) 10.3 -> 9.0, 6144 x 576 x 192
+    // (864) 8.7 -> 7.1, 4096 x 960 x 320 (960) 9.7 -> 8.5, 8192 x 512 x 2048 (1024) 28.4 -> 27.0; SwiGLU 2048 x 1024 x 256 (1024) 7.2 -> 6.4.
+    // With up to three per CU the third stage is worth 0 to 20 % (4096 x 512 x 2048, two per CU, 15.7 against 18.8), from five on there
+    // are further rounds either way (4096 x 1152 x 384, 1152 tiles, 11.3 against 11.9).
+    const int64_t tiles = tiles_of(shape_of(p, p.act), 64, 64);
+    if (tiles > 3 * 256 && tiles <= 4 * 256) return launch_tile_act<64, 64, 2, true>(p, stream);
+    return launch_tile_act<64, 64, 3, true>(p, stream);
+  }
   return gemm_persistent_launch(p, kind == PERSISTENT256 || kind == PERSISTENT256_192 ? 256 : 128,
                                 kind == PERSISTENT128_192 || kind == PERSISTENT256_192 ? 192 : 256, stream);
 }
 
-Shape shape_of(const GemmParams& p, int act) { return {p.M, p.N, p.K / BK, act, p.c_dtype == AERIS_F32, p.residual != nullptr, gemm_persistent_takes_192(p)}; }
 
 // vector epilogue: 8 / 16-byte accesses to C and the residual (4-element alignment of every row), to bias and gate rows
 bool vector_epilogue(const GemmParams& p) {

@@ -175,6 +175,18 @@ def test_gemm_tiles_of_192_columns(pkg, cuda, case):
     test_gemm_tile_edges(pkg, cuda, case)
 
 
+@pytest.mark.parametrize("case", [
+    (4100, 956, 320, None, True, 0, None, torch.bfloat16),             # 975 tiles of 64 x 64, ragged both ways
+    (6144, 576, 64, None, False, 3, torch.bfloat16, torch.bfloat16),   # 864, one k-tile
+    (2030, 1000, 256, "swiglu", False, 0, None, torch.bfloat16),       # 1024
+    (3137, 1024, 128, "gelu", True, 0, None, torch.bfloat16),          # 800, by erf
+    (4100, 956, 320, None, True, 2, None, torch.float32),              # 975, a batch boundary inside a tile
+], ids=lambda c: f"M{c[0]}_N{c[1]}_K{c[2]}_{c[3]}_g{c[5]}")
+def test_gemm_small_tiles_four_to_a_cu(pkg, cuda, case):
+    """Between three and four small tiles per CU: two k-tiles in LDS instead of three; errors as for the others."""
+    test_gemm_tile_edges(pkg, cuda, case)
+
+
 def test_gemm_heads_query_columns_end_inside_a_wave_of_96(pkg, cuda):
     """22 heads of 64: the query columns end in the fifteenth block of 96 columns.  Planes without a scale bit for bit, query planes
     to the rounding of the scaled value (half a bf16 ulp) against the unrounded product."""

@@ -3,10 +3,11 @@
 // For the problems that do not give the 256 x 256 persistent kernel (gemm_persistent.hip) enough tiles to fill the chip.
 // What bounds those is latency: a handful of k-tiles per workgroup, each a round trip to L2, and the first loads and the
 // epilogue on top of them.  Hence 64 x 64 tiles (four waves of 32 x 32, 48 KB of LDS: three workgroups per CU, free of each
-// other, so one's first loads and epilogue fall under another's main loop), three k-tiles in flight, every epilogue
+// other, so one's first loads and epilogue fall under another's main loop; 32 x 64 where there are not enough of those, and two
+// k-tiles where that lets a fourth run: launch_kind), three k-tiles in flight, every epilogue
 // operand requested ahead of the main loop, and little code (fetched cold: the kernel before this one, 128 x 128
 // register-staged with every epilogue option in one body, took 18-24 us for what takes 4-5 us here).  Measured before -> after:
-// 2048 x 128 x 128 17.9 -> 3.8 us, 2048 x 128 x 512 22.1 -> 5.0 us, 2048 x 256 x 1024 32.1 -> 7.1 us, 8192 x 256 x 256 25.0 ->
+// 2048 x 128 x 128 17.9 -> 3.4 us, 2048 x 128 x 512 22.1 -> 4.2 us, 2048 x 256 x 1024 32.1 -> 5.8 us, 8192 x 256 x 256 25.0 ->
 // 6.8 us.  128 x 128 tiles of the same kernel take what neither this size nor the persistent kernel can (odd N, unaligned
 // rows, W of 2 GiB and more, SiLU).
 //   - global loads go straight into LDS (buffer_load ... lds, 16 bytes per lane); a load instruction of a wave fetches
@@ -51,6 +52,7 @@ __device__ __forceinline__ void wait_barrier() {
 }  // namespace
 
 // VEC: C and the residual are accessed 4 / 8 columns at a time (N % 4 == 0, rows 4-element aligned); else one by one
+// BM 32, 64 or 128: of 32 rows a wave computes 16 x 32 of the tile and loads one block of A
 template <int BM, int BN, int STAGES, int ACT, bool OUT_F32, bool VEC>
 __global__ void __launch_bounds__(NT, 2) gemm_bf16_nt_tile_kernel(GemmParams p) {
   constexpr bool SWIGLU = ACT == AERIS_ACT_SWIGLU;
@@ -98,13 +100,16 @@ __global__ void __launch_bounds__(NT, 2) gemm_bf16_nt_tile_kernel(GemmParams p) 
   // the end exactly for the rows past the end.)
   constexpr int LD_MAX = A_LD > B_LD ? A_LD : B_LD;
   uint32_t ld_voff[LD_MAX];  // lane part of the source offset, per 8-row block
+  uint32_t a_voff0;          // of A's first block: tiles of 32 rows have one a wave, odd in the odd waves
   {
     const int dr = lane >> 4, pos = lane & 15;
+    auto voff = [&](int i, int odd) {
+      const int logical = pos ^ (odd * 4 + dr);
+      return (uint32_t)((i * 8 + dr * 2 + (logical >> 3)) * K * 2 + (logical & 7) * 16);
+    };
 #pragma unroll
-    for (int i = 0; i < LD_MAX; ++i) {
-      const int logical = pos ^ ((i & 1) * 4 + dr);
-      ld_voff[i] = (uint32_t)((i * 8 + dr * 2 + (logical >> 3)) * K * 2 + (logical & 7) * 16);
-    }
+    for (int i = 0; i < LD_MAX; ++i) ld_voff[i] = voff(i, i & 1);
+    a_voff0 = A_LD == 1 ? voff(0, wave & 1) : ld_voff[0];
   }
   auto rows_rsrc = [&](const uint16_t* base, int64_t row, int64_t limit, int count) {
     int64_t have = limit - row;
@@ -122,7 +127,7 @@ __global__ void __launch_bounds__(NT, 2) gemm_bf16_nt_tile_kernel(GemmParams p) 
     const uint32_t sa = lds0 + stage * STAGE + wave * (AR * 128), sw = lds0 + stage * STAGE + A_BYTES + wave * (BR * 128);
     const uint32_t k_off = (uint32_t)kt * (BK * 2);
 #pragma unroll
-    for (int i = 0; i < A_LD; ++i) lds_dma_load16(rs_a, sa + i * 1024, ld_voff[i], k_off);
+    for (int i = 0; i < A_LD; ++i) lds_dma_load16(rs_a, sa + i * 1024, i == 0 ? a_voff0 : ld_voff[i], k_off);
 #pragma unroll
     for (int i = 0; i < B_LD; ++i) lds_dma_load16(rs_w, sw + i * 1024, ld_voff[i], k_off);
   };
@@ -370,7 +375,7 @@ hipError_t launch_tile_act(const GemmParams& p, hipStream_t stream) {
     case AERIS_ACT_GELU:
       if (p.c_dtype == AERIS_F32) return launch_tile<BM, BN, STAGES, AERIS_ACT_GELU, true, VEC>(p, stream);
       // the polynomial: only as the last rows of a problem whose other rows take it, which are given to 64 x 64 tiles
-      return launch_tile<BM, BN, STAGES, BM == 64 ? AERIS_ACT_GELU : GEMM_ACT_GELU_ERF, false, VEC>(p, stream);
+      return launch_tile<BM, BN, STAGES, BM <= 64 ? AERIS_ACT_GELU : GEMM_ACT_GELU_ERF, false, VEC>(p, stream);
     case GEMM_ACT_GELU_ERF: return launch_tile<BM, BN, STAGES, GEMM_ACT_GELU_ERF, false, VEC>(p, stream);
     case AERIS_ACT_SWIGLU: GO(AERIS_ACT_SWIGLU);
     case AERIS_ACT_SILU: GO(AERIS_ACT_SILU);
@@ -393,7 +398,7 @@ template <int BM, int BN, int STAGES, bool VEC>
 hipError_t configure_tile() {
   hipError_t e = configure_tile_act<BM, BN, STAGES, VEC, AERIS_ACT_NONE>();
   if (e == hipSuccess) e = configure_tile_kernel<BM, BN, STAGES, VEC, AERIS_ACT_GELU, true>();
-  if (e == hipSuccess) e = configure_tile_kernel<BM, BN, STAGES, VEC, BM == 64 ? AERIS_ACT_GELU : GEMM_ACT_GELU_ERF, false>();
+  if (e == hipSuccess) e = configure_tile_kernel<BM, BN, STAGES, VEC, BM <= 64 ? AERIS_ACT_GELU : GEMM_ACT_GELU_ERF, false>();
   if (e == hipSuccess) e = configure_tile_kernel<BM, BN, STAGES, VEC, GEMM_ACT_GELU_ERF, false>();
   if (e == hipSuccess) e = configure_tile_act<BM, BN, STAGES, VEC, AERIS_ACT_SWIGLU>();
   if (e == hipSuccess) e = configure_tile_act<BM, BN, STAGES, VEC, AERIS_ACT_SILU>();
@@ -405,6 +410,7 @@ hipError_t configure_tile() {
 hipError_t gemm_configure_all() {
   hipError_t e = configure_tile<64, 64, 3, true>();
   if (e == hipSuccess) e = configure_tile<64, 64, 2, true>();
+  if (e == hipSuccess) e = configure_tile<32, 64, 3, true>();
   if (e == hipSuccess) e = configure_tile<128, 128, 2, true>();
   if (e == hipSuccess) e = configure_tile<128, 128, 2, false>();
   if (e == hipSuccess) e = gemm_persistent_configure();
@@ -494,6 +500,14 @@ hipError_t launch_kind(Kind kind, const GemmParams& p, hipStream_t stream) {
     // With up to three per CU the third stage is worth 0 to 20 % (4096 x 512 x 2048, two per CU, 15.7 against 18.8), from five on there
     // are further rounds either way (4096 x 1152 x 384, 1152 tiles, 11.3 against 11.9).
     const int64_t tiles = tiles_of(shape_of(p, p.act), 64, 64);
+    // Up to one tile per CU, the rate at which a CU brings in its k-tiles (16 KB each, about 37 bytes a clock) bounds the call: tiles of
+    // half the rows move 3 / 4 of the bytes per workgroup and twice as many of them share the CUs' loads.  64 -> 32 rows, us:
+    // 2048 x 256 x 256 (128 tiles of 64) 4.6 -> 3.8, x 1024 7.0 -> 5.8, 2048 x 384 x 1536 (192) 8.9 -> 8.4, 2500 x 384 x 1536 (240)
+    // 10.0 -> 8.9, 4096 x 256 x 256 (256) 4.9 -> 4.5.  Beyond, where some CU has two tiles of 64 anyway, that holds while first loads and
+    // epilogue weigh more than the loop: K = 512 and less, 6144 x 192 x 192 (288) 5.7 -> 4.9, 2500 x 512 x 512 (320) 6.8 -> 6.5,
+    // 4096 x 384 x 384 (384) 6.4 -> 6.2, but 2048 x 768 x 768 (384) 8.0 -> 8.2, 5000 x 320 x 320 (395) 6.3 -> 6.4; SwiGLU, whose tiles
+    // of 32 rows have half the result of the others, 2048 x 384 x 192 (384) 4.10 -> 4.14.
+    if (tiles <= 256 || (tiles <= 384 && p.K <= 512 && p.act != AERIS_ACT_SWIGLU)) return launch_tile_act<32, 64, 3, true>(p, stream);
     if (tiles > 3 * 256 && tiles <= 4 * 256) return launch_tile_act<64, 64, 2, true>(p, stream);
     return launch_tile_act<64, 64, 3, true>(p, stream);
   }
@@ -573,7 +587,7 @@ hipError_t gemm_launch(const void* A, const void* W, void* C, const void* bias, 
       persistent_ok = persistent_ok && !gate && !residual;
   }
   if (!persistent_ok)
-    return tiles_of(s, 128, 128) < 128 ? launch_tile_act<64, 64, 3, true>(p, stream) : launch_tile_act<128, 128, 2, true>(p, stream);
+    return tiles_of(s, 128, 128) < 128 ? launch_kind(TILE64, p, stream) : launch_tile_act<128, 128, 2, true>(p, stream);
   float one = 0.f;
   const Kind kind = best_kind(s, &one);
   // Whole rounds of 256-row tiles first, the rows of the last, partly filled round by smaller tiles in a launch of its own:

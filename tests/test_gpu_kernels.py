@@ -187,6 +187,21 @@ def test_gemm_small_tiles_four_to_a_cu(pkg, cuda, case):
     test_gemm_tile_edges(pkg, cuda, case)
 
 
+@pytest.mark.parametrize("case", [
+    (1, 4, 64, None, True, 0, None, torch.float32),                     # one row, four columns, one k-tile
+    (33, 68, 128, "swiglu", True, 0, None, torch.bfloat16),             # second row tile of one row
+    (2047, 256, 1024, None, True, 0, torch.float32, torch.float32),     # 128 tiles of 64, ragged rows
+    (2500, 196, 192, "gelu", True, 0, None, torch.bfloat16),            # 160, by erf or by the polynomial
+    (2048, 512, 576, None, True, 0, None, torch.bfloat16),              # 256
+    (2040, 572, 512, None, True, 3, torch.bfloat16, torch.bfloat16),    # 288, a batch boundary inside a tile
+    (6130, 252, 256, "silu", False, 0, None, torch.bfloat16),           # 384
+    (2048, 1152, 192, "gelu", True, 0, None, torch.bfloat16),           # 576: of 64 rows
+], ids=lambda c: f"M{c[0]}_N{c[1]}_K{c[2]}_{c[3]}_g{c[5]}")
+def test_gemm_tiles_of_32_rows(pkg, cuda, case):
+    """Up to one small tile per CU, and half as many again at K <= 512: tiles of 32 rows; errors as for the others."""
+    test_gemm_tile_edges(pkg, cuda, case)
+
+
 def test_gemm_heads_query_columns_end_inside_a_wave_of_96(pkg, cuda):
     """22 heads of 64: the query columns end in the fifteenth block of 96 columns.  Planes without a scale bit for bit, query planes
     to the rounding of the scaled value (half a bf16 ulp) against the unrounded product."""

@@ -4,8 +4,8 @@
 // One workgroup = a block of queries of one (window, head), 32 per wave; the keys of the window are streamed through LDS in
 // chunks of 64 with an online softmax.  How many waves and chunk buffers a workgroup has follows the window (the rule
 // stands at the launch):
-//   8 waves, 4 buffers   windows of more than 2048 tokens with head_dim 128, and few windows (head_dim 64: through registers): one
-//                        workgroup per CU, a barrier per two chunks
+//   8 waves, 4 buffers   windows of more than 2048 tokens with head_dim 128, and few windows: one workgroup per CU, a barrier per
+//                        two chunks
 //   4 waves, 2 buffers   the others: two workgroups per CU (head_dim 64: three), so that one's start - token table, Q, the first
 //                        chunk - and its output stores run beside another's sweep, and windows whose size is no multiple of
 //                        256 leave fewer waves without queries
@@ -21,8 +21,14 @@
 //   V chunk [64][HD]   global -> registers (4 keys x 8 d per thread) -> 4x8 register transpose -> LDS as
 //                      V^T [HD][64], key groups permuted so that a PV fragment is one ds_read_b128
 //   Q                  global -> registers (MFMA B operand), once
-//   S^T = K Q^T        v_mfma_f32_32x32x16_bf16; lane = one query, registers = keys
+//   S^T = K Q^T        v_mfma_f32_16x16x32_bf16; lane = one query, registers = keys
 //   O^T += V^T P^T     P^T straight from the S^T accumulator registers
+// What bounds it is the stream of MFMAs at the clock that the power budget leaves: with 32x32x16 MFMAs the loop without any exp2
+// and row sum was 4 % faster than with them, and two query groups a wave, which halve the LDS reads, 6 % slower.  The 16x16x32 shape
+// does the same FLOP per cycle and LDS bytes per FLOP at a higher clock.  32x32x16 -> 16x16x32, us: 360 x 720 tokens in 60 x 60 windows
+// with 8 x 128 3800 -> 3510, 120 x 120 with 12 x 128 333 -> 319; 20 x 20 windows, 3 x 128 320 -> 301; 8 x 16 182 -> 172; head_dim 64, 60 x 60
+// with 8 heads 2060 -> 1983, 6 x 6 with 6 202 -> 181.  (PV with the two query blocks of a V^T fragment back to back: 1.3 % of that; K Q^T
+// over four key blocks in turn, two or two pairs: 0.5 %; reading K fragments 3 or 4 ahead, raised wave priority: nothing.)
 // The query blocks of one (window, head) are placed on the same XCD (blockIdx % 8), so its K / V rows are fetched
 // into that XCD's L2 once and re-read from there by the other query blocks.
 #include "common.h"
@@ -84,12 +90,12 @@ struct StreamCfg {
 // transposing VALU work) and V stays row-major; the V^T fragments of P V then come from ds_read_b64_tr_b16, the LDS read that
 // transposes on the way out (within 16 lanes, source lane 4e + a reads 4 consecutive elements and result lane 4a + b
 // receives element b of source lanes a, 4 + a, 8 + a, 12 + a).  The 16-byte chunks of a row are XOR-swizzled.  head_dim 128,
-// rows of 256 B: K by row & 15 (conflict-free ds_read_b128 fragments), V by 4 (row & 3) (the 4 keys x 4 column groups that the
+// rows of 256 B: K by row & 15 (conflict-free ds_read_b128 fragments), V by 2 (row & 7) (the 8 keys x 2 chunks that the
 // two 16-lane halves of a transposing read's 32-lane pass gather - 16 pieces of 16 bytes - land on the 16 distinct slots of a
-// 256-byte bank period; with 2 (row & 3) the two halves shared eight).  head_dim 64, rows of 128 B: K over double rows
-// (off128()), V by 2 (row & 3), as in the one-window kernels.  Needs every byte offset inside an image's k / v plane to fit 32
-// bits (span_bytes; checked by the launcher); the register form, eight waves, takes what does not.  (head_dim 64, eight waves
-// either way: 360 x 720 tokens in 60 x 60 windows with 8 heads 2168 -> 2076 us; with 4 waves and 2 buffers 1978.)
+// 256-byte bank period).  head_dim 64, rows of 128 B: K over double rows (off128()), V by 2 ((row >> 1) & 3), which with the two rows
+// of a bank period are 16 slots again.  Needs every byte offset inside an image's k / v plane to fit 32
+// bits (span_bytes; checked by the launcher); the register form, eight waves, takes what does not (head_dim 64, 360 x 720 tokens in
+// 60 x 60 windows with 8 heads: 2160 us against 1983).
 template <int HD, bool DMA, int NWAVE, int NBUF>
 __global__ void __launch_bounds__(64 * NWAVE) __attribute__((amdgpu_waves_per_eu(2)))
 window_attention_stream_kernel(StreamParams p) {
@@ -97,8 +103,10 @@ window_attention_stream_kernel(StreamParams p) {
   using Cfg = StreamCfg<HD, NBUF>;
   constexpr int QB = 32 * NWAVE;  // queries per workgroup
   constexpr int CH = HD / 8;   // 16-byte chunks per head row
-  constexpr int KS = HD / 16;  // k16 steps of QK^T
-  constexpr int DB = HD / 32;  // 32-row blocks of O^T
+  constexpr int QN = 2;        // blocks of 16 queries per wave
+  constexpr int KS = HD / 32;  // k32 steps of QK^T
+  constexpr int KB = KC / 16;  // blocks of 16 keys per chunk
+  constexpr int DB = HD / 16;  // 16-row blocks of O^T
   constexpr int NT = 64 * NWAVE;
   constexpr int KIT = KC * CH / NT;                     // 16-byte K pieces per thread and chunk (1 or 2)
   constexpr int V_ITEMS = (KC / 4) * CH;                // (4 keys x 8 d) V pieces per chunk: 128 or 256
@@ -110,7 +118,7 @@ window_attention_stream_kernel(StreamParams p) {
   int* const redo = tok + ((p.ws_y * p.ws_x + 3) & ~3);    // set by a wave whose sums left the range of the fast sweep
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int l31 = lane & 31, hi = lane >> 5;
+  const int l15 = lane & 15, q4 = lane >> 4;
 
   // all query blocks of one (window, head) on one XCD
   const int xcd = blockIdx.x & 7, s_idx = blockIdx.x >> 3;
@@ -140,16 +148,19 @@ window_attention_stream_kernel(StreamParams p) {
   if (tid == 0) *redo = 0;
   __syncthreads();
 
-  // ---- Q fragments (B operand): lane = query, 8 consecutive d per k16 step
-  int qpos = qb * QB + wave * 32 + l31;
-  const bool q_valid = qpos < L;
-  if (!q_valid) qpos = L - 1;
-  const int64_t q_row = img_base + tok[qpos];
-  bf16x8 qf[KS];
-  {
-    const uint16_t* qp = p.qkv + head * p.head_stride + (uint64_t)(uint32_t)q_row * ld_qkv + hi * 8;
+  // ---- Q fragments (B operand): lane = query, 8 consecutive d per k32 step
+  bool q_valid[QN];
+  int64_t q_row[QN];
+  bf16x8 qf[QN][KS];
 #pragma unroll
-    for (int s = 0; s < KS; ++s) qf[s] = *reinterpret_cast<const bf16x8*>(qp + s * 16);
+  for (int n = 0; n < QN; ++n) {
+    int qpos = qb * QB + wave * 32 + n * 16 + l15;
+    q_valid[n] = qpos < L;
+    if (!q_valid[n]) qpos = L - 1;
+    q_row[n] = img_base + tok[qpos];
+    const uint16_t* qp = p.qkv + head * p.head_stride + (uint64_t)(uint32_t)q_row[n] * ld_qkv + q4 * 8;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) qf[n][s] = *reinterpret_cast<const bf16x8*>(qp + s * 32);
   }
   {
     // q is multiplied by scale * log2(e) once, here (the reference scales q in bf16 too, model.py:290): the
@@ -157,13 +168,15 @@ window_attention_stream_kernel(StreamParams p) {
     // producer of q has applied the factor in fp32 before its only rounding, and this is a multiplication by one
     const float c = p.q_prescaled ? 1.0f : p.scale * LOG2E;
 #pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      const u32x4 w = __builtin_bit_cast(u32x4, qf[s]);
-      u32x4 r;
+    for (int n = 0; n < QN; ++n)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) r[e] = pack_bf16x2(bf16_lo(w[e]) * c, bf16_hi(w[e]) * c);
-      qf[s] = __builtin_bit_cast(bf16x8, r);
-    }
+      for (int s = 0; s < KS; ++s) {
+        const u32x4 w = __builtin_bit_cast(u32x4, qf[n][s]);
+        u32x4 r;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) r[e] = pack_bf16x2(bf16_lo(w[e]) * c, bf16_hi(w[e]) * c);
+        qf[n][s] = __builtin_bit_cast(bf16x8, r);
+      }
   }
 
   const uint16_t* kbase = p.qkv + img_base * (int64_t)ld_qkv + p.part_stride + head * p.head_stride;
@@ -205,12 +218,12 @@ window_attention_stream_kernel(StreamParams p) {
       const int idx = tid + it * NT, key = idx / CH, c = idx % CH;
       *reinterpret_cast<u32x4*>(sK + (HD == 64 ? off128(key, c) : off256(key, c))) = kreg[it];
     }
-    // V: 4 keys x 8 d register transpose -> V^T[d][key].  Inside every block of 16 keys the four key groups are
-    // stored in the order 0, 2, 1, 3: the 8 keys one lane needs for a k16 step of PV (4hi..4hi+3 and
-    // 8+4hi..8+4hi+3, the accumulator layout of S^T) are then one aligned 16-byte chunk.
+    // V: 4 keys x 8 d register transpose -> V^T[d][key].  Inside every block of 32 keys the eight key groups are
+    // stored in the order 0, 4, 1, 5, 2, 6, 3, 7: the 8 keys one lane needs for a k32 step of PV (4 q4 .. 4 q4 + 3 and
+    // 16 + 4 q4 .., the accumulator layout of S^T) are then one aligned 16-byte chunk.
     if (v_item) {
       const int kg = v_kg, c = v_c;
-      const int pos = (kg & ~3) | (((kg & 1) << 1) | ((kg >> 1) & 1));
+      const int pos = (kg & ~7) | ((kg & 3) << 1) | ((kg >> 2) & 1);
 #pragma unroll
       for (int w = 0; w < 4; ++w) {  // word w holds d = 8c + 2w (low half) and 8c + 2w + 1 (high half)
         u32x2 lo, hi2;
@@ -245,54 +258,51 @@ window_attention_stream_kernel(StreamParams p) {
         const int rsub = lane >> 4, pc = lane & 15, row = 4 * ii + rsub;
         const uint32_t rowoff = row_offset(row);
         ok = rowoff + (uint32_t)((pc ^ (row & 15)) << 4);
-        ov = rowoff + (uint32_t)((pc ^ (4 * rsub)) << 4);
+        ov = rowoff + (uint32_t)((pc ^ (2 * (row & 7))) << 4);
       } else {
         const int pair = 4 * ii + (lane >> 4), logical = (lane & 15) ^ (pair & 7);  // K: off128(), double rows
         const int row_v = 8 * ii + (lane >> 3);
         ok = row_offset(2 * pair + (logical >> 3)) + (uint32_t)((logical & 7) << 4);
-        ov = row_offset(row_v) + (uint32_t)(((lane & 7) ^ (2 * (row_v & 3))) << 4);
+        ov = row_offset(row_v) + (uint32_t)(((lane & 7) ^ (2 * ((row_v >> 1) & 3))) << 4);
       }
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_k, (lds_vptr)(smem + buf * Cfg::K_BYTES + ii * 1024), 16, ok, 0, 0, 0);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_v, (lds_vptr)(smem + Cfg::V_BASE + buf * Cfg::V_BYTES + ii * 1024), 16, ov, 0, 0, 0);
     }
   };
-  // per-lane part of the transposing V reads: block of 16 lanes jb = lane >> 4 (d half jb & 1, key half jb >> 1),
-  // source lane 4e + a inside it reads V[key0 + 4 (jb >> 1) + e][32 db + 16 (jb & 1) + 4a ..]
-  typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4_t;
-  typedef __attribute__((address_space(3))) bf16x4_t* lds_bf16x4_ptr;
+  // per-lane part of the transposing V reads: of the 16 lanes q4, lane 4e + a reads V[key0 + 4 q4 + e][16 db + 4a ..]
   uint32_t v_tr[DB];
   if (DMA) {
-    const int jb = lane >> 4, e = (lane >> 2) & 3, a = lane & 3;
+    const int e = (lane >> 2) & 3, a = lane & 3, row = 4 * q4 + e;
 #pragma unroll
     for (int db = 0; db < DB; ++db) {
-      const int chunk = (4 * db + 2 * (jb & 1) + (a >> 1)) ^ (HD == 128 ? 4 * e : 2 * e);
-      v_tr[db] = (uint32_t)(Cfg::V_BASE + (4 * (jb >> 1) + e) * (HD * 2) + (chunk << 4) + (a & 1) * 8);
+      const int chunk = (2 * db + (a >> 1)) ^ (2 * (HD == 128 ? row & 7 : (row >> 1) & 3));
+      v_tr[db] = smem_addr + (uint32_t)(Cfg::V_BASE + row * (HD * 2) + (chunk << 4) + (a & 1) * 8);
       asm volatile("" : "+v"(v_tr[db]));
     }
   }
 
   // Fragment addresses = per-lane part (below, loop-invariant) + compile-time part (buffer, key block / row block):
-  //   K fragment of k16 step s, key block kb:  k_lane[s] + buf * K_BYTES + kb * 32 rows
-  //   V^T fragment of step, row block db:      v_lane[head_dim 128: step ^ db, else step] + V_BASE + buf * V_BYTES + db * 4096
+  //   K fragment of k32 step s, key block kb:  k_lane[s] + buf * K_BYTES + kb * 16 rows
+  //   V^T fragment of step, row block db:      v_lane[head_dim 128: 4 step ^ db, else step] + V_BASE + buf * V_BYTES + db * 2048
   // (the swizzles depend on the row only through bits that the block offsets leave alone)
   // (kept as opaque 32-bit LDS addresses: left to itself the compiler splits them again into a common and a per-step
   // part and adds the two in front of every read)
   typedef __attribute__((address_space(3))) const unsigned char* lds_cptr;
-  lds_cptr k_lane[KS], v_lane[4];
+  constexpr int VL = DMA ? 1 : HD == 128 ? 8 : 2;
+  lds_cptr k_lane[KS], v_lane[VL];
 #pragma unroll
   for (int sq = 0; sq < KS; ++sq) {
-    k_lane[sq] = (lds_cptr)(smem + (HD == 64 ? off128(l31, 2 * sq + hi) : off256(l31, 2 * sq + hi)));
+    k_lane[sq] = (lds_cptr)(smem + (HD == 64 ? off128(l15, 4 * sq + q4) : off256(l15, 4 * sq + q4)));
     asm volatile("" : "+v"(k_lane[sq]));
   }
 #pragma unroll
-  for (int sx = 0; sx < 4; ++sx) {
-    v_lane[sx] = (lds_cptr)(smem + Cfg::V_BASE +
-                 (HD == 128 ? (uint32_t)((l31 >> 1) * 256 + (l31 & 1) * 128) + (uint32_t)(((2 * sx) ^ hi ^ ((l31 >> 1) & 7) ^ (l31 >> 4)) << 4)
-                            : vt_off<HD>(l31, 2 * sx + hi)));
-    asm volatile("" : "+v"(v_lane[sx]));
+  for (int x = 0; x < VL; ++x) {
+    // vt_off(l15, chunk) with chunk = q4 ^ x (head_dim 128) or 4 x + q4; bits 4 to 6 of the row come in through x
+    v_lane[x] = (lds_cptr)(smem + Cfg::V_BASE + vt_off<HD>(l15, HD == 128 ? q4 ^ x : 4 * x + q4));
+    asm volatile("" : "+v"(v_lane[x]));
   }
-  float m = -INFINITY, l = 0.f;
-  f32x16 o[DB];
+  float m[QN], l[QN];
+  f32x4 o[QN][DB];
   // A wave whose 32 queries all lie past the window (last query block of a window whose size is not a multiple of 256)
   // only stages K / V and keeps the barriers; its MFMA and softmax work would be thrown away.
   const bool wave_active = qb * QB + wave * 32 < L;  // wave-uniform
@@ -302,12 +312,13 @@ window_attention_stream_kernel(StreamParams p) {
   // online form: running maximum m, accumulated output and sum rescaled whenever a maximum moves.
   auto sweep = [&](auto fast_tag) {
   constexpr bool FAST = decltype(fast_tag)::value;
-  m = -INFINITY;
-  l = 0.f;
 #pragma unroll
-  for (int db = 0; db < DB; ++db)
+  for (int n = 0; n < QN; ++n) {
+    m[n] = -INFINITY;
+    l[n] = 0.f;
 #pragma unroll
-    for (int e = 0; e < 16; ++e) o[db][e] = 0.f;
+    for (int db = 0; db < DB; ++db) o[n][db] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
 
   if (DMA) {
     issue_chunk(0, 0);
@@ -346,22 +357,22 @@ window_attention_stream_kernel(StreamParams p) {
     } else if (j + LEAD < nch) {
       load_chunk(j + LEAD);
     }
-    f32x16 acc[2];
+    f32x4 acc[QN][KB];
     if (wave_active) {
 
-    // ---- S^T = K Q^T for the 64 keys of the chunk: acc[kb][4g+i] = <k[key], q>, key = 64j + 32kb + 8g + 4hi + i
-    // The K fragments are read PF MFMAs ahead of their use (left to itself the compiler reads each one right before
-    // its MFMA and exposes the LDS latency every time).
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[kb][e] = 0.f;
+    // ---- S^T = K Q^T for the 64 keys of the chunk: acc[n][kb][i] = <k[key], q>, key = 64j + 16kb + 4 q4 + i, query 16n + l15
+    // The K fragments are read PF fragments ahead of their use (left to itself the compiler reads each one right before
+    // its MFMAs and exposes the LDS latency every time).
     {
-      constexpr int PF = 2, NS = 2 * KS;
+      constexpr int PF = 2, NS = KB * KS;
+      const f32x4 zero4 = {0.f, 0.f, 0.f, 0.f};
       bf16x8 kfr[PF + 1];
-      auto read_k = [&](int t) {  // rows 32 (t / KS) + l31, 16-byte chunk 2 (t % KS) + hi
+      // fragment t: the key blocks in turn, so that an accumulator is not needed again at once
+      auto step_of = [](int t) { return t / KB; };
+      auto block_of = [](int t) { return t % KB; };
+      auto read_k = [&](int t) {  // rows 16 kb + l15, 16-byte chunk 4 s + q4
         typedef __attribute__((address_space(3))) const bf16x8* frag_ptr;
-        return *(frag_ptr)(k_lane[t % KS] + u * Cfg::K_BYTES + (t / KS) * 32 * (HD * 2));
+        return *(frag_ptr)(k_lane[step_of(t)] + u * Cfg::K_BYTES + block_of(t) * 16 * (HD * 2));
       };
 #pragma unroll
       for (int t = 0; t < PF; ++t) kfr[t] = read_k(t);
@@ -369,97 +380,111 @@ window_attention_stream_kernel(StreamParams p) {
       for (int t = 0; t < NS; ++t) {
         if (t + PF < NS) kfr[(t + PF) % (PF + 1)] = read_k(t + PF);
         __builtin_amdgcn_sched_barrier(0);
-        acc[t / KS] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kfr[t % (PF + 1)], qf[t % KS], acc[t / KS], 0, 0, 0);
+#pragma unroll
+        for (int n = 0; n < QN; ++n)
+          acc[n][block_of(t)] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kfr[t % (PF + 1)], qf[n][step_of(t)], step_of(t) == 0 ? zero4 : acc[n][block_of(t)], 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
     if (j * KC + KC > L) {  // last, partial chunk (uniform): keys past the window do not take part
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
+      for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const int key = j * KC + kb * 32 + (e >> 2) * 8 + hi * 4 + (e & 3);
-          if (key >= L) acc[kb][e] = -INFINITY;
+        for (int i = 0; i < 4; ++i) {
+          const int key = j * KC + kb * 16 + q4 * 4 + i;
+          if (key >= L) {
+#pragma unroll
+            for (int n = 0; n < QN; ++n) acc[n][kb][i] = -INFINITY;
+          }
         }
     }
 
-    // PV step (kb, t2): k slots 0-3 <-> keys 32kb+16t2+4hi+(0..3); slots 4-7 <-> keys 32kb+16t2+8+4hi+(0..3): one V^T
-    // chunk per 32-row block of O^T.  The fragments of a step are read one step ahead of its MFMAs.
+    // PV step p (32 keys): k slots 0-3 <-> keys 32p + 4 q4 + (0..3); slots 4-7 <-> keys 32p + 16 + 4 q4 + (0..3): one V^T
+    // chunk per 16-row block of O^T.  The fragments of half of the row blocks are read ahead of the MFMAs of the half before.
     // DMA form: the transposing reads are inline assembly (the builtin form would make the compiler wait for the load
     // unit's pending loads of the next chunks in front of every one of them, see lds_read_tr16_b64); what they return
     // becomes usable in v_ready().
-    bf16x8 vfb[2][DB];
-    TrFrag vtr[2][DMA ? DB : 1];
-    auto load_v = [&](int step, int slot) {  // V^T rows 32 db + l31, chunk step * 2 + hi: vt_off(), taken apart
+    constexpr int DH = DB / 2, PARTS = KC / 32 * 2;  // row blocks of a half; halves of a chunk
+    bf16x8 vfb[2][DH];
+    TrFrag vtr[2][DMA ? DH : 1];
+    auto load_v = [&](int part, int slot) {
+      const int step = part >> 1;
 #pragma unroll
-      for (int db = 0; db < DB; ++db) {
-        if (DMA) {  // keys 16 step + 4 hi + (0..3) and 16 step + 8 + 4 hi + (0..3) of row-major V, transposed by the read
-          const uint32_t a0 = smem_addr + v_tr[db] + u * Cfg::V_BYTES + step * 16 * (HD * 2);
-          vtr[slot][DMA ? db : 0].lo = lds_read_tr16_b64<0>(a0);
-          vtr[slot][DMA ? db : 0].hi = lds_read_tr16_b64<8 * (HD * 2)>(a0);
+      for (int d = 0; d < DH; ++d) {
+        const int db = (part & 1) * DH + d;
+        if (DMA) {  // keys 32 step + 4 q4 + (0..3) and 32 step + 16 + 4 q4 + (0..3) of row-major V, transposed by the read
+          const uint32_t a0 = v_tr[db] + u * Cfg::V_BYTES + step * 32 * (HD * 2);
+          vtr[slot][DMA ? d : 0].lo = lds_read_tr16_b64<0>(a0);
+          vtr[slot][DMA ? d : 0].hi = lds_read_tr16_b64<16 * (HD * 2)>(a0);
         } else {
-          vfb[slot][db] = *(__attribute__((address_space(3))) const bf16x8*)(v_lane[HD == 128 ? step ^ db : step] + u * Cfg::V_BYTES + db * 4096);
+          vfb[slot][d] = *(__attribute__((address_space(3))) const bf16x8*)(v_lane[HD == 128 ? ((4 * step) ^ db) % VL : step % VL] + u * Cfg::V_BYTES + db * 2048);
         }
       }
     };
     auto v_ready = [&](int slot) {
       if (DMA) {
-        if constexpr (DB == 4) lds_tr_wait(vtr[slot][0], vtr[slot][DMA ? 1 : 0], vtr[slot][DMA ? 2 : 0], vtr[slot][DMA ? 3 : 0]);
+        if constexpr (DH == 4) lds_tr_wait(vtr[slot][0], vtr[slot][DMA ? 1 : 0], vtr[slot][DMA ? 2 : 0], vtr[slot][DMA ? 3 : 0]);
         else lds_tr_wait(vtr[slot][0], vtr[slot][DMA ? 1 : 0]);
 #pragma unroll
-        for (int db = 0; db < DB; ++db) vfb[slot][db] = tr_frag_value(vtr[slot][DMA ? db : 0]);
+        for (int d = 0; d < DH; ++d) vfb[slot][d] = tr_frag_value(vtr[slot][DMA ? d : 0]);
       }
     };
     load_v(0, 0);  // in flight during the softmax arithmetic below
 
     // ---- online softmax (exp2 domain): new row max, rescale what has been accumulated if any max moved
     if (!FAST) {
-      float cm = acc[0][0];
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
+      for (int n = 0; n < QN; ++n) {
+        float cm = acc[n][0][0];
 #pragma unroll
-        for (int e = 0; e < 16; e += 2) cm = fmaxf(fmaxf(cm, acc[kb][e]), acc[kb][e + 1]);
-      cm = fmaxf(cm, __shfl_xor(cm, 32, 64));
-      const float m_new = fmaxf(m, cm);
-      if (__builtin_amdgcn_ballot_w64(m_new > m) != 0) {
-        const float alpha = __builtin_amdgcn_exp2f(m - m_new);  // 0 for the first chunk (m = -inf)
-        l *= alpha;
+        for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
-        for (int db = 0; db < DB; ++db)
+          for (int i = 0; i < 4; i += 2) cm = fmaxf(fmaxf(cm, acc[n][kb][i]), acc[n][kb][i + 1]);
+        cm = fmaxf(cm, __shfl_xor(cm, 16, 64));
+        cm = fmaxf(cm, __shfl_xor(cm, 32, 64));
+        const float m_new = fmaxf(m[n], cm);
+        if (__builtin_amdgcn_ballot_w64(m_new > m[n]) != 0) {
+          const float alpha = __builtin_amdgcn_exp2f(m[n] - m_new);  // 0 for the first chunk (m = -inf)
+          l[n] *= alpha;
 #pragma unroll
-          for (int e = 0; e < 16; ++e) o[db][e] *= alpha;
-        m = m_new;
+          for (int db = 0; db < DB; ++db) o[n][db] *= alpha;
+          m[n] = m_new;
+        }
       }
     }
 
-    // ---- P = exp2(s) or exp2(s - m) for 16 keys at a time and O^T += V^T P^T: while the MFMAs of a step run, the P of the next
-    // step is formed (the VALU work hides the MFMAs) and its V^T fragments are read
-    uint32_t pkb[2][4];
-    auto exp_step = [&](int step, uint32_t (&pk)[4]) {
-      const int kb = step >> 1, t2 = step & 1;
+    // ---- P = exp2(s) or exp2(s - m) for 32 keys at a time and O^T += V^T P^T: while the MFMAs of a step run, the P of the next
+    // step is formed (the VALU work hides the MFMAs) and the V^T fragments of the next half are read
+    uint32_t pkb[2][QN][4];
+    auto exp_step = [&](int step, int n) {
 #pragma unroll
       for (int h = 0; h < 4; ++h) {
-        const int h2 = 4 * t2 + h;
-        const float e0 = __builtin_amdgcn_exp2f(FAST ? acc[kb][2 * h2] : acc[kb][2 * h2] - m);
-        const float e1 = __builtin_amdgcn_exp2f(FAST ? acc[kb][2 * h2 + 1] : acc[kb][2 * h2 + 1] - m);
-        pk[h] = pack_bf16x2(e0, e1);
-        l = dot2_ones(pk[h], l);  // the row sum of what PV multiplies: the rounded values, one instruction per pair
+        const float a0 = acc[n][2 * step + (h >> 1)][2 * (h & 1)], a1 = acc[n][2 * step + (h >> 1)][2 * (h & 1) + 1];
+        const float e0 = __builtin_amdgcn_exp2f(FAST ? a0 : a0 - m[n]);
+        const float e1 = __builtin_amdgcn_exp2f(FAST ? a1 : a1 - m[n]);
+        pkb[step & 1][n][h] = pack_bf16x2(e0, e1);
+        l[n] = dot2_ones(pkb[step & 1][n][h], l[n]);  // the row sum of what PV multiplies: the rounded values, one instruction per pair
       }
     };
-    exp_step(0, pkb[0]);
 #pragma unroll
-    for (int step = 0; step < 4; ++step) {
+    for (int n = 0; n < QN; ++n) exp_step(0, n);
+#pragma unroll
+    for (int part = 0; part < PARTS; ++part) {
+      const int step = part >> 1;
       __builtin_amdgcn_sched_barrier(0);
-      v_ready(step & 1);  // ahead of the next step's reads: the wait then covers reads issued a whole step ago only
-      if (step + 1 < 4) {
-        load_v(step + 1, (step + 1) & 1);
-        exp_step(step + 1, pkb[(step + 1) & 1]);
-      }
-      const uint32_t* pk = pkb[step & 1];
-      const u32x4 pw = {pk[0], pk[1], pk[2], pk[3]};
-      const bf16x8 pf = __builtin_bit_cast(bf16x8, pw);
+      v_ready(part & 1);  // ahead of the next half's reads: the wait then covers reads issued a whole half ago only
+      if (part + 1 < PARTS) load_v(part + 1, (part + 1) & 1);
+      if (step + 1 < KC / 32) exp_step(step + 1, part & 1);
 #pragma unroll
-      for (int db = 0; db < DB; ++db) o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vfb[step & 1][db], pf, o[db], 0, 0, 0);
+      for (int d = 0; d < DH; ++d) {
+#pragma unroll
+        for (int n = 0; n < QN; ++n) {
+          const u32x4 pw = {pkb[step & 1][n][0], pkb[step & 1][n][1], pkb[step & 1][n][2], pkb[step & 1][n][3]};
+          const bf16x8 pf = __builtin_bit_cast(bf16x8, pw);
+          f32x4& od = o[n][(part & 1) * DH + d];
+          od = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vfb[part & 1][d], pf, od, 0, 0, 0);
+        }
+      }
     }
     __builtin_amdgcn_sched_barrier(0);
     }  // wave_active
@@ -477,27 +502,34 @@ window_attention_stream_kernel(StreamParams p) {
   // Range check of the sweep without maximum: a row sum that left [2^-40, 2^100] (or is not a number) means logits
   // beyond what exp2 holds without the maximum; the workgroup then repeats the window's keys in the online form.
   {
-    const float lt = l + __shfl_xor(l, 32, 64);
-    const bool bad = wave_active && !(lt >= 0x1p-40f && lt <= 0x1p100f);
+    bool bad = false;
+#pragma unroll
+    for (int n = 0; n < QN; ++n) {
+      float lt = l[n] + __shfl_xor(l[n], 16, 64);
+      lt += __shfl_xor(lt, 32, 64);
+      bad = bad || (wave_active && !(lt >= 0x1p-40f && lt <= 0x1p100f));
+    }
     if (__builtin_amdgcn_ballot_w64(bad) != 0 && lane == 0) *redo = 1;
     __syncthreads();
     if (*redo != 0) sweep(std::false_type{});
   }
 
-  // ---- normalise and store: o[db][4g+i] = O[query][32db + 8g + 4hi + i]
-  l += __shfl_xor(l, 32, 64);
-  const float inv = __builtin_amdgcn_rcpf(l);
-  if (q_valid) {
-    uint16_t* op = p.out + q_row * inner + head * HD + hi * 4;
+  // ---- normalise and store: o[n][db][i] = O[query 16n + l15][16db + 4 q4 + i]
 #pragma unroll
-    for (int db = 0; db < DB; ++db)
+  for (int n = 0; n < QN; ++n) {
+    l[n] += __shfl_xor(l[n], 16, 64);
+    l[n] += __shfl_xor(l[n], 32, 64);
+    const float inv = __builtin_amdgcn_rcpf(l[n]);
+    if (q_valid[n]) {
+      uint16_t* op = p.out + q_row[n] * inner + head * HD + q4 * 4;
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
+      for (int db = 0; db < DB; ++db) {
         u32x2 w2;
-        w2.x = pack_bf16x2(o[db][g * 4] * inv, o[db][g * 4 + 1] * inv);
-        w2.y = pack_bf16x2(o[db][g * 4 + 2] * inv, o[db][g * 4 + 3] * inv);
-        *reinterpret_cast<u32x2*>(op + db * 32 + g * 8) = w2;
+        w2.x = pack_bf16x2(o[n][db][0] * inv, o[n][db][1] * inv);
+        w2.y = pack_bf16x2(o[n][db][2] * inv, o[n][db][3] * inv);
+        *reinterpret_cast<u32x2*>(op + db * 16) = w2;
       }
+    }
   }
 }
 
@@ -529,6 +561,7 @@ hipError_t launch_one(StreamParams p, int L, hipStream_t stream) {
 hipError_t attention_stream_configure_all() {
   hipError_t e = configure_one<64, false, 8, 4>();
   if (e == hipSuccess) e = configure_one<128, false, 8, 4>();
+  if (e == hipSuccess) e = configure_one<64, true, 8, 4>();
   if (e == hipSuccess) e = configure_one<64, true, 2, 1>();
   if (e == hipSuccess) e = configure_one<128, true, 2, 1>();
   if (e == hipSuccess) e = configure_one<64, true, 4, 2>();
@@ -555,18 +588,19 @@ hipError_t attention_stream_launch(const void* qkv, void* out, int B, int H, int
   const int64_t span = ((int64_t)H * W - 1) * tok_stride * 2 + (int64_t)head_dim * 2;
   p.span_bytes = span < ((int64_t)1 << 32) - 4096 ? (uint32_t)span : 0u;
   const bool dma = p.span_bytes != 0 && tok_stride > 0;
-  // Windows above 2048 tokens with head_dim 128: 8 waves where few workgroups share the chip (4 windows of 3600 with 12 heads:
-  // 308 us against 315), the same on a full grid (360 x 720: 5389, 5372).  Below, 4 waves (500 000 tokens x 3 heads, 8 -> 4 waves:
-  // L = 1395 1319 -> 1160 us, 960 965 -> 868, 400 633 -> 570, 192 427 -> 387, 128 398 -> 306), head_dim 64 for any L (500 000 x 6:
-  // L = 1395 1630 -> 1250), except where 8 waves are one workgroup per CU and 4 waves would be up to two: the chip is as full
-  // either way, and the two load every K / V chunk twice (`lone`, per XCD of 32 CUs; 8 -> 4 waves):
-  //   head_dim 128, units of 130 tokens  144: 10.9 -> 12.0 us   240: 12.3 -> 12.8   (the second workgroup has two queries)   192 tokens  144: 12.1 -> 12.0
-  //     400 tokens  72: 19.5 -> 20.1   120: 22.0 -> 22.2      900 tokens  48: 31.8 -> 32.9      1395  32: 41.8 -> 43.4      2048  24: 57.6 -> 60.0
-  //   head_dim 64, register form with 8 waves   900 tokens  40: 21.1 -> 21.3   1395  24: 27.4 -> 28.0   2048  24: 37.7 -> 38.5   3600  16: 63.5 -> 67.5
+  // Windows above 2048 tokens with head_dim 128: 8 waves (4 windows of 3600 with 12 heads: 320 us against 325; 360 x 720 with 8 heads
+  // 3530, 3615).  Below, 4 waves (250 000 tokens x 3 heads, 8 -> 4 waves: L = 1364 581 -> 550 us, 960 471 -> 460, 400 343 -> 304, 192 226 -> 206,
+  // 128 222 -> 174), head_dim 64 for any L (250 000 x 6: L = 1364 693 -> 600), except where 8 waves are one workgroup per CU and 4 waves would
+  // be up to two: the chip is as full either way, and the two load every K / V chunk twice (`lone`, per XCD of 32 CUs; 8 -> 4 waves):
+  //   head_dim 128, units of 130 tokens  144: 11.8 -> 12.8 us   240: 12.6 -> 13.9   (the second workgroup has two queries)   192 tokens  144: 13.4 -> 13.3
+  //     400 tokens  72: 21.6 -> 21.6   120: 23.6 -> 23.7      900 tokens  48: 36.9 -> 38.5      1395  32: 48.1 -> 49.9      2048  24: 66.9 -> 69.2
+  //   head_dim 64   130 tokens  144: 7.9 -> 8.5   192 tokens  144: 8.6 -> 8.5   400 tokens  72: 13.8 -> 13.9   120: 14.8 -> 15.0
+  //     900 tokens  40: 23.2 -> 23.8   64: 24.8 -> 25.8   1395  24: 30.7 -> 31.4   2048  24: 43.0 -> 44.7   3600  16: 71.5 -> 75.6
   const int64_t per_xcd = (p.n_units + 7) / 8, wgs4 = per_xcd * ((L + 127) / 128), wgs8 = per_xcd * ((L + 255) / 256);
   const bool lone = wgs8 <= 32 && wgs4 > 32;
   if (head_dim == 64) {
-    if (!dma || (lone && L > 1024)) return launch_one<64, false, 8, 4>(p, L, stream);
+    if (!dma) return launch_one<64, false, 8, 4>(p, L, stream);
+    if (lone && (L <= 160 || L > 256)) return launch_one<64, true, 8, 4>(p, L, stream);
     return L <= KC ? launch_one<64, true, 2, 1>(p, L, stream) : launch_one<64, true, 4, 2>(p, L, stream);
   }
   if (!dma) return launch_one<128, false, 8, 4>(p, L, stream);

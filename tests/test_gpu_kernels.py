@@ -537,6 +537,18 @@ def test_window_attention_streaming_workgroup_sizes(pkg, cuda, case):
     test_window_attention_streaming_parity(pkg, cuda, case)
 
 
+@pytest.mark.parametrize("case", [
+    # B, H, W, heads, head_dim, ws_y, ws_x, shift_y, shift_x: head_dim 64, so few windows that eight waves take them
+    (2, 26, 100, 4, 64, 13, 10, 6, 5),       # L = 130, 160 units: three chunks, the last one with two keys
+    (1, 48, 64, 36, 64, 16, 16, 8, 8),       # L = 256, 432 units: four waves again
+    (1, 38, 54, 12, 64, 19, 27, 0, 13),      # L = 513: nine chunks, the last one with one key
+    (2, 61, 61, 2, 64, 61, 61, 30, 30),      # L = 3721, 4 units
+], ids=lambda c: f"B{c[0]}_{c[1]}x{c[2]}_h{c[3]}x{c[4]}_ws{c[5]}x{c[6]}_s{c[7]}x{c[8]}")
+def test_window_attention_streaming_few_windows_hd64(pkg, cuda, case):
+    """Same oracle and tolerance as the other streaming cases."""
+    test_window_attention_streaming_parity(pkg, cuda, case)
+
+
 def test_window_attention_streaming_wide_rows_match_compact_hd64(pkg, cuda):
     """head_dim 64: rows of a [S, 3 * inner] matrix too wide for 32-bit offsets go through registers, a compact copy of
     some of its heads straight into LDS, bit for bit the same (the key order and the arithmetic per wave are)."""

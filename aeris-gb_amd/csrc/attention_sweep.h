@@ -338,4 +338,262 @@ __device__ __forceinline__ void store_attention_rows(uint16_t* op, const f32x16 
     }
 }
 
+// ---------------------------------------------------------------------------------------------
+// The same arithmetic in blocks of 16 queries and 16 keys (v_mfma_f32_16x16x32_bf16, lane = l15 + 16 q4): QN query blocks of a wave
+// against the window's keys, 32 a step.  Same work per cycle and LDS byte as the 32x32x16 shape at a higher clock, and a window
+// whose token count is an odd multiple of 16 (12x12) has no padded keys and a last wave of one query block instead of two.
+//   S^T block: acc[n][kb][i] is the logit (times log2 e) of key 16 kb + 4 q4 + i and query 16 n + l15.  The two key blocks of a
+//   step, packed, are the 8 k slots of P^T for O^T = V^T P^T: keys 32 p + 4 q4 + (0..3) and 32 p + 16 + 4 q4 + (0..3); a last
+//   single block is the 4 k slots of v_mfma_f32_16x16x16_bf16.
+//   o[n][db][i] = O[query 16 n + l15][16 db + 4 q4 + i].
+template <int WS_Y, int WS_X, bool HAS_BIAS, int PITCH = 2 * WS_X - 1>
+struct WindowLogits16 {
+  static constexpr int L = WS_Y * WS_X, KB = L / 16;
+  static constexpr float MASK_NEG = -100.0f * 1.4426950408889634f;  // the additive -100, in the exp2 domain
+  static_assert(WS_X % 4 == 0 && L % 16 == 0 && (WS_X == 8 || WS_X == 12 || WS_X == 16), "4 consecutive keys lie in one window row");
+  // Where a lane's 4 keys of a block stand relative to the block's first key: one way for windows of 8 and 16 columns, for 12 one
+  // per column (0, 4, 8) that a block can begin at.
+  static constexpr int WAYS = WS_X == 12 ? 3 : 1;
+  const unsigned char* bias_at[WAYS];
+  int q4;
+  bool my, mx;
+  int qiy, qix, sy, sx;
+
+  __device__ __forceinline__ WindowLogits16(const unsigned char* bias_lds, int qpos, int q4_, bool my_, bool mx_, int sy_, int sx_)
+      : q4(q4_), my(my_), mx(mx_), qiy(qpos / WS_X), qix(qpos % WS_X), sy(sy_), sx(sx_) {
+    const int sp = (2 * WS_Y - 2) * PITCH + 2 * WS_X - 2 - (qiy + WS_Y - 1) * PITCH - qix - (WS_X - 1);
+#pragma unroll
+    for (int w = 0; w < WAYS; ++w) bias_at[w] = bias_lds + (sp + rows_on(4 * w) * PITCH + column(4 * w) - 4 * w) * 16;
+  }
+  // of the lane's keys, the block beginning in column c0: window rows below the block's first, column
+  __device__ __forceinline__ int rows_on(int c0) const { return (c0 + 4 * q4) / WS_X; }
+  __device__ __forceinline__ int column(int c0) const { return (c0 + 4 * q4) % WS_X; }
+  __device__ __forceinline__ f32x4 start(int kb) const {
+    if (!HAS_BIAS) return f32x4{0.f, 0.f, 0.f, 0.f};
+    const int r0 = kb * 16 / WS_X, c0 = kb * 16 % WS_X;
+    const unsigned char* at = bias_at[0];
+    if (WAYS == 3) at = c0 == 0 ? bias_at[0] : c0 == 4 ? bias_at[1 % WAYS] : bias_at[2 % WAYS];
+    return *reinterpret_cast<const f32x4*>(at + (r0 * PITCH + c0) * 16);
+  }
+  __device__ __forceinline__ bool masked() const { return my || mx; }  // wave-uniform
+  __device__ __forceinline__ void mask(int kb, f32x4& a) const {
+    const int r0 = kb * 16 / WS_X, c0 = kb * 16 % WS_X;
+    const int kiy = r0 + rows_on(c0), kix = column(c0);
+    const bool ydiff = my && ((kiy < WS_Y - sy) != (qiy < WS_Y - sy));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const bool xdiff = mx && ((kix + i < WS_X - sx) != (qix < WS_X - sx));
+      if (ydiff || xdiff) a[i] += MASK_NEG;
+    }
+  }
+};
+
+// V^T fragments of head_dim 64 from a row-major V tile whose rows (128 B) have their 16-byte chunks XOR-swizzled by 2 ((key >> 1) & 3):
+// the 8 keys x 2 chunks that a 32-lane pass of the transposing read gathers lie on distinct banks.
+template <class Base>
+struct LoadVTransposed16 {
+  static constexpr int DB = 4;
+  uint32_t v_lane[DB];
+  __device__ __forceinline__ LoadVTransposed16(int lane, Base base) {
+    const int q4 = lane >> 4, e = (lane >> 2) & 3, a = lane & 3, row = 4 * q4 + e;
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+      v_lane[db] = base + (uint32_t)(row * 128 + (((2 * db + (a >> 1)) ^ (2 * ((row >> 1) & 3))) << 4) + (a & 1) * 8);
+  }
+  // keys 16 kb .. (low half) and, of a whole step, 16 kb + 16 .. (high half)
+  __device__ __forceinline__ void operator()(int kb, bool whole, TrFrag (&f)[DB]) const {
+#pragma unroll
+    for (int db = 0; db < DB; ++db) {
+      f[db].lo = lds_read_tr16_b64<0>(v_lane[db] + (uint32_t)kb * 2048u);
+      if (whole) f[db].hi = lds_read_tr16_b64<2048>(v_lane[db] + (uint32_t)kb * 2048u);
+    }
+  }
+};
+
+// `load_k(kb, s)` returns K's fragment: row 16 kb + l15, 8 elements from 32 s + 8 q4; `lg[n]` are the logits' start values and mask.
+// Otherwise as attention_sweep: one sweep without a row maximum, sums checked, the two-pass form for what leaves the range.
+template <int QN, class Logits, class LoadK, class LoadV, class Mid>
+__device__ __forceinline__ void attention_sweep16(const Logits (&lg)[QN], const LoadK& load_k, const LoadV& load_v, const Mid& mid,
+                                                  const bf16x8 (&qf)[QN][2], f32x4 (&o)[QN][4], float (&sum)[QN]) {
+  constexpr int KB = Logits::KB, NP = (KB + 1) / 2, DB = 4, KS = 2;
+  typedef __attribute__((ext_vector_type(4))) short s16x4;
+  const f32x4 zero4 = {0.f, 0.f, 0.f, 0.f};
+  auto blocks = [](int p) { return 2 * p + 2 <= KB ? 2 : 1; };  // key blocks of a step
+  auto pv_half = [](const u32x2& v, uint32_t p0, uint32_t p1, const f32x4& c) {
+    return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, v), __builtin_bit_cast(s16x4, u32x2{p0, p1}), c, 0, 0, 0);
+  };
+  {
+    f32x4 acc[2][QN][2];
+    bf16x8 kf[2][2][KS];
+    auto read_k = [&](int p) {
+#pragma unroll
+      for (int b = 0; b < blocks(p); ++b)
+#pragma unroll
+        for (int s = 0; s < KS; ++s) kf[p & 1][b][s] = load_k(2 * p + b, s);
+    };
+    auto start = [&](int p) {
+#pragma unroll
+      for (int b = 0; b < blocks(p); ++b)
+#pragma unroll
+        for (int n = 0; n < QN; ++n) acc[p & 1][n][b] = lg[n].start(2 * p + b);
+    };
+    auto qk = [&](int p) {
+#pragma unroll
+      for (int s = 0; s < KS; ++s)
+#pragma unroll
+        for (int b = 0; b < blocks(p); ++b)
+#pragma unroll
+          for (int n = 0; n < QN; ++n)
+            acc[p & 1][n][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[p & 1][b][s], qf[n][s], acc[p & 1][n][b], 0, 0, 0);
+    };
+#pragma unroll
+    for (int n = 0; n < QN; ++n) sum[n] = 0.f;
+    read_k(0);
+    start(0);
+    if (NP > 1) {
+      read_k(1);
+      start(1);
+    }
+    TrFrag vraw[DB];
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0), see below
+    __builtin_amdgcn_sched_barrier(0);
+    load_v(0, KB > 1, vraw);
+    __builtin_amdgcn_sched_barrier(0);
+    qk(0);
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+      const bool whole = blocks(p) == 2;
+      __builtin_amdgcn_sched_barrier(0);
+      mid(p);
+      // This step's V^T reads, then the next step's S^T.  The K fragments and bias vectors of the latter, requested a step ago, are waited
+      // for ahead of the reads: the compiler's own wait would count the assembly reads in.  (Behind the MFMAs the reads could return into
+      // registers that the first of two MFMAs on an accumulator is still writing: the shape's chains need not stay in one register.)
+      if (p > 0) {
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+        __builtin_amdgcn_sched_barrier(0);
+        load_v(2 * p, whole, vraw);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if (p + 1 < NP) qk(p + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      if (p + 2 < NP) read_k(p + 2);
+      if (lg[0].masked()) {
+#pragma unroll
+        for (int n = 0; n < QN; ++n)
+#pragma unroll
+          for (int b = 0; b < (whole ? 2 : 1); ++b) lg[n].mask(2 * p + b, acc[p & 1][n][b]);
+      }
+      uint32_t pk[QN][4];
+#pragma unroll
+      for (int n = 0; n < QN; ++n)
+#pragma unroll
+        for (int b = 0; b < (whole ? 2 : 1); ++b) {
+          const f32x4& a = acc[p & 1][n][b];
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            pk[n][2 * b + h] = pack_bf16x2(__builtin_amdgcn_exp2f(a[2 * h]), __builtin_amdgcn_exp2f(a[2 * h + 1]));
+            sum[n] = dot2_ones(pk[n][2 * b + h], sum[n]);  // the row sum of what PV multiplies: the rounded values
+          }
+        }
+      __builtin_amdgcn_sched_barrier(0);
+      if (whole) lds_tr_wait(vraw[0], vraw[1], vraw[2], vraw[3]);
+      else asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(vraw[0].lo), "+v"(vraw[1].lo), "+v"(vraw[2].lo), "+v"(vraw[3].lo));
+      if (p + 2 < NP) start(p + 2);
+#pragma unroll
+      for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int n = 0; n < QN; ++n) {
+          const f32x4 c = p == 0 ? zero4 : o[n][db];
+          if (whole)
+            o[n][db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(tr_frag_value(vraw[db]), __builtin_bit_cast(bf16x8, u32x4{pk[n][0], pk[n][1], pk[n][2], pk[n][3]}), c, 0, 0, 0);
+          else
+            o[n][db] = pv_half(vraw[db].lo, pk[n][0], pk[n][1], c);
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  bool out_of_range = false;
+#pragma unroll
+  for (int n = 0; n < QN; ++n) {
+    sum[n] += __shfl_xor(sum[n], 16, 64);
+    sum[n] += __shfl_xor(sum[n], 32, 64);
+    out_of_range = out_of_range || !(sum[n] >= 0x1p-40f && sum[n] <= 0x1p100f);  // true for NaN as well
+  }
+  if (__builtin_amdgcn_ballot_w64(out_of_range) != 0) {
+    float m[QN];
+#pragma unroll
+    for (int n = 0; n < QN; ++n) m[n] = -INFINITY;
+#pragma unroll 1
+    for (int pass = 0; pass < 2; ++pass) {
+      if (pass == 1) {
+#pragma unroll
+        for (int n = 0; n < QN; ++n) {
+          m[n] = fmaxf(m[n], __shfl_xor(m[n], 16, 64));
+          m[n] = fmaxf(m[n], __shfl_xor(m[n], 32, 64));
+          sum[n] = 0.f;
+#pragma unroll
+          for (int db = 0; db < DB; ++db) o[n][db] = zero4;
+        }
+      }
+#pragma unroll 1
+      for (int kb = 0; kb < KB; ++kb) {
+        f32x4 a[QN];
+#pragma unroll
+        for (int n = 0; n < QN; ++n) a[n] = lg[n].start(kb);
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+          const bf16x8 f = load_k(kb, s);
+#pragma unroll
+          for (int n = 0; n < QN; ++n) a[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f, qf[n][s], a[n], 0, 0, 0);
+        }
+        if (lg[0].masked()) {
+#pragma unroll
+          for (int n = 0; n < QN; ++n) lg[n].mask(kb, a[n]);
+        }
+        if (pass == 0) {
+#pragma unroll
+          for (int n = 0; n < QN; ++n) m[n] = fmaxf(fmaxf(fmaxf(m[n], a[n][0]), fmaxf(a[n][1], a[n][2])), a[n][3]);
+        } else {
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int n = 0; n < QN; ++n) asm volatile("s_nop 15\n\ts_nop 15" : "+v"(a[n]));  // (no MFMA is writing a register when the reads below are issued)
+          TrFrag vraw[DB];
+          load_v(kb, false, vraw);
+          asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(vraw[0].lo), "+v"(vraw[1].lo), "+v"(vraw[2].lo), "+v"(vraw[3].lo));
+#pragma unroll
+          for (int n = 0; n < QN; ++n) {
+            uint32_t pk[2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+              pk[h] = pack_bf16x2(__builtin_amdgcn_exp2f(a[n][2 * h] - m[n]), __builtin_amdgcn_exp2f(a[n][2 * h + 1] - m[n]));
+              sum[n] = dot2_ones(pk[h], sum[n]);
+            }
+#pragma unroll
+            for (int db = 0; db < DB; ++db) o[n][db] = pv_half(vraw[db].lo, pk[0], pk[1], o[n][db]);
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int n = 0; n < QN; ++n) {
+      sum[n] += __shfl_xor(sum[n], 16, 64);
+      sum[n] += __shfl_xor(sum[n], 32, 64);
+    }
+  }
+}
+
+// Normalise and store a query block's rows: v_permlane16_swap on the pieces of row blocks 2m and 2m + 1 leaves lane (l15, q4) with 8
+// consecutive elements, 32 m + 16 (q4 & 1) + 8 (q4 >> 1) .., of row l15: 64 contiguous bytes per row and instruction.  `op` points at the
+// row's head slice.  Two store instructions, issued by every lane for which `valid` holds.
+__device__ __forceinline__ void store_attention_rows16(uint16_t* op, const f32x4 (&o)[4], float sum, int q4, bool valid) {
+  const float inv = __builtin_amdgcn_rcpf(sum);
+#pragma unroll
+  for (int m = 0; m < 2; ++m) {
+    const f32x4 a = o[2 * m] * inv, b = o[2 * m + 1] * inv;
+    const auto rx = __builtin_amdgcn_permlane16_swap(pack_bf16x2(a[0], a[1]), pack_bf16x2(b[0], b[1]), false, false);
+    const auto ry = __builtin_amdgcn_permlane16_swap(pack_bf16x2(a[2], a[3]), pack_bf16x2(b[2], b[3]), false, false);
+    if (valid) *reinterpret_cast<u32x4*>(op + 32 * m + 16 * (q4 & 1) + 8 * (q4 >> 1)) = u32x4{rx[0], ry[0], rx[1], ry[1]};
+  }
+}
+
 }  // namespace aeris

@@ -27,6 +27,7 @@
 #include "common.h"
 #include "attention_sweep.h"
 #include "kernels.h"
+#include <type_traits>
 
 namespace aeris {
 
@@ -43,6 +44,7 @@ struct AttnParams {
   int use_mask;
   float scale;
   int q_prescaled;  // q already holds q * scale * log2(e) (the producing GEMM scaled it in fp32 before its only rounding)
+  int rotate;  // persistent form: see persist_rotation
 };
 
 template <int WS_Y, int WS_X, int HD, bool HAS_BIAS>
@@ -434,11 +436,16 @@ struct AttnPersistCfg {
 
 constexpr int attn_persist_threads(int ws_y, int ws_x) { return ((ws_y * ws_x + 31) / 32) * 64; }
 
-template <int WS_Y, int WS_X, bool HAS_BIAS>
+template <int WS_Y, int WS_X, bool HAS_BIAS, bool S16, bool ROTATES>
 __global__ void __launch_bounds__(attn_persist_threads(WS_Y, WS_X))
 window_attention_persist_kernel(AttnParams p, int n_units) {
   using Cfg = AttnPersistCfg<WS_Y, WS_X, HAS_BIAS>;
-  constexpr int HD = 64, KS = 4, DB = 2;
+  constexpr int HD = 64;
+  // S16: windows of an odd multiple of 16 tokens (12x12) in blocks of 16 queries and keys: no padded keys, and the last wave, the
+  // second one of its SIMD, has half of the others' work.  (Compute alone takes two thirds of the time there, memory at the rate of a
+  // copy the same.)  64800 tokens x 8 heads 64.3 -> 59.5 us, 259200 231 -> 210, 2 x 259200 x 16 884 -> 837; persist_in_16s says where.
+  static_assert(!S16 || Cfg::L % 32 != 0, "otherwise there is nothing to gain");
+  constexpr int NB = S16 ? 2 : 1, KS = 4 / NB;  // query blocks of a wave, k steps of K Q^T
   constexpr int L = Cfg::L, NQ = Cfg::NQ, NT = Cfg::NT, TBL = Cfg::TBL, KVB = Cfg::KV_BYTES;
   static_assert(WS_X % 4 == 0, "groups of 4 consecutive keys must stay inside one window row");
   constexpr float LOG2E = 1.4426950408889634f;
@@ -454,24 +461,27 @@ window_attention_persist_kernel(AttnParams p, int n_units) {
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int l31 = lane & 31, hi = lane >> 5;
+  const int l31 = lane & 31, hi = lane >> 5, l15 = lane & 15, q4 = lane >> 4;
   const int H = p.H, W = p.W;
   const int inner = p.heads * HD;
   const uint32_t ld_qkv = (uint32_t)p.tok_stride;
   const int wpi = p.nWy * p.nWx;
   const int n_win = p.B * wpi;
 
-  const int u_begin = blockIdx.x, u_step = gridDim.x;
+  const int u_begin = blockIdx.x;
   if (u_begin >= n_units) return;
 
   const uint32_t plane_bytes = (uint32_t)p.B * (uint32_t)(H * W) * ld_qkv * 2u;  // < 2^32, checked by the caller
   const int rsub = lane >> 3, pc = lane & 7;
 
   // A unit = (head, batch entry, window row, window column), numbered window-fastest; everything about it is
-  // workgroup-uniform and lives in scalar registers.  A workgroup takes the units u_begin, u_begin + u_step, ...: the
+  // workgroup-uniform and lives in scalar registers.  The workgroups take one unit each of as many in a row: the
   // windows on the wrapped border of a shifted grid (a whole window row; their mask arithmetic makes them the slow
-  // ones) are then spread over all workgroups instead of filling the ranges of a few.  The successor of a unit
-  // follows by adding the digits of u_step with carries, without a division.
+  // ones) are then spread over all workgroups instead of filling the ranges of a few.  From one such round to the next the workgroups
+  // move on by p.rotate units (ROTATES, persist_rotation; a form of its own, since the scalar registers are short: 2 to 3 % for 8x8 windows
+  // and small grids).
+  // The successor of a unit follows by adding the digits of the step, of which there are two, with carries, without a division.
+  const int n_wg = gridDim.x, rotate = ROTATES ? p.rotate : 0;
   struct Unit { int head, b, wy, wx; };
   auto decode = [&](int u) {
     Unit r;
@@ -483,8 +493,10 @@ window_attention_persist_kernel(AttnParams p, int n_units) {
     r.wx = wrem - r.wy * p.nWx;
     return r;
   };
-  const Unit step = decode(u_step);
-  auto successor = [&](Unit r) {
+  const Unit step_on = decode(n_wg + rotate), step_back = decode(rotate);  // the latter: past the end of the row of workgroups
+  auto successor = [&](Unit r, bool back) {
+    Unit step = step_on;
+    if (ROTATES && back) step = step_back;
     r.wx += step.wx;
     int carry = r.wx >= p.nWx;
     r.wx -= carry ? p.nWx : 0;
@@ -514,13 +526,14 @@ window_attention_persist_kernel(AttnParams p, int n_units) {
   // K and V of unit `un` -> buffer set `set`: instruction pair ii fills rows 8 ii .. 8 ii + 7 of both tiles; a wave
   // issues pairs wave, wave + NQ, ...  Per pair and lane: key, and the byte offsets of its K / V chunk relative to
   // the window's first token (un-wrapped windows).
+  auto v_swizzle = [](int key) { return 2 * (S16 ? (key >> 1) & 3 : key & 3); };
   uint32_t kv_relk[DMA_PER_WAVE], kv_relv[DMA_PER_WAVE];
 #pragma unroll
   for (int j = 0; j < DMA_PER_WAVE; ++j) {
     const int key = (wave + j * NQ) * 8 + rsub;
     const uint32_t rel = (uint32_t)((key / WS_X) * W + key % WS_X) * (ld_qkv * 2u);
     kv_relk[j] = rel + (uint32_t)((pc ^ ((key >> 1) & 7)) << 4);
-    kv_relv[j] = rel + (uint32_t)((pc ^ (2 * (key & 3))) << 4);
+    kv_relv[j] = rel + (uint32_t)((pc ^ v_swizzle(key)) << 4);
   }
   // The loads of a unit: descriptors and the window's base offset (kv_prepare), then one buffer_load ... lds per
   // call of kv_issue.  They are issued back to back right after the unit barrier.  (Spreading them over the key-block
@@ -549,21 +562,29 @@ window_attention_persist_kernel(AttnParams p, int n_units) {
     const int key = ii * 8 + rsub;
     uint32_t off = kv_base + (is_v ? kv_relv[j] : kv_relk[j]);
     if (kv_wraps)  // wave-uniform: windows on the wrapped border of a shifted grid
-      off = token_row(kv_unit, key) * (ld_qkv * 2u) + (uint32_t)((pc ^ (is_v ? 2 * (key & 3) : (key >> 1) & 7)) << 4);
+      off = token_row(kv_unit, key) * (ld_qkv * 2u) + (uint32_t)((pc ^ (is_v ? v_swizzle(key) : (key >> 1) & 7)) << 4);
     unsigned char* dst = smem + set * 2 * KVB + is_v * KVB + ii * 1024;
     __builtin_amdgcn_raw_ptr_buffer_load_lds(is_v ? kv_rs_v : kv_rs_k, (lds_ptr)dst, 16, off, 0, 0, 0);
   };
-  int qpos = wave * 32 + l31;
-  const bool q_valid = qpos < L;
-  if (!q_valid) qpos = L - 1;
-  const int qiy = qpos / WS_X, qix = qpos % WS_X;
-  const uint32_t q_rel = (uint32_t)(qiy * W + qix);
-  // Q fragments of this wave's query group (B operand: lane = query, 8 consecutive d per k16 step)
-  auto load_q = [&](const Unit& un, bf16x8 (&q)[KS], uint32_t& tok) {
-    tok = window_wraps(un) ? token_row(un, qpos) : window_base(un) + q_rel;
-    const uint16_t* qp = p.qkv + un.head * p.head_stride + (uint64_t)tok * ld_qkv + hi * 8;
+  // Q fragments of this wave's queries (B operand: lane = query, 8 consecutive d per k step).  A wave of one block of 16: the other
+  // one's rows are clamped to the last and not used.
+  const bool one_block = S16 && wave == NQ - 1;
+  int qpos[NB];
+  uint32_t q_rel[NB];
 #pragma unroll
-    for (int s2 = 0; s2 < KS; ++s2) q[s2] = *reinterpret_cast<const bf16x8*>(qp + s2 * 16);
+  for (int n = 0; n < NB; ++n) {
+    qpos[n] = wave * 32 + (S16 ? n * 16 + l15 : l31);
+    if (qpos[n] > L - 1) qpos[n] = L - 1;
+    q_rel[n] = (uint32_t)(qpos[n] / WS_X * W + qpos[n] % WS_X);
+  }
+  auto load_q = [&](const Unit& un, bf16x8 (&q)[NB][KS], uint32_t (&tok)[NB]) {
+#pragma unroll
+    for (int n = 0; n < NB; ++n) {
+      tok[n] = window_wraps(un) ? token_row(un, qpos[n]) : window_base(un) + q_rel[n];
+      const uint16_t* qp = p.qkv + un.head * p.head_stride + (uint64_t)tok[n] * ld_qkv + (S16 ? q4 : hi) * 8;
+#pragma unroll
+      for (int s2 = 0; s2 < KS; ++s2) q[n][s2] = *reinterpret_cast<const bf16x8*>(qp + s2 * (HD / KS));
+    }
   };
   auto build_bias = [&](int head) {
     if (HAS_BIAS) build_bias_lds<TBL>(sB, p.table, p.heads, head, tid, NT);
@@ -582,30 +603,37 @@ window_attention_persist_kernel(AttnParams p, int n_units) {
   const bool late_issuer = STAGGER_KB > 0 && wave >= NQ / 2;
   Unit cur = decode(u_begin);
   int bias_head = cur.head;
-  bf16x8 q_cur[KS], q_nxt[KS];
-  uint32_t tok_cur, tok_nxt = 0;
+  bf16x8 q_cur[NB][KS], q_nxt[NB][KS];
+  uint32_t tok_cur[NB], tok_nxt[NB];
   load_q(cur, q_cur, tok_cur);
   kv_prepare(cur);
 #pragma unroll
   for (int i = 0; i < N_DMA; ++i) kv_issue(i, 0);
   build_bias(bias_head);
 #pragma unroll
-  for (int s2 = 0; s2 < KS; ++s2) q_nxt[s2] = q_cur[s2];
+  for (int n = 0; n < NB; ++n) {
+    tok_nxt[n] = tok_cur[n];
+#pragma unroll
+    for (int s2 = 0; s2 < KS; ++s2) q_nxt[n][s2] = q_cur[n][s2];
+  }
 
-  int set = 1;
-  for (int u = u_begin; u < n_units; u += u_step) {
+  int set = 1, place = u_begin;  // place in the round
+  for (int u = u_begin, u_next; u < n_units; u = u_next) {
     set ^= 1;
-    const bool more = u + u_step < n_units;
-    const Unit nxt = successor(cur);
+    const bool back = ROTATES && place + rotate >= n_wg;
+    place += rotate - (back ? n_wg : 0);
+    u_next = u + rotate + (back ? 0 : n_wg);
+    const bool more = u_next < n_units;
+    const Unit nxt = successor(cur, back);
     if (HAS_BIAS && cur.head != bias_head) {  // workgroup-uniform and rare: the walk crosses into the next head
       __syncthreads();
       build_bias(cur.head);
       bias_head = cur.head;
     }
-    // this wave's loads of unit u (and its bias writes) have landed; only the 4 output stores of the unit before may
+    // this wave's loads of unit u (and its bias writes) have landed; only the output stores of the unit before, four (of a wave of one block two), may
     // still be outstanding (vector memory operations complete in order)
-    static_assert(DB * 2 == 4, "the vmcnt(4) below counts the DB * 2 output stores a wave issues per unit");
     if (u == u_begin) __builtin_amdgcn_s_waitcnt(0x0070);
+    else if (one_block) __builtin_amdgcn_s_waitcnt(0x0072);  // vmcnt(2) lgkmcnt(0)
     else __builtin_amdgcn_s_waitcnt(0x0074);  // vmcnt(4) lgkmcnt(0)
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
@@ -623,44 +651,73 @@ window_attention_persist_kernel(AttnParams p, int n_units) {
     const unsigned char* sV = sK + KVB;
     const bool my = p.use_mask && p.sy > 0 && cur.wy == p.nWy - 1;
     const bool mx = p.use_mask && p.sx > 0 && cur.wx == p.nWx - 1;
-    const WindowLogits<WS_Y, WS_X, HAS_BIAS> logits(sB, qpos, hi, my, mx, p.sy, p.sx);
-    bf16x8 qf[KS];
-#pragma unroll
-    for (int s2 = 0; s2 < KS; ++s2) qf[s2] = q_cur[s2];
     if (!p.q_prescaled) {
 #pragma unroll
-      for (int s2 = 0; s2 < KS; ++s2) {
-        u32x4 w = __builtin_bit_cast(u32x4, q_cur[s2]);
+      for (int n = 0; n < NB; ++n)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) w[e] = pack_bf16x2(bf16_lo(w[e]) * cq, bf16_hi(w[e]) * cq);
-        qf[s2] = __builtin_bit_cast(bf16x8, w);
-      }
+        for (int s2 = 0; s2 < KS; ++s2) {
+          u32x4 w = __builtin_bit_cast(u32x4, q_cur[n][s2]);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) w[e] = pack_bf16x2(bf16_lo(w[e]) * cq, bf16_hi(w[e]) * cq);
+          q_cur[n][s2] = __builtin_bit_cast(bf16x8, w);
+        }
     }
-    auto load_k = [&](int kb, bf16x8 (&f)[KS]) {
-#pragma unroll
-      for (int s2 = 0; s2 < KS; ++s2) f[s2] = *reinterpret_cast<const bf16x8*>(sK + k_off<64>(kb * 32 + l31, s2 * 2 + hi));
-    };
     const uint32_t v_addr = smem_addr + (uint32_t)(set * 2 * KVB + KVB);
-    auto v_step = [&](int step) { return v_addr + (uint32_t)step * 2048u; };
-    const LoadVTransposed<DB, decltype(v_step)> load_v(lane, v_step);
-    auto mid = [&](int kb) {  // the late issuers' share of the next unit's loads, STAGGER_KB key blocks into this unit
+    auto mid = [&](int kb) {  // the late issuers' share of the next unit's loads, STAGGER_KB steps of 32 keys into this unit
       if (STAGGER_KB > 0 && kb == STAGGER_KB && late_issuer && more) {
 #pragma unroll
         for (int i = 0; i < N_DMA; ++i) kv_issue(i, set ^ 1);
         __builtin_amdgcn_sched_barrier(0);
       }
     };
-    f32x16 o[DB];
-    float sum;
-    attention_sweep<NQ, KS, DB, HAS_BIAS>(logits, load_k, load_v, mid, qf, o, sum);
-    // Always DB * 2 stores per wave and unit (the wait at the top of the loop counts them); rows past the window store
-    // their (recomputed, identical) last row again.  (64 bytes per row and instruction through a further
-    // v_permlane16_swap, and the same for the Q loads, measured no faster.)
-    store_attention_rows<DB>(p.out + (uint64_t)tok_cur * (uint32_t)inner + cur.head * HD + hi * 8, o, sum, true);
-    cur = nxt;
-    tok_cur = tok_nxt;
+    uint16_t* const out = p.out + cur.head * HD;
+    // Always the same stores (the wait at the top of the loop counts them); rows past the window store their (recomputed, identical)
+    // last row again.
+    if constexpr (S16) {
+      const unsigned char* const k_lane[2] = {sK + k_off<64>(l15, q4), sK + k_off<64>(l15, 4 + q4)};
+      auto load_k = [&](int kb, int s2) { return *reinterpret_cast<const bf16x8*>(k_lane[s2] + kb * 2048); };  // 16 rows of 128 B
+      const LoadVTransposed16<uint32_t> load_v(lane, v_addr);
+      auto run = [&](auto qn_c) {
+        constexpr int QN = decltype(qn_c)::value;
+        using Logits = WindowLogits16<WS_Y, WS_X, HAS_BIAS>;
+        auto logits_of = [&](int n) { return Logits(sB, qpos[n], q4, my, mx, p.sy, p.sx); };
+        f32x4 o[QN][4];
+        float sum[QN];
+        if constexpr (QN == 2) {
+          const Logits logits[2] = {logits_of(0), logits_of(1)};
+          attention_sweep16<2>(logits, load_k, load_v, mid, q_cur, o, sum);
+        } else {
+          const Logits logits[1] = {logits_of(0)};
+          const bf16x8 q1[1][KS] = {{q_cur[0][0], q_cur[0][1]}};
+          attention_sweep16<1>(logits, load_k, load_v, mid, q1, o, sum);
+        }
 #pragma unroll
-    for (int s2 = 0; s2 < KS; ++s2) q_cur[s2] = q_nxt[s2];
+        for (int n = 0; n < QN; ++n) store_attention_rows16(out + (uint64_t)tok_cur[n] * (uint32_t)inner, o[n], sum[n], q4, true);
+      };
+      if (one_block) run(std::integral_constant<int, 1>{});
+      else run(std::integral_constant<int, 2>{});
+    } else {
+      constexpr int DB = 2;
+      const WindowLogits<WS_Y, WS_X, HAS_BIAS> logits(sB, qpos[0], hi, my, mx, p.sy, p.sx);
+      auto load_k = [&](int kb, bf16x8 (&f)[KS]) {
+#pragma unroll
+        for (int s2 = 0; s2 < KS; ++s2) f[s2] = *reinterpret_cast<const bf16x8*>(sK + k_off<64>(kb * 32 + l31, s2 * 2 + hi));
+      };
+      auto v_step = [&](int step) { return v_addr + (uint32_t)step * 2048u; };
+      const LoadVTransposed<DB, decltype(v_step)> load_v(lane, v_step);
+      f32x16 o[DB];
+      float sum;
+      attention_sweep<NQ, KS, DB, HAS_BIAS>(logits, load_k, load_v, mid, q_cur[0], o, sum);
+      // (64 bytes per row and instruction through a further v_permlane16_swap, and the same for the Q loads, measured no faster.)
+      store_attention_rows<DB>(out + (uint64_t)tok_cur[0] * (uint32_t)inner + hi * 8, o, sum, true);
+    }
+    cur = nxt;
+#pragma unroll
+    for (int n = 0; n < NB; ++n) {
+      tok_cur[n] = tok_nxt[n];
+#pragma unroll
+      for (int s2 = 0; s2 < KS; ++s2) q_cur[n][s2] = q_nxt[n][s2];
+    }
   }
 }
 
@@ -671,8 +728,8 @@ window_attention_persist_kernel(AttnParams p, int n_units) {
 // workgroup's CU nearly empty: six workgroups per CU (33792 tokens x 12 heads of 64 53.4 -> 34.6 us (four per CU: 37.4, eight: 36.8),
 // 2048 x 4 5.9 -> 4.8 us), and for 12x12 windows of which every CU gets one at most (4608 tokens x 4 heads 9.0 -> 7.9 us).  Five waves
 // beside five others do not spread over four SIMDs: 12x12 windows with more units than CUs have one workgroup of the kernel for
-// single units each (260 units 10.8 us, here 14.2; 480 12.7, here 15.6; without a table 288 units 8.4 and 9.5), from two per CU on the
-// persistent kernel (3600 units 65.5 us, here 85).
+// single units each (260 units 10.8 us, here 14.2; 480 12.7, here 15.6; without a table 288 units 8.4 and 9.5), from two and a half per CU on
+// the persistent kernel (3600 units 59 us, here 85).
 // What follows from the lane is worked out per unit: kept across units it filled the registers of a third wave per SIMD.  The bias
 // table holds only the vectors that a key group can start at (build_bias_rows_lds).
 template <int WS_Y, int WS_X, bool HAS_BIAS>
@@ -806,11 +863,14 @@ hipError_t attention_configure_all() {
   if (e != hipSuccess) return e;
   CFGD(12, 12, true) CFGD(12, 12, false) CFGD(16, 16, true) CFGD(16, 16, false)
 #undef CFGD
-#define CFGP(Y, Xx, Bi)                                                                                        \
-  e = hipFuncSetAttribute(reinterpret_cast<const void*>(window_attention_persist_kernel<Y, Xx, Bi>),            \
+#define CFGP(Y, Xx, Bi, S16, Ro)                                                                                      \
+  e = hipFuncSetAttribute(reinterpret_cast<const void*>(window_attention_persist_kernel<Y, Xx, Bi, S16, Ro>),   \
                           hipFuncAttributeMaxDynamicSharedMemorySize, AttnPersistCfg<Y, Xx, Bi>::SMEM);         \
   if (e != hipSuccess) return e;
-  CFGP(8, 8, true) CFGP(8, 8, false) CFGP(12, 12, true) CFGP(12, 12, false) CFGP(16, 16, true) CFGP(16, 16, false)
+  CFGP(8, 8, true, false, false) CFGP(8, 8, false, false, false)
+#define CFGP2(Xx, S16) CFGP(Xx, Xx, true, S16, false) CFGP(Xx, Xx, true, S16, true) CFGP(Xx, Xx, false, S16, false) CFGP(Xx, Xx, false, S16, true)
+  CFGP2(12, false) CFGP2(12, true) CFGP2(16, false)
+#undef CFGP2
 #undef CFGP
   {
     int dev = 0, cus = 0;
@@ -834,6 +894,42 @@ static bool walk_8x8(const AttnParams& p, bool has_bias) {
   return mib <= (has_bias ? 312 : 272) || (has_bias && windows < 4 * (int64_t)g_attn_cus);
 }
 
+// By how many units the workgroups of the persistent form move on from one round to the next.  The windows on the wrapped border of a
+// shifted grid take longer; where the window count and the number of workgroups share so large a factor that a workgroup meets fewer
+// than eight different windows, some of them would meet none but those.  0 -> 37 units, us: 96 x 192 in 12x12 windows, 14 heads, bias
+// 41.3 -> 35.6, four of 48 x 96, 20 heads 48.2 -> 44.1, 128 x 256 in 16x16 windows, 16 heads 73.3 -> 70.0; but 180 x 360 in 12x12 windows
+// (225 different ones), 8 heads 62.7 -> 66.5.  (40, which keeps a window's units on one XCD: 41.3 -> 38.4, 48.2 -> 49.0.)
+static bool wrapped_border(const AttnParams& p) { return p.use_mask && (p.sy > 0 || p.sx > 0); }
+static int persist_rotation(const AttnParams& p) {
+  constexpr int STEP = 37;
+  const int windows = p.B * p.nWy * p.nWx;
+  int a = windows, b = g_attn_cus;
+  while (b) {
+    const int t = a % b;
+    a = b;
+    b = t;
+  }
+  return wrapped_border(p) && windows / a < 8 && g_attn_cus > STEP ? STEP : 0;
+}
+
+// Whether the persistent form takes a window of an odd number of 16-token blocks (12x12) in blocks of 16: not where the mask, whose
+// arithmetic is the same either way, and the start-up weigh too much.  Blocks of 32 -> 16, us: 180 x 360, 8 heads 64.3 -> 59.5, shifted with
+// mask 65.7 -> 63.4, two heads 20.0 -> 19.9, with mask 21.3 -> 22.3; without a table 8 heads 55.9 -> 54.7, with mask 57.8 -> 55.4, three heads with
+// mask 25.6 -> 26.1; 96 x 192, 6 heads without a table 14.4 -> 14.5; 24 x 1200, 8 heads, mask (half of the windows on the border) 31.0 -> 31.7.
+static bool persist_in_16s(const AttnParams& p, bool has_bias, int64_t units) {
+  if (has_bias && !wrapped_border(p)) return true;
+  const int64_t all = (int64_t)p.nWy * p.nWx, inner = (int64_t)(p.nWy - (p.sy > 0)) * (p.nWx - (p.sx > 0));
+  return units >= 6 * (int64_t)g_attn_cus && (!wrapped_border(p) || 4 * inner >= 3 * all);
+}
+
+template <int WS_Y, int WS_X, bool HAS_BIAS, bool S16, bool ROTATES>
+static hipError_t launch_persist(const AttnParams& p, int64_t units, hipStream_t stream) {
+  using P = AttnPersistCfg<WS_Y, WS_X, HAS_BIAS>;
+  hipLaunchKernelGGL((window_attention_persist_kernel<WS_Y, WS_X, HAS_BIAS, S16, ROTATES>), dim3((unsigned)g_attn_cus), dim3(P::NT), P::SMEM, stream, p,
+                     (int)units);
+  return hipGetLastError();
+}
+
 template <int WS_Y, int WS_X, int HD, bool HAS_BIAS>
 static hipError_t launch_attn(const AttnParams& p, hipStream_t stream) {
   using Cfg = AttnCfg<WS_Y, WS_X, HD, HAS_BIAS>;
@@ -851,11 +947,20 @@ static hipError_t launch_attn(const AttnParams& p, hipStream_t stream) {
         return hipGetLastError();
       }
     }
-    if (grid >= 2 * (int64_t)g_attn_cus) {  // enough units for every CU to stream a few: the persistent form
-      using P = AttnPersistCfg<WS_Y, WS_X, HAS_BIAS>;
-      hipLaunchKernelGGL((window_attention_persist_kernel<WS_Y, WS_X, HAS_BIAS>), dim3((unsigned)g_attn_cus), dim3(P::NT), P::SMEM,
-                         stream, p, (int)grid);
-      return hipGetLastError();
+    // Enough units for every CU to stream a few: the persistent form.  12x12 windows from two and a half per CU on (one workgroup per unit ->
+    // persistent, us: 512 units 12.2 -> 12.6, with mask 13.3 -> 14.5; 640 16.5 -> 16.7, with mask 17.9 -> 18.6; 768 19.3 -> 17.3, with mask
+    // 20.5 -> 19.3), without a table and mask from two on (512 10.0 -> 10.5, 640 13.9 -> 13.5).
+    const int64_t cus = g_attn_cus;
+    if (WS_X == 12 ? 2 * grid > ((HAS_BIAS || wrapped_border(p)) ? 5 : 4) * cus : grid >= 2 * cus) {
+      AttnParams q = p;
+      q.rotate = persist_rotation(p);
+      if constexpr (WS_X == 8) return launch_persist<WS_Y, WS_X, HAS_BIAS, false, false>(q, grid, stream);
+      if constexpr (WS_Y * WS_X % 32 != 0) {
+        if (persist_in_16s(p, HAS_BIAS, grid))
+          return q.rotate ? launch_persist<WS_Y, WS_X, HAS_BIAS, true, true>(q, grid, stream) : launch_persist<WS_Y, WS_X, HAS_BIAS, true, false>(q, grid, stream);
+      }
+      if constexpr (WS_X > 8)
+        return q.rotate ? launch_persist<WS_Y, WS_X, HAS_BIAS, false, true>(q, grid, stream) : launch_persist<WS_Y, WS_X, HAS_BIAS, false, false>(q, grid, stream);
     }
     if constexpr (WS_X > 8) {
       using D = AttnDmaCfg<WS_Y, WS_X, HAS_BIAS>;
@@ -874,6 +979,7 @@ hipError_t attention_launch(const void* qkv, void* out, const void* bias_table, 
                             int q_prescaled, int64_t tok_stride, int64_t head_stride, int64_t part_stride,
                             hipStream_t stream) {
   AttnParams p;
+  p.rotate = 0;
   p.q_prescaled = q_prescaled;
   p.tok_stride = tok_stride; p.head_stride = head_stride; p.part_stride = part_stride;
   p.qkv = reinterpret_cast<const uint16_t*>(qkv);

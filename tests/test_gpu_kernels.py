@@ -414,6 +414,25 @@ def test_window_attention_several_workgroups_per_cu(pkg, cuda, case, prescaled):
     test_window_attention_planes_parity(pkg, cuda, case, prescaled)
 
 
+@pytest.mark.parametrize("prescaled", [True, False], ids=["qscaled", "qraw"])
+@pytest.mark.parametrize("case", [
+    (5, 24, 24, 32, 64, 12, 6, True, True, 1.0),      # 640 units, two and a half per CU: the most that have a workgroup each
+    (5, 24, 24, 33, 64, 12, 6, True, True, 1.0),      # 660: persistent, workgroups move on between rounds (20 windows, 5 different ones each)
+    (1, 96, 192, 6, 64, 12, 6, False, True, 1.0),     # 128 windows: every workgroup would meet one
+    (1, 120, 192, 5, 64, 12, 0, True, False, 1.0),    # in blocks of 16: with a table and no mask from the start ...
+    (1, 132, 204, 9, 64, 12, 0, False, False, 1.0),   # ... otherwise from six units per CU on
+    (1, 132, 204, 9, 64, 12, 6, True, True, 1.0),     # 187 windows: no moving on
+    (1, 120, 192, 10, 64, 12, 5, True, True, 1.0),    # 160: both; a border that cuts key groups
+    (1, 132, 204, 9, 64, 12, 6, True, True, 6.0),     # two-pass form
+    (1, 132, 204, 9, 64, 12, 0, False, False, 8.0),
+    (1, 128, 256, 5, 64, 16, 8, True, True, 1.0),     # 16x16, 128 windows, moving on
+], ids=lambda c: f"B{c[0]}_{c[1]}x{c[2]}_h{c[3]}_ws{c[5]}_s{c[6]}_b{int(c[7])}m{int(c[8])}_x{c[9]:g}")
+def test_window_attention_persistent_forms(pkg, cuda, case, prescaled):
+    """12x12 windows in blocks of 16 queries and keys, and workgroups that move on between rounds: same oracle and tolerance as the
+    other head-plane cases."""
+    test_window_attention_planes_parity(pkg, cuda, case, prescaled)
+
+
 STREAM_CASES = [
     # B, H, W, heads, head_dim, ws_y, ws_x, shift_y, shift_x  -- shapes only the streaming kernel takes
     (1, 120, 120, 2, 128, 60, 60, 30, 30),   # the reference's window: 3600 tokens, head_dim 128 (model.py:22-27), shifted

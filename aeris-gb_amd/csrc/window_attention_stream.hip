@@ -27,7 +27,7 @@
 // and row sum was 4 % faster than with them, and two query groups a wave, which halve the LDS reads, 6 % slower.  The 16x16x32 shape
 // does the same FLOP per cycle and LDS bytes per FLOP at a higher clock.  32x32x16 -> 16x16x32, us: 360 x 720 tokens in 60 x 60 windows
 // with 8 x 128 3800 -> 3510, 120 x 120 with 12 x 128 333 -> 319; 20 x 20 windows, 3 x 128 320 -> 301; 8 x 16 182 -> 172; head_dim 64, 60 x 60
-// with 8 heads 2060 -> 1983, 6 x 6 with 6 202 -> 181.  (PV with the two query blocks of a V^T fragment back to back: 1.3 % of that; K Q^T
+// with 8 heads 2060 -> 1983, 6 x 6 with 6 202 -> 181 (before the wider output stores).  (PV with the two query blocks of a V^T fragment back to back: 1.3 % of that; K Q^T
 // over four key blocks in turn, two or two pairs: 0.5 %; reading K fragments 3 or 4 ahead, raised wave priority: nothing.)
 // The query blocks of one (window, head) are placed on the same XCD (blockIdx % 8), so its K / V rows are fetched
 // into that XCD's L2 once and re-read from there by the other query blocks.
@@ -520,15 +520,16 @@ window_attention_stream_kernel(StreamParams p) {
     l[n] += __shfl_xor(l[n], 16, 64);
     l[n] += __shfl_xor(l[n], 32, 64);
     const float inv = __builtin_amdgcn_rcpf(l[n]);
-    if (q_valid[n]) {
-      uint16_t* op = p.out + q_row[n] * inner + head * HD + q4 * 4;
+    uint16_t* op = p.out + q_row[n] * inner + head * HD + 16 * (q4 & 1) + 8 * (q4 >> 1);
+    // 8 consecutive elements a lane: v_permlane16_swap on the pieces of two row blocks.  The address unit takes one lane's piece a cycle
+    // here (neighbouring lanes are different rows), 8 or 16 bytes alike: 4 elements a lane -> 8, us: 360 x 720 tokens, 3 heads x 128 in 8 x 8
+    // windows 156 -> 145, 20 x 20 300 -> 283; 6 x 64, 8 x 16 164 -> 152; two of 60 x 104 in 12 x 8 windows, 3 x 128 11.5 -> 10.8.
 #pragma unroll
-      for (int db = 0; db < DB; ++db) {
-        u32x2 w2;
-        w2.x = pack_bf16x2(o[n][db][0] * inv, o[n][db][1] * inv);
-        w2.y = pack_bf16x2(o[n][db][2] * inv, o[n][db][3] * inv);
-        *reinterpret_cast<u32x2*>(op + db * 16) = w2;
-      }
+    for (int m2 = 0; m2 < DB / 2; ++m2) {
+      const f32x4 a = o[n][2 * m2] * inv, c = o[n][2 * m2 + 1] * inv;
+      const auto rx = __builtin_amdgcn_permlane16_swap(pack_bf16x2(a[0], a[1]), pack_bf16x2(c[0], c[1]), false, false);
+      const auto ry = __builtin_amdgcn_permlane16_swap(pack_bf16x2(a[2], a[3]), pack_bf16x2(c[2], c[3]), false, false);
+      if (q_valid[n]) *reinterpret_cast<u32x4*>(op + m2 * 32) = u32x4{rx[0], ry[0], rx[1], ry[1]};
     }
   }
 }

@@ -751,6 +751,26 @@ def _unhooked(module, cls):
 _AS_DEFINED.update({LocalAERIS: LocalAERIS.forward, InputStage: InputStage.forward})
 
 
+def _stored(part):
+    """Whether the part's weight and bias are what its parameter table holds, not made or chosen at the access."""
+    p = getattr(part, "_parameters", {})
+    return (type(part) in _AS_TORCH and type(p.get("weight")) is nn.Parameter and type(p.get("bias")) in _STORED and
+            ("bias" in p or not ("bias" in part.__dict__ or "bias" in part._buffers)))
+
+
+def _stored_block(block, opts):
+    """Whether looking at a block once tells what every later look would: all that its record holds are stored parameters, of
+    modules of the types that this file makes."""
+    n1, attn, n2, ff = list(block._modules.values())[:4]
+    if type(attn) is not Attention or type(ff) is not (FeedForward if opts.mlp == "swiglu" else Mlp):
+        return False
+    up, down = ("w1", "w2") if opts.mlp == "swiglu" else ("fc1", "fc2")
+    parts = n1, n2, attn._modules.get("to_qkv"), attn._modules.get("wo"), ff._modules.get(up), ff._modules.get(down)
+    # (norms of two types: the call converts one at every look)
+    return (all(map(_stored, parts)) and n1._parameters["weight"].dtype is n2._parameters["weight"].dtype and
+            type(attn._parameters.get("relative_position_bias_table", attn.__dict__.get("relative_position_bias_table", attn))) in _STORED)
+
+
 class CallsAhead:
     """The denoiser calls of one draw, made by the sampler one after the other without anything of the caller's in between: what
     depends on the noise level alone, the modulation vectors, is computed for several levels at a time (the matrices are read
@@ -789,7 +809,7 @@ class CallsAhead:
             self.calls = list(self._block_calls(tok, mods))
         calls = self.calls
         hidden = torch.empty_like(tok) if len(calls) == 1 else tok
-        if any(c.computed or c.config != calls[0].config for c in calls):
+        if any(c.config != calls[0].config for c in calls):
             _run_blocks(self._block_calls(tok, mods), tok, hidden)
         elif calls:
             at = ops.BLOCK_MODULATION
@@ -801,10 +821,13 @@ class CallsAhead:
 
 def calls_ahead(model, levels):
     """``CallsAhead`` for a draw with ``model`` at the noise levels f32 [n], None where each call has to look again at what the
-    model's modules are: a model of another class, one with hooks or methods of the caller's, weights that are computed."""
+    model's modules are: a model of another class, one with hooks or methods of the caller's, weights that are computed or that
+    modules of the caller's return."""
     if not (_unhooked(model, LocalAERIS) and _unhooked(model._modules.get("input_stage"), InputStage) and
             _unhooked(model._modules.get("output_stage"), OutputStage) and _plain(model.output_stage, OutputStage) and
-            all(type(layer) is SwinLayer and _own_blocks(layer) for layer in model.layers) and ops._ordinary_execution()):
+            all(type(layer) is SwinLayer and _own_blocks(layer) and
+                all(_stored_block(block, layer.opts) for block in layer._modules["modulelist"]._modules.values()) for layer in model.layers) and
+            ops._ordinary_execution()):
         return None
     return CallsAhead(model, levels)
 

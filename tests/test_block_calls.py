@@ -1,5 +1,7 @@
 """What the Python side of the blocks hands to the native library, recorded on the CPU: nothing is launched, so the calls
 that must be refused ahead of a launch can be made here."""
+import weakref
+
 import pytest
 import torch
 
@@ -278,8 +280,6 @@ def test_a_modulation_mlp_with_more_in_its_sequence(pkg, calls):
 @pytest.mark.parametrize("whole_model", [False, True])
 def test_computed_weights_live_one_block_at_a_time(pkg, calls, monkeypatch, whole_model):
     """Weights that a parametrisation computes at the access exist for their own block only, not for all blocks of a call."""
-    import weakref
-
     import torch.nn.utils.parametrize as parametrize
     made, most = [], []
 
@@ -517,18 +517,58 @@ def test_a_draw_with_parts_of_the_callers_looks_at_every_call(pkg, calls, monkey
 
 
 def test_a_draw_with_computed_weights_makes_them_at_every_call(pkg, calls, monkeypatch):
-    made = []
+    """... once per call, and holds one block's at a time: as the calls one by one do."""
+    made, most = [], []
 
     class Made(torch.nn.Module):
         def forward(self, w):
-            made.append(1)
-            return w.clone()
+            r = w.clone()
+            made.append(weakref.ref(r))
+            return r
 
     def change(s):
-        torch.nn.utils.parametrize.register_parametrization(s.model.layers[1].modulelist[0][1].wo, "weight", Made())
+        for layer in s.model.layers:
+            torch.nn.utils.parametrize.register_parametrization(layer.modulelist[0][1].wo, "weight", Made())
+        record = pkg._lib.call
+
+        def call(name, *args):
+            record(name, *args)
+            most.append(sum(r() is not None for r in made))
+        monkeypatch.setattr(pkg._lib, "call", call)
         del made[:]
+    names = draw_of(pkg, calls, monkeypatch, change, steps=2, layers=4)
+    assert names.count("aeris_blocks_fwd") == 12 and len(made) == 12 and max(most) == 1, (len(made), most)
+
+
+@pytest.mark.parametrize("part", ["to_qkv", "w2", "norm"])
+def test_a_draw_asks_a_part_of_the_callers_at_every_call(pkg, calls, monkeypatch, part):
+    """A replaced part whose weight is a property (weights that are swapped in, say) may return another one each time."""
+    class Swapped(torch.nn.Module):
+        def __init__(self, weight):
+            super().__init__()
+            self.a, self.b, self.asked = torch.nn.Parameter(weight.detach().clone()), torch.nn.Parameter(weight.detach().clone()), 0
+
+        @property
+        def weight(self):
+            self.asked += 1
+            return self.a if self.asked % 2 else self.b
+
+    parts = []
+
+    def change(s):
+        n1, attn, _, ff = list(s.model.layers[1].modulelist[0])[:4]
+        if part == "norm":
+            parts.append(Swapped(n1.weight))
+            s.model.layers[1].modulelist[0][0] = parts[0]
+        else:
+            owner = attn if part == "to_qkv" else ff
+            parts.append(Swapped(getattr(owner, part).weight))
+            setattr(owner, part, parts[0])
     names = draw_of(pkg, calls, monkeypatch, change, steps=2)
-    assert names.count("aeris_blocks_fwd") == 6 and len(made) >= 3
+    size, at = pkg.ops.BLOCK_RECORD.size, {"norm": 0, "to_qkv": 4, "w2": 10}[part]
+    given = [pkg.ops.BLOCK_RECORD.unpack(c[1][1][size:2 * size])[at] for c in calls if c[0] == "aeris_blocks_fwd"]
+    a, b = parts[0].a.data_ptr(), parts[0].b.data_ptr()
+    assert names.count("aeris_blocks_fwd") == 3 and parts[0].asked == 3 and given == [a, b, a]
 
 
 def test_an_empty_model_draws(pkg, calls, monkeypatch):

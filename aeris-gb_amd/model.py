@@ -749,6 +749,8 @@ def _unhooked(module, cls):
 
 
 _AS_DEFINED.update({LocalAERIS: LocalAERIS.forward, InputStage: InputStage.forward})
+# what a denoiser call asks of its layers, as this file defines it
+_LAYER_METHODS = {k: getattr(SwinLayer, k) for k in ("modulations", "block_calls", "_block_call")}
 
 
 def _stored(part):
@@ -825,9 +827,9 @@ def calls_ahead(model, levels):
     modules of the caller's return."""
     if not (_unhooked(model, LocalAERIS) and _unhooked(model._modules.get("input_stage"), InputStage) and
             _unhooked(model._modules.get("output_stage"), OutputStage) and _plain(model.output_stage, OutputStage) and
-            all(type(layer) is SwinLayer and _own_blocks(layer) and
+            all(type(layer) is SwinLayer and not _LAYER_METHODS.keys() & layer.__dict__.keys() and _own_blocks(layer) and
                 all(_stored_block(block, layer.opts) for block in layer._modules["modulelist"]._modules.values()) for layer in model.layers) and
-            ops._ordinary_execution()):
+            all(getattr(SwinLayer, k) is f for k, f in _LAYER_METHODS.items()) and ops._ordinary_execution()):
         return None
     return CallsAhead(model, levels)
 

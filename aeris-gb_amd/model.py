@@ -743,9 +743,11 @@ class LocalAERIS(nn.Module):
 
 
 def _unhooked(module, cls):
-    """Whether the module is ``cls`` as it is, its forward called by nobody but this file: no forward of its own, no hook."""
+    """Whether the module is ``cls`` as it is, its forward called by nobody but this file: no forward of its own, no hook, not
+    compiled in place (``nn.Module.compile``)."""
     return not (type(module) is not cls or "forward" in module.__dict__ or cls.forward is not _AS_DEFINED[cls] or module._forward_hooks or
-                module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks)
+                module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks or
+                module._compiled_call_impl is not None)
 
 
 _AS_DEFINED.update({LocalAERIS: LocalAERIS.forward, InputStage: InputStage.forward})

@@ -485,7 +485,8 @@ def test_a_draw_computes_the_modulation_of_several_levels_at_once(pkg, calls, mo
 
 
 @pytest.mark.parametrize("what", ["model_hook", "input_hook", "output_hook", "modulation_hook", "core", "model_class", "model_forward",
-                                  "sampler_class", "sampler_method", "advance", "modulations", "block_calls", "_block_call", "layer_class"])
+                                  "sampler_class", "sampler_method", "advance", "modulations", "block_calls", "_block_call", "layer_class",
+                                  "model_compiled", "input_compiled"])
 def test_a_draw_with_parts_of_the_callers_looks_at_every_call(pkg, calls, monkeypatch, what):
     seen = []
 
@@ -506,6 +507,9 @@ def test_a_draw_with_parts_of_the_callers_looks_at_every_call(pkg, calls, monkey
             m.__class__ = type("Mine", (pkg.LocalAERIS,), {"forward": lambda self, *a, **kw: seen.append(1) or pkg.LocalAERIS.forward(self, *a, **kw)})
         elif what == "model_forward":
             m.forward = lambda *a, **kw: seen.append(1) or pkg.LocalAERIS.forward(m, *a, **kw)
+        elif what in ("model_compiled", "input_compiled"):  # (a compiler that calls what it is given)
+            monkeypatch.setattr(torch, "compile", lambda f, *a, **kw: lambda *a, **kw: seen.append(1) or f(*a, **kw))
+            (m if what == "model_compiled" else m.input_stage).compile()
         elif what in ("modulations", "block_calls", "_block_call"):
             layer, plain = m.layers[0], getattr(pkg.SwinLayer, what)
             setattr(layer, what, lambda *a: seen.append(1) or plain(layer, *a))

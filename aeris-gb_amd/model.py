@@ -762,16 +762,21 @@ def _stored(part):
             ("bias" in p or not ("bias" in part.__dict__ or "bias" in part._buffers)))
 
 
-def _stored_block(block, opts):
-    """Whether looking at a block once tells what every later look would: all that its record holds are stored parameters, of
-    modules of the types that this file makes."""
+def _record_parts(block, opts):
+    """The modules whose parameters a block's record holds, None in the place of those that are not where this file puts them."""
     n1, attn, n2, ff = list(block._modules.values())[:4]
+    up, down = ("w1", "w2") if opts.mlp == "swiglu" else ("fc1", "fc2")
+    return n1, attn, n2, ff, attn._modules.get("to_qkv"), attn._modules.get("wo"), ff._modules.get(up), ff._modules.get(down)
+
+
+def _stored_block(block, opts):
+    """Whether looking at a block once tells what every later look would, as long as its parameters stay where they are: all that
+    its record holds are stored parameters, of modules of the types that this file makes."""
+    n1, attn, n2, ff, *linears = _record_parts(block, opts)
     if type(attn) is not Attention or type(ff) is not (FeedForward if opts.mlp == "swiglu" else Mlp):
         return False
-    up, down = ("w1", "w2") if opts.mlp == "swiglu" else ("fc1", "fc2")
-    parts = n1, n2, attn._modules.get("to_qkv"), attn._modules.get("wo"), ff._modules.get(up), ff._modules.get(down)
     # (norms of two types: the call converts one at every look)
-    return (all(map(_stored, parts)) and n1._parameters["weight"].dtype is n2._parameters["weight"].dtype and
+    return (all(map(_stored, (n1, n2, *linears))) and n1._parameters["weight"].dtype is n2._parameters["weight"].dtype and
             type(attn._parameters.get("relative_position_bias_table", attn.__dict__.get("relative_position_bias_table", attn))) in _STORED)
 
 
@@ -780,6 +785,10 @@ class CallsAhead:
     depends on the noise level alone, the modulation vectors, is computed for several levels at a time (the matrices are read
     once for all of them, and a level that ends one step and begins the next is computed once), and what the blocks' modules
     hold is looked up once.  Same kernels on the same values as ``LocalAERIS.forward``: the same bits.  Lives as long as the draw.
+
+    Another thread may replace a parameter or move its storage meanwhile: each call asks whether the parameters are still the
+    ones, and where they were, that the blocks' records name, and from the first for which they are not on every call looks for
+    itself.  (The 24 parameters of four blocks: 5.5 us of host time; making their records: 54.)
     """
     LEVELS = 8  # levels at a time: the rows that the modulation kernel takes in one pass over a matrix
 
@@ -789,6 +798,10 @@ class CallsAhead:
         self.model, self.levels = model, levels
         self.layers = [(layer, half if i % 2 == 1 else (0, 0), layer.modulations()) for i, layer in enumerate(layers)]
         self.first, self.vectors, self.calls = 0, None, None
+        self.sublayers = sum(layer.sublayers for layer in layers)  # (in place but for a model of one block, as in the forward)
+        self.blocks = [(block, layer.opts) for layer in layers for block in layer._modules["modulelist"]._modules.values()]
+        tables = {id(part._parameters): part._parameters for block in self.blocks for part in _record_parts(*block)}
+        self.held = [(table, name, v, v.data_ptr()) for table in tables.values() for name, v in table.items() if v is not None]
 
     def _modulations(self, i, dim):
         """The modulation vectors of level i, f32 [1, N] each: those of the blocks, then the output stage's."""
@@ -797,6 +810,11 @@ class CallsAhead:
             modules = [m for _, _, own in self.layers for m in own]
             self.first, self.vectors = i, _modulation_vectors(modules, t, [_mlp_params(self.model.output_stage.modulation)])
         return [v[i - self.first:i - self.first + 1] for v in self.vectors]
+
+    def _as_held(self):
+        """Whether the blocks' parameters, and the bias tables in the one-kernel attention's form, are where the records say."""
+        return (all(table.get(name) is v and v.data_ptr() == at for table, name, v, at in self.held) and
+                all(not call.fused or block._modules["1"]._bias4() is call.keep[1] for (block, _), call in zip(self.blocks, self.calls or ())))
 
     def _block_calls(self, tok, mods):
         k = 0
@@ -809,13 +827,15 @@ class CallsAhead:
         model = self.model
         tok = model.input_stage._tokens(x, model.residual_dtype, cond, x_div)
         mods = self._modulations(i, tok.shape[-1])
-        if self.calls is None:
+        if self.calls is None and self.held:
             self.calls = list(self._block_calls(tok, mods))
+        if not self._as_held():
+            self.calls, self.held = None, []
         calls = self.calls
-        hidden = torch.empty_like(tok) if len(calls) == 1 else tok
-        if any(c.config != calls[0].config for c in calls):
+        hidden = torch.empty_like(tok) if self.sublayers == 1 else tok
+        if calls is None or any(c.config != calls[0].config for c in calls):
             _run_blocks(self._block_calls(tok, mods), tok, hidden)
-        elif calls:
+        else:
             at = ops.BLOCK_MODULATION
             records = [c.record for c in calls] if len(mods) == 1 else [
                 c.record[:at] + struct.pack("=Q", m.data_ptr()) + c.record[at + 8:] for c, m in zip(calls, mods)]

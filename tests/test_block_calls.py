@@ -581,6 +581,40 @@ def test_a_draw_asks_a_part_of_the_callers_at_every_call(pkg, calls, monkeypatch
     assert names.count("aeris_blocks_fwd") == 3 and parts[0].asked == 3 and given == [a, b, a]
 
 
+@pytest.mark.parametrize("window", [8, 16])  # the attention kernel's table; the one-kernel attention's
+@pytest.mark.parametrize("what", ["storage", "parameter", "table"])
+def test_a_draw_sees_parameters_that_move(pkg, calls, monkeypatch, window, what):
+    """Another thread may replace a parameter or its storage while a draw runs: the calls that follow take it where it is."""
+    torch.manual_seed(1)
+    model = pkg.LocalAERIS(None, 4, 256, 64, 512, (window, window), (16, 32), n_layers=4, model_in_channels=10, model_out_channels=4,
+                           preset="spec", mod_ways=2)
+    attn = model.layers[1].modulelist[0][1]
+    given, record = [], pkg._lib.call
+
+    def where():
+        table = attn.relative_position_bias_table
+        return attn.wo.weight.data_ptr(), table.data_ptr() if window == 8 else 0, attn._bias4().data_ptr() if window == 16 else 0
+
+    def call(name, *args):
+        record(name, *args)
+        if name != "aeris_blocks_fwd":
+            return
+        r = pkg.ops.BLOCK_RECORD.unpack(args[1][-pkg.ops.BLOCK_RECORD.size:])
+        given.append((r[6], r[12], r[13]) == where())
+        if len(given) in (1, 3):  # between the calls of the draw
+            if what == "table":
+                with torch.no_grad():
+                    attn.relative_position_bias_table = torch.nn.Parameter(attn.relative_position_bias_table + 1)
+            elif what == "parameter":
+                attn.wo.weight = torch.nn.Parameter(attn.wo.weight.detach().clone())
+            else:
+                attn.wo.weight.data = attn.wo.weight.detach().clone()
+    monkeypatch.setattr(pkg._lib, "call", call)
+    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: None)
+    pkg.TrigFlowSampler(model, n_steps=3, device="cpu").sample(torch.randn(1, 512, 6), torch.randn(1, 512, 4))
+    assert given == [True] * 5
+
+
 def test_an_empty_model_draws(pkg, calls, monkeypatch):
     names = draw_of(pkg, calls, monkeypatch, steps=2, layers=0)
     assert names.count("aeris_output_stage_fwd") == 3 and "aeris_blocks_fwd" not in names

@@ -19,7 +19,8 @@ registers, so two properties that it guarantees for its own instructions have to
    complete in order, so "at most N outstanding" covers everything older than the N youngest).  That only holds if N
    vector memory instructions really follow the loads on every path: the N youngest ones before the wait must be
    stores in the wait's own basic block (no label in between), so that no path can skip them.  (Checked wherever a
-   store is among them; the counted waits of the k-loops stand between loads only.)
+   store is among them; the counted waits of the k-loops stand between loads only, and those at the head of the persistent
+   attention kernel's loop in a block of their own: their counts are worked out from what the stores' functions issue.)
 
     python aeris-gb_amd/asm_check.py file.s [...]      # exit status 1 if a rule is broken
 

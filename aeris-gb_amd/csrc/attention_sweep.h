@@ -318,15 +318,16 @@ __device__ __forceinline__ void attention_sweep(const Logits& lg, const LoadK& l
 // Normalise and store the lane's output row: o[db][4g + i] = O[query][32 db + 8 g + 4 hi + i].  The two lanes of a
 // query (l31 and l31 + 32) each hold half of every 16-byte piece of the row; v_permlane32_swap on the pieces 2m and
 // 2m + 1 gives the lower lane all of piece 2m and the upper lane all of piece 2m + 1: 32 contiguous bytes per row and
-// instruction.  `op` points at element hi * 8 of the row's head slice.  DB * 2 store instructions, issued by every
-// lane for which `valid` holds.
+// instruction.  `op` points at element hi * 8 of the row's head slice.  attention_rows_stores(DB) store
+// instructions, issued by every lane for which `valid` holds.
+constexpr int attention_rows_stores(int db) { return db * 2; }
 template <int DB>
 __device__ __forceinline__ void store_attention_rows(uint16_t* op, const f32x16 (&o)[DB], float sum, bool valid) {
   const float inv = __builtin_amdgcn_rcpf(sum);
 #pragma unroll
   for (int db = 0; db < DB; ++db)
 #pragma unroll
-    for (int m = 0; m < 2; ++m) {
+    for (int m = 0; m < attention_rows_stores(1); ++m) {
       const int g0 = 2 * m, g1 = 2 * m + 1;
       const uint32_t x0 = pack_bf16x2(o[db][g0 * 4] * inv, o[db][g0 * 4 + 1] * inv);
       const uint32_t x1 = pack_bf16x2(o[db][g0 * 4 + 2] * inv, o[db][g0 * 4 + 3] * inv);
@@ -584,11 +585,13 @@ __device__ __forceinline__ void attention_sweep16(const Logits (&lg)[QN], const 
 
 // Normalise and store a query block's rows: v_permlane16_swap on the pieces of row blocks 2m and 2m + 1 leaves lane (l15, q4) with 8
 // consecutive elements, 32 m + 16 (q4 & 1) + 8 (q4 >> 1) .., of row l15: 64 contiguous bytes per row and instruction.  `op` points at the
-// row's head slice.  Two store instructions, issued by every lane for which `valid` holds.
+// row's head slice.  ATTENTION_ROWS16_STORES store instructions, issued by every lane for which `valid` holds.
+constexpr int ATTENTION_ROWS16_STORES = 2;
 __device__ __forceinline__ void store_attention_rows16(uint16_t* op, const f32x4 (&o)[4], float sum, int q4, bool valid) {
   const float inv = __builtin_amdgcn_rcpf(sum);
+  static_assert(ATTENTION_ROWS16_STORES * 32 == 64, "head_dim 64 in pieces of 32 elements");
 #pragma unroll
-  for (int m = 0; m < 2; ++m) {
+  for (int m = 0; m < ATTENTION_ROWS16_STORES; ++m) {
     const f32x4 a = o[2 * m] * inv, b = o[2 * m + 1] * inv;
     const auto rx = __builtin_amdgcn_permlane16_swap(pack_bf16x2(a[0], a[1]), pack_bf16x2(b[0], b[1]), false, false);
     const auto ry = __builtin_amdgcn_permlane16_swap(pack_bf16x2(a[2], a[3]), pack_bf16x2(b[2], b[3]), false, false);

@@ -389,7 +389,7 @@ __global__ void __launch_bounds__(QA_NT) qkv_window_attention_kernel(QkvAttnPara
     // pending when the k-loop is entered again (see gemm_persistent.hip).
     // The 4 output stores (the last vector memory operations of this phase; they write no register) drain under the
     // next unit's first slots, whose first counted wait covers them.
-    static_assert(DB * 2 == 4, "the wait below counts the output stores");
+    static_assert(attention_rows_stores(DB) == 4, "the wait below counts the output stores");
     __builtin_amdgcn_s_waitcnt(WAIT_VM4_LGKM0);
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);

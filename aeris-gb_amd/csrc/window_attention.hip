@@ -630,11 +630,13 @@ window_attention_persist_kernel(AttnParams p, int n_units) {
       build_bias(cur.head);
       bias_head = cur.head;
     }
-    // this wave's loads of unit u (and its bias writes) have landed; only the output stores of the unit before, four (of a wave of one block two), may
-    // still be outstanding (vector memory operations complete in order)
+    // this wave's loads of unit u (and its bias writes) have landed; only the output stores of the unit before may still be outstanding
+    // (vector memory operations complete in order): those of both query blocks, or of the one that the wave has
+    constexpr int BLOCK_STORES = S16 ? ATTENTION_ROWS16_STORES : attention_rows_stores(HD / 32);
+    static_assert(NB * BLOCK_STORES < 16, "bits 3:0 of the immediate: vmcnt; its other bits: lgkmcnt(0)");
     if (u == u_begin) __builtin_amdgcn_s_waitcnt(0x0070);
-    else if (one_block) __builtin_amdgcn_s_waitcnt(0x0072);  // vmcnt(2) lgkmcnt(0)
-    else __builtin_amdgcn_s_waitcnt(0x0074);  // vmcnt(4) lgkmcnt(0)
+    else if (one_block) __builtin_amdgcn_s_waitcnt(0x0070 | BLOCK_STORES);
+    else __builtin_amdgcn_s_waitcnt(0x0070 | (NB * BLOCK_STORES));
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
     if (more) {  // Q first: a later wait for it then does not have to wait for the K / V loads behind it
@@ -697,7 +699,7 @@ window_attention_persist_kernel(AttnParams p, int n_units) {
       if (one_block) run(std::integral_constant<int, 1>{});
       else run(std::integral_constant<int, 2>{});
     } else {
-      constexpr int DB = 2;
+      constexpr int DB = HD / 32;
       const WindowLogits<WS_Y, WS_X, HAS_BIAS> logits(sB, qpos[0], hi, my, mx, p.sy, p.sx);
       auto load_k = [&](int kb, bf16x8 (&f)[KS]) {
 #pragma unroll

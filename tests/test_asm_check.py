@@ -2,6 +2,7 @@
 hand-written snippets: each rule fires on the pattern it is for and stays quiet on the legal neighbours of that pattern."""
 import importlib.util
 import os
+import re
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 spec = importlib.util.spec_from_file_location("aeris_asm_check", os.path.join(ROOT, "aeris-gb_amd", "asm_check.py"))
@@ -115,3 +116,10 @@ def test_counted_wait_behind_stores():
     assert len(problems) == 1 and "not preceded by 4 stores" in problems[0]
     # the main loops' counted waits (no lgkmcnt(0) ... or vmcnt(0)) are not meant
     assert asm_check.check_text(kernel(["buffer_load_dwordx4 v2, s[44:47], s7 offen lds", "s_waitcnt vmcnt(0) lgkmcnt(0)"]))[0] == []
+
+
+def test_counted_waits_of_the_persistent_attention_follow_the_stores():
+    """A wait that leaves stores outstanding takes their number from the function that issues them, not from a literal."""
+    source = open(os.path.join(ROOT, "aeris-gb_amd", "csrc", "window_attention.hip")).read()
+    assert not re.findall(r"s_waitcnt\(0x007[1-9A-Fa-f]\)", source)
+    assert len(re.findall(r"s_waitcnt\(0x0070 \| \(?(?:NB \* )?BLOCK_STORES\)", source)) == 2

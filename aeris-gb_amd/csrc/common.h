@@ -157,7 +157,7 @@ __device__ __forceinline__ float gelu_erf_bf16_f(float x) {
 // erf-GELU for results that are rounded to bf16, for the problems whose epilogue is a sizeable part of a tile:
 // GELU(x) = max(x, 0) - a * 2^P(a), a = |x|, P the degree-4 polynomial for which 2^P is the minimax approximation of
 // 1 - Phi(a): log2 of the normal tail is nearly a parabola, so four coefficients do for it what a polynomial for Phi itself
-// needs seven for.  In fp32 against erfc in fp64 on [-12, 12]: at most 6.9e-6 |x| and 2.1e-5 absolute, 7.4e-6 of the 2-norm on
+// needs seven for.  In fp32 against erfc in fp64 on [-12, 12]: at most 6.9e-6 |x| and 2.2e-5 absolute, 7.4e-6 of the 2-norm on
 // normal inputs (the degree-6 polynomial in x^2 with clamps that stood here: 2.0e-4 |x| down to
 // -3.5, 8e-4 absolute below, 3.3e-5).  From 12 on a is held at 12, where 2^P = 9e-21: -inf goes to -1e-19, +inf stays; both
 // min and max hand NaN on.

@@ -172,7 +172,7 @@ int aeris_output_stage_noalloc_fwd(const void* x, int x_dtype, const void* gamma
  * at model.py:400-401.  Requires K % 64 == 0.
  * AERIS_ACT_GELU is the erf form, evaluated to the accuracy of the output type.  bf16 C where the problem has a chip's
  * worth of 256x256 tiles (M >= 256 and at least 256 tiles, N a multiple of 256 or >= 1024): the normal
- * tail as 2 to a polynomial, |error| <= 6.9e-6 |x| and 2.1e-5 absolute (a hundredth of half a bf16 ulp for x >= 0); -1e-19
+ * tail as 2 to a polynomial, |error| <= 6.9e-6 |x| and 2.2e-5 absolute (a hundredth of half a bf16 ulp for x >= 0); -1e-19
  * from -12 down.  Every other case: erf to 1.5e-7 absolute (f32 C), or GELU to
  * 4.1e-7 |x| before the rounding (bf16 C).  The forms agree to within one bf16 ulp of the result for x >= -1; all rows of a call
  * take the same one, and which one that is depends on the shape and alignment only, never on the data. */

@@ -435,13 +435,13 @@ namespace {
 // size too long, 24 576 x 192 x 192: 10.8 us against 8.7.)
 //
 // Tiles of 192 columns take 0.85-0.95 of the time of those of 256 for three quarters of the work, so they pay only where they need
-// no more rounds: N just over a multiple of 256, or a last round that is mostly empty.  256 -> 192 columns, us:
-//   256 rows   8192 x 1536 x 1536 (f32 C and residual) 45.1 -> 42.6, x 6144 126 -> 119; 9000 x 1152 x 1152 34.6 -> 32.2; 14400 x 1536 x 1536
-//              82.1 -> 76.3; 30000 x 576 x 576 43.8 -> 39.8; 10000 x 2304 x 768 (planes) 39.7 -> 37.1; 51840 x 320 x 1280 (bf16) 57.6 -> 53.3
-//   128 rows   12480 x 384 x 384 (f32) 14.6 -> 12.4, x 1088 22.3 -> 20.0
-//   more rounds: 64800 x 1536 x 512 97.5 -> 106, 64800 x 512 x 2048 (bf16) 118 -> 140, 518400 x 1536 x 1536 (f32) 2402 -> 2595
-// A bf16 residual is read in 64-byte pieces there, which short products wait for (51840 x 320 x 320 25.3 -> 27.1, 128 rows 32768 x 192 x
-// 768 17.4 -> 18.5), and short plain ones in tiles of 128 rows gain nothing (32768 x 576 x 192 17.7 -> 18.3).
+// no more rounds: N just over a multiple of 256, or a last round that is mostly empty.  256 -> 192 columns of the same height, us:
+//   256 rows   8192 x 1536 x 1536 (f32 C and residual) 42.4 -> 41.3, x 6144 117.3 -> 114.8; 9000 x 1152 x 1152 33.5 -> 31.4; 14400 x 1536 x 1536
+//              82.0 -> 70.7; 10000 x 2304 x 768 (bf16) 38.1 -> 32.1; 51840 x 320 x 1280 (bf16 residual) 53.0 -> 49.4; 32768 x 576 x 192 (bf16)
+//              16.8 -> 15.2
+//   128 rows   12480 x 384 x 384 (f32) 13.3 -> 12.6, x 1088 21.4 -> 20.1, 30000 x 576 x 576 38.5 -> 36.5 (256 rows: 43.1 -> 37.6)
+//   more rounds: 64800 x 1536 x 512 87.6 -> 101, 64800 x 512 x 2048 (bf16 residual) 113 -> 135
+// A bf16 residual is read in 64-byte pieces there, which short products wait for (51840 x 320 x 320 24.2 -> 25.0).
 enum Kind { TILE64, PERSISTENT128, PERSISTENT256, PERSISTENT128_192, PERSISTENT256_192 };
 
 struct Shape {
@@ -602,8 +602,13 @@ hipError_t gemm_launch(const void* A, const void* W, void* C, const void* bias, 
     rest.M = M - head.M;
     float t_rest = 0.f;
     const Kind rest_kind = best_kind(rest, &t_rest);
-    // (against tiles of 192 the estimate of two launches is too low: 14400 x 1536 x 1536 82.1 us, x 6144 253, in one 76.3 and 247)
-    if (estimate_us(PERSISTENT256, head) + t_rest < (kind == PERSISTENT256_192 ? 0.90f : 0.97f) * one) {
+    // Against one launch of 192-column tiles the sum of two estimates is too low, by 6 us at K = 1536 and 14 to 24 at K = 6144, while the
+    // one launch, whose CUs are never all busy to the end, takes 0.87 to 0.98 of its own.  f32 C and residual, N = 1536, us, one launch of
+    // 192 / two: K = 1536, M = 12544 65.7 / 70.2, 13312 67.1 / 74.1, 14400 70.7 / 78.2, 14848 71.4 / 78.5; K = 6144, M = 12544 233.7 /
+    // 226.1, 13312 232.8 / 233.5, 14400 244.6 / 239.4, 14848 247.7 / 239.1.  bf16, plain: 8192 x 2304 x 1024 38.4 / 39.7, 14400 x 1536 x
+    // 3072 100.6 / 109.0.
+    const float two = estimate_us(PERSISTENT256, head) + t_rest;
+    if (kind == PERSISTENT256_192 ? two + 3.0f < 0.88f * one : two < 0.97f * one) {
       const hipError_t e = launch_kind(PERSISTENT256, rows_of(p, 0, head.M), stream);
       return e != hipSuccess ? e : launch_kind(rest_kind, rows_of(p, head.M, rest.M), stream);
     }

@@ -3,6 +3,7 @@
 Tolerances: index maps bit-exact; bf16 results within relative L2 <= 1e-2 of the fp32 oracle
 (most kernels are far tighter, each bound is written at its assert).
 """
+import ctypes
 import math
 
 import numpy as np
@@ -177,6 +178,26 @@ def test_gemm_tile_edges(pkg, cuda, case):
 def test_gemm_tiles_of_192_columns(pkg, cuda, case):
     """Shapes that need no more rounds of 192-column tiles than of 256, at the edges of those tiles; errors as for the others."""
     test_gemm_tile_edges(pkg, cuda, case)
+
+
+@pytest.mark.parametrize("M,N,K,dtype,launches", [
+    (14400, 1536, 1536, torch.float32, 1),   # 192-column tiles, 70.7 us against 78.2
+    (12800, 1536, 1536, torch.float32, 1),   # 65.9 against 70.5
+    (14400, 1536, 6144, torch.float32, 2),   # 239.4 us against 244.6
+    (14400, 4608, 1536, None, 2),            # 147 against 164
+    (8192, 1536, 1536, torch.float32, 1),    # no full round
+])
+def test_gemm_rows_are_split_where_that_is_faster(pkg, cuda, M, N, K, dtype, launches):
+    """One launch or two (the rows beyond the last full round of 256 x 256 tiles in one of their own), whichever measured faster
+    at these shapes: counted as the nodes of a captured graph, which is not replayed."""
+    a, w = torch.zeros(M, K, dtype=torch.bfloat16, device=cuda), torch.zeros(N, K, dtype=torch.bfloat16, device=cuda)
+    out = torch.zeros(M, N, dtype=dtype or torch.bfloat16, device=cuda)
+    graph, nodes = torch.cuda.CUDAGraph(keep_graph=True), ctypes.c_size_t()
+    with torch.cuda.graph(graph):
+        pkg.ops.gemm(a, w, None, residual=out if dtype else None, out=out)
+    # (the HIP runtime that the library is linked with, torch's)
+    assert pkg._lib.lib().hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(nodes)) == 0
+    assert nodes.value == launches
 
 
 @pytest.mark.parametrize("case", [

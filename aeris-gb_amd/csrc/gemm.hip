@@ -366,6 +366,9 @@ hipError_t launch_tile(const GemmParams& p0, hipStream_t stream) {
   return hipGetLastError();
 }
 
+// SiLU has tiles of 64 x 64 below 128 of 128 x 128 only, fewer than 512: never the two-stage ones (launch_kind)
+constexpr bool takes_silu(int bm, int stages) { return !(bm == 64 && stages == 2); }
+
 template <int BM, int BN, int STAGES, bool VEC>
 hipError_t launch_tile_act(const GemmParams& p, hipStream_t stream) {
 #define GO(A)                                                                              \
@@ -378,7 +381,9 @@ hipError_t launch_tile_act(const GemmParams& p, hipStream_t stream) {
       return launch_tile<BM, BN, STAGES, BM <= 64 ? AERIS_ACT_GELU : GEMM_ACT_GELU_ERF, false, VEC>(p, stream);
     case GEMM_ACT_GELU_ERF: return launch_tile<BM, BN, STAGES, GEMM_ACT_GELU_ERF, false, VEC>(p, stream);
     case AERIS_ACT_SWIGLU: GO(AERIS_ACT_SWIGLU);
-    case AERIS_ACT_SILU: GO(AERIS_ACT_SILU);
+    case AERIS_ACT_SILU:
+      if constexpr (takes_silu(BM, STAGES)) GO(AERIS_ACT_SILU);
+      return hipErrorInvalidValue;
     default: GO(AERIS_ACT_NONE);
   }
 #undef GO
@@ -401,7 +406,9 @@ hipError_t configure_tile() {
   if (e == hipSuccess) e = configure_tile_kernel<BM, BN, STAGES, VEC, BM <= 64 ? AERIS_ACT_GELU : GEMM_ACT_GELU_ERF, false>();
   if (e == hipSuccess) e = configure_tile_kernel<BM, BN, STAGES, VEC, GEMM_ACT_GELU_ERF, false>();
   if (e == hipSuccess) e = configure_tile_act<BM, BN, STAGES, VEC, AERIS_ACT_SWIGLU>();
-  if (e == hipSuccess) e = configure_tile_act<BM, BN, STAGES, VEC, AERIS_ACT_SILU>();
+  if constexpr (takes_silu(BM, STAGES)) {
+    if (e == hipSuccess) e = configure_tile_act<BM, BN, STAGES, VEC, AERIS_ACT_SILU>();
+  }
   return e;
 }
 }  // namespace
@@ -447,7 +454,7 @@ enum Kind { TILE64, PERSISTENT128, PERSISTENT256, PERSISTENT128_192, PERSISTENT2
 struct Shape {
   int64_t M;
   int N, KT, act;
-  bool f32, res, w192;  // w192: tiles of 192 columns take the problem
+  bool f32, res, w192[2];  // w192: tiles of 128 / 256 rows x 192 columns take the problem
 };
 
 float epilogue_us(const Shape& s) {  // of a 256 x 256 tile
@@ -470,7 +477,7 @@ float estimate_us(Kind kind, const Shape& s) {
     const bool tall = kind == PERSISTENT256_192;
     const int bm = tall ? 256 : 128;
     auto rounds = [&](int bn) { return ((tiles_of(s, bm, bn) + 7) / 8 + 31) / 32; };
-    if (!s.w192 || rounds(192) > rounds(256) || !(s.f32 || (tall && (!s.res || s.KT >= 16)))) return 1e30f;
+    if (!s.w192[tall] || rounds(192) > rounds(256) || (s.res && !s.f32 && s.KT < 16)) return 1e30f;
     return (s.f32 ? (tall ? 0.93f : 0.88f) : 0.95f) * estimate_us(tall ? PERSISTENT256 : PERSISTENT128, s);
   }
   const int bm = kind == PERSISTENT256 ? 256 : 128;
@@ -490,7 +497,9 @@ Kind best_kind(const Shape& s, float* us) {
   return best;
 }
 
-Shape shape_of(const GemmParams& p, int act) { return {p.M, p.N, p.K / BK, act, p.c_dtype == AERIS_F32, p.residual != nullptr, gemm_persistent_takes_192(p)}; }
+Shape shape_of(const GemmParams& p, int act) {
+  return {p.M, p.N, p.K / BK, act, p.c_dtype == AERIS_F32, p.residual != nullptr, {gemm_persistent_takes_192(p, 128), gemm_persistent_takes_192(p, 256)}};
+}
 
 hipError_t launch_kind(Kind kind, const GemmParams& p, hipStream_t stream) {
   if (kind == TILE64) {

@@ -69,7 +69,7 @@ bool gemm_gelu_by_polynomial(const GemmParams& p);
 // persistent kernel (gemm_persistent.hip), tiles of tile_height (128 or 256) rows x tile_width (256, or 192 where
 // gemm_persistent_takes_192) columns; needs N % 4 == 0 and ldc % 4 == 0
 hipError_t gemm_persistent_configure();
-bool gemm_persistent_takes_192(const GemmParams& p);
+bool gemm_persistent_takes_192(const GemmParams& p, int tile_height);
 hipError_t gemm_persistent_launch(const GemmParams& p, int tile_height, int tile_width, hipStream_t stream);
 
 }  // namespace aeris

@@ -59,6 +59,7 @@ __global__ void __launch_bounds__(NT) gemm_bf16_nt_persistent_kernel(GemmParams 
   constexpr int A_LD = BM / 64;             // load instructions of a wave per k-tile of A (8 rows each); 4 for W
   constexpr int B_OFF = A_STAGES * A_BYTES;
   static_assert(!(PLAIN && RES_BF16) && !(OUT_F32 && RES_BF16), "RES_BF16 is a non-plain bf16-output form");
+  static_assert(BN == 256 || BM == 256 || RES_F32, "128 x 192 tiles: f32 C with an f32 residual alone");
   static_assert(!RES_F32 || (OUT_F32 && !PLAIN && !RES_BF16), "RES_F32 is a non-plain f32-output form");
   GemmParams p = p_in;
   if (RES_F32) p.res_dtype = AERIS_F32;
@@ -455,7 +456,7 @@ __global__ void __launch_bounds__(NT) gemm_bf16_nt_persistent_kernel(GemmParams 
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        if (u == 0 && UNITS > 1) load_res(1);  // once the first unit's accumulators are staged and their registers free
+        if (u == 0) load_res(1);  // once the first unit's accumulators are staged and their registers free
         f32x4 g0 = {1.f, 1.f, 1.f, 1.f}, g1 = g0;
         const int n_g0 = n < N - 4 ? n : N - 4, n_g1 = n + 4 < N - 4 ? n + 4 : N - 4;
         if (gate_tile) {
@@ -922,11 +923,13 @@ hipError_t configure_all() {
   if (e == hipSuccess) e = configure_act<BM, AERIS_ACT_SWIGLU>();
   if (e == hipSuccess) e = configure_one<BM, AERIS_ACT_NONE, true, false, false, true>();
   if (e == hipSuccess) e = configure_one<BM, GEMM_ACT_GELU_ERF, false, true>();
-  if (e == hipSuccess) e = configure_one<BM, AERIS_ACT_NONE, false, true, false, false, 192>();
-  if (e == hipSuccess) e = configure_one<BM, AERIS_ACT_GELU, false, true, false, false, 192>();
-  if (e == hipSuccess) e = configure_one<BM, GEMM_ACT_GELU_ERF, false, true, false, false, 192>();
-  if (e == hipSuccess) e = configure_one<BM, AERIS_ACT_NONE, false, false, true, false, 192>();
   if (e == hipSuccess) e = configure_one<BM, AERIS_ACT_NONE, true, false, false, true, 192>();
+  if constexpr (BM == 256) {
+    if (e == hipSuccess) e = configure_one<BM, AERIS_ACT_NONE, false, true, false, false, 192>();
+    if (e == hipSuccess) e = configure_one<BM, AERIS_ACT_GELU, false, true, false, false, 192>();
+    if (e == hipSuccess) e = configure_one<BM, GEMM_ACT_GELU_ERF, false, true, false, false, 192>();
+    if (e == hipSuccess) e = configure_one<BM, AERIS_ACT_NONE, false, false, true, false, 192>();
+  }
   return e;
 }
 
@@ -949,14 +952,20 @@ void launch_act(const GemmParams& p, dim3 grid, hipStream_t stream) {
 }
 
 template <int BM>
-void launch_192(const GemmParams& p, dim3 grid, hipStream_t stream) {
+hipError_t launch_192(const GemmParams& p, dim3 grid, hipStream_t stream) {
 #define GO(...) hipLaunchKernelGGL((gemm_bf16_nt_persistent_kernel<BM, 192, __VA_ARGS__>), grid, dim3(NT), smem_bytes(BM, 192), stream, p)
-  if (p.c_dtype == AERIS_F32) GO(AERIS_ACT_NONE, true, false, false, true);
-  else if (p.res_dtype >= 0) GO(AERIS_ACT_NONE, false, false, true);
-  else if (p.act == AERIS_ACT_GELU) GO(AERIS_ACT_GELU, false, true);
-  else if (p.act == GEMM_ACT_GELU_ERF) GO(GEMM_ACT_GELU_ERF, false, true);
-  else GO(AERIS_ACT_NONE, false, true);
+  if (p.c_dtype == AERIS_F32) {
+    GO(AERIS_ACT_NONE, true, false, false, true);
+  } else if constexpr (BM == 256) {
+    if (p.res_dtype >= 0) GO(AERIS_ACT_NONE, false, false, true);
+    else if (p.act == AERIS_ACT_GELU) GO(AERIS_ACT_GELU, false, true);
+    else if (p.act == GEMM_ACT_GELU_ERF) GO(GEMM_ACT_GELU_ERF, false, true);
+    else GO(AERIS_ACT_NONE, false, true);
+  } else {
+    return hipErrorInvalidValue;
+  }
 #undef GO
+  return hipSuccess;
 }
 
 template <int BM>
@@ -979,8 +988,10 @@ hipError_t launch_bm(GemmParams p, int bn, hipStream_t stream) {
     p.rpb_magic = (uint32_t)((((uint64_t)1 << p.rpb_shift) + (uint64_t)p.rows_per_batch - 1) / (uint64_t)p.rows_per_batch);
   }
   const dim3 grid(8 * p.bpx);
-  if (bn == 192) launch_192<BM>(p, grid, stream);
-  else if (p.act == AERIS_ACT_SWIGLU) launch_act<BM, AERIS_ACT_SWIGLU>(p, grid, stream);
+  if (bn == 192) {
+    const hipError_t e = launch_192<BM>(p, grid, stream);
+    if (e != hipSuccess) return e;
+  } else if (p.act == AERIS_ACT_SWIGLU) launch_act<BM, AERIS_ACT_SWIGLU>(p, grid, stream);
   else if (p.act == GEMM_ACT_GELU_ERF)
     hipLaunchKernelGGL((gemm_bf16_nt_persistent_kernel<BM, 256, GEMM_ACT_GELU_ERF, false, true>), grid, dim3(NT), smem_bytes(BM, 256), stream, p);
   else if (p.act == AERIS_ACT_GELU) launch_act<BM, AERIS_ACT_GELU>(p, grid, stream);
@@ -1001,7 +1012,8 @@ hipError_t gemm_persistent_launch(const GemmParams& p, int tile_height, int tile
   return tile_height == 128 ? launch_bm<128>(p, tile_width, stream) : launch_bm<256>(p, tile_width, stream);
 }
 
-bool gemm_persistent_takes_192(const GemmParams& p) {
+bool gemm_persistent_takes_192(const GemmParams& p, int tile_height) {
+  if (tile_height != 256 && p.c_dtype != AERIS_F32) return false;
   if (p.act == AERIS_ACT_GELU || p.act == GEMM_ACT_GELU_ERF) return p.c_dtype == AERIS_BF16 && !p.gate && p.res_dtype < 0;
   if (p.act != AERIS_ACT_NONE) return false;
   if (p.c_dtype == AERIS_F32) return p.res_dtype == AERIS_F32 && !p.split;

@@ -55,8 +55,8 @@ class _timed:
 
 
 def gemm_uses_big_tiles(M, N, act=None):
-    """Whether the problem has a chip's worth of 256x256 tiles (csrc/gemm.hip's choice is then the 256x256 kernel for all
-    rows but at most the last partial round's); used to label timings."""
+    """Whether the problem has a chip's worth of 256x256 tiles (csrc/gemm.hip's choice is then the persistent kernel, mostly with such
+    tiles, for all rows but at most the last partial round's); used to label timings."""
     bn = 128 if act == "swiglu" else 256
     return M >= 256 and (N % bn == 0 or N >= 4 * bn) and ((M + 255) // 256) * ((N + bn - 1) // bn) >= 256 and N % 4 == 0
 
@@ -367,7 +367,7 @@ def gemm(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, 
             raise RuntimeError("residual has the wrong size")
     big = gemm_uses_big_tiles(M, N, act) and act != "silu"
     tag = "gemm_small"
-    if big:  # one tag per instantiation of the persistent kernel ("plain": neither gate nor residual in the epilogue;
+    if big:  # one tag per epilogue of the persistent kernel, whatever tiles it takes ("plain": neither gate nor residual in the epilogue;
         # "res": bf16 output with a bf16 residual)
         res_bf16 = residual is not None and residual.dtype == torch.bfloat16 and out.dtype == torch.bfloat16
         tag = (f"gemm_256x256_{act or 'none'}_{'f32' if out.dtype == torch.float32 else 'bf16'}"

@@ -2,6 +2,7 @@
 declares, validates arguments on the host (no GPU touched), and its index-map hooks are bit-exact
 against the oracle.  The module layer keeps the reference's state_dict layout."""
 import ctypes
+import importlib.util
 import os
 import re
 
@@ -24,6 +25,18 @@ def test_library_exports_every_declared_symbol(pkg):
         assert hasattr(lib, name), f"{name} declared in include/aeris_hip.h but not exported"
     assert declared == set(pkg._lib.SIGNATURES), "ctypes signature table and header disagree"
     assert lib.aeris_version() >= 1
+
+
+def test_kernels_named_by_the_benchmark_are_in_the_library(pkg):
+    """Each kernel<arguments> of bench.py's record, in the mangled form of its template arguments (numbers and truth values)."""
+    spec = importlib.util.spec_from_file_location("bench", os.path.join(ROOT, "bench.py"))
+    bench = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(bench)
+    library = open(pkg._lib.LIB_PATH, "rb").read()
+    for name in bench.KERNEL_NAMES.values():
+        kernel, args = re.match(r"(\w+)<([^>]*)>", name).groups()
+        code = "".join({"true": "Lb1E", "false": "Lb0E"}.get(a, f"Li{a}E") for a in args.split(", "))
+        assert f"{kernel}I{code}E".encode() in library, name
 
 
 CASES = [(1, 4, 8, 2, 4, 0, 0), (1, 4, 8, 2, 4, 1, 2), (2, 6, 6, 3, 2, 1, 1), (1, 32, 64, 8, 8, 4, 4),

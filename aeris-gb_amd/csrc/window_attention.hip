@@ -471,6 +471,7 @@ window_attention_persist_kernel(AttnParams p, int n_units) {
   const int u_begin = blockIdx.x;
   if (u_begin >= n_units) return;
 
+  // (as rows of a [tokens, 3 inner] matrix a part's slice of a head begins further in: its last row ends where the matrix does)
   const uint32_t plane_bytes = (uint32_t)p.B * (uint32_t)(H * W) * ld_qkv * 2u;  // < 2^32, checked by the caller
   const int rsub = lane >> 3, pc = lane & 7;
 
@@ -918,11 +919,18 @@ static int persist_rotation(const AttnParams& p) {
 // arithmetic is the same either way, and the start-up weigh too much.  Blocks of 32 -> 16, us: 180 x 360, 8 heads 64.3 -> 59.5, shifted with
 // mask 65.7 -> 63.4, two heads 20.0 -> 19.9, with mask 21.3 -> 22.3; without a table 8 heads 55.9 -> 54.7, with mask 57.8 -> 55.4, three heads with
 // mask 25.6 -> 26.1; 96 x 192, 6 heads without a table 14.4 -> 14.5; 24 x 1200, 8 heads, mask (half of the windows on the border) 31.0 -> 31.7.
+// Blocks of 16 take the sums in another order than blocks of 32, so the answer follows the shape alone: q, k, v as rows of a [tokens, 3 inner]
+// matrix go the same way as head planes and give the same bits (180 x 360, 8 heads as rows: 90.9 us before, 58.4 now), and
+// both keep to blocks of 32 where offsets in such rows take more than 32 bits
+// (720 x 1440, 16 heads: 1889 us, in blocks of 16 1685).  (With the unit count a result changes in its rounding: a member alone against the same
+// one in a batch by 1.3e-5 of its 2-norm.)
 static bool persist_in_16s(const AttnParams& p, bool has_bias, int64_t units) {
   if (has_bias && !wrapped_border(p)) return true;
   const int64_t all = (int64_t)p.nWy * p.nWx, inner = (int64_t)(p.nWy - (p.sy > 0)) * (p.nWx - (p.sx > 0));
   return units >= 6 * (int64_t)g_attn_cus && (!wrapped_border(p) || 4 * inner >= 3 * all);
 }
+
+constexpr int64_t OFFSETS_32 = 0xFFFFFFF0u;  // bytes that the offsets of loads into LDS reach
 
 template <int WS_Y, int WS_X, bool HAS_BIAS, bool S16, bool ROTATES>
 static hipError_t launch_persist(const AttnParams& p, int64_t units, hipStream_t stream) {
@@ -936,9 +944,19 @@ template <int WS_Y, int WS_X, int HD, bool HAS_BIAS>
 static hipError_t launch_attn(const AttnParams& p, hipStream_t stream) {
   using Cfg = AttnCfg<WS_Y, WS_X, HD, HAS_BIAS>;
   const int64_t grid = (int64_t)p.B * p.nWy * p.nWx * p.heads;
+  const int64_t tokens = (int64_t)p.B * p.H * p.W, cus = g_attn_cus;
+  // Enough units for every CU to stream a few: the persistent form.  12x12 windows from two and a half per CU on (one workgroup per unit ->
+  // persistent, us: 512 units 12.2 -> 12.6, with mask 13.3 -> 14.5; 640 16.5 -> 16.7, with mask 17.9 -> 18.6; 768 19.3 -> 17.3, with mask
+  // 20.5 -> 19.3), without a table and mask from two on (512 10.0 -> 10.5, 640 13.9 -> 13.5).
+  const bool persist = WS_X == 12 ? 2 * grid > ((HAS_BIAS || wrapped_border(p)) ? 5 : 4) * cus : grid >= 2 * cus;
+  AttnParams q = p;
+  if constexpr (HD == 64) q.rotate = persist_rotation(p);
+  if constexpr (HD == 64 && WS_Y * WS_X % 32 != 0) {
+    if (persist && tokens * 3 * p.heads * HD * 2 < OFFSETS_32 && persist_in_16s(p, HAS_BIAS, grid))
+      return q.rotate ? launch_persist<WS_Y, WS_X, HAS_BIAS, true, true>(q, grid, stream) : launch_persist<WS_Y, WS_X, HAS_BIAS, true, false>(q, grid, stream);
+  }
   // head_dim 64 with every offset inside a q / k / v plane below 2^32 bytes: K and V straight into LDS
-  if (HD == 64 && p.head_stride >= (int64_t)p.B * p.H * p.W * p.tok_stride &&
-      (int64_t)p.B * p.H * p.W * p.tok_stride * 2 < (int64_t)0xFFFFFFF0u) {
+  if (HD == 64 && p.head_stride >= tokens * p.tok_stride && tokens * p.tok_stride * 2 < OFFSETS_32) {
     if constexpr (WS_X < 16) {
       constexpr int PER_CU = 6;
       if (WS_X == 8 ? walk_8x8(p, HAS_BIAS) : grid <= g_attn_cus) {
@@ -949,18 +967,8 @@ static hipError_t launch_attn(const AttnParams& p, hipStream_t stream) {
         return hipGetLastError();
       }
     }
-    // Enough units for every CU to stream a few: the persistent form.  12x12 windows from two and a half per CU on (one workgroup per unit ->
-    // persistent, us: 512 units 12.2 -> 12.6, with mask 13.3 -> 14.5; 640 16.5 -> 16.7, with mask 17.9 -> 18.6; 768 19.3 -> 17.3, with mask
-    // 20.5 -> 19.3), without a table and mask from two on (512 10.0 -> 10.5, 640 13.9 -> 13.5).
-    const int64_t cus = g_attn_cus;
-    if (WS_X == 12 ? 2 * grid > ((HAS_BIAS || wrapped_border(p)) ? 5 : 4) * cus : grid >= 2 * cus) {
-      AttnParams q = p;
-      q.rotate = persist_rotation(p);
+    if (persist) {
       if constexpr (WS_X == 8) return launch_persist<WS_Y, WS_X, HAS_BIAS, false, false>(q, grid, stream);
-      if constexpr (WS_Y * WS_X % 32 != 0) {
-        if (persist_in_16s(p, HAS_BIAS, grid))
-          return q.rotate ? launch_persist<WS_Y, WS_X, HAS_BIAS, true, true>(q, grid, stream) : launch_persist<WS_Y, WS_X, HAS_BIAS, true, false>(q, grid, stream);
-      }
       if constexpr (WS_X > 8)
         return q.rotate ? launch_persist<WS_Y, WS_X, HAS_BIAS, false, true>(q, grid, stream) : launch_persist<WS_Y, WS_X, HAS_BIAS, false, false>(q, grid, stream);
     }

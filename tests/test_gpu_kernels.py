@@ -464,6 +464,24 @@ def test_window_attention_persistent_forms(pkg, cuda, case, prescaled):
     test_window_attention_planes_parity(pkg, cuda, case, prescaled)
 
 
+def test_window_attention_12x12_alone_and_in_a_batch(pkg, cuda):
+    """600 units of one member have a workgroup each and blocks of 32, 1800 of three the persistent form and blocks of 16: another
+    order of the same sums, so a member alone and in a batch agree to the rounding of the results (at most 2^-7 / sqrt(12) of the
+    2-norm for either side).  Equal members of one batch have equal results."""
+    B, H, W, heads, hd, ws, sh = 3, 96, 180, 5, 64, 12, 6
+    g = torch.Generator().manual_seed(2)
+    one = bf(torch.randn(3 * heads, H * W, hd, generator=g)).to(cuda)
+    table = bf(0.7 * torch.randn((2 * ws - 1) ** 2, heads, generator=g)).to(cuda)
+
+    def run(qkv, b):
+        return pkg.ops.window_attention(qkv, b, (H, W), heads, hd, (ws, ws), (sh, sh), table, True, head_planes=True).view(b, H * W, -1)
+    alone, batch = run(one, 1), run(one.repeat(1, B, 1), B)
+    assert torch.equal(batch[0], batch[1]) and torch.equal(batch[0], batch[2])
+    err = rel_l2(batch[0], alone[0])
+    print(f"12x12 attention, a member in a batch against alone: rel-L2 {err:.3e}")
+    assert err <= math.sqrt(2.0) * 2.3e-3, err
+
+
 STREAM_CASES = [
     # B, H, W, heads, head_dim, ws_y, ws_x, shift_y, shift_x  -- shapes only the streaming kernel takes
     (1, 120, 120, 2, 128, 60, 60, 30, 30),   # the reference's window: 3600 tokens, head_dim 128 (model.py:22-27), shifted
@@ -628,6 +646,10 @@ HEAD_PLANE_CASES = [
     (1, 160, 160, 24, 64, 16, 16, 8, True, True),   # the 256x256 GEMM tiles write the planes
     (1, 120, 120, 2, 128, 60, 60, 30, False, False),
     (2, 40, 60, 3, 64, 20, 20, 10, False, False),
+    (1, 132, 204, 9, 64, 12, 12, 6, True, True),    # 12x12 windows in blocks of 16
+    (1, 120, 192, 5, 64, 12, 12, 0, True, False),
+    (1, 120, 192, 5, 64, 12, 12, 6, True, True),    # ... in blocks of 32: the mask, few units
+    (1, 420, 420, 64, 64, 12, 12, 6, True, True),   # ... and offsets in the rows that take more than 32 bits
 ]
 
 

@@ -437,9 +437,10 @@ namespace {
 //     8192, 1024, 1024      29.2 (32)      26.0 (22)     34.5 (41)    256 tiles of 128 rows: one round
 //     8192, 1536, 1536      43.7 (42)      50.1 (53)     64.6 (79)    192 tiles of 256 rows: one round
 //    14400, 1536, 6144     259  (269)     264  (264)    497  (570)    342 tiles of 256 rows: two rounds
-// (Over 487 shapes, M 1024 .. 51 840, N and K 192 .. 4096, every epilogue, all forms and the 128 x 128 tiles of the tile kernel
-// timed: the choice takes 0.2 % longer than the fastest form on average, 24 % at most, where the small tiles are kept one
-// size too long, 24 576 x 192 x 192: 10.8 us against 8.7.)
+// (Over 740 shapes, M 1024 .. 54 000, N 192 .. 6144, K 192 .. 6144, every epilogue, all forms timed: the choice takes 1.0 % longer than the
+// fastest form on average, more than 5 % at 56 of them, 22 % at most: 2500 x 2048 x 256 with bf16 residual 11.9 us in small tiles, 9.8 in
+// tiles of 128 rows; GELU the other way, 4096 x 1152 x 1024 20.8 against 18.2 in small tiles, whose estimate is from before they had 32 rows
+// or two stages.)
 //
 // Tiles of 192 columns take 0.85-0.95 of the time of those of 256 for three quarters of the work, so they pay only where they need
 // no more rounds: N just over a multiple of 256, or a last round that is mostly empty.  256 -> 192 columns of the same height, us:
@@ -600,8 +601,8 @@ hipError_t gemm_launch(const void* A, const void* W, void* C, const void* bias, 
   float one = 0.f;
   const Kind kind = best_kind(s, &one);
   // Whole rounds of 256-row tiles first, the rows of the last, partly filled round by smaller tiles in a launch of its own:
-  // the rows are split, nothing else.  (14400 x 4608 x 1536: 1026 tiles, two more than four rounds of 256: 177 -> 162 us;
-  // 14400 x 1536 x 6144: 342 tiles: 268 -> 256 us.)
+  // the rows are split, nothing else.  (14400 x 4608 x 1536: 1026 tiles, two more than four rounds of 256: 164 -> 147 us;
+  // 14400 x 1536 x 6144: 342 tiles: 264 -> 239 us.)
   const int bn_out = act == AERIS_ACT_SWIGLU ? 128 : 256;
   const int64_t tiles_n = (N + bn_out - 1) / bn_out, tiles = tiles_of(s, 256, 256);
   const int64_t panels = (tiles - 1) / 256 * 256 / tiles_n;  // row panels of the rounds before the last
@@ -611,11 +612,12 @@ hipError_t gemm_launch(const void* A, const void* W, void* C, const void* bias, 
     rest.M = M - head.M;
     float t_rest = 0.f;
     const Kind rest_kind = best_kind(rest, &t_rest);
-    // Against one launch of 192-column tiles the sum of two estimates is too low, by 6 us at K = 1536 and 14 to 24 at K = 6144, while the
-    // one launch, whose CUs are never all busy to the end, takes 0.87 to 0.98 of its own.  f32 C and residual, N = 1536, us, one launch of
-    // 192 / two: K = 1536, M = 12544 65.7 / 70.2, 13312 67.1 / 74.1, 14400 70.7 / 78.2, 14848 71.4 / 78.5; K = 6144, M = 12544 233.7 /
-    // 226.1, 13312 232.8 / 233.5, 14400 244.6 / 239.4, 14848 247.7 / 239.1.  bf16, plain: 8192 x 2304 x 1024 38.4 / 39.7, 14400 x 1536 x
-    // 3072 100.6 / 109.0.
+    // Against one launch of 192-column tiles the sum of two estimates is too low, by 6 to 11 us at K = 1536 and 14 to 24 at K = 6144, while
+    // the one launch, whose CUs are never all busy to the end, takes 0.87 to 0.99 of its own.  With 3 us and 0.88 the choice takes 0.2 %
+    // longer than the faster of the two over 255 shapes, 7 % at most (with 0.90 of the plain sum 1.9 and 14).  f32 C and residual, N = 1536,
+    // us, one launch of 192 / two: K = 1536, M = 12544 65.7 / 70.2, 13312 67.1 / 74.1, 14400 70.7 / 78.2, 14848 71.4 / 78.5; K = 6144, M =
+    // 12544 233.7 / 226.1, 13312 232.8 / 233.5, 14400 244.6 / 239.4, 14848 247.7 / 239.1.  bf16, plain: 8192 x 2304 x 1024 38.4 / 39.7,
+    // 14400 x 1536 x 3072 100.6 / 109.0.
     const float two = estimate_us(PERSISTENT256, head) + t_rest;
     if (kind == PERSISTENT256_192 ? two + 3.0f < 0.88f * one : two < 0.97f * one) {
       const hipError_t e = launch_kind(PERSISTENT256, rows_of(p, 0, head.M), stream);

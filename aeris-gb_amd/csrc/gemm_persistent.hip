@@ -18,8 +18,8 @@
 //     8192 x 1024 x 1024 with f32 residual 29.8 -> 26 us, 12480 x 384 x 1088 27.8 -> 22 us; per FLOP they are 30 % slower
 //   - tiles of 192 columns (waves four by two, 64 or 32 rows x 96 columns each: 10 fragment reads for 24 MFMAs where two by four
 //     would need 11) where N or the last round leaves tiles of 256 partly empty: 8192 x 1536 x 6144 with f32 residual is 192 tiles on
-//     256 CUs, 126 -> 119 us as 256 of them; 12480 x 384 x 384 14.6 -> 12.4.  A tile takes 0.85 of a full one's time, which the choice of
-//     form (gemm.hip) weighs
+//     256 CUs, 117 -> 115 us as 256 of them; 14400 x 1536 x 1536 82.0 -> 70.7.  A tile takes 0.85-0.95 of a full one's time; the choice of
+//     form (gemm.hip) weighs 0.88 (128 rows), 0.93 (f32 C) and 0.95.  128 rows: f32 C with an f32 residual alone
 //   - tiles are ordered so that the workgroups resident on one XCD (blockIdx % 8) cover a contiguous chunk, 4 row
 //     panels x all column tiles at a time: few distinct A / W k-slices per step compete for that XCD's 4 MB L2
 //   - the epilogue stages through the idle A stage (wave-private 4 KB): fragments (4 consecutive n per lane) are
